@@ -333,6 +333,52 @@ def test_delta_rule_in_chunks(K, G, H, d, dv):
     assert bool((state[[1, 4, 5]] == 3.0).all())
 
 
+def _delta_run(K, lens, G, H, d, dv, max_q, seed, ctx=0, edit=None, tail=()):
+    """The kernel's read-outs and states for sequences of these lengths and the plain recurrence in 64 bits for the same inputs
+    (`edit` changes them first), all on the GPU. States start from random ones where ctx > 0."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    r = lambda *shape: torch.randn(*shape, device="cuda", generator=g)
+    B, T = len(lens), sum(lens)
+    unit = lambda x: torch.nn.functional.normalize(x, dim=-1).reshape(T, -1)
+    y = torch.cat([unit(r(T, G, d)) * d ** -0.5, unit(r(T, G, d)), r(T, H * dv)], dim=1)
+    z, A_log, dtb, S0 = r(T, 2 * H), r(H) * 0.5, r(H) * 0.5, r(B, H, d, dv) * 0.3
+    if edit:
+        edit(y, z, A_log, dtb)
+    qs, cx, sl = ragged(lens, [ctx] * B, list(range(B)))
+    state, o = S0.clone(), torch.full((T, H * dv), 9.0, device="cuda")
+    K.delta_rule(o, y, z, state, A_log, dtb, qs, cx, sl, G, H, d, dv, 0, H, max_q, *tail)
+    beta, decay = torch.sigmoid(z[:, :H].double()), torch.exp(-torch.exp(A_log.double()) * torch.nn.functional.softplus(z[:, H:].double() + dtb.double()))
+    heads = lambda x: x.reshape(T, G, d).double().repeat_interleave(H // G, 1)
+    q, k, v = heads(y[:, :G * d]), heads(y[:, G * d:2 * G * d]), y[:, 2 * G * d:].reshape(T, H, dv).double()
+    ref, S_ref, t = torch.zeros(T, H, dv, device="cuda", dtype=torch.float64), [], 0
+    for b, n in enumerate(lens):
+        S = S0[b].double() if ctx else torch.zeros(H, d, dv, device="cuda", dtype=torch.float64)
+        for t in range(t, t + n):
+            S = S * decay[t][:, None, None]
+            S = S + k[t][:, :, None] * (beta[t][:, None] * (v[t] - (k[t][:, :, None] * S).sum(1)))[:, None]
+            ref[t] = (q[t][:, :, None] * S).sum(1)
+        t += n > 0
+        S_ref.append(S)
+    return o.reshape(T, H, dv), state, ref, torch.stack(S_ref)
+
+
+def rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+@gpu
+@pytest.mark.parametrize("n,G,H,d,dv", [(64, 4, 16, 128, 128), (300, 2, 8, 128, 64), (700, 4, 8, 64, 64)])
+def test_delta_rule_in_chunks_is_no_less_exact(K, n, G, H, d, dv):
+    """Against 64 bits, portions in chunks have no more error than the same portions token by token (which `max_q` 2 asks for), in the
+    read-outs and in the states they leave. Measured: 0.73 to 0.77 and 0.96 to 0.98 of it (with one 32-bit chain throughout: 1.04 to
+    1.12 and 1.09 to 1.13)."""
+    def error(max_q):
+        runs = [_delta_run(K, [n] * 3, G, H, d, dv, max_q, seed) for seed in range(4)]
+        return [rel(torch.cat([r[i] for r in runs]), torch.cat([r[i + 2] for r in runs])) for i in (0, 1)]
+    chunks, tokens = error(n), error(2)
+    assert chunks[0] <= 0.9 * tokens[0] and chunks[1] <= tokens[1], (chunks, tokens)
+
+
 @gpu
 def test_unit_heads_and_gated_headnorm(K):
     T, heads, d = 6, 5, 13
