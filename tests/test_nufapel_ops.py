@@ -442,3 +442,51 @@ def test_recurrences_one_token(rule, H, d, dv):
         assert float((a - b).abs().max()) <= 4 * d * 2.0 ** -24 * 8 * max(1.0, float(b.abs().max())), what
     idle = [1, 4, 5, 6]
     assert torch.equal(got[0][1][idle], state[idle]), "states of idle slots"
+
+
+@gpu
+@pytest.mark.parametrize("rule,H,d,dv", [(0, 4, 64, 64), (0, 8, 128, 128), (1, 8, 128, 128), (1, 4, 64, 64), (1, 4, 256, 256), (1, 4, 33, 20), (2, 16, 128, 128)])
+def test_recurrences_one_token_are_no_less_exact(rule, H, d, dv):
+    """Against 64 bits, a step of one token a sequence has no more error than the kernels for any number of tokens (which `max_q` 3 asks
+    for), in the read-outs and in the states.  Measured: read-outs 0.6 to 0.9 of it, states 0.8 (matrix memory) and 1.000 (the others,
+    whose only rounding of a state is the same).  One 32-bit chain of all a thread's rows: up to 1.6 and 1.8 of it."""
+    from distributed_llm_inference_amd import ops
+    K = ops.load()
+    g = torch.Generator(device="cuda").manual_seed(6)
+    r = lambda *shape: torch.randn(*shape, device="cuda", generator=g)
+    B, n, ints = 64, H * d, lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    q0, ctx, sl, NC = ints(range(B + 1)), ints([3] * B), ints(range(B)), dv + (rule == 1)
+    S0, z, wz = r(B, H, d, NC) * 0.3, r(B, 3 * n + H * dv + 2 * H), r(B, n)
+    D = lambda x, k=d: x.double().reshape(B, H, k)
+    if rule == 0:
+        ba, w0 = r(n) * 0.5, r(n) * 0.5
+        call = lambda o, st, q: K.state_scan(0, o, z, wz, st, None, ba, w0, q0, ctx, sl, H, d, d, 0, n, 2 * n, 3 * n, 0, 0, 1.0, 1.0, q, False)
+        q, k, v, a = D(z[:, :n]), D(z[:, n:2 * n]), D(z[:, 2 * n:3 * n]), torch.sigmoid(D(z[:, 3 * n:4 * n]) + ba.double().view(H, d))
+        w = torch.exp(-math.exp(-0.5) * torch.sigmoid(D(wz) + w0.double().view(H, d)))
+        u = k / torch.sqrt((k * k).sum(-1, keepdim=True) + 1e-6)
+        S = w[..., None] * S0.double() - (a * u)[..., None] * (u[..., None] * S0.double()).sum(2)[:, :, None] + k[..., None] * v[:, :, None]
+    elif rule == 1:
+        c, b, m0 = 2 * n + H * dv, torch.cat([r(H), r(H) + 3]), r(B, H).abs()
+        call = lambda o, st, q: K.state_scan(1, o, z, None, st, m0[..., None].expand(B, H, 128).contiguous(), b, None, q0, ctx, sl, H, d, dv, 0, n, 2 * n,
+                                             0, c, c + H, 15.0, d ** -0.5, q, False)
+        q, k, v = D(z[:, :n]) * d ** -0.5, D(z[:, n:2 * n]), torch.cat([D(z[:, 2 * n:c], dv), torch.ones(B, H, 1, device="cuda").double()], -1)
+        li = 15 * torch.tanh((z[:, c:c + H] + b[:H].double()) / 15)
+        lf = torch.nn.functional.logsigmoid(15 * torch.tanh((z[:, c + H:c + 2 * H] + b[H:].double()) / 15)) + m0
+        m = torch.maximum(lf, li)
+        S = torch.exp(lf - m)[..., None, None] * S0.double() + torch.exp(li - m)[..., None, None] * k[..., None] * v[:, :, None]
+    else:
+        A, dt = r(H) * 0.5, r(H) * 0.5
+        y = torch.cat([torch.nn.functional.normalize(z[:, :2 * n].reshape(B, 2 * H, d), dim=-1).reshape(B, -1), z[:, 2 * n:2 * n + H * dv]], 1)
+        call = lambda o, st, q: K.delta_rule(o, y, z, st, A, dt, q0, ctx, sl, H, H, d, dv, 0, H, q)
+        q, k, v = D(y[:, :n]), D(y[:, n:2 * n]), D(y[:, 2 * n:], dv)
+        S = S0.double() * torch.exp(-torch.exp(A.double()) * torch.nn.functional.softplus(z[:, H:2 * H].double() + dt.double()))[..., None, None]
+        S = S + k[..., None] * (torch.sigmoid(z[:, :H].double())[..., None] * (v - (k[..., None] * S).sum(2)))[:, :, None]
+    ref = (q[..., None] * S).sum(2)
+
+    def error(max_q):
+        st, o = S0.clone(), torch.zeros(B, H * (dv + 2 * (rule == 1)), device="cuda")
+        call(o, st, max_q)
+        rel = lambda a, b: float((a.double() - b).norm() / b.norm())
+        return rel(o.view(B, H, -1)[..., :NC], ref), rel(st, S)
+    one, many = error(1), error(3)
+    assert one[0] <= 0.95 * many[0] and one[1] <= 1.002 * many[1], (one, many)
