@@ -887,7 +887,7 @@ void delta_rule(Tensor o, const Tensor& y, const Tensor& z, Tensor state, const 
   DLIA_CHECK(z.size(0) >= T && col_beta + Hv <= z.size(1) && col_a + Hv <= z.size(1) && col_beta >= 0 && col_a >= 0, "delta_rule: gate columns");
   DLIA_CHECK(state.dim() == 4 && state.size(1) == Hv && state.size(2) == d && state.size(3) == dv, "delta_rule: state [slots, Hv, d, dv]");
   DLIA_CHECK(A_log.numel() == Hv && dt_bias.numel() == Hv && q_start.numel() >= B + 1 && slots.numel() >= B, "delta_rule: per-head / per-sequence vectors");
-  if (max_q <= 1 && B > 0 && dlia_scan_decode(2, o.data_ptr<float>(), o.stride(0), y.data_ptr<float>(), C, z.data_ptr<float>(), z.stride(0), nullptr, 0,
+  if (max_q <= 1 && dlia_scan_decode(2, o.data_ptr<float>(), o.stride(0), y.data_ptr<float>(), C, z.data_ptr<float>(), z.stride(0), nullptr, 0,
                                      state.data_ptr<float>(), nullptr, A_log.data_ptr<float>(), dt_bias.data_ptr<float>(), q_start.data_ptr<int>(),
                                      ctx.data_ptr<int>(), slots.data_ptr<int>(), (int)B, (int)Hv, (int)(Hv / G), (int)d, (int)dv, (int)state.size(0),
                                      0, (int)(G * d), (int)(2 * G * d), (int)col_a, (int)col_beta, 0.f, 1.f, cur_stream()) == 0)

@@ -165,6 +165,11 @@ void biased_attention(Tensor out, const Tensor& qkv, const Tensor& kcache, const
 
 int64_t state_scan_blocks(int64_t d, int64_t ncols) { return dlia_state_scan_blocks((int)d, (int)ncols); }
 
+// the kernel that a step of single tokens takes, by its sizes: 1 scan_decode.hip, 0 the general one
+int64_t scan_route(int64_t rule, int64_t B, int64_t H, int64_t d, int64_t dv) {
+  return dlia_scan_decode_takes((int)rule, (long)B, (int)H, (int)d, (int)dv);
+}
+
 void state_scan(int64_t rule, Tensor o, const Tensor& z, OptTensor wz, Tensor state, const std::optional<Tensor>& mstate,
                 const Tensor& b0, OptTensor b1, const Tensor& q_start, const Tensor& ctx, const Tensor& slots, int64_t H, int64_t d,
                 int64_t dv, int64_t col_q, int64_t col_k, int64_t col_v, int64_t col_a, int64_t col_i, int64_t col_f, double cap,
@@ -195,7 +200,7 @@ void state_scan(int64_t rule, Tensor o, const Tensor& z, OptTensor wz, Tensor st
     DLIA_CHECK(mstate->dim() == 3 && mstate->size(0) == state.size(0) && mstate->size(1) == H && mstate->size(2) == 128, "state_scan: mstate [slots, H, 128]");
     mp = mstate->data_ptr<float>();
   }
-  if (max_q <= 1 && B > 0 &&
+  if (max_q <= 1 &&
       dlia_scan_decode((int)rule, o.data_ptr<float>(), o.stride(0), z.data_ptr<float>(), z.stride(0), z.data_ptr<float>(), z.stride(0), wzp, ldw,
                        state.data_ptr<float>(), const_cast<float*>(mp), b0.data_ptr<float>(), b1.has_value() ? b1->data_ptr<float>() : nullptr,
                        q_start.data_ptr<int>(), ctx.data_ptr<int>(), slots.data_ptr<int>(), (int)B, (int)H, 1, (int)d, (int)dv, (int)state.size(0),
@@ -344,6 +349,7 @@ TORCH_LIBRARY_FRAGMENT(dlia, m) {
   m.def("softcap(Tensor(a!) logits, int vocab, float cap) -> ()");
   m.def("biased_attention(Tensor(a!) out, Tensor qkv, Tensor kcache, Tensor vcache, Tensor tok_pos, Tensor tok_seq, Tensor block_table, int H, int G, int d, int dv, float scale, Tensor? temp, Tensor? bias, Tensor? sink, Tensor? gate) -> ()");
   m.def("state_scan_blocks(int d, int ncols) -> int");
+  m.def("scan_route(int rule, int B, int H, int d, int dv) -> int");
   m.def("state_scan(int rule, Tensor(a!) o, Tensor z, Tensor? wz, Tensor(b!) state, Tensor(c!)? mstate, Tensor b0, Tensor? b1, Tensor q_start, Tensor ctx, Tensor slots, int H, int d, int dv, int col_q, int col_k, int col_v, int col_a, int col_i, int col_f, float cap, float qscale, int max_q, bool quick) -> ()");
   m.def("moe_route(Tensor(a!) sel, Tensor(b!) wts, Tensor logits, int top, int groups, int keep, float scale, Tensor? correction=None, bool softmax=False, int group_rank=2, bool renorm=True) -> ()");
   m.def("moe_plan(Tensor(a!) tiles, Tensor(b!) row_tok, Tensor(c!) pair_row, Tensor sel, int pairs, int top, int E, int tile_rows, Tensor? wts=None, Tensor(d!)? row_w=None) -> ()");
@@ -371,4 +377,5 @@ TORCH_LIBRARY_IMPL(dlia, CUDA, m) {
 
 TORCH_LIBRARY_IMPL(dlia, CompositeExplicitAutograd, m) {
   m.impl("state_scan_blocks", &state_scan_blocks);
+  m.impl("scan_route", &scan_route);
 }

@@ -156,6 +156,7 @@ void dlia_delta_chunks(float* o, const float* y, const float* z, float* state, c
 void dlia_memory_chunks(float* o, long ldo, const float* z, long ldz, float* state, float* mstate, const float* b0, const int* q_start,
                         const int* ctx, const int* slots, float* ws, int B, int H, int d, int dv, int state_rows, int col_q, int col_k,
                         int col_v, int col_i, int col_f, float cap, float qscale, int max_q, hipStream_t stream);
+int dlia_scan_decode_takes(int rule, long B, int H, int d, int dv);
 // scan_decode.hip: one token per sequence through the recurrences (rule 0, 1 as in state_scan, 2 the delta rule); 1: not taken
 int dlia_scan_decode(int rule, float* o, long ldo, const float* x, long ldx, const float* z, long ldz, const float* wz, long ldw, float* state,
                      float* mstate, const float* b0, const float* b1, const int* q_start, const int* ctx, const int* slots, int B, int H, int per,

@@ -179,6 +179,15 @@ __global__ __launch_bounds__(1024) void memory_decode_kernel(DecScanArgs p) {
 
 using dlia::DecScanArgs;
 
+// The sizes that take the step kernels. The memory's workgroup owns a (head, sequence) whole, so few of them on wide states leave most of the
+// chip without work: 8 heads of 128 x 257, 4 / 6 / 8 sequences 11.2 / 11.6 / 11.9 us against 10.2 / 11.9 / 12.7 of the general kernel's column
+// blocks, 2 of 512 x 257, 8 / 24 sequences 28 / 37 against 22 / 64 (64 x 257: 7.7 against 9.9 from one sequence on).
+extern "C" int dlia_scan_decode_takes(int rule, long B, int H, int d, int dv) {
+  if (B <= 0 || B > 65535) return 0;
+  if (rule == 1) return d <= 512 && dv <= 256 && (dv <= 128 || d <= 64 || B * H >= 48);
+  return d == dv && (d == 128 || (rule == 0 && d == 64));
+}
+
 // Steps of single tokens. 0: launched; 1: sizes or layout that the general kernels take.
 extern "C" int dlia_scan_decode(int rule, float* o, long ldo, const float* x, long ldx, const float* z, long ldz, const float* wz, long ldw,
                                 float* state, float* mstate, const float* b0, const float* b1, const int* q_start, const int* ctx,
@@ -186,10 +195,9 @@ extern "C" int dlia_scan_decode(int rule, float* o, long ldo, const float* x, lo
                                 int col_b, float cap, float qscale, hipStream_t stream) {
   const DecScanArgs p{o, ldo, x, ldx, z, ldz, wz, ldw, state, mstate, b0, b1, q_start, ctx, slots, H, per, d, dv, state_rows, col_q, col_k, col_v,
                       col_a, col_b, cap, qscale};
-  if (B > 65535) return 1;
+  if (!dlia_scan_decode_takes(rule, B, H, d, dv)) return 1;
   auto al = [](const void* q) { return (uintptr_t)q % 16 == 0; };
   if (rule == 1) {
-    if (d > 512 || dv > 256) return 1;
     // Row groups: every row in flight with up to 1024 threads while the chip has fewer workgroups than two a CU, batches of rows with
     // 256 from there on, a thread per row at least. 16 heads of 128 x 129, 4 / 16 / 64 / 160 sequences: 9.1 / 12.0 / 45.8 / 103 us with
     // 1024 threads, 12.3 / 15.9 / 38.3 / 88 with 256.
@@ -200,10 +208,9 @@ extern "C" int dlia_scan_decode(int rule, float* o, long ldo, const float* x, lo
     hipLaunchKernelGGL(dlia::memory_decode_kernel, dim3(H, B), dim3(CT * (rg < 2 ? 2 : rg)), 0, stream, p);
     return 0;
   }
-  if (d != dv || ldx % 4 || ldo % 4 || col_v % 4 || !al(x) || !al(o) || !al(state)) return 1;
-  if (rule == 0 && d == 128) hipLaunchKernelGGL((dlia::scan_decode_kernel<0, 128>), dim3(H, B), dim3(256), 0, stream, p);
-  else if (rule == 0 && d == 64) hipLaunchKernelGGL((dlia::scan_decode_kernel<0, 64>), dim3(H, B), dim3(256), 0, stream, p);
-  else if (rule == 2 && d == 128) hipLaunchKernelGGL((dlia::scan_decode_kernel<2, 128>), dim3(H, B), dim3(256), 0, stream, p);
-  else return 1;
+  if (ldx % 4 || ldo % 4 || col_v % 4 || !al(x) || !al(o) || !al(state)) return 1;
+  if (rule == 2) hipLaunchKernelGGL((dlia::scan_decode_kernel<2, 128>), dim3(H, B), dim3(256), 0, stream, p);
+  else if (d == 128) hipLaunchKernelGGL((dlia::scan_decode_kernel<0, 128>), dim3(H, B), dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL((dlia::scan_decode_kernel<0, 64>), dim3(H, B), dim3(256), 0, stream, p);
   return 0;
 }

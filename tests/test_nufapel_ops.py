@@ -444,6 +444,15 @@ def test_recurrences_one_token(rule, H, d, dv):
     assert torch.equal(got[0][1][idle], state[idle]), "states of idle slots"
 
 
+@pytest.mark.parametrize("rule,B,H,d,dv,step", [
+    (1, 4, 8, 128, 256, 0), (1, 6, 8, 128, 256, 1), (1, 4, 4, 256, 256, 0), (1, 12, 4, 256, 256, 1), (1, 8, 2, 512, 256, 0), (1, 24, 2, 512, 256, 1),
+    (1, 1, 2, 64, 256, 1), (1, 1, 16, 128, 128, 1), (1, 1, 4, 512, 64, 1), (1, 60, 4, 513, 64, 0), (1, 60, 4, 64, 257, 0), (1, 65536, 1, 64, 64, 0), (0, 1, 4, 64, 64, 1),
+    (0, 1, 4, 128, 128, 1), (0, 1, 4, 32, 32, 0), (2, 1, 16, 128, 128, 1), (2, 256, 4, 64, 64, 0), (2, 64, 8, 64, 128, 0), (2, 64, 8, 128, 64, 0)])
+def test_one_token_steps_take_the_kernel_that_measured_faster(rule, B, H, d, dv, step):
+    from distributed_llm_inference_amd import ops
+    assert ops.load(build_if_missing=True).scan_route(rule, B, H, d, dv) == step
+
+
 @gpu
 @pytest.mark.parametrize("rule,H,d,dv", [(0, 4, 64, 64), (0, 8, 128, 128), (1, 8, 128, 128), (1, 4, 64, 64), (1, 4, 256, 256), (1, 4, 33, 20), (2, 16, 128, 128)])
 def test_recurrences_one_token_are_no_less_exact(rule, H, d, dv):
