@@ -380,6 +380,15 @@ def test_delta_rule_in_chunks_is_no_less_exact(K, n, G, H, d, dv):
 
 
 @gpu
+def test_delta_rule_in_chunks_longer_than_announced(K):
+    """A portion longer than `max_q` says runs all of its tokens, in chunks as token by token."""
+    for lens, max_q in [([200, 3, 64], 64), ([1, 49, 100], 50)]:
+        o, state, ref, S = _delta_run(K, lens, 1, 2, 64, 32, max_q, 7, ctx=4)
+        close(o, ref, 2e-5)
+        close(state, S, 2e-5)
+
+
+@gpu
 def test_unit_heads_and_gated_headnorm(K):
     T, heads, d = 6, 5, 13
     x = rnd(T, heads * d + 3, seed=1)
