@@ -380,6 +380,19 @@ def test_delta_rule_in_chunks_is_no_less_exact(K, n, G, H, d, dv):
 
 
 @gpu
+@pytest.mark.parametrize("log_a", [5.0, 60.0, 100.0])
+def test_delta_rule_in_chunks_forgets_all(K, log_a):
+    """Decays of exactly zero between tokens that keep e^-1 of the state (for the largest `log_a`: all of them, exp(A_log) being infinite)."""
+    def edit(y, z, A_log, dtb):
+        A_log[0], dtb[0] = log_a, 0.0
+        z[:, 2] = -min(log_a, 60.0)
+        z[5::7, 2] = 30.0
+    o, state, ref, S = _delta_run(K, [100, 64], 1, 2, 64, 32, 100, 8, ctx=4, edit=edit)
+    close(o, ref, 2e-5)
+    close(state, S, 2e-5)
+
+
+@gpu
 def test_delta_rule_in_chunks_longer_than_announced(K):
     """A portion longer than `max_q` says runs all of its tokens, in chunks as token by token."""
     for lens, max_q in [([200, 3, 64], 64), ([1, 49, 100], 50)]:
