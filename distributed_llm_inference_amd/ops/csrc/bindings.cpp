@@ -899,7 +899,7 @@ void delta_rule(Tensor o, const Tensor& y, const Tensor& z, Tensor state, const 
     Tensor ws = at::empty({dlia_chunk_scan_ws((int)T, (int)B, (int)Hv)}, y.options());
     dlia_delta_chunks(o.data_ptr<float>(), y.data_ptr<float>(), z.data_ptr<float>(), state.data_ptr<float>(), A_log.data_ptr<float>(),
                       dt_bias.data_ptr<float>(), q_start.data_ptr<int>(), ctx.data_ptr<int>(), slots.data_ptr<int>(), ws.data_ptr<float>(),
-                      (int)B, (int)G, (int)Hv, (int)d, (int)dv, (int)C, z.stride(0), (int)col_beta, (int)col_a, (int)state.size(0), (int)max_q,
+                      (int)T, (int)B, (int)G, (int)Hv, (int)d, (int)dv, (int)C, z.stride(0), (int)col_beta, (int)col_a, (int)state.size(0),
                       cur_stream());
     return;
   }

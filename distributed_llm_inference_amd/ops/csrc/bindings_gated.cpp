@@ -213,9 +213,9 @@ void state_scan(int64_t rule, Tensor o, const Tensor& z, OptTensor wz, Tensor st
       col_v % 4 == 0 && (uintptr_t)z.data_ptr<float>() % 16 == 0) {
     Tensor ws = at::empty({dlia_chunk_scan_ws((int)T, (int)B, (int)H)}, o.options());
     dlia_memory_chunks(o.data_ptr<float>(), o.stride(0), z.data_ptr<float>(), z.stride(0), state.data_ptr<float>(), const_cast<float*>(mp),
-                       b0.data_ptr<float>(), q_start.data_ptr<int>(), ctx.data_ptr<int>(), slots.data_ptr<int>(), ws.data_ptr<float>(), (int)B,
-                       (int)H, (int)d, (int)dv, (int)state.size(0), (int)col_q, (int)col_k, (int)col_v, (int)col_i, (int)col_f, (float)cap,
-                       (float)qscale, (int)max_q, cur_stream());
+                       b0.data_ptr<float>(), q_start.data_ptr<int>(), ctx.data_ptr<int>(), slots.data_ptr<int>(), ws.data_ptr<float>(), (int)T,
+                       (int)B, (int)H, (int)d, (int)dv, (int)state.size(0), (int)col_q, (int)col_k, (int)col_v, (int)col_i, (int)col_f, (float)cap,
+                       (float)qscale, cur_stream());
     return;
   }
   const int rc = dlia_state_scan((int)rule, o.data_ptr<float>(), o.stride(0), z.data_ptr<float>(), z.stride(0), wzp, ldw,

@@ -150,12 +150,12 @@ long dlia_chunk_scan_ws(int T, int B, int H);
 // chunk_scan.hip: the delta rule over prompt portions on the matrix cores; d 64 or 128, dv and all row lengths and columns of y in
 // 16-byte pieces (dv a multiple of 16), ws of dlia_chunk_scan_ws floats
 void dlia_delta_chunks(float* o, const float* y, const float* z, float* state, const float* A_log, const float* dt_bias,
-                       const int* q_start, const int* ctx, const int* slots, float* ws, int B, int G, int Hv, int d, int dv, int C,
-                       long ldz, int col_beta, int col_a, int state_rows, int max_q, hipStream_t stream);
+                       const int* q_start, const int* ctx, const int* slots, float* ws, int T, int B, int G, int Hv, int d, int dv, int C,
+                       long ldz, int col_beta, int col_a, int state_rows, hipStream_t stream);
 // the matrix memory likewise (z rows and the columns of q, k, v in 16-byte pieces)
 void dlia_memory_chunks(float* o, long ldo, const float* z, long ldz, float* state, float* mstate, const float* b0, const int* q_start,
-                        const int* ctx, const int* slots, float* ws, int B, int H, int d, int dv, int state_rows, int col_q, int col_k,
-                        int col_v, int col_i, int col_f, float cap, float qscale, int max_q, hipStream_t stream);
+                        const int* ctx, const int* slots, float* ws, int T, int B, int H, int d, int dv, int state_rows, int col_q, int col_k,
+                        int col_v, int col_i, int col_f, float cap, float qscale, hipStream_t stream);
 int dlia_scan_decode_takes(int rule, long B, int H, int d, int dv);
 // scan_decode.hip: one token per sequence through the recurrences (rule 0, 1 as in state_scan, 2 the delta rule); 1: not taken
 int dlia_scan_decode(int rule, float* o, long ldo, const float* x, long ldx, const float* z, long ldz, const float* wz, long ldw, float* state,
