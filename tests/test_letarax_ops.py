@@ -393,6 +393,25 @@ def test_delta_rule_in_chunks_forgets_all(K, log_a):
 
 
 @gpu
+@pytest.mark.parametrize("what", ["q", "k", "v", "beta", "decay"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_delta_rule_in_chunks_keeps_a_bad_value_to_later_tokens(K, what, value):
+    """A value that is no number or infinite in token 41 of the first sequence (head 1, or the key head of heads 0 and 1; value column 5)
+    leaves the read-outs and states finite where they are token by token: earlier tokens, other heads, sequences and columns."""
+    G, H, d, dv = 2, 4, 64, 32
+    def edit(y, z, A_log, dtb):
+        if what in "qkv":
+            y[41, {"q": 3, "k": G * d + 3, "v": 2 * G * d + dv + 5}[what]] = value
+        else:
+            z[41, {"beta": 1, "decay": H + 1}[what]] = value
+    chunks, tokens = (_delta_run(K, [100, 70], G, H, d, dv, q, 9, ctx=4, edit=edit) for q in (100, 2))
+    for a, b in zip(chunks[:2], tokens[:2]):
+        assert torch.equal(a.isfinite(), b.isfinite()) and bool(a.isfinite().any())
+        close(a[a.isfinite()], b[a.isfinite()], 2e-5)
+    assert bool(chunks[0][:41].isfinite().all()) and bool(chunks[0][100:].isfinite().all())
+
+
+@gpu
 def test_delta_rule_in_chunks_longer_than_announced(K):
     """A portion longer than `max_q` says runs all of its tokens, in chunks as token by token."""
     for lens, max_q in [([200, 3, 64], 64), ([1, 49, 100], 50)]:

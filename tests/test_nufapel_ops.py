@@ -203,6 +203,31 @@ def test_matrix_memory_in_chunks_hip(H, d, dv, cap):
     assert bool((state[[3, 4, 6]] == 3.0).all()) and bool((mstate[[3, 4, 6]] == -5.0).all())
 
 
+@gpu
+@pytest.mark.parametrize("col", ["q", "k", "v", "i", "f"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_matrix_memory_in_chunks_keeps_a_bad_value_to_later_tokens(col, value):
+    """A value that is no number or infinite in token 41 leaves the read-outs and states finite where they are token by token."""
+    from distributed_llm_inference_amd import ops
+    K = ops.load()
+    H, d, dv, lens = 2, 64, 32, [100, 70]
+    T, n, c = sum(lens), H * d, 2 * H * d + H * dv
+    g = torch.Generator(device="cuda").manual_seed(12)
+    z, b0 = torch.randn(T, c + 2 * H, device="cuda", generator=g), torch.randn(2 * H, device="cuda", generator=g)
+    z[41, {"q": d + 3, "k": n + d + 3, "v": 2 * n + dv + 5, "i": c + 1, "f": c + H + 1}[col]] = value
+    q0, ctx, sl = _meta(lens, [3, 4], [0, 1])
+    got = []
+    for max_q in (100, 2):
+        st, ms = torch.ones(2, H, d, dv + 1, device="cuda"), torch.zeros(2, H, 128, device="cuda")
+        o = torch.zeros(T, H * (dv + 2), device="cuda")
+        K.state_scan(1, o, z, None, st, ms, b0, None, q0, ctx, sl, H, d, dv, 0, n, 2 * n, 0, c, c + H, 15.0, d ** -0.5, max_q, False)
+        got.append((o.view(T, H, dv + 2)[..., :dv + 1], st))
+    for a, b in zip(*got):
+        assert torch.equal(a.isfinite(), b.isfinite()) and bool(a.isfinite().any())
+        _close(a[a.isfinite()], b[a.isfinite()], 2e-5)
+    assert bool(got[0][0][:41].isfinite().all()) and bool(got[0][0][100:].isfinite().all())
+
+
 # ---- attention with distance bias, head temperature, learned sink, head gate ---------------------------------------------
 def _attn_case(T, H, G, d, dv, rows, far, seed, scale=None, low=False):
     g = torch.Generator().manual_seed(seed)
