@@ -527,7 +527,7 @@ class HybridGpuStage(GpuStage):
         if self.canon:
             return self._layers_canon(wk, T, B, tok_pos, tok_seq, q_start, ctx, slots, max_q)
         if self.post:
-            return self._layers_post(wk, T, B, tok_pos, tok_seq, q_start, ctx, slots, max_q)
+            return self._layers_post(wk, T, B, tok_pos, tok_seq, q_start, ctx, slots, max_q, lead_decode)
         if self.par:
             return self._layers_par(wk, T, B, tok_pos, tok_seq, q_start, ctx, slots, max_q)
         if self.gated:
@@ -584,7 +584,7 @@ class HybridGpuStage(GpuStage):
                 self._mm(wk, z, xn, p, "w_in")
                 K.short_conv(y, z, carry, p["conv_w"], q_start, ctx, slots, max_q)
                 K.unit_heads(y[:, :2 * qn], 2 * G, d, G, d ** -0.5, 1e-6)
-                K.delta_rule(o, y, z, state, p["A_log"], p["dt_bias"], q_start, ctx, slots, G, Hh, d, dv, C + vn, C + vn + Hh, max_q)
+                K.delta_rule(o, y, z, state, p["A_log"], p["dt_bias"], q_start, ctx, slots, G, Hh, d, dv, C + vn, C + vn + Hh, max_q, lead_decode)
                 K.gated_headnorm(mixed, o, z[:, C:C + vn], p["o_norm_w"], Hh, dv, eps)
             self._mm(wk, yo, mixed, p, "w_o")
             nxt = self.layers[li + 1]["ln1_w"] if li + 1 < n_layers else None
@@ -767,7 +767,7 @@ class HybridGpuStage(GpuStage):
                                        p["temp"], p["bias"], p["sink"], gate)
                 self._mm(wk, ya, mixed, p, "w_o")
                 K.state_scan(1, o, z, None, self.rec[ri][0], self.rec[ri][1], p["b_if"], None, q_start, ctx, slots, b.heads, b.dim, b.vdim,
-                             c_q, c_k, c_v, 0, c_i, c_i + b.heads, b.gate_cap, b.scale, max_q, self.wmode == "bf16")
+                             c_q, c_k, c_v, 0, c_i, c_i + b.heads, b.gate_cap, b.scale, max_q, self.wmode == "bf16", lead_decode)
                 K.headnorm_gate(mixed2, o, z[:, c_rg:c_rg + bv], p["o_norm_w"], b.heads, b.vdim, 2, eps)
                 yb = view(wk.yb, self._cols(p, "w_o"))
                 self._mm(wk, yb, mixed2, p, "w_o_r")
@@ -1121,7 +1121,7 @@ class HybridGpuStage(GpuStage):
             row_tok=z(32 * tiles, i32), eact=z(32 * tiles * ef, at), ey=z(32 * tiles * H), part=z(part), ws=z(ws_floats + 4096),
             head_x=torch.zeros(B, H, device=dev, dtype=at), logits=torch.zeros(B, self.vocab_pad, device=dev), cmax=None, guided=False)
 
-    def _layers_post(self, wk, T: int, B: int, tok_pos, tok_seq, q_start, ctx, slots, max_q: int):
+    def _layers_post(self, wk, T: int, B: int, tok_pos, tok_seq, q_start, ctx, slots, max_q: int, lead_decode: int):
         K, eps, H = self.K, self.spec.norm_eps, self.spec.hidden_size
         h, xn = wk.h[:T], wk.xn[:T]
         view = lambda buf, cols: buf[:T * cols].view(T, cols)
@@ -1166,7 +1166,7 @@ class HybridGpuStage(GpuStage):
                 K.multi_attention(mixed, qf, kd, kc, vc, 0, tok_pos, tok_seq, table, Hh, kd, dv, 1, scale, a.window or 0, 0, 0.0, 0.0,
                                   1.0, eps, gate, a.chunk, p["sink"])
             K.state_scan(1, o, z, None, self.rec[li][0], self.rec[li][1], p["b_if"], None, q_start, ctx, slots, b.heads, b.dim, b.vdim,
-                         c_q, c_k, c_v, 0, c_i, c_f, b.gate_cap, b.scale, max_q, self.wmode == "bf16")
+                         c_q, c_k, c_v, 0, c_i, c_f, b.gate_cap, b.scale, max_q, self.wmode == "bf16", lead_decode)
             K.headnorm_gate(mixed2, o, z[:, c_rg:c_rg + bv], p["o_norm_w"], b.heads, b.vdim, 2, eps)
             ya = view(wk.ya, self._cols(p, "w_o"))
             self._mm(wk, ya, both, p, "w_o")

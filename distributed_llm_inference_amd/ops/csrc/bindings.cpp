@@ -874,9 +874,10 @@ void unit_heads(Tensor x, int64_t heads, int64_t d, int64_t scaled_heads, double
                   cur_stream());
 }
 
+// `lead`: so many sequences at the front have one token each (decode tokens that ride in front of prompt portions)
 void delta_rule(Tensor o, const Tensor& y, const Tensor& z, Tensor state, const Tensor& A_log, const Tensor& dt_bias,
                 const Tensor& q_start, const Tensor& ctx, const Tensor& slots, int64_t G, int64_t Hv, int64_t d, int64_t dv,
-                int64_t col_beta, int64_t col_a, int64_t max_q) {
+                int64_t col_beta, int64_t col_a, int64_t max_q, int64_t lead) {
   DLIA_ON_DEVICE_OF(o);
   check_f32(o, "o"); check_f32(y, "y"); check_f32(state, "state"); check_f32(A_log, "A_log"); check_f32(dt_bias, "dt_bias");
   check_mat(z, "z");
@@ -887,27 +888,29 @@ void delta_rule(Tensor o, const Tensor& y, const Tensor& z, Tensor state, const 
   DLIA_CHECK(z.size(0) >= T && col_beta + Hv <= z.size(1) && col_a + Hv <= z.size(1) && col_beta >= 0 && col_a >= 0, "delta_rule: gate columns");
   DLIA_CHECK(state.dim() == 4 && state.size(1) == Hv && state.size(2) == d && state.size(3) == dv, "delta_rule: state [slots, Hv, d, dv]");
   DLIA_CHECK(A_log.numel() == Hv && dt_bias.numel() == Hv && q_start.numel() >= B + 1 && slots.numel() >= B, "delta_rule: per-head / per-sequence vectors");
-  if (max_q <= 1 && dlia_scan_decode(2, o.data_ptr<float>(), o.stride(0), y.data_ptr<float>(), C, z.data_ptr<float>(), z.stride(0), nullptr, 0,
-                                     state.data_ptr<float>(), nullptr, A_log.data_ptr<float>(), dt_bias.data_ptr<float>(), q_start.data_ptr<int>(),
-                                     ctx.data_ptr<int>(), slots.data_ptr<int>(), (int)B, (int)Hv, (int)(Hv / G), (int)d, (int)dv, (int)state.size(0),
-                                     0, (int)(G * d), (int)(2 * G * d), (int)col_a, (int)col_beta, 0.f, 1.f, cur_stream()) == 0)
-    return;
-  // Prompt portions in chunks on the matrix cores; decode steps, other sizes and unaligned rows token by token. The line: one
-  // sequence of 33 / 64 / 2048 tokens (32 heads of 128) takes 18 / 27 / 780 us token by token and 18 / 22 / 224 in chunks, 64
-  // sequences of 33 tokens 406 and 407, 16 of 128 337 and 229.
-  if (max_q >= 48 && (d == 64 || d == 128) && dv % 16 == 0 && C % 4 == 0 && (uintptr_t)y.data_ptr<float>() % 16 == 0) {
-    Tensor ws = at::empty({dlia_chunk_scan_ws((int)T, (int)B, (int)Hv)}, y.options());
-    dlia_delta_chunks(o.data_ptr<float>(), y.data_ptr<float>(), z.data_ptr<float>(), state.data_ptr<float>(), A_log.data_ptr<float>(),
-                      dt_bias.data_ptr<float>(), q_start.data_ptr<int>(), ctx.data_ptr<int>(), slots.data_ptr<int>(), ws.data_ptr<float>(),
-                      (int)T, (int)B, (int)G, (int)Hv, (int)d, (int)dv, (int)C, z.stride(0), (int)col_beta, (int)col_a, (int)state.size(0),
-                      cur_stream());
-    return;
-  }
-  const int rc = dlia_delta_rule(o.data_ptr<float>(), y.data_ptr<float>(), z.data_ptr<float>(), state.data_ptr<float>(),
-                                 A_log.data_ptr<float>(), dt_bias.data_ptr<float>(), q_start.data_ptr<int>(), ctx.data_ptr<int>(),
-                                 slots.data_ptr<int>(), (int)B, (int)G, (int)Hv, (int)d, (int)dv, (int)C, z.stride(0), (int)col_beta,
-                                 (int)col_a, (int)state.size(0), (int)max_q, cur_stream());
-  DLIA_CHECK(rc == 0, "delta_rule: key size ", d, " is beyond what the kernel holds in registers (512)");
+  // `n` sequences from the b-th on, token by token: single tokens by the step kernel where it takes their sizes
+  auto by_token = [&](int64_t b, int64_t n, int64_t longest) {
+    const int *q0 = q_start.data_ptr<int>() + b, *cx = ctx.data_ptr<int>() + b, *sl = slots.data_ptr<int>() + b;
+    if (longest <= 1 && dlia_scan_decode(2, o.data_ptr<float>(), o.stride(0), y.data_ptr<float>(), C, z.data_ptr<float>(), z.stride(0), nullptr, 0,
+                                         state.data_ptr<float>(), nullptr, A_log.data_ptr<float>(), dt_bias.data_ptr<float>(), q0, cx, sl, (int)n,
+                                         (int)Hv, (int)(Hv / G), (int)d, (int)dv, (int)state.size(0), 0, (int)(G * d), (int)(2 * G * d),
+                                         (int)col_a, (int)col_beta, 0.f, 1.f, cur_stream()) == 0)
+      return;
+    const int rc = dlia_delta_rule(o.data_ptr<float>(), y.data_ptr<float>(), z.data_ptr<float>(), state.data_ptr<float>(), A_log.data_ptr<float>(),
+                                   dt_bias.data_ptr<float>(), q0, cx, sl, (int)n, (int)G, (int)Hv, (int)d, (int)dv, (int)C, z.stride(0),
+                                   (int)col_beta, (int)col_a, (int)state.size(0), (int)longest, cur_stream());
+    DLIA_CHECK(rc == 0, "delta_rule: key size ", d, " is beyond what the kernel holds in registers (512)");
+  };
+  const bool aligned = C % 4 == 0 && (uintptr_t)y.data_ptr<float>() % 16 == 0;
+  const int route = aligned ? dlia_chunk_scan_route(2, B, lead, T, max_q, (int)Hv, (int)d, (int)dv) : 0;
+  if (route == 0) return by_token(0, B, max_q);
+  const int64_t b = route == 2 ? lead : 0, n = B - b;
+  if (b) by_token(0, b, 1);
+  Tensor ws = at::empty({dlia_chunk_scan_ws((int)T, (int)n, (int)Hv)}, y.options());
+  dlia_delta_chunks(o.data_ptr<float>(), y.data_ptr<float>(), z.data_ptr<float>(), state.data_ptr<float>(), A_log.data_ptr<float>(),
+                    dt_bias.data_ptr<float>(), q_start.data_ptr<int>() + b, ctx.data_ptr<int>() + b, slots.data_ptr<int>() + b, ws.data_ptr<float>(),
+                    (int)T, (int)n, (int)G, (int)Hv, (int)d, (int)dv, (int)C, z.stride(0), (int)col_beta, (int)col_a, (int)state.size(0),
+                    cur_stream());
 }
 
 }  // namespace
@@ -927,7 +930,7 @@ TORCH_LIBRARY(dlia, m) {
   m.def("short_conv(Tensor(a!) y, Tensor z, Tensor(b!) carry, Tensor taps, Tensor q_start, Tensor ctx, Tensor slots, int max_q) -> ()");
   m.def("short_conv_act(Tensor(a!) y, Tensor z, Tensor(b!) carry, Tensor taps, Tensor? bias, Tensor q_start, Tensor ctx, Tensor slots, int max_q, bool silu) -> ()");
   m.def("unit_heads(Tensor(a!) x, int heads, int d, int scaled_heads, float mult, float eps) -> ()");
-  m.def("delta_rule(Tensor(a!) o, Tensor y, Tensor z, Tensor(b!) state, Tensor A_log, Tensor dt_bias, Tensor q_start, Tensor ctx, Tensor slots, int G, int Hv, int d, int dv, int col_beta, int col_a, int max_q) -> ()");
+  m.def("delta_rule(Tensor(a!) o, Tensor y, Tensor z, Tensor(b!) state, Tensor A_log, Tensor dt_bias, Tensor q_start, Tensor ctx, Tensor slots, int G, int Hv, int d, int dv, int col_beta, int col_a, int max_q, int lead=0) -> ()");
   m.def("norm(Tensor(a!) out, Tensor(b!) x, Tensor? delta, Tensor? partial, int splits, Tensor? pbias, Tensor w, Tensor? b, Tensor? row_idx, float eps, int mode) -> ()");
   m.def("embed(Tensor(a!) out, Tensor ids, Tensor? pos, Tensor wte, Tensor? wpe) -> ()");
   m.def("rope_kvwrite(Tensor(a!) qkv, Tensor? partial, int splits, Tensor? pbias, Tensor(b!) kv_cache, Tensor cos, Tensor sin, Tensor tok_pos, Tensor tok_seq, Tensor block_table, int Hq, int Hkv, int D, bool use_rope) -> ()");

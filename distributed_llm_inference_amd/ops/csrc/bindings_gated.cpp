@@ -165,15 +165,19 @@ void biased_attention(Tensor out, const Tensor& qkv, const Tensor& kcache, const
 
 int64_t state_scan_blocks(int64_t d, int64_t ncols) { return dlia_state_scan_blocks((int)d, (int)ncols); }
 
-// the kernel that a step of single tokens takes, by its sizes: 1 scan_decode.hip, 0 the general one
-int64_t scan_route(int64_t rule, int64_t B, int64_t H, int64_t d, int64_t dv) {
-  return dlia_scan_decode_takes((int)rule, (long)B, (int)H, (int)d, (int)dv);
+// the kernels that a step takes, by its sizes (rule 2: the gated delta rule): 0 the general one, 1 scan_decode.hip, 2 chunk_scan.hip, 3 that one
+// behind a step of single tokens for the `lead` ones at the front
+int64_t scan_route(int64_t rule, int64_t B, int64_t H, int64_t d, int64_t dv, int64_t T, int64_t max_q, int64_t lead) {
+  if (max_q <= 1) return dlia_scan_decode_takes((int)rule, (long)B, (int)H, (int)d, (int)dv);
+  const int r = dlia_chunk_scan_route((int)rule, (long)B, (long)lead, (long)T, (long)max_q, (int)H, (int)d, (int)dv);
+  return r ? r + 1 : 0;
 }
 
+// `lead`: so many sequences at the front have one token each (decode tokens that ride in front of prompt portions)
 void state_scan(int64_t rule, Tensor o, const Tensor& z, OptTensor wz, Tensor state, const std::optional<Tensor>& mstate,
                 const Tensor& b0, OptTensor b1, const Tensor& q_start, const Tensor& ctx, const Tensor& slots, int64_t H, int64_t d,
                 int64_t dv, int64_t col_q, int64_t col_k, int64_t col_v, int64_t col_a, int64_t col_i, int64_t col_f, double cap,
-                double qscale, int64_t max_q, bool quick) {
+                double qscale, int64_t max_q, bool quick, int64_t lead) {
   DLIA_ON_DEVICE_OF(o);
   check_fmat(o, "o"); check_fmat(z, "z"); check_f32(state, "state"); check_f32(b0, "b0");
   check_i32(q_start, "q_start"); check_i32(ctx, "ctx"); check_i32(slots, "slots");
@@ -200,30 +204,31 @@ void state_scan(int64_t rule, Tensor o, const Tensor& z, OptTensor wz, Tensor st
     DLIA_CHECK(mstate->dim() == 3 && mstate->size(0) == state.size(0) && mstate->size(1) == H && mstate->size(2) == 128, "state_scan: mstate [slots, H, 128]");
     mp = mstate->data_ptr<float>();
   }
-  if (max_q <= 1 &&
-      dlia_scan_decode((int)rule, o.data_ptr<float>(), o.stride(0), z.data_ptr<float>(), z.stride(0), z.data_ptr<float>(), z.stride(0), wzp, ldw,
-                       state.data_ptr<float>(), const_cast<float*>(mp), b0.data_ptr<float>(), b1.has_value() ? b1->data_ptr<float>() : nullptr,
-                       q_start.data_ptr<int>(), ctx.data_ptr<int>(), slots.data_ptr<int>(), (int)B, (int)H, 1, (int)d, (int)dv, (int)state.size(0),
-                       (int)col_q, (int)col_k, (int)col_v, (int)(rule == 0 ? col_a : col_f), (int)col_i, (float)cap, (float)qscale, cur_stream()) == 0)
-    return;
-  // Matrix memory over prompt portions: in chunks on the matrix cores. The line: one sequence of 48 / 64 / 2048 tokens (16 heads of
-  // 128) takes 19 / 24 / 595 us token by token and 14 / 14 / 168 in chunks, 16 sequences of 128 tokens 125 and 121, but 64 of 48
-  // tokens 174 and 250: with several rounds of workgroups no chain is waited for, and a chunk kernel's workgroup has a CU to itself.
-  if (rule == 1 && max_q >= (B * H * (dv / 16 + 1) <= 1024 ? 48 : 128) && (d == 64 || d == 128) && dv % 16 == 0 && dv <= 512 && z.stride(0) % 4 == 0 && col_q % 4 == 0 && col_k % 4 == 0 &&
-      col_v % 4 == 0 && (uintptr_t)z.data_ptr<float>() % 16 == 0) {
-    Tensor ws = at::empty({dlia_chunk_scan_ws((int)T, (int)B, (int)H)}, o.options());
-    dlia_memory_chunks(o.data_ptr<float>(), o.stride(0), z.data_ptr<float>(), z.stride(0), state.data_ptr<float>(), const_cast<float*>(mp),
-                       b0.data_ptr<float>(), q_start.data_ptr<int>(), ctx.data_ptr<int>(), slots.data_ptr<int>(), ws.data_ptr<float>(), (int)T,
-                       (int)B, (int)H, (int)d, (int)dv, (int)state.size(0), (int)col_q, (int)col_k, (int)col_v, (int)col_i, (int)col_f, (float)cap,
-                       (float)qscale, cur_stream());
-    return;
-  }
-  const int rc = dlia_state_scan((int)rule, o.data_ptr<float>(), o.stride(0), z.data_ptr<float>(), z.stride(0), wzp, ldw,
-                                 state.data_ptr<float>(), const_cast<float*>(mp), b0.data_ptr<float>(),
-                                 b1.has_value() ? b1->data_ptr<float>() : nullptr, q_start.data_ptr<int>(), ctx.data_ptr<int>(),
-                                 slots.data_ptr<int>(), (int)B, (int)H, (int)d, (int)dv, (int)state.size(0), (int)col_q, (int)col_k,
-                                 (int)col_v, (int)col_a, (int)col_i, (int)col_f, (float)cap, (float)qscale, (int)max_q, quick ? 1 : 0, cur_stream());
-  DLIA_CHECK(rc == 0, "state_scan: key size ", d, " / value size ", dv, " beyond what the kernel splits (1024 rows, 128 column blocks)");
+  // `n` sequences from the b-th on, token by token: single tokens by the step kernel where it takes their sizes
+  auto by_token = [&](int64_t b, int64_t n, int64_t longest) {
+    const int *q0 = q_start.data_ptr<int>() + b, *cx = ctx.data_ptr<int>() + b, *sl = slots.data_ptr<int>() + b;
+    const float* b1p = b1.has_value() ? b1->data_ptr<float>() : nullptr;
+    if (longest <= 1 && dlia_scan_decode((int)rule, o.data_ptr<float>(), o.stride(0), z.data_ptr<float>(), z.stride(0), z.data_ptr<float>(), z.stride(0),
+                                         wzp, ldw, state.data_ptr<float>(), const_cast<float*>(mp), b0.data_ptr<float>(), b1p, q0, cx, sl, (int)n, (int)H,
+                                         1, (int)d, (int)dv, (int)state.size(0), (int)col_q, (int)col_k, (int)col_v,
+                                         (int)(rule == 0 ? col_a : col_f), (int)col_i, (float)cap, (float)qscale, cur_stream()) == 0)
+      return;
+    const int rc = dlia_state_scan((int)rule, o.data_ptr<float>(), o.stride(0), z.data_ptr<float>(), z.stride(0), wzp, ldw, state.data_ptr<float>(),
+                                   const_cast<float*>(mp), b0.data_ptr<float>(), b1p, q0, cx, sl, (int)n, (int)H, (int)d, (int)dv,
+                                   (int)state.size(0), (int)col_q, (int)col_k, (int)col_v, (int)col_a, (int)col_i, (int)col_f, (float)cap,
+                                   (float)qscale, (int)longest, quick ? 1 : 0, cur_stream());
+    DLIA_CHECK(rc == 0, "state_scan: key size ", d, " / value size ", dv, " beyond what the kernel splits (1024 rows, 128 column blocks)");
+  };
+  const bool aligned = z.stride(0) % 4 == 0 && col_q % 4 == 0 && col_k % 4 == 0 && col_v % 4 == 0 && (uintptr_t)z.data_ptr<float>() % 16 == 0;
+  const int route = rule == 1 && aligned ? dlia_chunk_scan_route(1, B, lead, T, max_q, (int)H, (int)d, (int)dv) : 0;
+  if (route == 0) return by_token(0, B, max_q);
+  const int64_t b = route == 2 ? lead : 0, n = B - b;
+  if (b) by_token(0, b, 1);
+  Tensor ws = at::empty({dlia_chunk_scan_ws((int)T, (int)n, (int)H)}, o.options());
+  dlia_memory_chunks(o.data_ptr<float>(), o.stride(0), z.data_ptr<float>(), z.stride(0), state.data_ptr<float>(), const_cast<float*>(mp),
+                     b0.data_ptr<float>(), q_start.data_ptr<int>() + b, ctx.data_ptr<int>() + b, slots.data_ptr<int>() + b, ws.data_ptr<float>(),
+                     (int)T, (int)n, (int)H, (int)d, (int)dv, (int)state.size(0), (int)col_q, (int)col_k, (int)col_v, (int)col_i, (int)col_f,
+                     (float)cap, (float)qscale, cur_stream());
 }
 
 void moe_route(Tensor sel, Tensor wts, const Tensor& logits, int64_t top, int64_t groups, int64_t keep, double scale, OptTensor correction,
@@ -349,8 +354,8 @@ TORCH_LIBRARY_FRAGMENT(dlia, m) {
   m.def("softcap(Tensor(a!) logits, int vocab, float cap) -> ()");
   m.def("biased_attention(Tensor(a!) out, Tensor qkv, Tensor kcache, Tensor vcache, Tensor tok_pos, Tensor tok_seq, Tensor block_table, int H, int G, int d, int dv, float scale, Tensor? temp, Tensor? bias, Tensor? sink, Tensor? gate) -> ()");
   m.def("state_scan_blocks(int d, int ncols) -> int");
-  m.def("scan_route(int rule, int B, int H, int d, int dv) -> int");
-  m.def("state_scan(int rule, Tensor(a!) o, Tensor z, Tensor? wz, Tensor(b!) state, Tensor(c!)? mstate, Tensor b0, Tensor? b1, Tensor q_start, Tensor ctx, Tensor slots, int H, int d, int dv, int col_q, int col_k, int col_v, int col_a, int col_i, int col_f, float cap, float qscale, int max_q, bool quick) -> ()");
+  m.def("scan_route(int rule, int B, int H, int d, int dv, int T=0, int max_q=1, int lead=0) -> int");
+  m.def("state_scan(int rule, Tensor(a!) o, Tensor z, Tensor? wz, Tensor(b!) state, Tensor(c!)? mstate, Tensor b0, Tensor? b1, Tensor q_start, Tensor ctx, Tensor slots, int H, int d, int dv, int col_q, int col_k, int col_v, int col_a, int col_i, int col_f, float cap, float qscale, int max_q, bool quick, int lead=0) -> ()");
   m.def("moe_route(Tensor(a!) sel, Tensor(b!) wts, Tensor logits, int top, int groups, int keep, float scale, Tensor? correction=None, bool softmax=False, int group_rank=2, bool renorm=True) -> ()");
   m.def("moe_plan(Tensor(a!) tiles, Tensor(b!) row_tok, Tensor(c!) pair_row, Tensor sel, int pairs, int top, int E, int tile_rows, Tensor? wts=None, Tensor(d!)? row_w=None) -> ()");
   m.def("moe_route_plan(Tensor(a!) sel, Tensor(b!) wts, Tensor logits, int top, int groups, int keep, float scale, Tensor? correction, bool softmax, int group_rank, bool renorm, Tensor(c!) tiles, Tensor(d!) row_tok, Tensor(e!) pair_row, int E, int tile_rows, Tensor(f!)? row_w) -> ()");

@@ -146,6 +146,8 @@ void dlia_short_conv(float* y, const float* z, float* carry, const float* taps, 
                      const int* slots, int B, int max_q, int C, int K, long ldz, int state_rows, const float* bias, int silu,
                      hipStream_t stream);
 void dlia_unit_heads(float* x, int T, int heads, int d, long ld, int scaled_heads, float mult, float eps, hipStream_t stream);
+int dlia_scan_decode_takes(int rule, long B, int H, int d, int dv);
+int dlia_chunk_scan_route(int rule, long B, long lead, long T, long max_q, int H, int d, int dv);
 long dlia_chunk_scan_ws(int T, int B, int H);
 // chunk_scan.hip: the delta rule over prompt portions on the matrix cores; d 64 or 128, dv and all row lengths and columns of y in
 // 16-byte pieces (dv a multiple of 16), ws of dlia_chunk_scan_ws floats
@@ -156,7 +158,6 @@ void dlia_delta_chunks(float* o, const float* y, const float* z, float* state, c
 void dlia_memory_chunks(float* o, long ldo, const float* z, long ldz, float* state, float* mstate, const float* b0, const int* q_start,
                         const int* ctx, const int* slots, float* ws, int T, int B, int H, int d, int dv, int state_rows, int col_q, int col_k,
                         int col_v, int col_i, int col_f, float cap, float qscale, hipStream_t stream);
-int dlia_scan_decode_takes(int rule, long B, int H, int d, int dv);
 // scan_decode.hip: one token per sequence through the recurrences (rule 0, 1 as in state_scan, 2 the delta rule); 1: not taken
 int dlia_scan_decode(int rule, float* o, long ldo, const float* x, long ldx, const float* z, long ldz, const float* wz, long ldw, float* state,
                      float* mstate, const float* b0, const float* b1, const int* q_start, const int* ctx, const int* slots, int B, int H, int per,
