@@ -205,7 +205,7 @@ __global__ __launch_bounds__(256) void glu_act_kernel(OT* __restrict__ act, long
   act[m * lda + c] = (OT)v;
 }
 
-// Row tiles of the plan: 32 rows. Where experts have several of them (fp32 prompts above all) a workgroup of four waves covers one
+// Row tiles of the plan: 32 rows. Where experts have several of them and the blocks fill the chip (fp32 prompts above all) a workgroup of four waves covers one
 // row tile by 128 (up) or 256 (down) output columns; a wave holds both 16-row halves of the tile against its 32 (64) columns, so
 // every fragment it loads feeds two or more MFMAs, and the fragments of the next k-step are on their way while the current ones
 // are multiplied.
@@ -421,8 +421,9 @@ __global__ __launch_bounds__(64 * NW) void moe_stream_kernel(OT* __restrict__ ou
           for (int g = 0; g < NG * NJ; ++g) acc[i][g] = mma_frag(T{}, f.a[u][i], f.w[u][g], acc[i][g]);
     };
     // Piece c of the wave's share; each workgroup begins elsewhere in K and goes round. A K of no more pieces than waves stays with
-    // one of them: there is little to share, and its sums are then formed in the order of the wide blocks (a row's result does not
-    // depend on which of the two its step took).
+    // one of them: its sums are then formed in the order of the wide blocks, so that for such K (up to 512 in 16 bits, 128 in 32) a row's
+    // result does not depend on which of the two its step took; for longer K it may, in the last bits. It costs next to nothing where a
+    // launch is all there is (4.5 to 5 us either way) and up to 1.7 of 8 us in the gated fp32 form, 1.7 of 16 in the 16-bit one (512 x 512).
     const int total = (K + CH - 1) / CH, turn = total > NW ? (blockIdx.x * 4 + e) % total : 0, step = total > NW ? NW : 1;
     if (wave >= step) return;
     auto at = [&](int c) { const int k = c + turn; return (k >= total ? k - total : k) * CH; };
@@ -761,9 +762,15 @@ static void launch_moe_stream(OT* out, const T* x, const T* w0, const T* w1, con
 #undef DLIA_ST
 }
 
-// Row tiles that share their experts' weights in the caches: from four full tiles an expert on the wide column blocks are faster (8
-// experts, two a token, 2048 x 2048 fp32: 500 tokens 335 us wide and 301 as a stream, 900 tokens 492 and 537).
-static bool moe_wide(int max_tiles, int experts) { return max_tiles - experts > 4 * experts; }
+// Steps that run in wide column blocks (128 columns of gate and up, 256 of the down projection, a workgroup a CU) and not as a stream of the
+// weights: experts of more than four tiles, and blocks that fill their rounds over the 256 CUs. A round takes what it takes however few its
+// blocks (8 experts, two a token, 2048 x 2048 fp32, down: 96 to 107 us), a stream goes by the rows (0.48 us a block's worth): 700 / 1000 /
+// 1400 / 2048 tokens 187 / 303 / 306 / 527 us in blocks and 179 / 250 / 339 / 485 as a stream. Gate and up gain by blocks in a single full
+// round alone (1900 tokens, one of 4 experts, 1024 x 512: 60 against 64 us; the above, 1000 / 1400 tokens: 579 / 707 against 421 / 576).
+extern "C" int dlia_moe_wide(int max_tiles, int experts, int cols, int down) {
+  const long blocks = (long)(max_tiles - experts / 2) * ((cols + (down ? 255 : 127)) / (down ? 256 : 128)), rounds = (blocks + 255) / 256;
+  return max_tiles - experts > 4 * experts && blocks * 10 > rounds * 256 * 9 && (down || rounds == 1);
+}
 
 extern "C" void dlia_moe_up(void* act, const void* x, const void* wg, const void* wu, int f32, const int* tiles, const int* row_tok,
                             int max_tiles, int experts, int F, int K, long ldx, long lda, float limit, int tile_rows, const float* row_w,
@@ -777,11 +784,11 @@ extern "C" void dlia_moe_up(void* act, const void* x, const void* wg, const void
   const int vec = f32 ? 4 : 8;
   const int ok = K % vec == 0 && ldx % vec == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)wg % 16 == 0 && (uintptr_t)wu % 16 == 0;
   if (f32) {
-    if (moe_wide(max_tiles, experts)) launch_moe_up<float, float, 2>(act, x, wg, wu, tiles, row_tok, max_tiles, F, K, ldx, lda, limit, ok, row_w, stream);
+    if (dlia_moe_wide(max_tiles, experts, F, 0)) launch_moe_up<float, float, 2>(act, x, wg, wu, tiles, row_tok, max_tiles, F, K, ldx, lda, limit, ok, row_w, stream);
     else if (wg) launch_moe_stream<float, float, 1>((float*)act, (const float*)x, (const float*)wg, (const float*)wu, tiles, row_tok, max_tiles, experts, F, K, ldx, lda, limit, ok, row_w, stream);
     else launch_moe_stream<float, float, 2>((float*)act, (const float*)x, (const float*)wu, nullptr, tiles, row_tok, max_tiles, experts, F, K, ldx, lda, limit, ok, row_w, stream);
   } else {
-    if (moe_wide(max_tiles, experts)) launch_moe_up<dlia::bf16, dlia::bf16, 2>(act, x, wg, wu, tiles, row_tok, max_tiles, F, K, ldx, lda, limit, ok, row_w, stream);
+    if (dlia_moe_wide(max_tiles, experts, F, 0)) launch_moe_up<dlia::bf16, dlia::bf16, 2>(act, x, wg, wu, tiles, row_tok, max_tiles, F, K, ldx, lda, limit, ok, row_w, stream);
     else if (wg) launch_moe_stream<dlia::bf16, dlia::bf16, 1>((dlia::bf16*)act, (const dlia::bf16*)x, (const dlia::bf16*)wg, (const dlia::bf16*)wu, tiles, row_tok, max_tiles, experts, F, K, ldx, lda, limit, ok, row_w, stream);
     else launch_moe_stream<dlia::bf16, dlia::bf16, 2>((dlia::bf16*)act, (const dlia::bf16*)x, (const dlia::bf16*)wu, nullptr, tiles, row_tok, max_tiles, experts, F, K, ldx, lda, limit, ok, row_w, stream);
   }
@@ -797,10 +804,10 @@ extern "C" void dlia_moe_down(float* y, const void* act, const void* wd, int f32
   const int vec = f32 ? 4 : 8;
   const int ok = F % vec == 0 && lda % vec == 0 && (uintptr_t)act % 16 == 0 && (uintptr_t)wd % 16 == 0;
   if (f32) {
-    if (moe_wide(max_tiles, experts)) launch_moe_down<float, 4>(y, act, wd, tiles, row_tok, max_tiles, H, F, lda, ok, stream);
+    if (dlia_moe_wide(max_tiles, experts, H, 1)) launch_moe_down<float, 4>(y, act, wd, tiles, row_tok, max_tiles, H, F, lda, ok, stream);
     else launch_moe_stream<float, float, 0>(y, (const float*)act, (const float*)wd, nullptr, tiles, row_tok, max_tiles, experts, H, F, lda, (long)H, 0.f, ok, nullptr, stream);
   } else {
-    if (moe_wide(max_tiles, experts)) launch_moe_down<dlia::bf16, 4>(y, act, wd, tiles, row_tok, max_tiles, H, F, lda, ok, stream);
+    if (dlia_moe_wide(max_tiles, experts, H, 1)) launch_moe_down<dlia::bf16, 4>(y, act, wd, tiles, row_tok, max_tiles, H, F, lda, ok, stream);
     else launch_moe_stream<dlia::bf16, float, 0>(y, (const dlia::bf16*)act, (const dlia::bf16*)wd, nullptr, tiles, row_tok, max_tiles, experts, H, F, lda, (long)H, 0.f, ok, nullptr, stream);
   }
 }

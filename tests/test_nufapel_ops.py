@@ -326,9 +326,20 @@ MOE = [(50, 32, 6, 2, 24, 3, 2, 1.5, 1.0), (600, 128, 8, 2, 64, 2, 1, 2.0, 1.5),
        # 128-row tiles by 256 weight rows (gate and up; then down): 13, 33 and 66 steps of the ring, ragged last column blocks
        (1100, 416, 3, 2, 1056, 1, 1, 1.0, 7.0), (1100, 2112, 3, 2, 96, 1, 1, 1.0, 7.0),
        # row tiles of 32 as a weight stream: a token or two, whole and ragged pieces, K beyond one turn of the waves; then one and two
-       # column tiles a wave with half tiles empty; then the wide blocks' whole and masked pieces
+       # column tiles a wave with half tiles empty; then many tiles an expert with whole and masked pieces
        (1, 512, 3, 2, 88, 1, 1, 1.0, 7.0), (3, 1152, 4, 1, 1100, 1, 1, 1.0, 7.0), (40, 64, 6, 2, 4100, 1, 1, 1.0, 7.0), (60, 200, 2, 1, 64, 1, 1, 1.0, 7.0),
-       (300, 128, 2, 1, 256, 1, 1, 1.0, 7.0), (300, 72, 2, 1, 40, 1, 1, 1.0, 7.0)]
+       (300, 128, 2, 1, 256, 1, 1, 1.0, 7.0), (300, 72, 2, 1, 40, 1, 1, 1.0, 7.0),
+       # the wide blocks (a full round of them): gate and up with whole and masked pieces, then the down projection
+       (450, 128, 2, 1, 1900, 1, 1, 1.0, 7.0), (450, 72, 2, 1, 1900, 1, 1, 1.0, 7.0), (450, 3700, 2, 1, 64, 1, 1, 1.0, 7.0), (450, 3700, 2, 1, 40, 1, 1, 1.0, 7.0)]
+
+
+@pytest.mark.parametrize("T,E,top,cols,down,wide", [
+    (513, 4, 1, 256, True, False), (1900, 4, 1, 256, True, False), (513, 8, 2, 512, True, False), (1900, 8, 2, 512, True, True),      # 13.4 against 29 us wide, ..., 14 / 17, 125 / 112
+    (1000, 8, 2, 2048, True, False), (1400, 8, 2, 2048, True, True), (2048, 8, 2, 2048, True, False), (500, 8, 2, 2048, True, False),
+    (1400, 8, 2, 2048, False, False), (1900, 4, 1, 512, False, True), (450, 2, 1, 1900, False, True), (450, 2, 1, 3700, True, True)])
+def test_experts_wide_blocks_where_they_measured_faster(T, E, top, cols, down, wide):
+    from distributed_llm_inference_amd import ops
+    assert ops.load(build_if_missing=True).moe_wide((T * top + 31) // 32 + E, E, cols, down) == wide
 
 
 @pytest.mark.parametrize("T,W,E,top,ff,groups,keep,scale,limit", MOE)
