@@ -746,13 +746,14 @@ template <typename T, typename OT, int KIND>
 static void launch_moe_stream(OT* out, const T* x, const T* w0, const T* w1, const int* tiles, const int* row_tok, int max_tiles, int experts, int N,
                               int K, long ldx, long ldo, float limit, int ok, const float* row_w, hipStream_t stream) {
   // One column tile a wave where the gated kernel would have too few workgroups to fill the chip three a CU, or hardly a row each (2048 x
-  // 2048, 64 tokens: 27.6 us against 30.7; 3584 x 4096, 4 tokens: 51 against 58, 64 tokens 101 against 96); fp32 pieces are half as
-  // deep and its workgroups last longer (64 tokens: 68 against 60).
+  // 2048, 64 tokens: 27.6 us against 30.7; 3584 x 4096, 4 tokens: 51 against 58, 64 tokens 101 against 96; by the row tiles there
+  // are, not the experts: 2048 x 2048, 300 / 400 tokens in 19 / 25 tiles 86 / 107 us against 70 / 89); fp32 pieces are half as deep and its
+  // workgroups last longer (64 tokens: 68 against 60).
 #define DLIA_ST(FAST, U, NJ)                                                                                                               \
   hipLaunchKernelGGL((dlia::moe_stream_kernel<T, OT, KIND, FAST, 4, U, NJ>), dim3((N + 16 * NJ - 1) / (16 * NJ), max_tiles), dim3(256), 0, \
                      stream, out, x, w0, w1, tiles, row_tok, N, K, ldx, ldo, limit, ok, row_w)
   if constexpr (KIND == 1 && sizeof(T) == 2)
-    if (max_tiles - experts <= 1 || (long)(N + 31) / 32 * experts < 768) {
+    if (max_tiles - experts <= 1 || (long)(N + 31) / 32 * (max_tiles - experts / 2) < 768) {
       if (ok && K % (256 / (int)sizeof(T)) == 0) DLIA_ST(true, 4, 1);
       else DLIA_ST(false, 4, 1);
       return;

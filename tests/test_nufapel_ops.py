@@ -328,7 +328,7 @@ MOE = [(50, 32, 6, 2, 24, 3, 2, 1.5, 1.0), (600, 128, 8, 2, 64, 2, 1, 2.0, 1.5),
        # row tiles of 32 as a weight stream: a token or two, whole and ragged pieces, K beyond one turn of the waves; then one and two
        # column tiles a wave with half tiles empty; then many tiles an expert with whole and masked pieces
        (1, 512, 3, 2, 88, 1, 1, 1.0, 7.0), (3, 1152, 4, 1, 1100, 1, 1, 1.0, 7.0), (40, 64, 6, 2, 4100, 1, 1, 1.0, 7.0), (60, 200, 2, 1, 64, 1, 1, 1.0, 7.0),
-       (300, 128, 2, 1, 256, 1, 1, 1.0, 7.0), (300, 72, 2, 1, 40, 1, 1, 1.0, 7.0),
+       (300, 128, 2, 1, 256, 1, 1, 1.0, 7.0), (300, 72, 2, 1, 40, 1, 1, 1.0, 7.0), (330, 192, 3, 1, 2048, 1, 1, 1.0, 7.0),
        # the wide blocks (a full round of them): gate and up with whole and masked pieces, then the down projection
        (450, 128, 2, 1, 1900, 1, 1, 1.0, 7.0), (450, 72, 2, 1, 1900, 1, 1, 1.0, 7.0), (450, 3700, 2, 1, 64, 1, 1, 1.0, 7.0), (450, 3700, 2, 1, 40, 1, 1, 1.0, 7.0)]
 
