@@ -390,7 +390,9 @@ __global__ __launch_bounds__(256) void multi_attention_kernel(
 // 16-entry tiles. Bound by what a CU takes from the caches (512 KB a round at key rows of 512 and four value heads of 128). Against a
 // wave per (token, head) with a key row per lane (16 bytes of 64 rows a load): 16 heads on key rows of 512, values 4 x 128, a prompt
 // of 300 / 2000 tokens 309 -> 77 / 9330 -> 1440 us, 24 sequences of 1000 tokens 944 -> 194, one 608 -> 184. Error against 64 bits,
-// mean over rows: 3.5e-7 -> 2.9e-7, 6.9e-7 -> 4.1e-7 (sums in four parts, and by rounds of 128 keys).
+// mean over rows: 3.5e-7 -> 2.9e-7, 6.9e-7 -> 4.1e-7 (sums in four parts, and by rounds of 128 keys). Below 16 keys, where the contexts of a
+// batch can only be for its first tokens, the two barriers and the copy of the queries cost 0.5 to 1 us more than that wave (8 heads of
+// 64 on two key rows, 6 keys: 7.7 -> 8.8 us), with a value head per head 2.5 to 4 (10 keys: 8.6 -> 11.9); at 31 keys 14.6 -> 10.
 template <int UPW>
 __global__ __launch_bounds__(512) void multi_rows_kernel(
     float* __restrict__ out, long ldo, const float* __restrict__ q, long ldq, int q_head, const float* __restrict__ kcache, int k_row,
@@ -412,10 +414,8 @@ __global__ __launch_bounds__(512) void multi_rows_kernel(
     for (int i = threadIdx.x; i < nr * dv; i += blockDim.x) out[(long)t * ldo + (long)h0 * dv + i] = 0.f;
     return;
   }
-  for (int i = threadIdx.x; i < 16 * d; i += blockDim.x) {
-    const int r = i / d, c = i % d;
-    qs[r * LQ + c] = r < nr ? q[(long)t * ldq + (long)(h0 + r) * q_head + c] * scale : 0.f;
-  }
+  for (int r = wave; r < 16; r += NW)
+    for (int c = lane; c < d; c += 64) qs[r * LQ + c] = r < nr ? q[(long)t * ldq + (long)(h0 + r) * q_head + c] * scale : 0.f;
   __syncthreads();
   const int* table = block_table + (long)slot * max_blocks;
   int lo = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
@@ -458,25 +458,29 @@ __global__ __launch_bounds__(512) void multi_rows_kernel(
       const int nsub = min(NW, (j_hi - j0) / 16 + 1);
       float p[NW][4], bm = -INFINITY;
 #pragma unroll
-      for (int sub = 0; sub < NW; ++sub)
+      for (int sub = 0; sub < NW; ++sub) {
+        if (sub >= nsub) break;                      // (a part round)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int key = sub * 16 + kq * 4 + i;
           p[sub][i] = B[key] >= 0 ? S[key * LS + r16] : -INFINITY;      // (keys beyond the last have no block)
           bm = fmaxf(bm, p[sub][i]);
         }
+      }
       bm = fmaxf(bm, __shfl_xor(bm, 16, 64));
       bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
       const float m_new = fmaxf(m, bm);
       const float corr = m == -INFINITY ? 0.f : expf(m - m_new);
       float add = 0.f;
 #pragma unroll
-      for (int sub = 0; sub < NW; ++sub)
+      for (int sub = 0; sub < NW; ++sub) {
+        if (sub >= nsub) break;                      // (a part round)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           p[sub][i] = p[sub][i] == -INFINITY ? 0.f : expf(p[sub][i] - m_new);
           add += p[sub][i];
         }
+      }
       l = l * corr + add;
       m = m_new;
 #pragma unroll
