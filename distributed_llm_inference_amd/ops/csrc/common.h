@@ -111,7 +111,7 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
 // restored: the kernels that use this have no other user of M0. Every piece counts in vmcnt.
 template <int NP>
 __device__ __forceinline__ void lds_dma_run(const void* const (&g)[NP], unsigned lds_addr) {
-  static_assert(NP == 1 || NP == 2 || NP == 3 || NP == 4 || NP == 6 || NP == 8, "pieces per run");
+  static_assert(NP == 1 || NP == 2 || NP == 3 || NP == 4 || NP == 8, "pieces per run");
   auto at = [&](int q, int off) { return reinterpret_cast<const char*>(g[q]) - off; };
   if constexpr (NP == 8)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
@@ -127,14 +127,6 @@ __device__ __forceinline__ void lds_dma_run(const void* const (&g)[NP], unsigned
                  "global_load_lds_dwordx4 %1, off\n\tglobal_load_lds_dwordx4 %2, off offset:1024\n\t"
                  "global_load_lds_dwordx4 %3, off offset:2048\n\tglobal_load_lds_dwordx4 %4, off offset:3072"
                  :: "s"(lds_addr), "v"(at(0, 0)), "v"(at(1, 1024)), "v"(at(2, 2048)), "v"(at(3, 3072)) : "memory", "m0");
-  else if constexpr (NP == 6)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
-                 "global_load_lds_dwordx4 %1, off offset:-2048\n\tglobal_load_lds_dwordx4 %2, off offset:-1024\n\t"
-                 "global_load_lds_dwordx4 %3, off\n\tglobal_load_lds_dwordx4 %4, off offset:1024\n\t"
-                 "global_load_lds_dwordx4 %5, off offset:2048\n\tglobal_load_lds_dwordx4 %6, off offset:3072"
-                 :: "s"(lds_addr + 2048), "v"(at(0, -2048)), "v"(at(1, -1024)), "v"(at(2, 0)), "v"(at(3, 1024)),
-                    "v"(at(4, 2048)), "v"(at(5, 3072))
-                 : "memory", "m0");
   else if constexpr (NP == 3)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
                  "global_load_lds_dwordx4 %1, off\n\tglobal_load_lds_dwordx4 %2, off offset:1024\n\t"
@@ -147,13 +139,19 @@ __device__ __forceinline__ void lds_dma_run(const void* const (&g)[NP], unsigned
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" :: "s"(lds_addr), "v"(at(0, 0)) : "memory", "m0");
 }
-// any number of pieces: runs of 8, then 4, 2, 1
+// waits until no more than N vector memory accesses of the wave (pieces among them) are on their way
+template <int N>
+__device__ __forceinline__ void wait_pieces() {
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
+}
+
+// any of these numbers of pieces: one run, or two of 8
 template <int NP>
 __device__ __forceinline__ void lds_dma_pieces(const void* const (&g)[NP], unsigned lds_addr) {
-  if constexpr (NP <= 4 || NP == 6 || NP == 8) {
+  if constexpr (NP <= 4 || NP == 8) {
     lds_dma_run<NP>(g, lds_addr);
   } else {
-    static_assert(NP == 16, "1, 2, 4, 8 or 16 pieces");
+    static_assert(NP == 16, "1 to 4, 8 or 16 pieces");
     const void* lo[8]; const void* hi[8];
 #pragma unroll
     for (int q = 0; q < 8; ++q) { lo[q] = g[q]; hi[q] = g[8 + q]; }

@@ -486,11 +486,6 @@ __global__ __launch_bounds__(64 * NW) void moe_stream_kernel(OT* __restrict__ ou
 // KIND 0: down; 1: gate and up; 2: up alone (the square of relu).
 constexpr int kBigStages = 6;
 
-template <int N>
-__device__ __forceinline__ void wait_pieces() {
-  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
-}
-
 template <int KIND, int BN>
 __global__ __launch_bounds__(512) void moe_big_kernel(bf16* __restrict__ act_out, float* __restrict__ y_out, const bf16* __restrict__ a,
                                                       const bf16* __restrict__ w0, const bf16* __restrict__ w1,
