@@ -661,8 +661,12 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(float* __restrict__ ou
   for (int r = 0; r < top; ++r) {
     const int row = pair_row[(long)t * top + r];
     const float w = wts[(long)t * top + r];
-    if (row < 0 && !x) continue;
-    const Unit<V> a = ldu<V>(row >= 0 ? y + (long)row * H + c : x + (long)t * ldx + c);
+    Unit<V> a;
+    if (row >= 0 || x) a = ldu<V>(row >= 0 ? y + (long)row * H + c : x + (long)t * ldx + c);
+    else {      // (zeros times the weight: one that is no number shows)
+#pragma unroll
+      for (int e = 0; e < V; ++e) a.v[e] = 0.f;
+    }
 #pragma unroll
     for (int e = 0; e < V; ++e) s.v[e] += w * a.v[e];
   }

@@ -386,6 +386,24 @@ def test_routed_ff_hip(T, W, E, top, ff, groups, keep, scale, limit, dt):
         _close(out, ref, 2e-4 if dt == "fp32" else 3e-2, f"row tiles of {tr}")
 
 
+@gpu
+@pytest.mark.parametrize("H", [64, 37])
+def test_weighted_sum_of_choices_without_a_row(H):
+    """A choice without a row adds its weight times the token, or times nothing: then a weight that is no number still shows."""
+    from distributed_llm_inference_amd import ops
+    K = ops.load()
+    y, x = _dev(torch.randn(4, H, generator=torch.Generator().manual_seed(1))), _dev(torch.randn(3, H, generator=torch.Generator().manual_seed(2)))
+    pair_row = torch.tensor([0, -1, 2, 3, -1, -1], dtype=torch.int32, device="cuda")
+    wts = torch.tensor([0.5, 2.0, 0.25, -1.0, float("nan"), 1.0], device="cuda")
+    out = torch.full((3, H), 9.0, device="cuda")
+    K.moe_combine(out, y, pair_row, wts, 2)
+    _close(out[:2], torch.stack([0.5 * y[0], 0.25 * y[2] - y[3]]), 1e-6)
+    assert bool(out[2].isnan().all())
+    K.moe_combine(out, y, pair_row, wts, 2, x)
+    _close(out[:2], torch.stack([0.5 * y[0] + 2.0 * x[0], 0.25 * y[2] - y[3]]), 1e-6)
+    assert bool(out[2].isnan().all())
+
+
 # ---- norms, gates, activations ---------------------------------------------------------------------------------------------
 def test_dyt_and_gelu_torch():
     g = torch.Generator().manual_seed(7)
