@@ -784,6 +784,11 @@ void gemm_any(Tensor out, const Tensor& x, const Tensor& w, OptTensor bias, int6
                 (int)K, x.stride(0), w.stride(0), out.stride(0), (int)epi, cur_stream());
 }
 
+// the kernel that gemm_any or gemm_blocks takes by its sizes where its rows are in whole 16-byte pieces (`dlia_gemm_any_form`)
+int64_t gemm_any_form(int64_t M, int64_t N, int64_t K, int64_t blocks, bool f32, int64_t epi) {
+  return dlia_gemm_any_form((int)M, (int)N, (int)K, (int)blocks, f32, (int)epi);
+}
+
 void gated_gelu(Tensor act, const Tensor& gu) {
   DLIA_ON_DEVICE_OF(act);
   check_bf16(act, "act"); check_bf16(gu, "gu"); check_rows(act, "act"); check_rows(gu, "gu");
@@ -925,6 +930,7 @@ TORCH_LIBRARY(dlia, m) {
   m.def("paged_attention_capped(Tensor(a!) out, Tensor q, Tensor kv_cache, Tensor q_start, Tensor ctx_lens, Tensor block_table, Tensor? slots, int max_q_len, int Hq, int Hkv, int D, float scale, int window, float softcap, Tensor? gate) -> ()");
   m.def("value_mix(Tensor(a!) qkv, Tensor(b!) vfirst, Tensor? lam, int mix, int v_off, int v_cols) -> ()");
   m.def("gemm_any(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int epi) -> ()");
+  m.def("gemm_any_form(int M, int N, int K, int blocks, bool f32, int epi) -> int");
   m.def("kv_store(Tensor qkv, Tensor(a!)? vfirst, Tensor? lam, int mix, Tensor(b!) kcache, Tensor(c!) vcache, Tensor tok_pos, Tensor tok_seq, Tensor block_table, int G, int d, int dv, int q_cols) -> ()");
   m.def("window_attention(Tensor(a!) out, Tensor qkv, Tensor kcache, Tensor vcache, Tensor tok_pos, Tensor tok_seq, Tensor block_table, int H, int G, int d, int dv, float scale, int window, bool sink) -> ()");
   m.def("short_conv(Tensor(a!) y, Tensor z, Tensor(b!) carry, Tensor taps, Tensor q_start, Tensor ctx, Tensor slots, int max_q) -> ()");
@@ -997,5 +1003,6 @@ TORCH_LIBRARY_IMPL(dlia, CompositeExplicitAutograd, m) {
   m.impl("large_gemm_kernel", &large_gemm_kernel);
   m.impl("gemm_ws_floats", &gemm_ws_floats);
   m.impl("gemm_config", &gemm_config);
+  m.impl("gemm_any_form", &gemm_any_form);
   m.impl("attention_ws_floats", &attention_ws_floats);
 }

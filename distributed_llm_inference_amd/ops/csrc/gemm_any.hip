@@ -347,46 +347,59 @@ __global__ __launch_bounds__(256) void gated_gelu_kernel(bf16* __restrict__ act,
   st16(act + (long)m * lda + c, pack8(g));
 }
 
+}  // namespace dlia
+
+// The kernel that a product takes where its rows are in whole 16-byte pieces: 0 the general one, 1 the weight stream, a tile of BM x BN with KG groups
+// of waves as 1000 BM + 10 BN + KG. The tile is the one whose rounds over the 256 CUs take least; what a round of each costs relative to 64 x
+// 64 is measured (fp32, K 4096: 77, 60, 45 and 25 us; 28 where a CU has one 32 x 32 tile to itself). bf16 chooses by the same numbers: of
+// 159 shapes (17 to 2048 rows, N and K 64 to 8192) of either type the tile taken was within 8 % of the best of the four, but for 400 rows,
+// N 8192, K 2048 (bf16 40 us where 64 x 64 takes 34, fp32 166 and 152).
+extern "C" int dlia_gemm_any_form(int M, int N, int K, int blocks, int f32, int epi) {
+  const int bk = f32 ? 32 : 64;
+  if (M <= 16 && K >= 8 * bk) return 1;
+  if (K % bk) return 0;
+  auto rounds = [&](int bm, int bn) { return (int)(((long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * blocks + 255) / 256); };
+  const int r66 = rounds(64, 64), r46 = rounds(48, 64), r36 = rounds(32, 64), r33 = rounds(32, 32);
+  const double t66 = r66, t46 = epi == 0 ? r46 * 0.77 : 1e30, t36 = r36 * 0.58, t33 = epi == 0 ? (r33 == 1 ? 0.36 : r33 * 0.33) : 1e30;
+  const bool split = K >= 16 * bk;             // (below that the rings are filled once or twice: nothing to hide)
+  const double best = r66 > 8 ? t66 : fmin(fmin(t66, t46), fmin(t36, t33));        // (with many rounds the last one is small change)
+  if (t66 == best) return split && r66 == 1 ? 64642 : 64641;
+  if (t36 == best) return split && r36 == 1 ? 32642 : 32641;
+  if (t46 == best) return split && r46 == 1 ? 48642 : 48641;
+  return split && r33 == 1 ? 32324 : split && r33 == 2 ? 32322 : 32321;
+}
+
+namespace dlia {
+
 #define DLIA_ANY_ARGS (OT*)C, (const T*)A, (const T*)W, bias, M, N, K, lda, ldw, ldc
 
 template <typename T, typename OT, int EPI>
 static void launch_any_epi(void* C, const void* A, const void* W, const float* bias, int M, int N, int K, long lda, long ldw, long ldc,
                            hipStream_t stream, int blocks, long a_step, long w_step, long c_step) {
-  constexpr int VEC = 16 / sizeof(T), BK = 128 / sizeof(T);
+  constexpr int VEC = 16 / sizeof(T);
   const int vec_ok = K % VEC == 0 && lda % VEC == 0 && ldw % VEC == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 &&
                      a_step % VEC == 0 && w_step % VEC == 0;
-  if (vec_ok && M <= 16 && K >= 8 * BK) {
+  const int form = vec_ok ? dlia_gemm_any_form(M, N, K, blocks, sizeof(T) == 4, EPI) : 0;
+  if (form == 1) {
     constexpr int NT = EPI == 0 ? 1 : 2;
     hipLaunchKernelGGL((gemm_any_rows_kernel<T, OT, EPI, NT>), dim3((N + 16 * NT - 1) / (16 * NT), 1, blocks), dim3(512), 0, stream, DLIA_ANY_ARGS, a_step, w_step, c_step);
     return;
   }
-  if (vec_ok && K % BK == 0) {
+  if (form) {
     const int wide = N % 8 == 0 && ldc % 8 == 0 && c_step % 8 == 0 && (uintptr_t)C % 16 == 0;
-    // The tile whose rounds over the 256 CUs take least; what a round of each costs relative to 64 x 64 is measured (fp32, K 4096:
-    // 77, 60, 45 and 25 us; 28 where a CU has one 32 x 32 tile to itself). bf16 chooses by the same numbers: of 159 shapes (17 to 2048
-    // rows, N and K 64 to 8192) of either type the tile taken was within 8 % of the best of the four, but for 400 rows, N 8192, K 2048
-    // (bf16 40 us where 64 x 64 takes 34, fp32 166 and 152).
-    auto rounds = [&](int bm, int bn) { return (int)(((long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * blocks + 255) / 256); };
-    const int r66 = rounds(64, 64), r46 = rounds(48, 64), r36 = rounds(32, 64), r33 = rounds(32, 32);
-    const double t66 = r66, t46 = EPI == 0 ? r46 * 0.77 : 1e30, t36 = r36 * 0.58, t33 = EPI == 0 ? (r33 == 1 ? 0.36 : r33 * 0.33) : 1e30;
-    const bool split = K >= 16 * BK;             // (below that the rings are filled once or twice: nothing to hide)
 #define DLIA_ANY_TILE(BM, BN, KG, E)                                                                                                       \
   hipLaunchKernelGGL((gemm_any_tile_kernel<T, OT, E, BM, BN, KG>), dim3((N + BN - 1) / BN, (M + BM - 1) / BM, blocks), dim3(256 * KG), 0, \
                      stream, DLIA_ANY_ARGS, wide, a_step, w_step, c_step)
-    const double best = r66 > 8 ? t66 : fmin(fmin(t66, t46), fmin(t36, t33));        // (with many rounds the last one is small change)
-    if (t66 == best) {
-      if (split && r66 == 1) DLIA_ANY_TILE(64, 64, 2, EPI);
-      else DLIA_ANY_TILE(64, 64, 1, EPI);
-    } else if (t36 == best) {
-      if (split && r36 == 1) DLIA_ANY_TILE(32, 64, 2, EPI);
-      else DLIA_ANY_TILE(32, 64, 1, EPI);
-    } else if (t46 == best) {
-      if (split && r46 == 1) DLIA_ANY_TILE(48, 64, 2, 0);
-      else DLIA_ANY_TILE(48, 64, 1, 0);
-    } else {
-      if (split && r33 == 1) DLIA_ANY_TILE(32, 32, 4, 0);
-      else if (split && r33 == 2) DLIA_ANY_TILE(32, 32, 2, 0);
-      else DLIA_ANY_TILE(32, 32, 1, 0);
+    switch (form) {
+      case 64642: DLIA_ANY_TILE(64, 64, 2, EPI); break;
+      case 64641: DLIA_ANY_TILE(64, 64, 1, EPI); break;
+      case 32642: DLIA_ANY_TILE(32, 64, 2, EPI); break;
+      case 32641: DLIA_ANY_TILE(32, 64, 1, EPI); break;
+      case 48642: DLIA_ANY_TILE(48, 64, 2, 0); break;
+      case 48641: DLIA_ANY_TILE(48, 64, 1, 0); break;
+      case 32324: DLIA_ANY_TILE(32, 32, 4, 0); break;
+      case 32322: DLIA_ANY_TILE(32, 32, 2, 0); break;
+      default: DLIA_ANY_TILE(32, 32, 1, 0);
     }
 #undef DLIA_ANY_TILE
     return;

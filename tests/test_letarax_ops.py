@@ -99,12 +99,25 @@ def test_gemm_any(K, dt, tol, M, N, Kd):
         close(out16, O.linear(x.cpu(), w.cpu()), 1e-2)
 
 
+TILED = [(1, 16, 512), (16, 34, 520), (15, 2050, 2056),               # the weight stream: its least K, K beyond whole chunks, a ragged last tile
+         (17, 36, 512), (33, 4100, 64), (300, 2048, 1024),            # tiles of 32 and 48 rows, one and several K groups, one stage
+         (64, 2048, 1088), (65, 64, 192), (301, 8192, 256), (200, 2056, 1024), (1000, 1030, 320),
+         (512, 2048, 1024), (500, 2040, 1088), (2000, 4100, 128), (1030, 4096, 320), (2336, 224, 1024)]      # tiles of 64 rows; two groups on 32 x 32
+GATED = [(9, 48, 1024), (40, 48, 1024), (70, 528, 320), (250, 2048, 1024), (250, 1040, 1088), (700, 4112, 192)]
+
+
+def test_gemm_any_shapes_reach_every_kernel():
+    from distributed_llm_inference_amd import ops
+    form = ops.load(build_if_missing=True).gemm_any_form
+    for f32 in (False, True):
+        assert {form(M, N, K, 1, f32, 0) for M, N, K in TILED} == {1, 64642, 64641, 48642, 48641, 32642, 32641, 32324, 32322, 32321}
+        assert {form(M, 2 * F, K, 1, f32, 1) for M, F, K in GATED} == {1, 64642, 64641, 32642, 32641}
+        assert form(40, 64, 100, 1, f32, 0) == 0
+
+
 @gpu
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("M,N,Kd", [
-    (1, 16, 512), (16, 34, 520), (15, 2050, 2056),               # the weight stream: its least K, K beyond whole chunks, a ragged last tile
-    (17, 36, 512), (33, 4100, 64), (300, 2048, 1024),            # tiles of 32 and 48 rows, one and several K groups, one stage
-    (64, 2048, 1088), (65, 64, 192), (301, 8192, 256), (200, 2056, 1024), (1000, 1030, 320)])
+@pytest.mark.parametrize("M,N,Kd", TILED)
 def test_gemm_any_tiles_and_weight_stream(K, dt, M, N, Kd):
     """A sum of K products in fp32, in any order: every entry within K roundings of the sum of the magnitudes (and, where the
     output is 16 bits wide, within one more of bf16)."""
@@ -125,7 +138,7 @@ def test_gemm_any_tiles_and_weight_stream(K, dt, M, N, Kd):
 
 @gpu
 @pytest.mark.parametrize("dt,tol", [(torch.float32, 5e-6), (torch.bfloat16, 1e-2)])
-@pytest.mark.parametrize("M,F,Kd", [(9, 48, 1024), (40, 48, 1024), (70, 528, 320)])
+@pytest.mark.parametrize("M,F,Kd", GATED)
 def test_gemm_any_gated_tiles(K, dt, tol, M, F, Kd):
     test_gemm_any_gated(K, dt, tol, M, F, Kd)
 

@@ -233,6 +233,38 @@ def test_recurrent_unit_hip(W, nb, taps, over_workgroups):
     close(torch.cat(got_b), ref_b, 5e-5)
 
 
+BLOCKS = [(16, 48, 512, 3), (9, 40, 520, 4), (40, 36, 128, 3), (300, 72, 1088, 5), (200, 448, 128, 32), (1900, 448, 128, 32), (500, 1020, 1024, 2)]
+
+
+def test_block_products_reach_streams_and_tiles():
+    from distributed_llm_inference_amd import ops
+    form = ops.load(build_if_missing=True).gemm_any_form
+    for f32 in (False, True):
+        assert {form(M, N, k, nb, f32, 0) for M, N, k, nb in BLOCKS} >= {1, 64642, 64641, 48641, 32324, 32321}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("dt,ot", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32), (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("M,N,k,nb", BLOCKS)
+def test_block_products_streams_and_tiles_hip(M, N, k, nb, dt, ot, bias):
+    """Every block against 64 bits, read from and written into rows with gaps between the blocks. A sum of k products in fp32, in any order:
+    within k roundings of the sum of the magnitudes (one more for the bias, and one of bf16 where the output is)."""
+    K, dev, xs, os_ = _K(), "cuda", k + 16, N + 8
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    x, w = torch.randn(M, nb * xs, device=dev, generator=g).to(dt), torch.randn(nb, N, k, device=dev, generator=g).to(dt)
+    b = torch.randn(nb * N, device=dev, generator=g) if bias else None
+    out = torch.full((M, nb * os_), 7.0, device=dev, dtype=ot)
+    K.gemm_blocks(out, x, w, b, xs, os_)
+    for i in range(nb):
+        xi, wi = x[:, i * xs:i * xs + k].double(), w[i].double()
+        bi = b[i * N:(i + 1) * N].double() if bias else torch.zeros(N, device=dev, dtype=F64)
+        ref, mag = xi @ wi.t() + bi, xi.abs() @ wi.abs().t() + bi.abs()
+        bound = (k + 1) * 2.0 ** -24 * mag + (2.0 ** -8 * ref.abs() if ot == torch.bfloat16 else 0.0)
+        assert bool(((out[:, i * os_:i * os_ + N].double() - ref).abs() <= bound).all()), i
+        assert bool((out[:, i * os_ + N:(i + 1) * os_] == 7.0).all()), i
+
+
 @pytest.mark.gpu
 def test_block_products_activation_and_scale_hip():
     K, dev = _K(), "cuda"
