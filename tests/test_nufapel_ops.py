@@ -387,6 +387,52 @@ def test_routed_ff_hip(T, W, E, top, ff, groups, keep, scale, limit, dt):
 
 
 @gpu
+@pytest.mark.parametrize("kind,N", [(0, 160), (0, 2112), (1, 104), (1, 1056), (2, 160), (2, 2112)])      # (128 and 256 weight rows a tile)
+@pytest.mark.parametrize("k", [32, 160, 192, 320, 352, 384, 416, 768])
+def test_experts_of_prompts_at_the_edges_of_their_ring(kind, N, k):
+    """The 128-row tiles of the three forms (0 down, 1 gate and up, 2 squared ReLU on weighted rows) on both widths, with K on either side of
+    where the ring's rounds of six steps begin and end. Pre-activations are sums of k products in fp32: within k + 1 roundings of the sum of
+    the magnitudes; what an activation makes of that (silu and its slope: 1.1) and, for 16-bit results, one more rounding."""
+    from distributed_llm_inference_amd import ops
+    K = ops.load()
+    T, top, E, tr = 1100, 2, 3, 128
+    g = torch.Generator(device="cuda").manual_seed(k + N)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    nt = (T * top + tr - 1) // tr + E
+    sel = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(t))[:top] for t in range(T)]).reshape(-1).int().cuda()
+    wts, row_w = torch.rand(T * top, device="cuda", generator=g) + 0.5, torch.full((tr * nt,), float("nan"), device="cuda")
+    tiles, row_tok, pair_row = (torch.full((n,), 77777, dtype=torch.int32, device="cuda") for n in (1 + nt, tr * nt, T * top))
+    K.moe_plan(tiles, row_tok, pair_row, sel, T * top, top, E, tr, wts, row_w)
+    bf = torch.bfloat16
+    x, w, w2 = r(tr * nt if kind == 0 else T, k).to(bf), (r(E, N, k) * k ** -0.5).to(bf), (r(E, N, k) * k ** -0.5).to(bf)
+    out = torch.full((tr * nt, N), 3.0, device="cuda", dtype=torch.float32 if kind == 0 else bf)
+    if kind == 0:
+        K.moe_down(out, x, w, tiles, row_tok, nt, tr)
+    else:
+        K.moe_up(out, x, w if kind == 1 else None, w2, tiles, row_tok, nt, 0.0, tr, row_w if kind == 2 else None)
+    tok, ex, eps = row_tok.long(), tiles[1:].long().repeat_interleave(tr), (k + 1) * 2.0 ** -24
+    assert int((tok[:int(tiles[0]) * tr] >= 0).sum()) == T * top
+    for e in range(E):
+        rows = torch.nonzero((tok >= 0) & (ex == e) & (torch.arange(tr * nt, device="cuda") < int(tiles[0]) * tr)).squeeze(1)
+        a = (x[rows] if kind == 0 else x[tok[rows]]).double()
+        if kind == 2:
+            a = a * row_w[rows].double()[:, None]
+        p, m = a @ w[e].double().t(), eps * (a.abs() @ w[e].double().abs().t())
+        q, n = a @ w2[e].double().t(), (eps + 2.0 ** -23) * (a.abs() @ w2[e].double().abs().t())
+        if kind == 0:
+            ref, bound = p, m
+        elif kind == 1:
+            s = p * torch.sigmoid(p)
+            ref, bound = s * q, 1.1 * m * (q.abs() + n) + s.abs() * n
+        else:
+            u = torch.relu(q)
+            ref, bound = u * u, 2 * u * n + n * n
+        if kind:
+            bound = bound + (2.0 ** -8 + 2.0 ** -20) * ref.abs()
+        assert bool(((out[rows].double() - ref).abs() <= bound).all()), e
+
+
+@gpu
 @pytest.mark.parametrize("H", [64, 37])
 def test_weighted_sum_of_choices_without_a_row(H):
     """A choice without a row adds its weight times the token, or times nothing: then a weight that is no number still shows."""
