@@ -653,6 +653,17 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(float* __restrict__ ou
                                                           const int* __restrict__ pair_row, const float* __restrict__ wts,
                                                           int H, int top, long ldo, const float* __restrict__ x, long ldx) {
   const int t = blockIdx.x, c = (blockIdx.y * 256 + threadIdx.x) * V;
+  if constexpr (V == 1) {      // (a loop: with many rows a workgroup each; 4096 rows of 1030 11.9 us, 14.4 with one for every 256 columns)
+    for (int i = c; i < H; i += gridDim.y * 256) {
+      float s = 0.f;
+      for (int r = 0; r < top; ++r) {
+        const int row = pair_row[(long)t * top + r];
+        s += wts[(long)t * top + r] * (row >= 0 ? y[(long)row * H + i] : (x ? x[(long)t * ldx + i] : 0.f));
+      }
+      out[(long)t * ldo + i] = s;
+    }
+    return;
+  }
   if (c >= H) return;
   Unit<V> s;
 #pragma unroll
@@ -818,7 +829,7 @@ extern "C" void dlia_moe_combine(float* out, const float* y, const int* pair_row
   if (H % 4 == 0 && ldo % 4 == 0 && ldx % 4 == 0 && dlia::al16_(out) && dlia::al16_(y) && dlia::al16_(x))
     hipLaunchKernelGGL(dlia::moe_combine_kernel<4>, dim3(T, (H + 1023) / 1024), dim3(256), 0, stream, out, y, pair_row, wts, H, top, ldo, x, ldx);
   else
-    hipLaunchKernelGGL(dlia::moe_combine_kernel<1>, dim3(T, (H + 255) / 256), dim3(256), 0, stream, out, y, pair_row, wts, H, top, ldo, x, ldx);
+    hipLaunchKernelGGL(dlia::moe_combine_kernel<1>, dim3(T, T > 1024 ? 1 : (H + 255) / 256), dim3(256), 0, stream, out, y, pair_row, wts, H, top, ldo, x, ldx);
 }
 
 extern "C" void dlia_moe_table_plan(int* tiles, int* row_tok, int* pair_row, const int* tables, const int* ids, const int* desc, int layers,

@@ -433,21 +433,22 @@ def test_experts_of_prompts_at_the_edges_of_their_ring(kind, N, k):
 
 
 @gpu
-@pytest.mark.parametrize("H", [64, 37])
-def test_weighted_sum_of_choices_without_a_row(H):
+@pytest.mark.parametrize("times", [1, 400])
+@pytest.mark.parametrize("H", [64, 37, 300, 1030])
+def test_weighted_sum_of_choices_without_a_row(H, times):
     """A choice without a row adds its weight times the token, or times nothing: then a weight that is no number still shows."""
     from distributed_llm_inference_amd import ops
     K = ops.load()
-    y, x = _dev(torch.randn(4, H, generator=torch.Generator().manual_seed(1))), _dev(torch.randn(3, H, generator=torch.Generator().manual_seed(2)))
-    pair_row = torch.tensor([0, -1, 2, 3, -1, -1], dtype=torch.int32, device="cuda")
-    wts = torch.tensor([0.5, 2.0, 0.25, -1.0, float("nan"), 1.0], device="cuda")
-    out = torch.full((3, H), 9.0, device="cuda")
-    K.moe_combine(out, y, pair_row, wts, 2)
-    _close(out[:2], torch.stack([0.5 * y[0], 0.25 * y[2] - y[3]]), 1e-6)
-    assert bool(out[2].isnan().all())
-    K.moe_combine(out, y, pair_row, wts, 2, x)
-    _close(out[:2], torch.stack([0.5 * y[0] + 2.0 * x[0], 0.25 * y[2] - y[3]]), 1e-6)
-    assert bool(out[2].isnan().all())
+    y, x = _dev(torch.randn(4, H, generator=torch.Generator().manual_seed(1))), _dev(torch.randn(3, H, generator=torch.Generator().manual_seed(2)).repeat(times, 1))
+    pair_row = torch.tensor([0, -1, 2, 3, -1, -1], dtype=torch.int32, device="cuda").repeat(times)
+    wts = torch.tensor([0.5, 2.0, 0.25, -1.0, float("nan"), 1.0], device="cuda").repeat(times)
+    for with_x in (False, True):
+        out = torch.full((3 * times, H), 9.0, device="cuda")
+        K.moe_combine(out, y, pair_row, wts, 2, *([x] if with_x else []))
+        first = 0.5 * y[0] + 2.0 * x[0] if with_x else 0.5 * y[0]
+        for t in range(0, 3 * times, 3):
+            _close(out[t:t + 2], torch.stack([first, 0.25 * y[2] - y[3]]), 1e-6)
+        assert bool(out[2::3].isnan().all())
 
 
 # ---- norms, gates, activations ---------------------------------------------------------------------------------------------
