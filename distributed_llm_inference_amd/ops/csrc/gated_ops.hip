@@ -189,7 +189,9 @@ __global__ __launch_bounds__(256) void softcap_kernel(float* __restrict__ z, lon
 extern "C" void dlia_embed_pos32(float* out, const int* ids, const int* pos, const void* table, const void* ptable, int f32, int T,
                                  int H, int vocab, int max_pos, hipStream_t stream) {
   if (T <= 0) return;
-  const int vec = H % 4 == 0 && dlia::al16_(out) && dlia::al16_(table) && dlia::al16_(ptable), nt = vec ? dlia::row_shape(T, H).threads : 128;
+  // (many wide rows, where the bytes are the time, keep the walk of single entries: 4096 rows of 8192 32 us, 39 in units of four)
+  const int vec = H % 4 == 0 && dlia::al16_(out) && dlia::al16_(table) && dlia::al16_(ptable) && !(T > 2048 && H > 4096);
+  const int nt = vec ? dlia::row_shape(T, H).threads : 128;
   if (f32)
     hipLaunchKernelGGL(dlia::embed_pos32_kernel<float>, dim3(T), dim3(nt), 0, stream, out, ids, pos, (const float*)table,
                        (const float*)ptable, H, vocab, max_pos, vec);
