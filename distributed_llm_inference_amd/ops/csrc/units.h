@@ -37,13 +37,14 @@ __device__ __forceinline__ Unit<4> ldu4(const bf16* p) {
 // ... (NR of them). Rows go through memory once in each direction; a walk of single floats that re-reads what it wrote is three
 // serial passes of 16 (width 4096, 256 threads) dependent accesses each, and with a workgroup per row of a decode step that chain,
 // not the bytes, is the kernel's time. Steps of few rows take as many threads as there are units (one unit each, one memory
-// latency per pass); with many rows the chip is full anyway and 4 units per thread keep the reductions short.
+// latency per pass); with many rows (more than `per_cu` threads a CU) the chip is full anyway and 4 units per thread keep the reductions short.
 struct RowShape { int threads, nr; };
-inline RowShape row_shape(int rows, int H) {
+inline RowShape row_shape(int rows, int H, int per_cu = 1024) {
   const int units = H / 4;
   int threads = 64;
-  if (rows <= 512) while (threads < units && threads < 1024) threads <<= 1;
-  else while (threads * 4 < units && threads < 1024) threads <<= 1;
+  while (threads < units && threads < 1024) threads <<= 1;
+  if (rows > 512 && (long)rows * threads > 256 * per_cu)
+    for (threads = 64; threads * 4 < units && threads < 1024;) threads <<= 1;
   return {threads, (units + threads - 1) / threads <= 1 ? 1 : 4};
 }
 inline bool row_fits(int H) { return H % 4 == 0 && H <= 16384; }

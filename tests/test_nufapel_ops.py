@@ -466,13 +466,19 @@ def test_row_kernels_widths_hip(W):
 
 
 @gpu
+@pytest.mark.parametrize("T,W", [(600, 1000), (1030, 256), (2100, 576), (600, 4096)])
+def test_row_kernels_many_rows_hip(T, W):
+    """One unit of a row a thread and four, on both sides of the lines by rows."""
+    test_row_kernels_hip(W, T)
+
+
+@gpu
 @pytest.mark.parametrize("W", [40, 256, 1000])
-def test_row_kernels_hip(W):
+def test_row_kernels_hip(W, T=13):
     from distributed_llm_inference_amd import ops
     K = ops.load()
     g = torch.Generator().manual_seed(8)
     rn = lambda *s: torch.randn(*s, generator=g, dtype=F64)
-    T = 13
     x, ya, yb, gl = rn(T, W) * 2, rn(T, W), rn(T, W) * 5, rn(T, W + 8)
     wa, wb, gb, step, nw, nb = (rn(W) for _ in range(6))
     y = 0.5 * (O.rms_unit(ya, 1e-5) * wa + O.rms_unit(yb, 1e-5) * wb)
