@@ -360,6 +360,7 @@ extern "C" int dlia_gemm_any_form(int M, int N, int K, int blocks, int f32, int 
   if (K % bk) return 0;
   auto rounds = [&](int bm, int bn) { return (int)(((long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * blocks + 255) / 256); };
   const int r66 = rounds(64, 64), r46 = rounds(48, 64), r36 = rounds(32, 64), r33 = rounds(32, 32);
+  if (K == bk && r66 >= 4) return 0;           // (a single stage and the chip full: 32 products of 1000 rows, N 448, K 64 29.9 us, the general kernel 26.5)
   const double t66 = r66, t46 = epi == 0 ? r46 * 0.77 : 1e30, t36 = r36 * 0.58, t33 = epi == 0 ? (r33 == 1 ? 0.36 : r33 * 0.33) : 1e30;
   const bool split = K >= 16 * bk;             // (below that the rings are filled once or twice: nothing to hide)
   const double best = r66 > 8 ? t66 : fmin(fmin(t66, t46), fmin(t36, t33));        // (with many rounds the last one is small change)
