@@ -30,6 +30,7 @@
 #include "common.h"
 #include "frag.h"
 #include <type_traits>
+#include <algorithm>
 #include "units.h"
 #include "launch.h"
 
@@ -738,10 +739,10 @@ static void launch_moe_down(float* y, const void* act, const void* wd, const int
 template <int KIND>
 static void launch_moe_big(void* act, float* y, const void* a, const void* w0, const void* w1, const int* tiles, const int* row_tok,
                            int max_tiles, int experts, int N, int K, long lda, long ldo, float limit, const float* row_w, hipStream_t stream) {
-  // 256 or 128 weight rows by the rounds over the 256 CUs that about max_tiles - experts / 2 row tiles make (a round of the narrow
-  // form costs 0.6 of one of the wide form: 520 tokens, 2 of 8 experts, width and expert 2048: gate and up 41 us wide and 54
+  // 256 or 128 weight rows by the rounds over the 256 CUs that about max_tiles - experts / 2 row tiles make, one an expert at least (a round of
+  // the narrow form costs 0.6 of one of the wide form: 520 tokens, 2 of 8 experts, width and expert 2048: gate and up 41 us wide and 54
   // narrow, down 33 and 23)
-  const int cols = KIND == 1 ? 2 * N : N, likely = max_tiles - experts / 2 - 1 > 0 ? max_tiles - experts / 2 - 1 : 1;
+  const int cols = KIND == 1 ? 2 * N : N, likely = std::max(max_tiles - experts / 2 - 1, experts);
   const int r256 = ((cols + 255) / 256 * likely + 255) / 256, r128 = ((cols + 127) / 128 * likely + 255) / 256;
 #define DLIA_BIG(BN)                                                                                                                    \
   hipLaunchKernelGGL((dlia::moe_big_kernel<KIND, BN>), dim3((N + (KIND == 1 ? BN / 2 : BN) - 1) / (KIND == 1 ? BN / 2 : BN) * max_tiles), \
