@@ -423,8 +423,8 @@ __global__ __launch_bounds__(64 * NW) void moe_stream_kernel(OT* __restrict__ ou
     };
     // Piece c of the wave's share; each workgroup begins elsewhere in K and goes round. A K of no more pieces than waves stays with
     // one of them: its sums are then formed in the order of the wide blocks, so that for such K (up to 512 in 16 bits, 128 in 32) a row's
-    // result does not depend on which of the two its step took; for longer K it may, in the last bits. It costs next to nothing where a
-    // launch is all there is (4.5 to 5 us either way) and up to 1.7 of 8 us in the gated fp32 form, 1.7 of 16 in the 16-bit one (512 x 512).
+    // result does not depend on which of the two its step took; for longer K it may, in the last bits. (Steps of few workgroups alone:
+    // there a launch is all there is, 4.5 to 5 us either way.)
     const int total = (K + CH - 1) / CH, turn = total > NW ? (blockIdx.x * 4 + e) % total : 0, step = total > NW ? NW : 1;
     if (wave >= step) return;
     auto at = [&](int c) { const int k = c + turn; return (k >= total ? k - total : k) * CH; };
@@ -753,6 +753,12 @@ static void launch_moe_big(void* act, float* y, const void* a, const void* w0, c
 #undef DLIA_BIG
 }
 
+// About how many row tiles of 32 a step has: its pairs' and half a tile an expert, one an expert at least where there are four pairs for each
+static int likely_tiles(int max_tiles, int experts) {
+  const int most = max_tiles - experts;
+  return std::max(std::min(max_tiles - experts / 2, 32 * most), 8 * most >= experts ? experts : 0);
+}
+
 template <typename T, typename OT, int KIND>
 static void launch_moe_stream(OT* out, const T* x, const T* w0, const T* w1, const int* tiles, const int* row_tok, int max_tiles, int experts, int N,
                               int K, long ldx, long ldo, float limit, int ok, const float* row_w, hipStream_t stream) {
@@ -764,7 +770,7 @@ static void launch_moe_stream(OT* out, const T* x, const T* w0, const T* w1, con
   hipLaunchKernelGGL((dlia::moe_stream_kernel<T, OT, KIND, FAST, 4, U, NJ>), dim3((N + 16 * NJ - 1) / (16 * NJ), max_tiles), dim3(256), 0, \
                      stream, out, x, w0, w1, tiles, row_tok, N, K, ldx, ldo, limit, ok, row_w)
   if constexpr (KIND == 1 && sizeof(T) == 2)
-    if (max_tiles - experts <= 1 || (long)(N + 31) / 32 * (max_tiles - experts / 2) < 768) {
+    if (max_tiles - experts <= 1 || (long)(N + 31) / 32 * likely_tiles(max_tiles, experts) < 768) {
       if (ok && K % (256 / (int)sizeof(T)) == 0) DLIA_ST(true, 4, 1);
       else DLIA_ST(false, 4, 1);
       return;
@@ -784,6 +790,42 @@ extern "C" int dlia_moe_wide(int max_tiles, int experts, int cols, int down) {
   return max_tiles - experts > 4 * experts && blocks * 10 > rounds * 256 * 9 && (down || rounds == 1);
 }
 
+// Steps of a short K (kind as in the stream, which leaves such a K to one of a workgroup's four waves and pays for whole pieces): column blocks of
+// 64 (1), or the wide ones (2) where experts have more than four tiles, as soon as the stream's workgroups are more than a round or two; before
+// that its launch is the shorter one. Stream against blocks, 314 shapes of K up to 512 bf16, 128 fp32, by the stream's workgroups as estimated here:
+// gated, above 512 0.93 to 3.7 of the blocks' time, on average 1.35 (32 tokens, one of 32 experts of 4096, K 40: 24 against 6.5 us; 1400 tokens, two of 16
+// of 3584, K 200: 105 against 50), in 16 bits 0.76 to 0.9 up to 512 and with whole pieces up to 1024; the other kinds, from 1024 on, 0.92 to 1.39 where K is at most 192 bytes, down
+// 0.66 to 1.0 above that, squared ReLU 0.98 to 1.25 with masked pieces; with many tiles the wide ones up to 256 in fp32 too: gated, K 256, 111 against 99 us, down, K 64, 35 against 27.
+extern "C" int dlia_moe_short(int max_tiles, int experts, int cols, int K, int f32, int kind) {
+  const int bytes = K * (f32 ? 4 : 2), most = max_tiles - experts;
+  if (bytes > 1024) return 0;
+  const long tiles = likely_tiles(max_tiles, experts);
+  const bool narrow = kind == 1 && !f32 && (most <= 1 || (cols + 31) / 32 * tiles < 768);
+  const long groups = (narrow ? (cols + 15) / 16 : (cols + 31) / 32) * tiles;
+  if (most > 4 * experts && groups >= 4096 && (kind || bytes <= 512)) return 2;
+  if (f32 && bytes > 512) return 0;
+  if (kind == 1 ? groups <= (narrow && bytes % 256 == 0 ? 1024 : 512) : groups < 1024 || (bytes > 192 && (kind == 0 || bytes % 128 == 0))) return 0;
+  return most > 4 * experts ? 2 : 1;
+}
+
+template <typename T>
+static void moe_up_rows(T* act, const T* x, const T* wg, const T* wu, const int* tiles, const int* row_tok, int max_tiles, int experts, int F, int K,
+                        long ldx, long lda, float limit, int ok, const float* row_w, hipStream_t stream) {
+  const int few = dlia_moe_short(max_tiles, experts, F, K, sizeof(T) == 4, wg ? 1 : 2);
+  if (few == 1) launch_moe_up<T, T, 1>(act, x, wg, wu, tiles, row_tok, max_tiles, F, K, ldx, lda, limit, ok, row_w, stream);
+  else if (few || dlia_moe_wide(max_tiles, experts, F, 0)) launch_moe_up<T, T, 2>(act, x, wg, wu, tiles, row_tok, max_tiles, F, K, ldx, lda, limit, ok, row_w, stream);
+  else if (wg) launch_moe_stream<T, T, 1>(act, x, wg, wu, tiles, row_tok, max_tiles, experts, F, K, ldx, lda, limit, ok, row_w, stream);
+  else launch_moe_stream<T, T, 2>(act, x, wu, nullptr, tiles, row_tok, max_tiles, experts, F, K, ldx, lda, limit, ok, row_w, stream);
+}
+template <typename T>
+static void moe_down_rows(float* y, const T* act, const T* wd, const int* tiles, const int* row_tok, int max_tiles, int experts, int H, int F,
+                          long lda, int ok, hipStream_t stream) {
+  const int few = dlia_moe_short(max_tiles, experts, H, F, sizeof(T) == 4, 0);
+  if (few == 1) launch_moe_down<T, 1>(y, act, wd, tiles, row_tok, max_tiles, H, F, lda, ok, stream);
+  else if (few || dlia_moe_wide(max_tiles, experts, H, 1)) launch_moe_down<T, 4>(y, act, wd, tiles, row_tok, max_tiles, H, F, lda, ok, stream);
+  else launch_moe_stream<T, float, 0>(y, act, wd, nullptr, tiles, row_tok, max_tiles, experts, H, F, lda, (long)H, 0.f, ok, nullptr, stream);
+}
+
 extern "C" void dlia_moe_up(void* act, const void* x, const void* wg, const void* wu, int f32, const int* tiles, const int* row_tok,
                             int max_tiles, int experts, int F, int K, long ldx, long lda, float limit, int tile_rows, const float* row_w,
                             hipStream_t stream) {
@@ -795,15 +837,11 @@ extern "C" void dlia_moe_up(void* act, const void* x, const void* wg, const void
   }
   const int vec = f32 ? 4 : 8;
   const int ok = K % vec == 0 && ldx % vec == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)wg % 16 == 0 && (uintptr_t)wu % 16 == 0;
-  if (f32) {
-    if (dlia_moe_wide(max_tiles, experts, F, 0)) launch_moe_up<float, float, 2>(act, x, wg, wu, tiles, row_tok, max_tiles, F, K, ldx, lda, limit, ok, row_w, stream);
-    else if (wg) launch_moe_stream<float, float, 1>((float*)act, (const float*)x, (const float*)wg, (const float*)wu, tiles, row_tok, max_tiles, experts, F, K, ldx, lda, limit, ok, row_w, stream);
-    else launch_moe_stream<float, float, 2>((float*)act, (const float*)x, (const float*)wu, nullptr, tiles, row_tok, max_tiles, experts, F, K, ldx, lda, limit, ok, row_w, stream);
-  } else {
-    if (dlia_moe_wide(max_tiles, experts, F, 0)) launch_moe_up<dlia::bf16, dlia::bf16, 2>(act, x, wg, wu, tiles, row_tok, max_tiles, F, K, ldx, lda, limit, ok, row_w, stream);
-    else if (wg) launch_moe_stream<dlia::bf16, dlia::bf16, 1>((dlia::bf16*)act, (const dlia::bf16*)x, (const dlia::bf16*)wg, (const dlia::bf16*)wu, tiles, row_tok, max_tiles, experts, F, K, ldx, lda, limit, ok, row_w, stream);
-    else launch_moe_stream<dlia::bf16, dlia::bf16, 2>((dlia::bf16*)act, (const dlia::bf16*)x, (const dlia::bf16*)wu, nullptr, tiles, row_tok, max_tiles, experts, F, K, ldx, lda, limit, ok, row_w, stream);
-  }
+  if (f32)
+    moe_up_rows((float*)act, (const float*)x, (const float*)wg, (const float*)wu, tiles, row_tok, max_tiles, experts, F, K, ldx, lda, limit, ok, row_w, stream);
+  else
+    moe_up_rows((dlia::bf16*)act, (const dlia::bf16*)x, (const dlia::bf16*)wg, (const dlia::bf16*)wu, tiles, row_tok, max_tiles, experts, F, K, ldx, lda,
+                limit, ok, row_w, stream);
 }
 
 extern "C" void dlia_moe_down(float* y, const void* act, const void* wd, int f32, const int* tiles, const int* row_tok,
@@ -815,13 +853,8 @@ extern "C" void dlia_moe_down(float* y, const void* act, const void* wd, int f32
   }
   const int vec = f32 ? 4 : 8;
   const int ok = F % vec == 0 && lda % vec == 0 && (uintptr_t)act % 16 == 0 && (uintptr_t)wd % 16 == 0;
-  if (f32) {
-    if (dlia_moe_wide(max_tiles, experts, H, 1)) launch_moe_down<float, 4>(y, act, wd, tiles, row_tok, max_tiles, H, F, lda, ok, stream);
-    else launch_moe_stream<float, float, 0>(y, (const float*)act, (const float*)wd, nullptr, tiles, row_tok, max_tiles, experts, H, F, lda, (long)H, 0.f, ok, nullptr, stream);
-  } else {
-    if (dlia_moe_wide(max_tiles, experts, H, 1)) launch_moe_down<dlia::bf16, 4>(y, act, wd, tiles, row_tok, max_tiles, H, F, lda, ok, stream);
-    else launch_moe_stream<dlia::bf16, float, 0>(y, (const dlia::bf16*)act, (const dlia::bf16*)wd, nullptr, tiles, row_tok, max_tiles, experts, H, F, lda, (long)H, 0.f, ok, nullptr, stream);
-  }
+  if (f32) moe_down_rows(y, (const float*)act, (const float*)wd, tiles, row_tok, max_tiles, experts, H, F, lda, ok, stream);
+  else moe_down_rows(y, (const dlia::bf16*)act, (const dlia::bf16*)wd, tiles, row_tok, max_tiles, experts, H, F, lda, ok, stream);
 }
 
 extern "C" void dlia_moe_combine(float* out, const float* y, const int* pair_row, const float* wts, int T, int H, int top, long ldo,

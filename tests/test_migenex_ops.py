@@ -183,7 +183,7 @@ def test_activations_hip(dtype, F):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("H,ff,experts,top,T", [(40, 24, 5, 2, 33), (64, 32, 3, 3, 7), (36, 10, 1, 1, 20), (128, 64, 8, 2, 700), (96, 160, 6, 1, 1100), (24, 16, 40, 4, 50)])
+@pytest.mark.parametrize("H,ff,experts,top,T", [(40, 24, 5, 2, 33), (64, 32, 3, 3, 7), (36, 10, 1, 1, 20), (128, 64, 8, 2, 700), (96, 160, 6, 1, 1100), (24, 16, 40, 4, 50), (40, 3000, 16, 2, 64), (32, 3000, 16, 2, 64)])
 def test_routed_feed_forward_hip(dtype, H, ff, experts, top, T):
     """route -> plan with the weights at the rows -> the gateless experts on weighted inputs -> sum in the boundary kernel, with a
     shared expert; both tile sizes; buffers full of garbage beforehand."""

@@ -330,7 +330,18 @@ MOE = [(50, 32, 6, 2, 24, 3, 2, 1.5, 1.0), (600, 128, 8, 2, 64, 2, 1, 2.0, 1.5),
        (1, 512, 3, 2, 88, 1, 1, 1.0, 7.0), (3, 1152, 4, 1, 1100, 1, 1, 1.0, 7.0), (40, 64, 6, 2, 4100, 1, 1, 1.0, 7.0), (60, 200, 2, 1, 64, 1, 1, 1.0, 7.0),
        (300, 128, 2, 1, 256, 1, 1, 1.0, 7.0), (300, 72, 2, 1, 40, 1, 1, 1.0, 7.0), (330, 192, 3, 1, 2048, 1, 1, 1.0, 7.0),
        # the wide blocks (a full round of them): gate and up with whole and masked pieces, then the down projection
-       (450, 128, 2, 1, 1900, 1, 1, 1.0, 7.0), (450, 72, 2, 1, 1900, 1, 1, 1.0, 7.0), (450, 3700, 2, 1, 64, 1, 1, 1.0, 7.0), (450, 3700, 2, 1, 40, 1, 1, 1.0, 7.0)]
+       (450, 128, 2, 1, 1900, 1, 1, 1.0, 7.0), (450, 72, 2, 1, 1900, 1, 1, 1.0, 7.0), (450, 3700, 2, 1, 64, 1, 1, 1.0, 7.0), (450, 3700, 2, 1, 40, 1, 1, 1.0, 7.0),
+       # a short K and many tiles: column blocks of 64, masked and whole steps, up and down
+       (64, 40, 16, 2, 1500, 1, 1, 1.0, 7.0), (64, 64, 16, 2, 1500, 1, 1, 1.0, 7.0), (64, 4100, 16, 2, 40, 1, 1, 1.0, 7.0), (64, 4096, 16, 2, 32, 1, 1, 1.0, 7.0)]
+
+
+@pytest.mark.parametrize("T,E,top,cols,K,f32,kind,form", [
+    (64, 16, 2, 1500, 40, False, 1, 1), (64, 16, 2, 1500, 64, True, 1, 1), (64, 16, 2, 900, 64, True, 1, 0), (64, 16, 2, 4100, 40, False, 0, 1), (64, 16, 2, 4100, 40, True, 0, 1), (64, 16, 2, 3000, 40, True, 2, 1),
+    (32, 32, 1, 4096, 40, False, 1, 1), (200, 64, 2, 3584, 200, False, 1, 1), (1400, 16, 2, 3584, 200, False, 1, 2), (800, 4, 2, 3584, 256, True, 1, 2),
+    (2048, 8, 4, 1024, 64, True, 0, 2), (16, 32, 1, 512, 512, False, 1, 0), (4, 2, 1, 4096, 256, False, 1, 0), (800, 32, 2, 3584, 384, False, 0, 0), (64, 8, 2, 3584, 4096, False, 1, 0)])
+def test_experts_short_k_takes_the_blocks_where_they_measured_faster(T, E, top, cols, K, f32, kind, form):
+    from distributed_llm_inference_amd import ops
+    assert ops.load(build_if_missing=True).moe_short((T * top + 31) // 32 + E, E, cols, K, f32, kind) == form
 
 
 @pytest.mark.parametrize("T,E,top,cols,down,wide", [
