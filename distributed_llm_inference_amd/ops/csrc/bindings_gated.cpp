@@ -328,6 +328,11 @@ int64_t moe_short(int64_t max_tiles, int64_t experts, int64_t cols, int64_t K, b
   return dlia_moe_short((int)max_tiles, (int)experts, (int)cols, (int)K, f32, (int)kind);
 }
 
+// whether a step in row tiles of 128 runs in pairs of them (cols: weight rows, gate and up together)
+bool moe_pairs(int64_t max_tiles, int64_t experts, int64_t cols, int64_t K) {
+  return dlia_moe_pairs((int)max_tiles, (int)experts, (int)cols, (int)K) != 0;
+}
+
 void moe_down(Tensor y, const Tensor& act, const Tensor& wd, const Tensor& tiles, const Tensor& row_tok, int64_t max_tiles, int64_t tile_rows) {
   DLIA_ON_DEVICE_OF(y);
   check_f32(y, "y"); check_act(act, "act"); check_mat(act, "act"); check_act(wd, "wd"); check_i32(tiles, "tiles"); check_i32(row_tok, "row_tok");
@@ -371,6 +376,7 @@ TORCH_LIBRARY_FRAGMENT(dlia, m) {
   m.def("moe_route_plan(Tensor(a!) sel, Tensor(b!) wts, Tensor logits, int top, int groups, int keep, float scale, Tensor? correction, bool softmax, int group_rank, bool renorm, Tensor(c!) tiles, Tensor(d!) row_tok, Tensor(e!) pair_row, int E, int tile_rows, Tensor(f!)? row_w) -> ()");
   m.def("moe_up(Tensor(a!) act, Tensor x, Tensor? wg, Tensor wu, Tensor tiles, Tensor row_tok, int max_tiles, float limit, int tile_rows, Tensor? row_w=None) -> ()");
   m.def("moe_wide(int max_tiles, int experts, int cols, bool down) -> bool");
+  m.def("moe_pairs(int max_tiles, int experts, int cols, int K) -> bool");
   m.def("moe_short(int max_tiles, int experts, int cols, int K, bool f32, int kind) -> int");
   m.def("moe_down(Tensor(a!) y, Tensor act, Tensor wd, Tensor tiles, Tensor row_tok, int max_tiles, int tile_rows) -> ()");
   m.def("moe_combine(Tensor(a!) out, Tensor y, Tensor pair_row, Tensor wts, int top, Tensor? x=None) -> ()");
@@ -396,5 +402,6 @@ TORCH_LIBRARY_IMPL(dlia, CompositeExplicitAutograd, m) {
   m.impl("state_scan_blocks", &state_scan_blocks);
   m.impl("scan_route", &scan_route);
   m.impl("moe_wide", &moe_wide);
+  m.impl("moe_pairs", &moe_pairs);
   m.impl("moe_short", &moe_short);
 }

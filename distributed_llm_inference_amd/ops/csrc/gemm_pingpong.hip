@@ -46,6 +46,7 @@
 #include "common.h"
 #include "gemm_common.h"
 #include "launch.h"
+#include "pingpong.h"
 
 // Diagnostic builds only (bench/pp_ablate.py): PP_ABL is a mask of parts of the main loop to leave
 // out — 1 DMA issue, 2 fragment reads, 4 barriers, 8 MFMAs. Results are then wrong on purpose; what
@@ -56,35 +57,10 @@
 
 namespace dlia {
 
-constexpr int kPPThreads = 512;
-constexpr int kPPHalf = 16384;                   // bytes of one half-tile
 constexpr int kPPLds = 8 * kPPHalf;              // 2 K-tiles x {A0, B0, B1, A1}
 constexpr int kPPSlab = 256 * 256;               // floats of one partial tile
 constexpr int kPPCounters = 4096;                // counter words at the end of the workspace (two per output tile)
 
-// Two 1 KiB pieces, global -> LDS, under ONE setting of M0: lane l of piece i lands at
-// lds_addr + 1024 i + 16 l and reads g_i + 16 bytes per lane as set up by the caller. The second
-// piece uses the instruction's immediate offset, which advances the global AND the LDS address, so
-// its source pointer is passed 1024 bytes low. Why one setting: a write to M0 waits until every
-// earlier LDS-DMA instruction of the wave has read it, ~180 cycles after issue — with M0 written
-// (and restored) around every piece a wave issues one piece per ~180 cycles and a CU takes 32 bytes
-// per cycle from L2, with four pieces per setting 63 (bench/l2_lds_bw.hip). M0 is not restored:
-// nothing else in this kernel uses it (no other LDS-DMA, no indexed register access).
-__device__ __forceinline__ void pp_dma_pair(const void* g0, const void* g1_minus_1k, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\t"
-               "global_load_lds_dwordx4 %2, off offset:1024"
-               :: "s"(lds_addr), "v"(g0), "v"(g1_minus_1k) : "memory", "m0");
-}
-template <int N>
-__device__ __forceinline__ void pp_wait_vm() {
-  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-__device__ __forceinline__ void pp_barrier() {
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-}
 __device__ __forceinline__ void pp_loop_barrier() {
   if constexpr (!(PP_ABL & 4)) pp_barrier();
   else __builtin_amdgcn_sched_barrier(0);

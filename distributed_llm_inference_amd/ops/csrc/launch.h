@@ -200,6 +200,9 @@ void dlia_moe_route_plan(int* sel, float* wts, const float* logits, long ld, int
 // wg null: experts without a gate, act = relu(x . Wu)^2; row_w: what the rows' inputs are multiplied by
 void dlia_moe_up(void* act, const void* x, const void* wg, const void* wu, int f32, const int* tiles, const int* row_tok,
                  int max_tiles, int experts, int F, int K, long ldx, long lda, float limit, int tile_rows, const float* row_w, hipStream_t stream);
+int dlia_moe_pairs(int max_tiles, int experts, int cols, int K);
+void dlia_moe_pingpong(int kind, void* act, float* y, const void* a, const void* w0, const void* w1, const int* tiles, const int* row_tok,
+                       int max_tiles, int experts, int N, int K, long lda, long ldo, float limit, const float* row_w, hipStream_t stream);
 int dlia_moe_short(int max_tiles, int experts, int cols, int K, int f32, int kind);
 int dlia_moe_wide(int max_tiles, int experts, int cols, int down);
 void dlia_moe_down(float* y, const void* act, const void* wd, int f32, const int* tiles, const int* row_tok, int max_tiles, int experts,

@@ -26,8 +26,9 @@
 //   moe_combine  out[t, :] = sum over the token's choices of weight * y[row, :], in the order of the choices (fp32); a choice
 //                without a row (an identity expert) contributes weight * x[t, :].
 // Operands are bf16 (16x16x32 MFMA) or fp32 (16x16x4 MFMA, true 32-bit): fragments read straight from the K-contiguous rows in steps
-// with few rows, through an LDS ring in prompt steps (128-row tiles).
+// with few rows, through an LDS ring in prompt steps (128-row tiles; in pairs of an expert's tiles where that fills the chip, moe_pingpong.hip).
 #include "common.h"
+#include "expert_act.h"
 #include "frag.h"
 #include <type_traits>
 #include <algorithm>
@@ -39,17 +40,6 @@ namespace dlia {
 constexpr int kMoeMaxExperts = 256;
 constexpr int kMoeRows = 32;           // rows of a plan tile (steps with few rows), kMoeBigRows for the LDS-tiled kernel
 constexpr int kMoeBigRows = 128;
-
-// An expert's activation from its gate and up pre-activations.
-__device__ __forceinline__ float expert_act(float g, float u, float limit) {
-  if (limit > 0.f) {
-    const float gv = fminf(g, limit), uv = fminf(fmaxf(u, -limit), limit);
-    return gv / (1.f + expf(-1.702f * gv)) * (uv + 1.f);
-  }
-  return g / (1.f + expf(-g)) * u;
-}
-
-__device__ __forceinline__ float relu2(float u) { const float r = fmaxf(u, 0.f); return r * r; }
 
 __device__ __forceinline__ void route_token(int t, int* __restrict__ sel, float* __restrict__ wts, const float* __restrict__ logits, long ld,
                                             int E, int top, int groups, int keep, float scale, const float* __restrict__ corr, int softmax,
@@ -743,6 +733,10 @@ static void launch_moe_big(void* act, float* y, const void* a, const void* w0, c
   // the narrow form costs 0.6 of one of the wide form: 520 tokens, 2 of 8 experts, width and expert 2048: gate and up 41 us wide and 54
   // narrow, down 33 and 23)
   const int cols = KIND == 1 ? 2 * N : N, likely = std::max(max_tiles - experts / 2 - 1, experts);
+  if (dlia_moe_pairs(max_tiles, experts, cols, K)) {
+    dlia_moe_pingpong(KIND, act, y, a, w0, w1, tiles, row_tok, max_tiles, experts, N, K, lda, ldo, limit, row_w, stream);
+    return;
+  }
   const int r256 = ((cols + 255) / 256 * likely + 255) / 256, r128 = ((cols + 127) / 128 * likely + 255) / 256;
 #define DLIA_BIG(BN)                                                                                                                    \
   hipLaunchKernelGGL((dlia::moe_big_kernel<KIND, BN>), dim3((N + (KIND == 1 ? BN / 2 : BN) - 1) / (KIND == 1 ? BN / 2 : BN) * max_tiles), \

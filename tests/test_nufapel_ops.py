@@ -443,6 +443,62 @@ def test_experts_of_prompts_at_the_edges_of_their_ring(kind, N, k):
         assert bool(((out[rows].double() - ref).abs() <= bound).all()), e
 
 
+@pytest.mark.parametrize("T,E,top,cols,K,pairs", [
+    (1900, 8, 2, 7168, 4096, True), (1900, 8, 2, 4096, 3584, True), (800, 8, 2, 7168, 4096, True), (800, 8, 2, 4096, 3584, False),        # 343 against 242 us in pairs, 151 / 109, 178 / 129, 81 / 86
+    (1900, 8, 1, 3584, 4096, False), (1900, 8, 1, 4096, 3584, True), (1900, 8, 2, 2048, 1792, False), (1900, 8, 2, 4096, 3616, False),    # 79 / 82, 132 / 86, 45 / 50, ...
+    (1900, 32, 2, 2048, 2048, True), (885, 4, 2, 2048, 1024, False), (1062, 8, 4, 7168, 1024, True), (1062, 8, 4, 1024, 3584, False)])    # 97 / 63, 17 / 30, 123 / 103, 56 / 71
+def test_experts_tiles_in_pairs_where_they_measured_faster(T, E, top, cols, K, pairs):
+    from distributed_llm_inference_amd import ops
+    assert ops.load(build_if_missing=True).moe_pairs((T * top + 127) // 128 + E, E, cols, K) == pairs
+
+
+@gpu
+@pytest.mark.parametrize("counts,kind,N", [([1, 128, 129, 256, 300, 700], 0, 8200), ([1, 128, 129, 256, 300, 700], 1, 4100), ([700, 0, 129, 1, 257, 384], 2, 8200),
+                                           ([(37 * i) % 401 for i in range(80)], 0, 640), ([(37 * i) % 401 for i in range(80)], 1, 328)])      # (more than 64 tiles)
+@pytest.mark.parametrize("k", [64, 128, 192, 256, 320, 448])
+def test_experts_of_prompts_in_pairs_of_tiles(counts, kind, N, k):
+    """Pairs of 128-row tiles and odd tiles by themselves, experts without a row, ragged last column blocks, K of one K-tile and more. Bounds as
+    above: sums of k products in fp32, what the activation makes of them, one rounding of 16-bit results."""
+    from distributed_llm_inference_amd import ops
+    K = ops.load()
+    E, T, tr, bf = len(counts), sum(counts), 128, torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(k + N)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    nt = (T + tr - 1) // tr + E
+    assert K.moe_pairs(nt, E, 2 * N if kind == 1 else N, k)
+    sel = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=torch.Generator().manual_seed(k))].int().cuda()
+    wts, row_w = torch.rand(T, device="cuda", generator=g) + 0.5, torch.full((tr * nt,), float("nan"), device="cuda")
+    tiles, row_tok, pair_row = (torch.full((n,), 77777, dtype=torch.int32, device="cuda") for n in (1 + nt, tr * nt, T))
+    K.moe_plan(tiles, row_tok, pair_row, sel, T, 1, E, tr, wts, row_w)
+    x, w, w2 = r(tr * nt if kind == 0 else T, k).to(bf), (r(E, N, k) * k ** -0.5).to(bf), (r(E, N, k) * k ** -0.5).to(bf)
+    out = torch.full((tr * nt, N), 3.0, device="cuda", dtype=torch.float32 if kind == 0 else bf)
+    if kind == 0:
+        K.moe_down(out, x, w, tiles, row_tok, nt, tr)
+    else:
+        K.moe_up(out, x, w if kind == 1 else None, w2, tiles, row_tok, nt, 0.0, tr, row_w if kind == 2 else None)
+    assert bool((out[int(tiles[0]) * tr:] == 3.0).all())                      # (nothing behind the tiles there are)
+    eps = (k + 1) * 2.0 ** -24
+    for e in range(E):
+        at = torch.nonzero(sel == e).squeeze(1)
+        rows = pair_row[at].long()
+        a = (x[rows] if kind == 0 else x[at]).double()
+        if kind == 2:
+            a = a * wts[at].double()[:, None]
+        p, m = a @ w[e].double().t(), eps * (a.abs() @ w[e].double().abs().t())
+        q, n = a @ w2[e].double().t(), (eps + 2.0 ** -23) * (a.abs() @ w2[e].double().abs().t())
+        if kind == 0:
+            ref, bound = p, m
+        elif kind == 1:
+            s = p * torch.sigmoid(p)
+            ref, bound = s * q, 1.1 * m * (q.abs() + n) + s.abs() * n
+        else:
+            u = torch.relu(q)
+            ref, bound = u * u, 2 * u * n + n * n
+        if kind:
+            bound = bound + (2.0 ** -8 + 2.0 ** -20) * ref.abs()
+        assert bool(((out[rows].double() - ref).abs() <= bound).all()), e
+
+
 @gpu
 @pytest.mark.parametrize("times", [1, 400])
 @pytest.mark.parametrize("H", [64, 37, 300, 1030])
