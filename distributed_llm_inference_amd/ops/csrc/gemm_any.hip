@@ -110,15 +110,17 @@ __device__ __forceinline__ void mma_tiles(float, const u32x4 (&a)[MT], const u32
 }
 
 // A BM x BN tile of C per workgroup, both operand panels through a ring of four LDS stages of 128 bytes of K. The general
-// kernel issues its next fragment loads only when the last ones have been used, so every k-step waits for L2; here three
-// stages are on their way while one is multiplied. A stage is rows of 128 bytes, written by direct LDS loads (1 KiB = 8 rows a
-// piece, whole cache lines of eight rows); the 16-byte chunk c of row r sits at c ^ (r % 8), so that the 16 rows a fragment
-// read touches fall on different banks (the swizzle is applied to the address each lane loads FROM). Rows beyond M or N
-// repeat the last one: their products are never stored.
+// kernel issues its next fragment loads only when the last ones have been used, so every k-step waits for L2; here a wave holds
+// the fragments of stage s when the barrier opens, asks for those of stage s + 1 and for the loads of stage s + 4 (into the slot that
+// everybody has just read), and multiplies: the matrix cores have work at once. (Before, the fragments were read behind the barrier: the
+// table's middle column.) A stage is rows of 128 bytes, written by direct LDS loads (1 KiB = 8 rows a piece, whole cache lines of eight
+// rows); the 16-byte chunk c of row r sits at c ^ (r / 2 % 8), so that the 16 rows a fragment read touches fall on different banks, of
+// which two rows fill all (the swizzle is applied to the address each lane loads FROM). Rows beyond M or N repeat the last one: their
+// products are never stored.
 // Bound by the fp32 matrix rate in fp32 (a 64 x 64 tile needs 16 bytes of L2 and 32 of LDS per cycle and CU) and by how evenly
-// the tiles fall on the CUs. fp32, general kernel -> this one: 300 rows, N 8192, K 2048 172 -> 116 us; N 2048, K 8192 355 ->
-// 126 us; 1024 rows, N = K = 4096 476 -> 307 us (112 TFLOP/s). bf16: 1024 rows, N = K = 4096 233 -> 68 us; 32 products of 1900
-// rows, N 448, K 128 61 -> 35 us.
+// the tiles fall on the CUs. us, general kernel -> fragments behind the barrier -> this one, fp32: 300 rows, N 8192, K 2048 172 -> 118 -> 99;
+// N 2048, K 8192 355 -> 128 -> 111; 1024 rows, N = K = 4096 476 -> 317 -> 277 (124 TFLOP/s), 2048 rows 612 -> 515; 64 rows, N 8192, K 2048
+// 27 -> 22. bf16: 1024 rows, N = K = 4096 233 -> 61 -> 50; 32 products of 1900 rows, N 448, K 128 61 -> 35 -> 35, N 128, K 448 54 -> 28 -> 23.
 //
 // KG > 1: the stages are dealt out to KG groups of four waves with a ring each, whose tiles meet in LDS at the end. One tile
 // per CU is one wave per SIMD, and a stage is then mostly waiting (barrier, first fragment read).
@@ -145,21 +147,22 @@ __global__ __launch_bounds__(256 * KG) void gemm_any_tile_kernel(OT* __restrict_
 #pragma unroll
   for (int q = 0; q < P; ++q) {
     const int row = (wave * P + q) * 8 + (lane >> 3);
-    const int chunk = (lane & 7) ^ (row & 7);
+    const int chunk = (lane & 7) ^ ((row >> 1) & 7);
     src[q] = row < BMP ? A + (long)min(m0 + row, M - 1) * lda + chunk * VEC : W + (long)min(n0 + row - BMP, N - 1) * ldw + chunk * VEC;
   }
   const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)ring + wave * P * 1024;
-  // stage i of this group: K-step i KG + group
+  // stage i of this group: K-step i KG + group (asked for in order: the sources walk along)
   const int steps = K / BK, nk = (steps - group + KG - 1) / KG, rounds = (steps + KG - 1) / KG;
-  auto fetch = [&](int i) {
-    const unsigned to = __builtin_amdgcn_readfirstlane(lds_base + (i % kAnyStages) * kStage);
+#pragma unroll
+  for (int q = 0; q < P; ++q) src[q] += group * BK;
+  auto fetch = [&](int slot) {
     const void* g[P];
 #pragma unroll
-    for (int q = 0; q < P; ++q) g[q] = src[q] + ((long)i * KG + group) * BK;
-    lds_dma_run<P>(g, to);
+    for (int q = 0; q < P; ++q) { g[q] = src[q]; src[q] += KG * BK; }
+    lds_dma_run<P>(g, __builtin_amdgcn_readfirstlane(lds_base + slot * kStage));
   };
 #pragma unroll
-  for (int i = 0; i < kAnyStages - 1; ++i)
+  for (int i = 0; i < kAnyStages; ++i)
     if (i < nk) fetch(i);
   f32x4 acc[MT][NT];
 #pragma unroll
@@ -167,26 +170,67 @@ __global__ __launch_bounds__(256 * KG) void gemm_any_tile_kernel(OT* __restrict_
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
-  for (int s = 0; s < rounds; ++s) {
-    // stage s has landed (own pieces: the stages behind it may still be on their way), everybody is done with stage s - 1
-    if (nk - 1 - s >= 2) wait_pieces<2 * P>();
-    else if (nk - 1 - s == 1) wait_pieces<P>();
-    else wait_pieces<0>();
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (s >= nk) continue;                                        // (the last round of a group that has one stage less)
-    if (s + kAnyStages - 1 < nk) fetch(s + kAnyStages - 1);
-    const char* st = ring + (s % kAnyStages) * kStage;
+  struct Frags { u32x4 a[2][MT], b[2][NT]; };
+  const int at = r16 * 128, sw = (r16 >> 1) & 7;                  // (tiles start at multiples of 16 rows: the swizzle is the lane's own)
+  auto read = [&](Frags& f, int slot) {
+    const char* st = ring + slot * kStage + at;
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
-      u32x4 a[MT], b[NT];
+      const int c = ((kk * 4 + kq) ^ sw) << 4;
 #pragma unroll
-      for (int i = 0; i < MT; ++i) { const int row = wm + i * 16 + r16; a[i] = ld16(st + row * 128 + (((kk * 4 + kq) ^ (row & 7)) << 4)); }
+      for (int i = 0; i < MT; ++i) f.a[kk][i] = ld16(st + (wm + i * 16) * 128 + c);
 #pragma unroll
-      for (int j = 0; j < NT; ++j) { const int row = BMP + wn + j * 16 + r16; b[j] = ld16(st + row * 128 + (((kk * 4 + kq) ^ (row & 7)) << 4)); }
-      mma_tiles<MT, NT>(T{}, a, b, acc);
+      for (int j = 0; j < NT; ++j) f.b[kk][j] = ld16(st + (BMP + wn + j * 16) * 128 + c);
     }
+  };
+  // own reads are done and own pieces have landed; the barrier makes it everybody's
+  auto meet = [] {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto landed = [&](int behind) {                                 // all but the last `behind` stages asked for
+    if (behind >= 3) wait_pieces<3 * P>();
+    else if (behind == 2) wait_pieces<2 * P>();
+    else if (behind == 1) wait_pieces<P>();
+    else wait_pieces<0>();
+  };
+  Frags f0, f1;
+  landed(nk - 1);
+  meet();
+  read(f0, 0);
+  auto multiply = [&](const Frags& f) {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) mma_tiles<MT, NT>(T{}, f.a[kk], f.b[kk], acc);
+  };
+  // (a group may have one stage less than the others: it then reads a slot that nothing was asked for, and does not multiply it)
+  auto step = [&](int s, const Frags& now, Frags& next) {
+    landed(nk - 2 - s < 2 ? nk - 2 - s : 2);
+    meet();
+    read(next, (s + 1) % kAnyStages);
+    if (s + kAnyStages < nk) fetch(s % kAnyStages);               // (everybody holds stage s)
+    multiply(now);
+  };
+  // Rounds of four stages with nothing conditional in them (a branch around the loads makes the compiler wait for the fragments just
+  // asked for); what is left goes step by step.
+  auto steady = [&](int slot, const Frags& now, Frags& next) {
+    wait_pieces<2 * P>();
+    meet();
+    read(next, (slot + 1) % kAnyStages);
+    fetch(slot);
+    multiply(now);
+  };
+  static_assert(kAnyStages == 4, "the slots of a round of steps");
+  int s = 0;
+  const int least = steps / KG;                                   // (stages that every group has)
+  for (; s + 2 * kAnyStages - 1 < least; s += kAnyStages) { steady(0, f0, f1); steady(1, f1, f0); steady(2, f0, f1); steady(3, f1, f0); }
+  for (; s + 2 < rounds; s += 2) { step(s, f0, f1); step(s + 1, f1, f0); }
+  if (s + 1 < rounds) {
+    step(s, f0, f1);
+    if (KG == 1 || s + 1 < nk) multiply(f1);
+  } else if (KG == 1 || s < nk) {
+    multiply(f0);
   }
   if constexpr (KG > 1) {
     f32x4* part = reinterpret_cast<f32x4*>(lds);                  // [group - 1][wave][tile][lane]
@@ -360,10 +404,10 @@ extern "C" int dlia_gemm_any_form(int M, int N, int K, int blocks, int f32, int 
   if (K % bk) return 0;
   auto rounds = [&](int bm, int bn) { return (int)(((long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * blocks + 255) / 256); };
   const int r66 = rounds(64, 64), r46 = rounds(48, 64), r36 = rounds(32, 64), r33 = rounds(32, 32);
-  if (K == bk && r66 >= 4) return 0;           // (a single stage and the chip full: 32 products of 1000 rows, N 448, K 64 29.9 us, the general kernel 26.5)
   const double t66 = r66, t46 = epi == 0 ? r46 * 0.77 : 1e30, t36 = r36 * 0.58, t33 = epi == 0 ? (r33 == 1 ? 0.36 : r33 * 0.33) : 1e30;
+  if (f32 && K == bk && r66 >= 4) return 0;    // (a single stage and the chip full: 2048 rows, N 4096, K 32 19.1 us, the general kernel 16.4)
   const bool split = K >= 16 * bk;             // (below that the rings are filled once or twice: nothing to hide)
-  const double best = r66 > 8 ? t66 : fmin(fmin(t66, t46), fmin(t36, t33));        // (with many rounds the last one is small change)
+  const double best = r66 > 6 ? t66 : fmin(fmin(t66, t46), fmin(t36, t33));        // (with many rounds the last one is small change: 32 products of 1900 rows, N 128, K 448 23 us, in tiles of 48 rows 27)
   if (t66 == best) return split && r66 == 1 ? 64642 : 64641;
   if (t36 == best) return split && r36 == 1 ? 32642 : 32641;
   if (t46 == best) return split && r46 == 1 ? 48642 : 48641;
