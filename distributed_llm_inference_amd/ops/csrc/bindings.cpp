@@ -428,6 +428,8 @@ void gemm_a8w8(Tensor out, const Tensor& xq, const Tensor& xscale, const Tensor&
   }
 }
 
+// 256 x 256 tiles per XCD in front of those that run as halves of 128 rows, -1: none do (ktiles: 128-byte pieces of a row of x)
+int64_t gemm_large_whole(int64_t M, int64_t N, int64_t ktiles, bool alone) { return dlia_gemm_pingpong_whole((int)M, (int)N, (int)ktiles, alone); }
 int64_t gemm_splitk(int64_t M, int64_t N, int64_t K) { return dlia_gemm_skinny_splitk((int)M, (int)N, (int)K); }
 
 // [ntw, splitk] the weight-streaming kernel would use for this shape
@@ -949,6 +951,7 @@ TORCH_LIBRARY(dlia, m) {
   m.def("quant_rows(Tensor(a!) q, Tensor(b!) scale, Tensor x) -> ()");
   m.def("gemm_config(int M, int N, int K, int epi, bool allow_split) -> int[]");
   m.def("gemm_splitk(int M, int N, int K) -> int");
+  m.def("gemm_large_whole(int M, int N, int ktiles, bool alone) -> int");
   m.def("large_gemm_kernel(int which) -> int");
   m.def("gemm_ws_floats(int M, int N, int K) -> int");
   m.def("attention_ws_floats(int B, int max_q_len, int Hq, int Hkv, int D, int splits) -> int");
@@ -1000,6 +1003,7 @@ TORCH_LIBRARY_IMPL(dlia, CUDA, m) {
 
 TORCH_LIBRARY_IMPL(dlia, CompositeExplicitAutograd, m) {
   m.impl("gemm_splitk", &gemm_splitk);
+  m.impl("gemm_large_whole", &gemm_large_whole);
   m.impl("large_gemm_kernel", &large_gemm_kernel);
   m.impl("gemm_ws_floats", &gemm_ws_floats);
   m.impl("gemm_config", &gemm_config);

@@ -20,6 +20,7 @@ struct GemmParams {
   int act;                    // 0 none, 1 swiglu (gate tile, up tile interleaved), 2 gelu_tanh
   int out_f32;
   int partial_only;           // write fp32 partials even when splitk == 1 (a consumer kernel sums them)
+  int full_items;             // gemm_pingpong.hip only: tiles per XCD that run whole, those behind them as halves; -1: no halves
   int group_n;                // gemm_rows.hip only: column blocks per workgroup-order group (set by its launcher)
   int* counters;              // gemm_pingpong.hip with splitk > 1: one arrival counter per output tile, zero between launches
   // gemm_pingpong.hip as the lm_head: besides the fp32 logits, the maximum of every 32-column chunk of every

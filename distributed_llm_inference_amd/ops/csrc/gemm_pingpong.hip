@@ -58,6 +58,7 @@
 namespace dlia {
 
 constexpr int kPPLds = 8 * kPPHalf;              // 2 K-tiles x {A0, B0, B1, A1}
+constexpr int kPPTailLds = 9 * kPPHalf;          // ... or 3 x {A0, B0, B1}
 constexpr int kPPSlab = 256 * 256;               // floats of one partial tile
 constexpr int kPPCounters = 4096;                // counter words at the end of the workspace (two per output tile)
 
@@ -81,8 +82,13 @@ typedef int i32x8 __attribute__((ext_vector_type(8)));
 // (220 instead of 256 VGPRs, a different main loop): with it compiled into every GEMM, bench.py's default point lost
 // 1.1 % (60.98 against 60.30 ms per step, four position-balanced runs each) — more than half of what the guided
 // sampler it serves brings.
-template <bool F8, bool CMAX = false>
+// TAIL: the tiles behind an XCD's last whole round run as two halves of 128 rows each, on twice as many workgroups (the launcher's rule;
+// never with K splits). A half walks K in two phases a K-tile, q0: A0 x B0, q1: A0 x B1, over three K-tiles of three half-tiles (144 KiB):
+// q0 of K-tile t asks for A0 and B0 of t + 2, q1 for its B1, into the slots that t - 1 was read from two phases before, and at q1 a wave
+// waits until only the four pieces it asked for in q0 may be on their way: all of t + 1 has landed.
+template <bool F8, bool CMAX = false, bool TAIL = false>
 __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams p) {
+  static_assert(!(CMAX && TAIL), "the chunk maxima of a half tile would need their own rows");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -95,10 +101,12 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
   const int nb = (p.ntiles + 15) >> 4;           // 256-column blocks (the last may have one column half only)
   // ... and the K splits of one tile are neighbours in that order: dispatched together, done together.
   const int within = blockIdx.x >> 3;
-  const int ks = within % p.splitk, rest = within / p.splitk;
+  const bool half = TAIL && within >= p.full_items;
+  const int ks = TAIL ? 0 : within % p.splitk, rest = TAIL ? (half ? p.full_items + ((within - p.full_items) >> 1) : within) : within / p.splitk;
   const int cb = (rest / mblocks) * 8 + (blockIdx.x & 7);
   if (cb >= nb) return;                          // grid padded to 8 column blocks; whole workgroup, before any barrier
-  const int mblk = rest % mblocks, mrow0 = mblk * 256;
+  const int mblk = rest % mblocks, mrow0 = mblk * 256 + (half ? ((within - p.full_items) & 1) * 128 : 0);
+  if (TAIL && mrow0 >= p.M) return;              // (the lower half of a last row block; whole workgroup)
   const int tiles_total = p.K >> (F8 ? 7 : 6), KT = tiles_total * 2;   // K-tile = 128 bytes of an x row
   const int per = (tiles_total + p.splitk - 1) / p.splitk;
   const int c0 = ks * per;
@@ -239,6 +247,49 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
     pp_loop_barrier();
   };
 
+  if (TAIL && half) {
+    auto fetch = [&](auto kind_c, int c, int slot) {          // kind 0 A0, 1 B0, 2 B1 of K-tile c, to half-tile `slot` of nine
+      constexpr int kind = decltype(kind_c)::value;
+      const long cc = min(c, n - 1);
+      const unsigned dst = lds0 + slot * kPPHalf + wave * 2048;
+      if constexpr (kind == 0) pp_dma_pair(asrc[0][0] + cc * 128, asrc[0][1] + cc * 128, dst);
+      else pp_dma_pair(bsrc[kind - 1] + cc * 2048, bsrc[kind - 1] + cc * 2048, dst);
+    };
+    auto half_phase = [&](auto q_c, int t, auto buf_c) {
+      constexpr int q = decltype(q_c)::value, here = decltype(buf_c)::value * 3, there = (decltype(buf_c)::value + 2) % 3 * 3;
+      if constexpr (q == 1) pp_wait_vm<4>();
+      const char* base = smem + (here + 1 + q) * kPPHalf + boff;
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) (q ? b1 : b0)[j][kk] = *reinterpret_cast<const u32x4*>(base + (j * 2 + kk) * 1024);
+      if constexpr (q == 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        const char* xb = smem + here * kPPHalf + xoff;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk)
+            af[i][kk] = *reinterpret_cast<const u32x4*>(xb + i * 2048 + (((F8 ? 2 * quad + kk : kk * 4 + quad) ^ sw) << 4));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (q == 0) { fetch(ic<0>{}, t + 2, there); fetch(ic<1>{}, t + 2, there + 1); }
+      else fetch(ic<2>{}, t + 2, there + 2);
+      pp_barrier();
+      cluster(acc[0][q], q ? b1 : b0);
+      pp_barrier();
+    };
+    fetch(ic<0>{}, 0, 0); fetch(ic<1>{}, 0, 1); fetch(ic<2>{}, 0, 2);
+    fetch(ic<0>{}, 1, 3); fetch(ic<1>{}, 1, 4); fetch(ic<2>{}, 1, 5);
+    pp_wait_vm<6>();
+    pp_barrier();
+    if (wr == 1) pp_barrier();
+    for (int t = 0; t < n; t += 3) {
+      half_phase(ic<0>{}, t, ic<0>{}); half_phase(ic<1>{}, t, ic<0>{});
+      if (t + 1 < n) { half_phase(ic<0>{}, t + 1, ic<1>{}); half_phase(ic<1>{}, t + 1, ic<1>{}); }
+      if (t + 2 < n) { half_phase(ic<0>{}, t + 2, ic<2>{}); half_phase(ic<1>{}, t + 2, ic<2>{}); }
+    }
+  } else {
   // prologue: K-tile 0 whole, A0 and B0 of K-tile 1
   issue(ic<0>{}, 0, 0); issue(ic<1>{}, 0, 0); issue(ic<2>{}, 0, 0); issue(ic<3>{}, 0, 0);
   issue(ic<0>{}, 1, 1); issue(ic<1>{}, 1, 1);
@@ -255,6 +306,7 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
       phase(ic<0>{}, t + 1, 1); phase(ic<1>{}, t + 1, 1); phase(ic<2>{}, t + 1, 1); phase(ic<3>{}, t + 1, 1);
     }
   }
+  }
   if (wr == 0) pp_loop_barrier();                // the barrier waves 4-7 took at the start
   pp_wait_vm<0>();                               // no DMA may land after the workgroup is gone
 
@@ -267,7 +319,7 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
         for (int b = 0; b < 4; ++b) o[a * 4 + b] = stamp_sum[a][b];
     }
   }
-  if (p.splitk > 1) {
+  if (!TAIL && p.splitk > 1) {
     // ---- sum the K splits of this tile ------------------------------------------------------
     // Each workgroup first draws a ticket from the tile's arrival counter. All but the last to
     // arrive store their accumulators (write-through, register order) to their slab and raise the
@@ -392,6 +444,7 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
       const bf16* const resp = p.residual + cb * 256 + cl * 8;     // (only dereferenced when there is a residual)
 #pragma unroll
       for (int hm = 0; hm < 2; ++hm) {
+        if (TAIL && half && hm) break;            // (a half tile; whole workgroup)
         pp_barrier();                             // the area is free: all DMA landed and fragments read / previous half read back
 #pragma unroll
         for (int hn = 0; hn < 2; ++hn)
@@ -447,11 +500,13 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
           }
       const int cl = lane & 15, rsub = lane >> 4;
       bf16* const outp = reinterpret_cast<bf16*>(p.out) + cb * 128 + cl * 8;
-      const int m0 = mrow0 + wave * 32 + rsub;
+      const int rows = TAIL && half ? 16 : 32;     // of a wave
+      const int m0 = mrow0 + wave * rows + rsub;
       pp_barrier();
 #pragma unroll
       for (int s = 0; s < 8; ++s) {
-        const int R = wave * 32 + s * 4 + rsub;
+        if (TAIL && half && s >= 4) break;
+        const int R = wave * rows + s * 4 + rsub;
         const float* row = st + R * 128;
         const f32x4 lo = *reinterpret_cast<const f32x4*>(row + (((2 * cl) ^ (R & 15)) << 2));
         const f32x4 hi = *reinterpret_cast<const f32x4*>(row + (((2 * cl + 1) ^ (R & 15)) << 2));
@@ -469,7 +524,7 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
   for (int hm = 0; hm < 2; ++hm)
 #pragma unroll
     for (int hn = 0; hn < 2; ++hn)
-      write_acc_tiles<4, 2, true>(p, acc[hm][hn], cb * 16 + hn * 8 + wc * 2, l15, quad, 0, mrow0 + hm * 128 + wr * 64);
+      if (!(TAIL && half && hm)) write_acc_tiles<4, 2, true>(p, acc[hm][hn], cb * 16 + hn * 8 + wc * 2, l15, quad, 0, mrow0 + hm * 128 + wr * 64);
 }
 
 
@@ -853,6 +908,17 @@ static int pp_splitk(int M, int N, int ktiles, int want = 0) {
   while (s > 1 && ktiles / s < 8) --s;
   return s < 1 ? 1 : s;
 }
+// Tiles per XCD that run whole in front of halves (TAIL), or -1: no halves. An XCD's 32 CUs take its tiles in rounds of 32; where the last round has
+// at most 16, its tiles go out as halves of 128 rows, which cost 0.55 (half the chip) to 0.8 (all of it) of a round: 1531 rows, N 14336, K 4096
+// (42 tiles) 162 -> 141 us, fp32 out 175 -> 150; 1290 rows (42) 160 -> 137; 2048 rows, N 28672 (112) 417 -> 402. With up to 16 tiles in all
+// the halves stand against K splits, whose sums cost 17 to 37 us whatever K is: 1024 rows, N = K =
+// 4096 47 -> 42 us, 2048 rows 63 -> 57, 300 rows 48 -> 39; K 14336 102 / 129, 173 / 182, 143 / 154. They meet between 79 and 126 K-tiles.
+// `alone`: the caller wants the chip filled (beside another stream's kernels an idle CU is theirs, and halves move more bytes a product).
+extern "C" int dlia_gemm_pingpong_whole(int M, int N, int ktiles, int alone) {
+  const int per_xcd = ((packed_ntiles(N) + 15) / 16 + 7) / 8 * ((M + 255) / 256), rest = per_xcd % 32;
+  if (!alone || rest == 0 || rest > 16) return -1;
+  return per_xcd > 32 || ktiles <= 80 ? per_xcd - rest : -1;
+}
 extern "C" int dlia_gemm_pingpong_splitk(int M, int N, int K) { return pp_splitk(M, N, K / 64); }
 // Workspace the split needs: slabs [tiles][S][256 x 256]; the arrival counters are the LAST
 // kPPCounters words of whatever workspace the caller hands over (so that workspaces shared with
@@ -866,16 +932,27 @@ extern "C" long dlia_gemm_pingpong_ws_floats(int M, int N, int K) {
 // bf16, M > 256 (any M is correct; below that the weight-streaming kernels are faster), K a
 // multiple of 64; `p` fully set up by the caller. p->splitk > 1 needs p->partial = slabs for
 // [tiles][splitk - 1] and p->counters = two zero words per tile (the kernel leaves them zero).
-template <bool F8, bool CMAX = false>
-static void launch_pingpong(const dlia::GemmParams* p, hipStream_t stream) {
+template <bool F8, bool CMAX = false, bool TAIL = false>
+static void launch_pingpong_kernel(const dlia::GemmParams* p, int workgroups, hipStream_t stream) {
+  constexpr int lds = TAIL ? kPPTailLds : kPPLds;
   static const bool once = [] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_pingpong_kernel<F8, CMAX>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, kPPLds);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_pingpong_kernel<F8, CMAX, TAIL>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     return true;
   }();
   (void)once;
+  hipLaunchKernelGGL((gemm_pingpong_kernel<F8, CMAX, TAIL>), dim3(workgroups), dim3(kPPThreads), lds, stream, *p);
+}
+template <bool F8, bool CMAX = false>
+static void launch_pingpong(const dlia::GemmParams* p, hipStream_t stream) {
   const int nb = (p->ntiles + 15) / 16, nb8 = (nb + 7) / 8 * 8, mblocks = (p->M + 255) / 256;
-  hipLaunchKernelGGL((gemm_pingpong_kernel<F8, CMAX>), dim3(nb8 * mblocks * p->splitk), dim3(kPPThreads), kPPLds, stream, *p);
+  if constexpr (!CMAX) {
+    if (p->full_items >= 0) {
+      launch_pingpong_kernel<F8, false, true>(p, 8 * (p->full_items + 2 * (nb8 / 8 * mblocks - p->full_items)), stream);
+      return;
+    }
+  }
+  launch_pingpong_kernel<F8, CMAX>(p, nb8 * mblocks * p->splitk, stream);
 }
 static void launch_quad(const dlia::GemmParams* p, hipStream_t stream) {
   static const bool once = [] {
@@ -908,9 +985,10 @@ extern "C" void dlia_gemm_large(void* out, const void* x, const void* wp, const 
   p.ldr = ldr; p.partial = workspace; p.M = M; p.N = N; p.K = K;
   p.ntiles = packed_ntiles(N);
   p.act = epi == 4 ? 1 : (epi == 5 ? 2 : 0);
-  p.out_f32 = out_f32; p.partial_only = 0; p.splitk = 1; p.group_n = 1; p.counters = nullptr;
+  p.out_f32 = out_f32; p.partial_only = 0; p.splitk = 1; p.group_n = 1; p.full_items = -1; p.counters = nullptr;
   if (dlia_gemm_large_choice(-1) == 2 && chunk_max == nullptr) { dlia_gemm_rows(&p, stream); return; }
-  const int s = pp_splitk(M, N, K / 64, wg_target);
+  p.full_items = chunk_max ? -1 : dlia_gemm_pingpong_whole(M, N, K / 64, wg_target > 128);
+  const int s = p.full_items >= 0 ? 1 : pp_splitk(M, N, K / 64, wg_target);
   const long tiles = (long)((M + 255) / 256) * ((p.ntiles + 15) / 16);
   if (workspace && s > 1 && ws_floats >= tiles * (s - 1) * kPPSlab + kPPCounters) {
     p.splitk = s;
@@ -933,9 +1011,10 @@ extern "C" void dlia_gemm_a8w8_large(void* out, const void* xq, const float* xsc
   p.ldr = ldr; p.partial = workspace; p.M = M; p.N = N; p.K = K;
   p.ntiles = packed_ntiles(N);
   p.act = epi == 4 ? 1 : (epi == 5 ? 2 : 0);
-  p.out_f32 = out_f32; p.partial_only = 0; p.splitk = 1; p.group_n = 1; p.counters = nullptr;
+  p.out_f32 = out_f32; p.partial_only = 0; p.splitk = 1; p.group_n = 1; p.full_items = -1; p.counters = nullptr;
   if (dlia_gemm_large_choice(-1) == 2) { p.partial = nullptr; dlia_gemm_rows_f8(&p, stream); return; }
-  const int s = pp_splitk(M, N, K / 128, wg_target);
+  p.full_items = dlia_gemm_pingpong_whole(M, N, K / 128, wg_target > 128);
+  const int s = p.full_items >= 0 ? 1 : pp_splitk(M, N, K / 128, wg_target);
   const long tiles = (long)((M + 255) / 256) * ((p.ntiles + 15) / 16);
   if (workspace && s > 1 && ws_floats >= tiles * (s - 1) * kPPSlab + kPPCounters) {
     p.splitk = s;

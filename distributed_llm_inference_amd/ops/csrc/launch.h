@@ -75,6 +75,7 @@ extern "C" void dlia_gemm_a8w8_large(void* out, const void* xq, const float* xsc
 int dlia_gemm_large_choice(int which);
 // the large-M kernel's in-launch split-K: factor for a shape, and the workspace floats it needs (slabs + counters)
 int dlia_gemm_pingpong_splitk(int M, int N, int K);
+int dlia_gemm_pingpong_whole(int M, int N, int ktiles, int alone);
 long dlia_gemm_pingpong_ws_floats(int M, int N, int K);
 
 // ---- attention.hip --------------------------------------------------------------------

@@ -497,6 +497,49 @@ def test_gemm_a8w8_large_kernels_agree_on_edge_shapes(K, which, shape):
         K.large_gemm_kernel(prev)
 
 
+@pytest.mark.parametrize("f8", [False, True], ids=["bf16", "e4m3"])
+@pytest.mark.parametrize("epi,f32", [(0, False), (0, True), (1, False), (2, False), (3, True), (4, False), (5, False)])
+@pytest.mark.parametrize("shape", [(1531, 14336, 1), (1290, 14200, 2), (300, 4096, 3), (257, 4000, 4), (2011, 4096, 5), (512, 2048, 7)])
+def test_gemm_large_m_halves_of_the_last_round(K, shape, epi, f32, f8):
+    """Tiles behind an XCD's last whole round as halves of 128 rows: every output element is the sum of the same products in the same order
+    as in whole tiles, so the bits are the same. 42 tiles an XCD, 4, 16 and 2; last row blocks of one half or less, ragged last
+    column blocks, one to seven K-tiles."""
+    M, N, kt = shape
+    Kd = kt * (128 if f8 else 64)
+    if not f8 and Kd % 128:
+        Kd, kt = Kd + 64, kt + 1                     # (the packed image wants whole pieces of 128)
+    N = N // 32 * 32
+    assert K.gemm_large_whole(M, N, kt, True) >= 0 and K.gemm_large_whole(M, N, kt, False) < 0
+    g = torch.Generator(device=DEV).manual_seed(M + N + epi)
+    n_out = N // 2 if epi == 4 else N
+    x, w = bf(torch.randn(M, Kd, device=DEV, generator=g)), torch.randn(N, Kd, device=DEV, generator=g) / math.sqrt(Kd)
+    bias, res = bf(torch.randn(n_out, device=DEV, generator=g)), bf(torch.randn(M, n_out, device=DEV, generator=g))
+    prev = K.large_gemm_kernel(0)
+    try:
+        outs = []
+        for target in (1, 256):
+            out = torch.full((M + 1, n_out), 7.0, device=DEV, dtype=torch.float32 if f32 else torch.bfloat16)
+            if f8:
+                xq, xs = torch.zeros(M, Kd, device=DEV, dtype=torch.uint8), torch.zeros(M, device=DEV)
+                K.quant_rows(xq, xs, x)
+                wp, sc = packing.pack_weight_a8w8(w)
+                K.gemm_a8w8(out[:M], xq, xs, wp, sc, bias, res, None, N, epi, target, 0)
+            else:
+                K.gemm(out[:M], x, packing.pack_weight(bf(w)), bias, res, None, N, epi, target, 0)
+            outs.append(out)
+        assert torch.equal(outs[0], outs[1]) and bool((outs[1][M] == 7.0).all()) and bool((outs[1][:M] != 7.0).any(0).all())
+    finally:
+        K.large_gemm_kernel(prev)
+
+
+def test_gemm_large_m_halves_where_they_measured_faster(K):
+    whole = K.gemm_large_whole          # us: whole tiles or K splits against halves
+    assert whole(1531, 14336, 64, True) == 32 and whole(2048, 28672, 64, True) == 96 and whole(1290, 14336, 64, True) == 32          # 162 / 141, 417 / 402, 160 / 137
+    assert whole(1024, 4096, 64, True) == 0 and whole(2048, 4096, 64, True) == 0 and whole(300, 14336, 64, True) == 0               # 47 / 42, 63 / 57, 57 / 44
+    assert whole(1024, 4096, 224, True) == -1 and whole(2048, 4096, 224, True) == -1 and whole(2048, 8192, 64, True) == -1          # 102 / 129, 173 / 182, full rounds
+    assert whole(2048, 6144, 64, True) == -1 and whole(1531, 14336, 64, False) == -1                                                # more than half a round; beside another stream
+
+
 def test_gemm_pingpong_exact_on_integer_data_with_asymmetric_operands(K):
     """Small integers are exact in bf16 and fp32: every output element must equal the integer product
     exactly, with an x that is not symmetric and weights that differ per column (a swapped row/column
