@@ -992,16 +992,37 @@ __global__ __launch_bounds__(64) void rglru_stretch_kernel(
 }
 
 // ---- activation, scaling ---------------------------------------------------------------------------------------------
-template <typename OT>
+// exp(v) - 1 - v for v <= 0: the series above -1/2 (what it leaves out is under 2^-29 of the value; expm1f(v) - v cancels there), the
+// hardware exponential below, with what its argument v log2(e) loses to rounding put back. Both are evaluated, some 16 instructions in all.
+__device__ __forceinline__ float exp_rest(float v) {
+  float c = 1.f / 362880.f;
+  const float inv[7] = {1.f / 40320.f, 1.f / 5040.f, 1.f / 720.f, 1.f / 120.f, 1.f / 24.f, 1.f / 6.f, 0.5f};
+#pragma unroll
+  for (int i = 0; i < 7; ++i) c = __builtin_fmaf(c, v, inv[i]);
+  const float w = fmaxf(v, -128.f), t = w * 1.44269502162933349609f;      // (nothing is left of the exponential there)
+  const float lost = __builtin_fmaf(w, 1.925963e-8f, __builtin_fmaf(w, 1.44269502162933349609f, -t));
+  const float e = __builtin_amdgcn_exp2f(t);       // log2(e) = 1.442695021629333 (its nearest float) + 1.925963e-8
+  const float x = __builtin_fmaf(e * 0.6931471805599453f, lost, e);
+  return v > -0.5f ? v * v * c : x - (1.f + v);
+}
+
+// V entries of a row per thread. Bound by its bytes: 1531 rows of 14336, bf16 out, 23 us (5.8 TB/s, half of them from the last-level
+// cache); 43 with an entry a thread and expm1f, whose two cases both run in a wave that holds both.
+template <typename OT, int V>
 __global__ __launch_bounds__(256) void xielu_kernel(OT* __restrict__ act, const float* __restrict__ z, int M, int F, long ldz,
                                                     long lda, const float* __restrict__ pq) {
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (long)M * F) return;
-  const int m = (int)(i / F), c = (int)(i % F);
+  const int units = F / V;
+  if (i >= (long)M * units) return;
+  const int m = (int)(i / units), c = (int)(i % units) * V;
   const float ap = pq[0], aq = pq[1];          // softplus(p), 1/2 + softplus(q)
-  const float v = z[(long)m * ldz + c];
-  const float r = v > 0.f ? ap * v * v + 0.5f * v : aq * (expm1f(v) - v) + 0.5f * v;
-  act[(long)m * lda + c] = (OT)r;
+  Unit<V> u = ldu<V>(z + (long)m * ldz + c);
+#pragma unroll
+  for (int e = 0; e < V; ++e) {
+    const float v = u.v[e];
+    u.v[e] = v > 0.f ? ap * v * v + 0.5f * v : aq * exp_rest(v) + 0.5f * v;
+  }
+  stu<V>(act + (long)m * lda + c, u);
 }
 
 __global__ __launch_bounds__(256) void scale_rows_kernel(float* __restrict__ x, int M, int N, long ld, float s) {
@@ -1156,9 +1177,12 @@ extern "C" void dlia_xielu(void* act, int out_f32, const float* z, int M, int F,
                            hipStream_t stream) {
   const long n = (long)M * F;
   if (n <= 0) return;
-  const dim3 grid((unsigned)((n + 255) / 256));
-  if (out_f32) hipLaunchKernelGGL(xielu_kernel<float>, grid, dim3(256), 0, stream, (float*)act, z, M, F, ldz, lda, pq);
-  else hipLaunchKernelGGL(xielu_kernel<bf16>, grid, dim3(256), 0, stream, (bf16*)act, z, M, F, ldz, lda, pq);
+  const bool wide = F % 4 == 0 && ldz % 4 == 0 && lda % 4 == 0 && al16_(z) && (uintptr_t)act % (out_f32 ? 16 : 8) == 0;
+  const dim3 grid((unsigned)((wide ? n / 4 : n) + 255) / 256);
+#define DLIA_XIELU(OT, V) hipLaunchKernelGGL((xielu_kernel<OT, V>), grid, dim3(256), 0, stream, (OT*)act, z, M, F, ldz, lda, pq)
+  if (out_f32) { if (wide) DLIA_XIELU(float, 4); else DLIA_XIELU(float, 1); }
+  else { if (wide) DLIA_XIELU(bf16, 4); else DLIA_XIELU(bf16, 1); }
+#undef DLIA_XIELU
 }
 
 extern "C" void dlia_scale_rows(float* x, int M, int N, long ld, float s, hipStream_t stream) {

@@ -292,6 +292,24 @@ def test_block_products_activation_and_scale_hip():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,F,ld", [(3, 1024, 1024), (5, 1022, 1024), (4, 260, 261), (1, 4, 4)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_xielu_rows_in_pieces_and_one_by_one(M, F, ld, dt):
+    """Whole pieces of four and rows that are not, both sides of where the negative branch changes, zeros and large magnitudes. Negative side: |q|
+    times two roundings of what the exponential and v leave, and of the sum's terms."""
+    K, dev = _K(), "cuda"
+    z = rnd(M, ld, seed=1, std=2.0)
+    z[0, :4] = torch.tensor([0.0, -0.5, -3e38, 100.0])            # (q 3e38 = 3.15e38 is below the largest float, 3.4e38: with 1.3 the sum is infinite in any fp32 form)
+    z = z.float()[:, :F]
+    act, pq = torch.full((M, F), 7.0, device=dev, dtype=dt), torch.tensor([0.8, 1.05])
+    K.xielu(act, z.to(dev), pq.to(dev))
+    v, (p, q) = z.to(F64), pq.to(F64)
+    ref = torch.where(v > 0, p * v * v, q * (torch.expm1(v.clamp(max=0)) - v)) + 0.5 * v
+    bound = 2.0 ** -22 * (torch.where(v > 0, p * v * v, q * (1 + v.abs())) + 0.5 * v.abs()) + (2.0 ** -8 * ref.abs() if dt == torch.bfloat16 else 0)
+    assert bool(((act.cpu().to(F64) - ref).abs() <= bound).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,G,d,dv,maps,window,keep,cap,dims,inter", [
     (4, 2, 16, 24, 2, 40, 5, 10.0, 8, True), (2, 1, 8, 8, 1, 0, 0, 0.0, 8, False), (3, 3, 24, 70, 2, 3, 50, 0.0, 4, True),
     (2, 2, 72, 130, 1, 33, 0, 3.0, 0, False), (6, 1, 40, 16, 2, 64, 1, 25.0, 10, True), (1, 1, 104, 300, 1, 0, 0, 0.0, 16, False),
