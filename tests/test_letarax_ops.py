@@ -283,6 +283,27 @@ def test_short_conv_kernel(K, Kt):
 
 
 @gpu
+@pytest.mark.parametrize("C", [4, 72, 1028, 2052])
+def test_short_conv_of_four_taps_in_pieces(K, C):
+    """Channels in whole pieces, portions on either side of the 8 tokens that a thread takes, beside a sequence that goes on behind them."""
+    T = 52
+    x, x2, taps = rnd(T, C + 4, seed=1), rnd(40, C + 4, seed=3), rnd(C, 4, seed=2)
+    ref, ref2 = (O.silu(O.causal_short_conv(v[:, :C], taps)) for v in (x, x2))
+    carry = torch.full((3, 3, C), 7.0, device="cuda")
+    outs, outs2, lo, lo2 = [], [], 0, 0
+    for n, n2 in [(1, 2), (2, 1), (7, 17), (8, 1), (9, 8), (17, 9), (8, 2)]:
+        z = dev(torch.cat([x[lo:lo + n], x2[lo2:lo2 + n2]]))
+        y = torch.full((n + n2, C), 9.0, device="cuda")
+        qs, ctx, sl = ragged([n, n2], [lo, lo2], [2, 0])
+        K.short_conv(y, z, carry, dev(taps), qs, ctx, sl, max(n, n2))
+        outs.append(y[:n].cpu())
+        outs2.append(y[n:].cpu())
+        lo, lo2 = lo + n, lo2 + n2
+    close(torch.cat(outs), ref, 1e-5)
+    close(torch.cat(outs2), ref2, 1e-5)
+
+
+@gpu
 @pytest.mark.parametrize("G,H,d,dv", [(1, 1, 7, 9), (2, 4, 32, 32), (2, 6, 16, 48), (1, 2, 160, 72), (1, 1, 128, 128), (3, 3, 64, 20)])
 def test_delta_rule_kernel(K, G, H, d, dv):
     T, C = 40, 2 * G * d + H * dv
