@@ -460,7 +460,7 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
 #pragma unroll
           for (int s = 0; s < 8; ++s) res[s] = ld16(resp + (long)min(m0 + 2 * s, p.M - 1) * p.ldr);
         }
-        pp_barrier();
+        pp_staged();
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
           const int R = wave * 16 + s * 2 + rsub;
@@ -502,7 +502,7 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
       bf16* const outp = reinterpret_cast<bf16*>(p.out) + cb * 128 + cl * 8;
       const int rows = TAIL && half ? 16 : 32;     // of a wave
       const int m0 = mrow0 + wave * rows + rsub;
-      pp_barrier();
+      pp_staged();
 #pragma unroll
       for (int s = 0; s < 8; ++s) {
         if (TAIL && half && s >= 4) break;

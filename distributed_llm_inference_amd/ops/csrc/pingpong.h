@@ -31,5 +31,10 @@ __device__ __forceinline__ void pp_barrier() {
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
 }
+// what the wave wrote to LDS is there, and everyone's behind the barrier (s_barrier alone does not wait for LDS writes)
+__device__ __forceinline__ void pp_staged() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  pp_barrier();
+}
 
 }  // namespace dlia
