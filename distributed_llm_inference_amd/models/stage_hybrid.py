@@ -592,7 +592,9 @@ class HybridGpuStage(GpuStage):
             K.norm32(xn if after_mixer is not None else None, h, yo, p["ln1b_w"], after_mixer, None, eps, 1.0)
             if ls.ff:
                 act = view(wk.act, p["ff_cols"])
-                if "w_gu_p" in p:
+                if "w_gu_p" in p and T > max(self.decode_rows, 256) and ls.ff % 16 == 0:
+                    K.gemm_act(act, xn, p["w_gu_p"], p.get("w_gu_b"), None, wk.ws, 2 * ls.ff, 1, 256)
+                elif "w_gu_p" in p:
                     gu = view(wk.gu, 2 * ls.ff)
                     self._mm(wk, gu, xn, p, "w_gu")
                     K.gated_gelu(act, gu)
@@ -995,8 +997,11 @@ class HybridGpuStage(GpuStage):
             self._mm(wk, ya, mixed, p, "w_o")
             if ls.ff:
                 z2, act, yb = view(wk.z2, self._cols(p, "w_up")), view(wk.act, ls.ff), view(wk.yb, self._cols(p, "w_down"))
-                self._mm(wk, z2, xn, p, "w_up")
-                K.xielu(act, z2, p["pq"])
+                if "w_up_p" in p and T > max(self.decode_rows, 256) and ls.ff % 256 == 0:
+                    K.gemm_act(act, xn, p["w_up_p"], None, p["pq"], wk.ws, ls.ff, 2, 256)
+                else:
+                    self._mm(wk, z2, xn, p, "w_up")
+                    K.xielu(act, z2, p["pq"])
                 self._mm(wk, yb, act, p, "w_down")
                 yb = yb[:, :H]
             nxt = self.layers[li + 1]["ln1_w"] if li + 1 < n_layers else None

@@ -330,6 +330,43 @@ static void gemm_impl(Tensor out, const Tensor& x, const Tensor& wp, OptTensor w
   }
 }
 
+// More than 256 rows and a feed-forward's activation: act 1 out [M, N / 2] = gelu_tanh(gate) * up (weight rows: gate, then up; bias [N]), act 2
+// out [M, N] = xIELU with coef [2] (fp32). `workgroups` as splitk of `gemm`.
+void gemm_act(Tensor out, const Tensor& x, const Tensor& wp, OptTensor bias, OptTensor coef, OptTensor workspace, int64_t N, int64_t act,
+              int64_t workgroups) {
+  DLIA_ON_DEVICE_OF(out);
+  check_bf16(x, "x"); check_rows(x, "x"); check_bf16(out, "out"); check_dev(wp, "wp");
+  const int64_t M = x.size(0), K = x.size(1), n_out = act == 1 ? N / 2 : N, n_pad = (N + 127) / 128 * 128;
+  DLIA_CHECK(M > 256, "gemm_act: more than 256 rows");
+  DLIA_CHECK(act == 1 || act == 2, "gemm_act: act 1 (gated GELU) or 2 (xIELU)");
+  DLIA_CHECK(K % 128 == 0 && N % (act == 1 ? 32 : 256) == 0, "gemm_act: K a multiple of 128, N of 32 (gated) or 256 (xIELU)");
+  DLIA_CHECK(wp.is_contiguous() && wp.numel() * wp.element_size() == n_pad * K * 2 && reinterpret_cast<uintptr_t>(wp.data_ptr()) % 16 == 0,
+             "gemm_act: packed weight size / alignment");
+  DLIA_CHECK(out.dim() == 2 && out.stride(1) == 1 && out.size(0) >= M && out.size(1) >= n_out, "gemm_act: out shape");
+  DLIA_CHECK(act == 1 || (out.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0), "gemm_act: out alignment");
+  const void* bp = nullptr; const float* cp = nullptr;
+  if (bias.has_value()) {
+    DLIA_CHECK(act == 1, "gemm_act: xIELU takes no bias");
+    check_bf16(*bias, "bias");
+    DLIA_CHECK(bias->is_contiguous() && bias->numel() >= N, "gemm_act: bias [N]");
+    bp = bias->data_ptr();
+  }
+  if (act == 2) {
+    DLIA_CHECK(coef.has_value(), "gemm_act: xIELU needs its coefficients");
+    check_f32(*coef, "coef");
+    DLIA_CHECK(coef->is_contiguous() && coef->numel() >= 2, "gemm_act: coef [2]");
+    cp = coef->data_ptr<float>();
+  }
+  float* wsp = nullptr; int64_t wsn = 0;
+  if (workspace.has_value()) {
+    check_f32(*workspace, "workspace");
+    DLIA_CHECK(workspace->is_contiguous(), "gemm workspace must be contiguous");
+    wsp = workspace->data_ptr<float>(); wsn = workspace->numel();
+  }
+  dlia_gemm_large_act(out.data_ptr(), x.data_ptr(), wp.data_ptr(), bp, cp, wsp, wsn, (int)M, (int)N, (int)K, x.stride(0), out.stride(0), (int)act,
+                      (int)workgroups, cur_stream());
+}
+
 void gemm(Tensor out, const Tensor& x, const Tensor& wp, OptTensor bias, OptTensor residual,
           OptTensor workspace, int64_t N, int64_t epi, int64_t splitk, int64_t ntw) {
   gemm_impl(out, x, wp, c10::nullopt, bias, residual, workspace, N, epi, splitk, ntw);
@@ -945,6 +982,7 @@ TORCH_LIBRARY(dlia, m) {
   m.def("rope_kvwrite8(Tensor(a!) qkv, Tensor? partial, int splits, Tensor? pbias, Tensor(b!) kv_cache, Tensor(c!) kv_scale, Tensor cos, Tensor sin, Tensor tok_pos, Tensor tok_seq, Tensor block_table, int Hq, int Hkv, int D, bool use_rope) -> ()");
   m.def("paged_attention8(Tensor(a!) out, Tensor qkv, Tensor kv_cache, Tensor kv_scale, Tensor q_start, Tensor ctx_lens, Tensor block_table, Tensor? slots, Tensor? partial, int max_q_len, int Hq, int Hkv, int D, float scale, int splits) -> ()");
   m.def("gemm(Tensor(a!) out, Tensor x, Tensor wp, Tensor? bias, Tensor? residual, Tensor? workspace, int N, int epi, int splitk, int ntw) -> ()");
+  m.def("gemm_act(Tensor(a!) out, Tensor x, Tensor wp, Tensor? bias, Tensor? coef, Tensor? workspace, int N, int act, int workgroups) -> ()");
   m.def("gemm_w8(Tensor(a!) out, Tensor x, Tensor wp, Tensor wscale, Tensor? bias, Tensor? residual, Tensor? workspace, int N, int epi, int splitk, int ntw) -> ()");
   m.def("gemm_a8w8(Tensor(a!) out, Tensor xq, Tensor xscale, Tensor wp, Tensor wscale, Tensor? bias, Tensor? residual, Tensor? workspace, int N, int epi, int splitk, int ntw) -> ()");
   m.def("norm_q(Tensor(a!) out_q, Tensor(b!) qscale, Tensor(c!) x, Tensor? delta, Tensor? partial, int splits, Tensor? pbias, Tensor w, Tensor? b, float eps, int mode) -> ()");
@@ -987,6 +1025,7 @@ TORCH_LIBRARY_IMPL(dlia, CUDA, m) {
   m.impl("rope_kvwrite8", &rope_kvwrite8);
   m.impl("paged_attention8", &paged_attention8);
   m.impl("gemm", &gemm);
+  m.impl("gemm_act", &gemm_act);
   m.impl("gemm_w8", &gemm_w8);
   m.impl("gemm_a8w8", &gemm_a8w8);
   m.impl("quant_rows", &quant_rows);

@@ -17,6 +17,7 @@ struct GemmParams {
   int M, N, K;                // N = number of GEMM columns (for swiglu: 2 * output columns)
   int ntiles;                 // packed n-tiles (N rounded up to the pack granule) / 16
   int splitk;
+  const float* coef = nullptr;   // gemm_pingpong.hip with xIELU: its two coefficients
   int act;                    // 0 none, 1 swiglu (gate tile, up tile interleaved), 2 gelu_tanh
   int out_f32;
   int partial_only;           // write fp32 partials even when splitk == 1 (a consumer kernel sums them)

@@ -44,6 +44,7 @@
 #include <cstdlib>
 #include <type_traits>
 #include "common.h"
+#include "fp32_math.h"
 #include "gemm_common.h"
 #include "launch.h"
 #include "pingpong.h"
@@ -86,7 +87,12 @@ typedef int i32x8 __attribute__((ext_vector_type(8)));
 // never with K splits). A half walks K in two phases a K-tile, q0: A0 x B0, q1: A0 x B1, over three K-tiles of three half-tiles (144 KiB):
 // q0 of K-tile t asks for A0 and B0 of t + 2, q1 for its B1, into the slots that t - 1 was read from two phases before, and at q1 a wave
 // waits until only the four pieces it asked for in q0 may be on their way: all of t + 1 has landed.
-template <bool F8, bool CMAX = false, bool TAIL = false>
+// ACT: the activation of a feed-forward in the epilogue, on the fp32 sums, instead of a launch that reads them back (an instantiation each, for the
+// registers' sake): 1 gelu_tanh(gate) * up from weights whose first N / 2 rows are the gate's: B0 takes gate columns and B1 the up columns of
+// the same places, so both meet in one wave; p.bias [N]. 2 xIELU with the coefficients p.coef [2], N a multiple of 256, rows of out in
+// 16-byte pieces. bf16 out. K 4096, width 14336, two launches against
+// one, 300 / 1531 / 2048 rows: gated 111 / 300 / 383 -> 101 / 271 / 350 us, xIELU (fp32 between the two) 60 / 169 / 222 -> 59 / 159 / 205.
+template <bool F8, bool CMAX = false, bool TAIL = false, int ACT = 0>
 __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams p) {
   static_assert(!(CMAX && TAIL), "the chunk maxima of a half tile would need their own rows");
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -132,7 +138,8 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
   const char* bsrc[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const int nt = cb_l * 16 + h * 8 + wave;
+    int nt = cb_l * 16 + h * 8 + wave;
+    if constexpr (ACT == 1) nt = cb * 8 + wave < p.N >> 5 ? (h ? p.N >> 5 : 0) + cb * 8 + wave : p.ntiles;
     bsrc[h] = reinterpret_cast<const char*>(p.wp) + ((long)(nt < p.ntiles ? nt : wave) * KT + (long)c0 * 2) * 1024 + lane * 16;
   }
   // kind: 0 A0, 1 B0, 2 B1, 3 A1 (the order of the stream); c = K-tile of this split; par = its LDS buffer
@@ -424,6 +431,55 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
         }
       }
   }
+  if constexpr (ACT == 1) {
+    float* const st = reinterpret_cast<float*>(smem);
+    const int F = p.N >> 1;
+    f32x4 bg[2], bu[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int col = cb * 128 + wc * 32 + j * 16 + quad * 4;
+      bg[j] = bu[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (p.bias && col < F) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { bg[j][e] = (float)p.bias[col + e]; bu[j][e] = (float)p.bias[F + col + e]; }
+      }
+    }
+    pp_barrier();                                  // the area is free
+#pragma unroll
+    for (int hm = 0; hm < 2; ++hm) {
+      if (TAIL && half && hm) break;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          f32x4 o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = gelu_tanh(acc[hm][0][i][j][e] + bg[j][e]) * (acc[hm][1][i][j][e] + bu[j][e]);
+          *reinterpret_cast<f32x4*>(st + (hm * 128 + wr * 64 + i * 16 + l15) * 128 + (((wc * 8 + j * 4 + quad) ^ l15) << 2)) = o;
+        }
+    }
+    pp_staged();
+    const int cl = lane & 15, rows = TAIL && half ? 16 : 32, col = cb * 128 + cl * 8;      // (rows of a wave)
+    const bool wide = (cb + 1) * 128 <= F && (p.ldo & 7) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      if (TAIL && half && s >= 4) break;
+      const int R = wave * rows + s * 4 + (lane >> 4), m = mrow0 + R;
+      const float* row = st + R * 128;
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(row + (((2 * cl) ^ (R & 15)) << 2));
+      const f32x4 hi = *reinterpret_cast<const f32x4*>(row + (((2 * cl + 1) ^ (R & 15)) << 2));
+      const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      bf16* const to = reinterpret_cast<bf16*>(p.out) + (long)m * p.ldo + col;
+      if (m >= p.M) continue;
+      if (wide) st16(to, pack8(v));
+      else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (col + e < F) to[e] = (bf16)v[e];
+      }
+    }
+    return;
+  }
   // ---- row-wise epilogue for what a Llama layer asks of this kernel ------------------------------------
   // bf16 out, the whole 256-column block inside N: plain (+ bias, GELU, + residual: QKV, O, down, GPT-2's MLP) and SwiGLU (gate / up).
   // In the accumulator layout a lane holds 4 columns of one row of a tile: a store writes 8 bytes per lane into 16
@@ -432,11 +488,12 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
   // on different banks — and every wave stores whole rows: 16 bytes per lane, two rows of 512 contiguous bytes (four
   // of 256 for SwiGLU) per instruction, the residual read the same way. Plain: one row half (128 x 256 fp32 = the
   // whole 128 KiB) at a time; SwiGLU: gate and up meet in registers, the 256 x 128 results are staged at once.
-  if (!p.out_f32 && (cb + 1) * 256 <= p.N && (PP_ABL & 4096) == 0 &&
+  const float ap = ACT == 2 ? p.coef[0] : 0.f, aq = ACT == 2 ? p.coef[1] : 0.f;
+  if (ACT == 2 || (!p.out_f32 && (cb + 1) * 256 <= p.N && (PP_ABL & 4096) == 0 &&
       (p.act != 1 || (p.residual == nullptr && p.bias == nullptr)) && ((p.ldo | p.ldr) & 7) == 0 &&
-      ((reinterpret_cast<uintptr_t>(p.out) | reinterpret_cast<uintptr_t>(p.residual) | reinterpret_cast<uintptr_t>(p.bias)) & 15) == 0) {
+      ((reinterpret_cast<uintptr_t>(p.out) | reinterpret_cast<uintptr_t>(p.residual) | reinterpret_cast<uintptr_t>(p.bias)) & 15) == 0)) {
     float* const st = reinterpret_cast<float*>(smem);
-    if (p.act != 1) {
+    if (ACT == 2 || p.act != 1) {
       const int cl = lane & 31, rsub = lane >> 5;
       float b8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       if (p.bias) unpack8(ld16(p.bias + cb * 256 + cl * 8), b8);
@@ -472,7 +529,10 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] += b8[e];
           }
-          if (p.act == 2) {
+          if constexpr (ACT == 2) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = xielu(v[e], ap, aq);
+          } else if (p.act == 2) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = gelu_tanh(v[e]);
           }
@@ -932,27 +992,27 @@ extern "C" long dlia_gemm_pingpong_ws_floats(int M, int N, int K) {
 // bf16, M > 256 (any M is correct; below that the weight-streaming kernels are faster), K a
 // multiple of 64; `p` fully set up by the caller. p->splitk > 1 needs p->partial = slabs for
 // [tiles][splitk - 1] and p->counters = two zero words per tile (the kernel leaves them zero).
-template <bool F8, bool CMAX = false, bool TAIL = false>
+template <bool F8, bool CMAX = false, bool TAIL = false, int ACT = 0>
 static void launch_pingpong_kernel(const dlia::GemmParams* p, int workgroups, hipStream_t stream) {
   constexpr int lds = TAIL ? kPPTailLds : kPPLds;
   static const bool once = [] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_pingpong_kernel<F8, CMAX, TAIL>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_pingpong_kernel<F8, CMAX, TAIL, ACT>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     return true;
   }();
   (void)once;
-  hipLaunchKernelGGL((gemm_pingpong_kernel<F8, CMAX, TAIL>), dim3(workgroups), dim3(kPPThreads), lds, stream, *p);
+  hipLaunchKernelGGL((gemm_pingpong_kernel<F8, CMAX, TAIL, ACT>), dim3(workgroups), dim3(kPPThreads), lds, stream, *p);
 }
-template <bool F8, bool CMAX = false>
+template <bool F8, bool CMAX = false, int ACT = 0>
 static void launch_pingpong(const dlia::GemmParams* p, hipStream_t stream) {
   const int nb = (p->ntiles + 15) / 16, nb8 = (nb + 7) / 8 * 8, mblocks = (p->M + 255) / 256;
   if constexpr (!CMAX) {
     if (p->full_items >= 0) {
-      launch_pingpong_kernel<F8, false, true>(p, 8 * (p->full_items + 2 * (nb8 / 8 * mblocks - p->full_items)), stream);
+      launch_pingpong_kernel<F8, false, true, ACT>(p, 8 * (p->full_items + 2 * (nb8 / 8 * mblocks - p->full_items)), stream);
       return;
     }
   }
-  launch_pingpong_kernel<F8, CMAX>(p, nb8 * mblocks * p->splitk, stream);
+  launch_pingpong_kernel<F8, CMAX, false, ACT>(p, nb8 * mblocks * p->splitk, stream);
 }
 static void launch_quad(const dlia::GemmParams* p, hipStream_t stream) {
   static const bool once = [] {
@@ -995,6 +1055,27 @@ extern "C" void dlia_gemm_large(void* out, const void* x, const void* wp, const 
     p.counters = reinterpret_cast<int*>(workspace + ws_floats - kPPCounters);
   }
   dlia_gemm_pingpong(&p, stream);
+}
+
+// The same with a feed-forward's activation: act 1 gelu_tanh(gate) * up, out [M, N / 2] (N / 2 a multiple of 16; weight rows: the gate's, then
+// the up projection's; bias [N] or null), act 2 xIELU, out [M, N], N a multiple of 256, coef [2]. bf16 out. Always the kernel above, whatever else is chosen.
+extern "C" void dlia_gemm_large_act(void* out, const void* x, const void* wp, const void* bias, const float* coef, float* workspace, long ws_floats,
+                                    int M, int N, int K, long ldx, long ldo, int act, int wg_target, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return;
+  GemmParams p;
+  p.x = (const bf16*)x; p.ldx = ldx; p.wp = (const u32x4*)wp; p.wscale = nullptr; p.xscale = nullptr; p.out = out; p.ldo = ldo;
+  p.bias = act == 1 ? (const bf16*)bias : nullptr; p.residual = nullptr; p.ldr = 0; p.coef = coef;
+  p.partial = workspace; p.M = M; p.N = N; p.K = K; p.ntiles = packed_ntiles(N);
+  p.act = 0; p.out_f32 = 0; p.partial_only = 0; p.splitk = 1; p.group_n = 1; p.counters = nullptr;
+  p.full_items = dlia_gemm_pingpong_whole(M, N, K / 64, wg_target > 128);
+  const int s = p.full_items >= 0 ? 1 : pp_splitk(M, N, K / 64, wg_target);
+  const long tiles = (long)((M + 255) / 256) * ((p.ntiles + 15) / 16);
+  if (workspace && s > 1 && ws_floats >= tiles * (s - 1) * kPPSlab + kPPCounters) {
+    p.splitk = s;
+    p.counters = reinterpret_cast<int*>(workspace + ws_floats - kPPCounters);
+  }
+  if (act == 1) launch_pingpong<false, false, 1>(&p, stream);
+  else launch_pingpong<false, false, 2>(&p, stream);
 }
 
 // The same for e4m3 x e4m3 (dlia_gemm_a8w8's contract: xq bytes [M, K] with row stride ldx BYTES,

@@ -1012,16 +1012,6 @@ __global__ __launch_bounds__(64) void rglru_stretch_kernel(
 }
 
 // ---- activation, scaling ---------------------------------------------------------------------------------------------
-// exp(v) - 1 - v for v <= 0: the series above -1/2 (what it leaves out is under 2^-29 of the value; expm1f(v) - v cancels there). Both cases are
-// evaluated, some 16 instructions in all.
-__device__ __forceinline__ float exp_rest(float v) {
-  float c = 1.f / 362880.f;
-  const float inv[7] = {1.f / 40320.f, 1.f / 5040.f, 1.f / 720.f, 1.f / 120.f, 1.f / 24.f, 1.f / 6.f, 0.5f};
-#pragma unroll
-  for (int i = 0; i < 7; ++i) c = __builtin_fmaf(c, v, inv[i]);
-  return v > -0.5f ? v * v * c : exp_c(v) - (1.f + v);
-}
-
 // V entries of a row per thread. Bound by its bytes: 1531 rows of 14336, bf16 out, 23 us (5.8 TB/s, half of them from the last-level
 // cache); 43 with an entry a thread and expm1f, whose two cases both run in a wave that holds both.
 template <typename OT, int V>
@@ -1034,10 +1024,7 @@ __global__ __launch_bounds__(256) void xielu_kernel(OT* __restrict__ act, const 
   const float ap = pq[0], aq = pq[1];          // softplus(p), 1/2 + softplus(q)
   Unit<V> u = ldu<V>(z + (long)m * ldz + c);
 #pragma unroll
-  for (int e = 0; e < V; ++e) {
-    const float v = u.v[e];
-    u.v[e] = v > 0.f ? ap * v * v + 0.5f * v : aq * exp_rest(v) + 0.5f * v;
-  }
+  for (int e = 0; e < V; ++e) u.v[e] = xielu(u.v[e], ap, aq);
   stu<V>(act + (long)m * lda + c, u);
 }
 

@@ -532,6 +532,39 @@ def test_gemm_large_m_halves_of_the_last_round(K, shape, epi, f32, f8):
         K.large_gemm_kernel(prev)
 
 
+@pytest.mark.parametrize("M,F,Kd,act", [(300, 80, 128, 1), (1531, 5504, 128, 1), (2011, 7168, 384, 1), (600, 1408, 1024, 1), (257, 144, 256, 1),
+                                        (300, 256, 128, 2), (1531, 14336, 128, 2), (600, 1536, 1024, 2), (2011, 2048, 384, 2)])
+@pytest.mark.parametrize("pad", [0, 4])
+def test_gemm_large_m_with_the_feed_forwards_activation(K, M, F, Kd, act, pad):
+    """Whole tiles, halves of the last round and K splits, ragged column blocks; rows of the gated form's output that are no whole 16-byte pieces.
+    Pre-activations are sums of Kd products in fp32; a slope of up to 1.13 (GELU) or 2 p |z| + 1.3 (xIELU) and one rounding behind them."""
+    if act == 2 and pad:
+        pad = 8
+    g = torch.Generator(device=DEV).manual_seed(M + F)
+    N = 2 * F if act == 1 else F
+    x, w = bf(torch.randn(M, Kd, device=DEV, generator=g)), bf(torch.randn(N, Kd, device=DEV, generator=g) / math.sqrt(Kd))
+    bias = bf(torch.randn(N, device=DEV, generator=g)) if act == 1 and M != 600 else None
+    coef = torch.tensor([0.9, 1.2], device=DEV)
+    ws = torch.zeros(int(K.gemm_ws_floats(M, N, Kd)) + 4096, device=DEV)
+    big = torch.full((M + 1, F + pad), 7.0, device=DEV, dtype=torch.bfloat16)
+    K.gemm_act(big[:M, :F], x, packing.pack_weight(w), bias, coef if act == 2 else None, ws, N, act, 256)
+    z = x.double() @ w.double().t() + (bias.double() if bias is not None else 0.0)
+    m = (Kd + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + 4.0)
+    if act == 1:
+        gt, u = z[:, :F], z[:, F:]
+        h = torch.nn.functional.gelu(gt, approximate="tanh")
+        want = h * u
+        err = 1.13 * m[:, :F] * (u.abs() + m[:, F:]) + (h.abs() + 2.0 ** -21 * gt.abs()) * m[:, F:] + 2.0 ** -20 * gt.abs() * u.abs()
+    else:
+        p, q = coef.double()
+        want = torch.where(z > 0, p * z * z, q * (torch.expm1(z.clamp(max=0)) - z)) + 0.5 * z
+        err = m * (2 * p * (z.abs() + m) + 1.3) + 2.0 ** -22 * (z * z + q * (1 + z.abs()))
+    out = big[:M, :F].double()
+    assert bool(((out - want).abs() <= err + 2.0 ** -8 * want.abs()).all())
+    assert bool((big[M] == 7.0).all()) and (not pad or bool((big[:, F:] == 7.0).all()))
+    assert int(ws[-4096:].view(torch.int32).abs().sum()) == 0
+
+
 def test_gemm_large_m_halves_where_they_measured_faster(K):
     whole = K.gemm_large_whole          # us: whole tiles or K splits against halves
     assert whole(1531, 14336, 64, True) == 32 and whole(2048, 28672, 64, True) == 96 and whole(1290, 14336, 64, True) == 32          # 162 / 141, 417 / 402, 160 / 137
