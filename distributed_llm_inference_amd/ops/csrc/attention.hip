@@ -500,9 +500,11 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
 // KV block through LDS. A (block, kv head) is K slab + V slab back to back in memory and already
 // in fragment order, so staging it is a linear copy (16 B per thread and piece) and a fragment
 // is one conflict-free ds_read_b128 at fragment*1 KiB + lane*16 (an e4m3 cache is widened to bf16
-// while it is staged, once per workgroup). Block k+1 is loaded global -> registers while block k
-// is computed, then written to the other buffer: one barrier per block.
-// No cross-wave merge, 33 KB of LDS, K/V are fetched once per 128 columns.
+// while it is staged, once per workgroup). A bf16 cache's blocks go straight into one of four LDS slots
+// while the blocks before them are computed, two at a time where nothing is masked: one barrier, one maximum and one
+// rescale per 64 keys. (Staged through registers block by block, as an e4m3 cache's still are: 64 heads on 8, 1024 tokens behind
+// 4096 241 -> 201 us, 0.77 PFLOP/s; 32 heads, 2048 tokens 85 -> 72, 8192 704 -> 671; five prompts of 400 28 -> 25.)
+// No cross-wave merge, 64 KB of LDS, K/V are fetched once per 128 columns.
 // Softmax work per score is cut to what the hardware needs: raw v_exp_f32 (results below the
 // normal range flush to zero, which a probability may), one FMA instead of subtract + multiply,
 // the causal mask only in blocks that can reach the wave's diagonal, the accumulator rescale only
@@ -533,7 +535,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnParams p) {
   constexpr int MEM_BYTES = KV8 ? BLOCK_BYTES / 2 : BLOCK_BYTES;      // ... and as stored in the cache
   constexpr int PIECES = MEM_BYTES / (256 * 16);
   static_assert(PIECES >= 1 && PIECES * 256 * 16 == MEM_BYTES, "a block is whole 16-byte pieces per thread");
-  constexpr int BUF = BLOCK_BYTES + 256;                              // + the block's 64 fp32 scales (KV8)
+  constexpr int BUF = BLOCK_BYTES + (KV8 ? 256 : 0);                  // + the block's 64 fp32 scales (KV8)
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, l15 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -625,13 +627,24 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnParams p) {
   }
 
   const int* table = p.block_table + (long)srow * p.max_blocks;
-  u32x4 stage[PIECES];
-  f32x4 sstage = {0.f, 0.f, 0.f, 0.f};
+  [[maybe_unused]] u32x4 stage[KV8 ? PIECES : 1];
+  [[maybe_unused]] f32x4 sstage = {0.f, 0.f, 0.f, 0.f};
+  [[maybe_unused]] const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  // bf16: a block is 4 NP pieces of 1 KiB, NP a wave, straight into LDS
+  [[maybe_unused]] auto bring = [&](int blk, int boff) {
+    blk = (srow_ok && blk >= 0 && blk < p.num_blocks) ? blk : 0;            // never a wild read
+    constexpr int NP = BLOCK_BYTES / 4096;
+    const char* src = reinterpret_cast<const char*>(p.kv) + kv_head_base(blk, kvh, p.Hkv, D, 0) * 2 + wave * (NP * 1024) + lane * 16;
+    const void* g[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) g[i] = src + i * 1024;
+    lds_dma_run<NP>(g, __builtin_amdgcn_readfirstlane(lds0 + boff + wave * (NP * 1024)));
+  };
   auto gload = [&](int blk) {
     blk = (srow_ok && blk >= 0 && blk < p.num_blocks) ? blk : 0;            // never a wild read
     const char* src = reinterpret_cast<const char*>(p.kv) + kv_head_base(blk, kvh, p.Hkv, D, 0) * (KV8 ? 1 : 2);
 #pragma unroll
-    for (int i = 0; i < PIECES; ++i) stage[i] = *reinterpret_cast<const u32x4*>(src + (i * 256 + tid) * 16);
+    for (int i = 0; i < (KV8 ? PIECES : 1); ++i) stage[i] = *reinterpret_cast<const u32x4*>(src + (i * 256 + tid) * 16);
     if constexpr (KV8) {
       if (tid < 16) sstage = *reinterpret_cast<const f32x4*>(p.kv_scale + kv_scale_base(blk, kvh, p.Hkv, 0) + tid * 4);
     }
@@ -641,13 +654,11 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnParams p) {
   // waves read plain bf16 fragments and the compute path is the bf16 one plus the two scale multiplies.
   auto lstore = [&](int boff) {
 #pragma unroll
-    for (int i = 0; i < PIECES; ++i) {
+    for (int i = 0; i < (KV8 ? PIECES : 0); ++i) {
       if constexpr (KV8) {
         const int run = i * 4 + (tid >> 6);
         *reinterpret_cast<u32x4*>(smem + boff + (2 * run) * 1024 + lane * 16) = fp8x8_to_bf16x8(stage[i][0], stage[i][1]);
         *reinterpret_cast<u32x4*>(smem + boff + (2 * run + 1) * 1024 + lane * 16) = fp8x8_to_bf16x8(stage[i][2], stage[i][3]);
-      } else {
-        *reinterpret_cast<u32x4*>(smem + boff + (i * 256 + tid) * 16) = stage[i];
       }
     }
     if constexpr (KV8) {
@@ -655,8 +666,10 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnParams p) {
     }
   };
 
-  auto process = [&](int kb, int boff, auto mask_c) {
+  // N neighbouring blocks (kb, kb + 1) side by side in LDS: one maximum, one rescale and one barrier for all of their keys
+  auto process = [&](int kb, int boff, auto mask_c, auto n_c) {
     constexpr bool MASK = decltype(mask_c)::value;
+    constexpr int N = decltype(n_c)::value;
     f32x4 sk[2], sv[2];
     if constexpr (KV8) {
 #pragma unroll
@@ -665,12 +678,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnParams p) {
         sv[kt] = *reinterpret_cast<const f32x4*>(smem + boff + BLOCK_BYTES + (kBlockTokens + kt * 16 + quad * 4) * 4);
       }
     }
-    f32x4 st[2][NT];
+    f32x4 st[2 * N][NT];
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
+    for (int kt = 0; kt < 2 * N; ++kt) {
       u32x4 kf[KS];
 #pragma unroll
-      for (int s = 0; s < KS; ++s) kf[s] = *reinterpret_cast<const u32x4*>(smem + boff + (kt * KS + s) * 1024 + lane * 16);
+      for (int s = 0; s < KS; ++s)
+        kf[s] = *reinterpret_cast<const u32x4*>(smem + boff + (kt >> 1) * BUF + ((kt & 1) * KS + s) * 1024 + lane * 16);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         f32x4 a = {0.f, 0.f, 0.f, 0.f};
@@ -680,14 +694,14 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnParams p) {
         st[kt][nt] = a;
       }
     }
-    u32x4 pf[NT];
+    u32x4 pf[N][NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       float mx = kNegInf;
       if constexpr (CAPPED) {
         if (p.cap > 0.f) {
 #pragma unroll
-          for (int kt = 0; kt < 2; ++kt)
+          for (int kt = 0; kt < 2 * N; ++kt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) st[kt][nt][r] = p.cap * tanh_exp(st[kt][nt][r] * p.inv_cap);
         }
@@ -696,7 +710,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnParams p) {
         if (p.temp || p.bias) {
           const int qabs = ctx + col_qpos[nt];
 #pragma unroll
-          for (int kt = 0; kt < 2; ++kt)
+          for (int kt = 0; kt < 2 * N; ++kt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const int dist = min(max(qabs - (kb * kBlockTokens + kt * 16 + quad * 4 + r), 0), p.bias_rows - 1);
@@ -707,7 +721,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnParams p) {
       if constexpr (MASK) {
         const int limit = col_qpos[nt] >= 0 ? ctx + col_qpos[nt] : -1;   // last visible key position
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+        for (int kt = 0; kt < 2 * N; ++kt)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int kpos = kb * kBlockTokens + kt * 16 + quad * 4 + r;
@@ -719,7 +733,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnParams p) {
           }
       } else {
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+        for (int kt = 0; kt < 2 * N; ++kt)
 #pragma unroll
           for (int r = 0; r < 4; ++r) mx = fmaxf(mx, st[kt][nt][r]);
       }
@@ -729,28 +743,34 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnParams p) {
       const float ms = m_safe * p.scale_log2;
       const float alpha = __builtin_amdgcn_exp2f(__builtin_fmaf(m[nt], p.scale_log2, -ms));     // m = -inf -> 0
       m[nt] = m_new;
-      float pv[8], rs = 0.f;
+      float pv[8 * N], rs = 0.f;
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
+      for (int kt = 0; kt < 2 * N; ++kt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kt][nt][r], p.scale_log2, -ms));   // masked: -inf -> 0
           rs += e;
-          pv[kt * 4 + r] = KV8 ? e * sv[kt][r] : e;       // V's per-key scale rides in P^T
+          pv[kt * 4 + r] = KV8 ? e * sv[kt & 1][r] : e;       // V's per-key scale rides in P^T
         }
       l[nt] = l[nt] * alpha + rs;
       if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[dt][nt] *= alpha;
       }
-      pf[nt] = pack8(pv);
+#pragma unroll
+      for (int u = 0; u < N; ++u) {
+        const float pu[8] = {pv[u * 8], pv[u * 8 + 1], pv[u * 8 + 2], pv[u * 8 + 3], pv[u * 8 + 4], pv[u * 8 + 5], pv[u * 8 + 6], pv[u * 8 + 7]};
+        pf[u][nt] = pack8(pu);
+      }
     }
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      const u32x4 vf = *reinterpret_cast<const u32x4*>(smem + boff + BLOCK_BYTES / 2 + dt * 1024 + lane * 16);
+    for (int u = 0; u < N; ++u)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) o[dt][nt] = mfma16(vf, pf[nt], o[dt][nt]);
-    }
+      for (int dt = 0; dt < DT; ++dt) {
+        const u32x4 vf = *reinterpret_cast<const u32x4*>(smem + boff + u * BUF + BLOCK_BYTES / 2 + dt * 1024 + lane * 16);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) o[dt][nt] = mfma16(vf, pf[u][nt], o[dt][nt]);
+      }
   };
 
   // The block table is read 64 entries at a time, one per lane; a block's entry is then a v_readlane:
@@ -761,7 +781,22 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnParams p) {
   // windowed: the walk starts at the block of the first key that the tile's first query still sees
   const int kb_lo = (WIN && p.window > 0 && tile_live) ? min(max(0, ctx + qp0 - p.window + 1) / kBlockTokens, nb) : 0;
   tbl_fill(kb_lo & ~63);
-  if (nb > kb_lo) { gload(tbl_at(kb_lo)); lstore((kb_lo & 1) * BUF); }
+  // Four slots: block kb lies in slot (kb - kb_lo) % 4. Blocks up to `upto` are on their way behind this call.
+  [[maybe_unused]] int brought = kb_lo;
+  [[maybe_unused]] auto bring_to = [&](int upto) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (brought >= upto) break;
+      if ((brought & 63) == 0) tbl_fill(brought);
+      bring(tbl_at(brought), ((brought - kb_lo) & 3) * BUF);
+      ++brought;
+    }
+  };
+  if constexpr (KV8) {
+    if (nb > kb_lo) { gload(tbl_at(kb_lo)); lstore((kb_lo & 1) * BUF); }
+  } else {
+    bring_to(min(nb, kb_lo + 2));
+  }
   // Everything loaded so far (the Q fragments, block 0) has landed before the loop starts: vmcnt is
   // one in-order counter, so a wait for a prologue load placed inside the loop would also wait for
   // the prefetch of the next block that was issued just before it.
@@ -789,14 +824,33 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnParams p) {
         gload(tbl_at(kb + 1));
       }
       // masked loop: a block whose first key is beyond the wave's last column is skipped altogether
-      if (wave_live && (!MASK || kb * kBlockTokens <= lim_last)) process(kb, boff, mask_c);
+      if (wave_live && (!MASK || kb * kBlockTokens <= lim_last)) process(kb, boff, mask_c, std::integral_constant<int, 1>{});
       if (kb + 1 < nb) lstore(BUF - boff);
       __syncthreads();
     }
   };
-  if constexpr (WIN) run(kb_lo, kb_mid, std::true_type{});
-  run(kb_mid, nb_full, std::false_type{});
-  run(nb_full, nb, std::true_type{});
+  if constexpr (KV8) {
+    if constexpr (WIN) run(kb_lo, kb_mid, std::true_type{});
+    run(kb_mid, nb_full, std::false_type{});
+    run(nb_full, nb, std::true_type{});
+  } else {
+    // Without a mask two blocks at a time, one maximum, one rescale and one barrier for their 64 keys; with one block by block. At a step
+    // its blocks have landed and every wave is done with the blocks before them; the two blocks behind the step's go into their slots.
+    int kb = kb_lo;
+    auto step = [&](auto mask_c, auto n_c) {
+      constexpr int N = decltype(n_c)::value;
+      if (N == 1 && brought > kb + 1) wait_pieces<BLOCK_BYTES / 4096>();      // (the block behind this one may still be on its way)
+      else wait_pieces<0>();
+      __syncthreads();
+      bring_to(min(nb, kb + N + 2));
+      if (wave_live && (!decltype(mask_c)::value || kb * kBlockTokens <= lim_last)) process(kb, ((kb - kb_lo) & 3) * BUF, mask_c, n_c);
+      kb += N;
+    };
+    if constexpr (WIN)
+      while (kb < kb_mid || (kb < nb_full && ((kb - kb_lo) & 1))) step(std::true_type{}, std::integral_constant<int, 1>{});
+    while (kb + 1 < nb_full) step(std::false_type{}, std::integral_constant<int, 2>{});
+    while (kb < nb) step(std::true_type{}, std::integral_constant<int, 1>{});
+  }
 
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
@@ -832,9 +886,9 @@ static inline bool capped(const AttnParams& p) { return p.cap > 0.f || p.egate; 
 template <int D>
 static void launch_prefill_attn(const AttnParams& p, hipStream_t stream) {
   const long nitems = p.xcd_map > 1 ? 8L * ((p.qtiles + p.xcd_map - 1) / p.xcd_map) : (long)p.B * p.Hkv * p.qtiles;
-  constexpr size_t smem = 2 * (4 * kBlockTokens * D + 256);      // two bf16 blocks + their scales
+  constexpr size_t smem8 = 2 * (4 * kBlockTokens * D + 256), smem = 4 * (4 * kBlockTokens * D);      // two bf16 blocks + their scales (e4m3 cache), or four blocks
   const bool win = p.window > 0 || p.sink;
-  if (p.kv_scale) hipLaunchKernelGGL((prefill_attn_kernel<D, true>), dim3((unsigned)nitems), dim3(256), smem, stream, p);
+  if (p.kv_scale) hipLaunchKernelGGL((prefill_attn_kernel<D, true>), dim3((unsigned)nitems), dim3(256), smem8, stream, p);
   else if (capped(p)) hipLaunchKernelGGL((prefill_attn_kernel<D, false, 2>), dim3((unsigned)nitems), dim3(256), smem, stream, p);
   else if (win)   hipLaunchKernelGGL((prefill_attn_kernel<D, false, 1>), dim3((unsigned)nitems), dim3(256), smem, stream, p);
   else            hipLaunchKernelGGL((prefill_attn_kernel<D, false>), dim3((unsigned)nitems), dim3(256), smem, stream, p);

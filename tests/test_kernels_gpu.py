@@ -497,6 +497,53 @@ def test_gemm_a8w8_large_kernels_agree_on_edge_shapes(K, which, shape):
         K.large_gemm_kernel(prev)
 
 
+@pytest.mark.parametrize("window", [0, 100, 517])
+@pytest.mark.parametrize("H,G,D", [(8, 2, 128), (4, 4, 64), (6, 2, 128)])
+@pytest.mark.parametrize("lens", [[(0, 200), (31, 129), (64, 300)], [(1985, 140), (2080, 133)], [(2016, 129), (0, 161), (1, 257)]])
+def test_prefill_attention_steps_of_two_blocks(K, lens, H, G, D, window):
+    """Portions whose key blocks are odd and even in number, first blocks of a window at odd places, more than the 64 blocks of which the table's
+    entries are held at a time. Weights are rounded to bf16 (8 significant bits: by up to 2^-8 of each, the sum is of the unrounded ones),
+    the result once more; the fp32 scores move a weight by less than 2^-11 of itself."""
+    g = torch.Generator(device=DEV).manual_seed(len(lens) + window)
+    B, tot = len(lens), sum(n for _, n in lens)
+    nb = [(c + n + 31) // 32 for c, n in lens]
+    cos, sin = (torch.ones(4096, D // 2, device=DEV), torch.zeros(4096, D // 2, device=DEV))      # (rows as they are)
+    kv = torch.zeros(sum(nb) + 1, G, 2, 32 * D, device=DEV, dtype=torch.bfloat16)
+    perm = torch.randperm(sum(nb), generator=torch.Generator().manual_seed(3)).int() + 1
+    table = torch.zeros(B, max(nb), dtype=torch.int32)
+    at = 0
+    for b in range(B):
+        table[b, :nb[b]] = perm[at:at + nb[b]]
+        at += nb[b]
+    table, i32 = table.to(DEV), lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    full = [bf(torch.randn(c + n, (H + 2 * G) * D, device=DEV, generator=g)) for c, n in lens]
+    for b, (c, n) in enumerate(lens):                  # the cache as the steps before left it, and this step's rows
+        pos = torch.arange(c + n, device=DEV, dtype=torch.int32)
+        K.rope_kvwrite(full[b].clone(), None, 1, None, kv, cos, sin, pos, torch.full_like(pos, b), table, H, G, D, False)
+    qkv = torch.cat([f[c:] for f, (c, n) in zip(full, lens)])
+    starts = [0]
+    for _, n in lens:
+        starts.append(starts[-1] + n)
+    out = torch.zeros(tot, H * D, device=DEV, dtype=torch.bfloat16)
+    scale = D ** -0.5
+    K.paged_attention_window(out, qkv, kv, i32(starts), i32([c for c, _ in lens]), table, i32(list(range(B))), None, max(n for _, n in lens), H, G, D,
+                             scale, 1, window, window > 0)
+    for b, (c, n) in enumerate(lens):
+        f = full[b].double()
+        i, j = torch.arange(c, c + n, device=DEV)[:, None], torch.arange(c + n, device=DEV)[None]
+        seen = (j <= i) & ((i - j < window) if window else True)
+        for h in range(H):
+            q, k = f[c:, h * D:(h + 1) * D], f[:, (H + h // (H // G)) * D:(H + h // (H // G) + 1) * D]
+            v = f[:, (H + G + h // (H // G)) * D:(H + G + h // (H // G) + 1) * D]
+            sc = (q @ k.t() * scale).masked_fill(~seen, float("-inf"))
+            if window:                                 # (one more score of 0 without a value)
+                sc = torch.cat([sc, torch.zeros(n, 1, device=DEV, dtype=torch.float64)], 1)
+            w = torch.softmax(sc, -1)[:, :c + n]
+            want, bound = w @ v, (2.0 ** -8 + 2.0 ** -11) * (w @ v.abs())
+            got = out[starts[b]:starts[b + 1], h * D:(h + 1) * D].double()
+            assert bool(((got - want).abs() <= bound + 2.0 ** -8 * want.abs() + 1e-6).all()), (b, h)
+
+
 @pytest.mark.parametrize("f8", [False, True], ids=["bf16", "e4m3"])
 @pytest.mark.parametrize("epi,f32", [(0, False), (0, True), (1, False), (2, False), (3, True), (4, False), (5, False)])
 @pytest.mark.parametrize("shape", [(1531, 14336, 1), (1290, 14200, 2), (300, 4096, 3), (257, 4000, 4), (2011, 4096, 5), (512, 2048, 7)])
