@@ -118,6 +118,7 @@ _CAPTURE_LOCK = threading.RLock()
 
 class GpuStage:
     backend = "hip"
+    _first_norm_enters = True        # (captured steps: the first norm reads the input buffer, the last fold writes the output buffer)
 
     def __init__(self, spec: ModelSpec, plan: StagePlan, weights: StageWeights, *, device="cuda",
                  max_slots: int = 256, max_seq_len: int = 2048, num_blocks: Optional[int] = None,
@@ -448,8 +449,8 @@ class GpuStage:
         return c
 
     def _layers(self, wk: _Work, T: int, B: int, tok_pos, tok_seq, q_start, ctx, slots, max_q: int, splits: int,
-                alone: bool = False, lead_decode: int = 0):
-        """Runs this stage's decoder layers on wk.h[:T]. Returns the pending split-K partial
+                alone: bool = False, lead_decode: int = 0, entry: Optional[torch.Tensor] = None):
+        """Runs this stage's decoder layers on wk.h[:T] (decode regime: or on the rows `entry`, which wk.h takes over). Returns the pending split-K partial
         (splits, bias) of the last down projection that the caller still has to fold into h
         (decode regime), or None when h is final. `lead_decode`: the first that many sequences of a
         ragged step are single decode tokens riding with prompt chunks; their attention runs on the
@@ -512,7 +513,10 @@ class GpuStage:
         pend = None
         for li, p in enumerate(self.layers):
             if "w_qkv" in p:
-                if pend is None:
+                if pend is None and entry is not None:
+                    x1 = None if fp8 else xn
+                    K.norm_enter(wk.xq[:T, :H] if fp8 else xn, wk.xs if fp8 else None, h, entry, p["ln1_w"], p.get("ln1_b"), s.norm_eps, nmode)
+                elif pend is None:
                     x1 = norm(None, 1, None, p["ln1_w"], p.get("ln1_b"))
                 else:
                     x1 = norm(ws, pend[0], pend[1], p["ln1_w"], p.get("ln1_b"))
@@ -700,17 +704,22 @@ class GpuStage:
     def _decode_body(self, st: _MicroBatchState):
         """One decode step over the micro-batch's static buffers (captured into the graph)."""
         K, B, wk = self.K, st.B, st.wk
+        entry = {}
         if self.plan.has_embed:
             self._embed_rows(wk, B, st.ids, st.ctx, st.slots)
+        elif self._first_norm_enters and B <= self.decode_rows and self.layers and "w_qkv" in self.layers[0]:
+            entry = {"entry": st.hidden_in}
         else:
             wk.h[:B].copy_(st.hidden_in)
-        pend = self._layers(wk, B, B, st.ctx, st.slots, self._arange[:B + 1], st.ctx, st.slots, 1, st.splits)
+        pend = self._layers(wk, B, B, st.ctx, st.slots, self._arange[:B + 1], st.ctx, st.slots, 1, st.splits, **entry)
         if self.plan.has_head:
             self._head(wk, self._arange, B, B, pend)
             # the thread that writes a row's token also advances the row's draw counter and context length and — single-stage
             # pipeline, where the feedback hop is local — puts the token into the next step's input ids
             K.sample_step(st.tokens, wk.logits[:B], wk.cmax[:B] if wk.guided else None, st.temperature, st.top_k, st.top_p,
                           st.seeds, st.steps, self.spec.vocab_size, st.ids if self.plan.has_embed else None, st.ctx)
+        elif self._first_norm_enters and pend is not None:
+            K.fold_out(st.hidden_out, wk.h[:B], wk.ws, pend[0], pend[1], st.ctx)
         else:
             self._fold(wk, B, pend)
             st.hidden_out.copy_(wk.h[:B])

@@ -121,6 +121,7 @@ class _HybridWork:
 
 class HybridGpuStage(GpuStage):
     backend = "hip"
+    _first_norm_enters = False
 
     def __init__(self, spec: ModelSpec, plan: StagePlan, weights: StageWeights, *, device="cuda", max_slots: int = 256,
                  max_seq_len: int = 2048, num_blocks: Optional[int] = None, max_tokens: int = 2048, max_batch: int = 64,

@@ -52,7 +52,7 @@ inline void check_rows(const Tensor& t, const char* name) {
 
 // out[r,:] = norm(x[row_idx[r] or r,:] (+addend -> x)) * w (+ b); mode 0 rms, 1 layernorm, 2 fold only.
 static void norm_impl(Tensor out, Tensor x, OptTensor delta, OptTensor partial, int64_t splits, OptTensor pbias,
-                      const Tensor& w, OptTensor b, OptTensor row_idx, double eps, int64_t mode, OptTensor qscale) {
+                      const Tensor& w, OptTensor b, OptTensor row_idx, double eps, int64_t mode, OptTensor qscale, bool enter = false) {
   DLIA_ON_DEVICE_OF(out);
   check_bf16(x, "x"); check_bf16(w, "w");
   check_rows(out, "out"); check_rows(x, "x");
@@ -105,7 +105,7 @@ static void norm_impl(Tensor out, Tensor x, OptTensor delta, OptTensor partial, 
     bp = b->data_ptr();
   }
   dlia_norm(out.data_ptr(), x.data_ptr(), dp, pp, (int)splits, pM, pb, w.data_ptr(), bp, ridx, (int)rows, (int)H,
-            x.stride(0), out.stride(0), (float)eps, (int)mode, qs, cur_stream());
+            x.stride(0), out.stride(0), (float)eps, (int)mode, qs, cur_stream(), enter ? 1 : 0);
 }
 
 void norm(Tensor out, Tensor x, OptTensor delta, OptTensor partial, int64_t splits, OptTensor pbias,
@@ -117,6 +117,31 @@ void norm(Tensor out, Tensor x, OptTensor delta, OptTensor partial, int64_t spli
 void norm_q(Tensor out_q, Tensor qscale, Tensor x, OptTensor delta, OptTensor partial, int64_t splits, OptTensor pbias,
             const Tensor& w, OptTensor b, double eps, int64_t mode) {
   norm_impl(out_q, x, delta, partial, splits, pbias, w, b, c10::nullopt, eps, mode, qscale);
+}
+
+// The first norm of a step whose input is kept apart from the residual stream: x <- src, out <- norm(x). qscale given: out is e4m3 bytes.
+void norm_enter(Tensor out, OptTensor qscale, Tensor x, const Tensor& src, const Tensor& w, OptTensor b, double eps, int64_t mode) {
+  DLIA_CHECK(mode == 0 || mode == 1, "norm_enter: RMSNorm (0) or LayerNorm (1)");
+  norm_impl(out, x, src, c10::nullopt, 1, c10::nullopt, w, b, c10::nullopt, eps, mode, qscale, true);
+}
+
+// out = x + the partial sums [splits, rows, H] (+ pbias); counter[row] += 1
+void fold_out(Tensor out, const Tensor& x, const Tensor& partial, int64_t splits, OptTensor pbias, Tensor counter) {
+  DLIA_ON_DEVICE_OF(out);
+  check_bf16(out, "out"); check_rows(out, "out"); check_bf16(x, "x"); check_rows(x, "x"); check_f32(partial, "partial"); check_i32(counter, "counter");
+  const int64_t rows = x.size(0), H = x.size(1);
+  DLIA_CHECK(H % 8 == 0 && out.size(0) >= rows && out.size(1) == H, "fold_out: out [rows, H], H a multiple of 8");
+  DLIA_CHECK(splits >= 1 && partial.is_contiguous() && partial.numel() >= splits * rows * H && reinterpret_cast<uintptr_t>(partial.data_ptr()) % 16 == 0,
+             "fold_out: partial workspace smaller than [splits, rows, H]");
+  DLIA_CHECK(counter.is_contiguous() && counter.numel() >= rows, "fold_out: a counter a row");
+  const void* pb = nullptr;
+  if (pbias.has_value()) {
+    check_bf16(*pbias, "pbias");
+    DLIA_CHECK(pbias->numel() == H && pbias->is_contiguous(), "pbias shape");
+    pb = pbias->data_ptr();
+  }
+  dlia_fold_out(out.data_ptr(), x.data_ptr(), partial.data_ptr<float>(), (int)splits, rows, pb, (int)rows, (int)H, x.stride(0), out.stride(0),
+                counter.data_ptr<int>(), cur_stream());
 }
 
 void embed(Tensor out, const Tensor& ids, OptTensor pos, const Tensor& wte, OptTensor wpe) {
@@ -977,6 +1002,8 @@ TORCH_LIBRARY(dlia, m) {
   m.def("unit_heads(Tensor(a!) x, int heads, int d, int scaled_heads, float mult, float eps) -> ()");
   m.def("delta_rule(Tensor(a!) o, Tensor y, Tensor z, Tensor(b!) state, Tensor A_log, Tensor dt_bias, Tensor q_start, Tensor ctx, Tensor slots, int G, int Hv, int d, int dv, int col_beta, int col_a, int max_q, int lead=0) -> ()");
   m.def("norm(Tensor(a!) out, Tensor(b!) x, Tensor? delta, Tensor? partial, int splits, Tensor? pbias, Tensor w, Tensor? b, Tensor? row_idx, float eps, int mode) -> ()");
+  m.def("norm_enter(Tensor(a!) out, Tensor(b!)? qscale, Tensor(c!) x, Tensor src, Tensor w, Tensor? b, float eps, int mode) -> ()");
+  m.def("fold_out(Tensor(a!) out, Tensor x, Tensor partial, int splits, Tensor? pbias, Tensor(b!) counter) -> ()");
   m.def("embed(Tensor(a!) out, Tensor ids, Tensor? pos, Tensor wte, Tensor? wpe) -> ()");
   m.def("rope_kvwrite(Tensor(a!) qkv, Tensor? partial, int splits, Tensor? pbias, Tensor(b!) kv_cache, Tensor cos, Tensor sin, Tensor tok_pos, Tensor tok_seq, Tensor block_table, int Hq, int Hkv, int D, bool use_rope) -> ()");
   m.def("rope_kvwrite8(Tensor(a!) qkv, Tensor? partial, int splits, Tensor? pbias, Tensor(b!) kv_cache, Tensor(c!) kv_scale, Tensor cos, Tensor sin, Tensor tok_pos, Tensor tok_seq, Tensor block_table, int Hq, int Hkv, int D, bool use_rope) -> ()");
@@ -1020,6 +1047,8 @@ TORCH_LIBRARY_IMPL(dlia, CUDA, m) {
   m.impl("unit_heads", &unit_heads);
   m.impl("delta_rule", &delta_rule);
   m.impl("norm", &norm);
+  m.impl("norm_enter", &norm_enter);
+  m.impl("fold_out", &fold_out);
   m.impl("embed", &embed);
   m.impl("rope_kvwrite", &rope_kvwrite);
   m.impl("rope_kvwrite8", &rope_kvwrite8);

@@ -15,7 +15,8 @@ constexpr int kNormThreads = 256;
 // MODE 0: RMSNorm, 1: LayerNorm (weight + bias), 2: no norm (only fold the addend into x).
 // SRC 0: x as is; 1: x += delta (bf16 [rows,H]); 2: x += sum_s partial[s] (+ pbias) where partial
 // is the fp32 [S][M][H] split-K output of the preceding GEMM — the reduction of those partials
-// costs no launch of its own. In modes 1/2 the updated residual stream is written back into x.
+// costs no launch of its own. In modes 1/2 the updated residual stream is written back into x. 3: x takes over delta's rows
+// (the step's input, kept apart from the stream) — the copy in front of the first norm without a launch.
 // QOUT: instead of bf16 rows, write the normalised row as OCP e4m3 bytes plus one fp32 scale
 // (max|y| / 448) per row — the input format of the fp8 x fp8 GEMM — saving a quantiser launch.
 template <int MODE, int SRC, bool QOUT>
@@ -34,7 +35,7 @@ __global__ __launch_bounds__(kNormThreads) void norm_kernel(
   float s1 = 0.f, s2 = 0.f;
   for (int i = threadIdx.x; i < nvec; i += kNormThreads) {
     float f[8];
-    unpack8(ld16(xr + i * 8), f);
+    unpack8(ld16((SRC == 3 ? delta + irow * ldx : xr) + i * 8), f);
     if (SRC == 1) {
       float d[8];
       unpack8(ld16(delta + irow * ldx + i * 8), d);
@@ -143,21 +144,56 @@ __global__ __launch_bounds__(kNormThreads) void norm_kernel(
   }
 }
 
+// The end of a captured step of a stage that sends its rows on: out = x + sum_s partial[s] (+ pbias), in the order of the norm above, and every row's
+// counter of cached tokens moves on. (Three launches before: the fold into x, a copy, the counters; 4 to 5 us each beside other stages' work.)
+__global__ __launch_bounds__(kNormThreads) void fold_out_kernel(bf16* __restrict__ out, const bf16* __restrict__ x, const float* __restrict__ partial,
+                                                                int splits, long pM, const bf16* __restrict__ pbias, int H, long ldx, long ldo,
+                                                                int* __restrict__ counter) {
+  const long row = blockIdx.x;
+  for (int i = threadIdx.x; i < (H >> 3); i += kNormThreads) {
+    float f[8];
+    unpack8(ld16(x + row * ldx + i * 8), f);
+    const float* pr = partial + row * H + i * 8;
+    const long ss = pM * (long)H;
+#pragma unroll 4
+    for (int s = 0; s < splits; ++s) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(pr + s * ss), c = *reinterpret_cast<const f32x4*>(pr + s * ss + 4);
+      f[0] += a[0]; f[1] += a[1]; f[2] += a[2]; f[3] += a[3];
+      f[4] += c[0]; f[5] += c[1]; f[6] += c[2]; f[7] += c[3];
+    }
+    if (pbias) {
+      float d[8];
+      unpack8(ld16(pbias + i * 8), d);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] += d[j];
+    }
+    st16(out + row * ldo + i * 8, pack8(f));
+  }
+  if (threadIdx.x == 0) counter[row] += 1;
+}
+
 }  // namespace dlia
 
 using namespace dlia;
 
+extern "C" void dlia_fold_out(void* out, const void* x, const float* partial, int splits, long pM, const void* pbias, int rows, int H, long ldx,
+                              long ldo, int* counter, hipStream_t stream) {
+  if (rows <= 0) return;
+  hipLaunchKernelGGL(fold_out_kernel, dim3(rows), dim3(kNormThreads), 0, stream, (bf16*)out, (const bf16*)x, partial, splits, pM, (const bf16*)pbias, H,
+                     ldx, ldo, counter);
+}
+
 // mode: 0 RMSNorm, 1 LayerNorm, 2 none (fold the addend into x only). Addend: `delta` (bf16) or
-// `partial` (fp32 [splits][pM][H] + optional bias), at most one of them.
+// `partial` (fp32 [splits][pM][H] + optional bias), at most one of them. enter: x becomes delta (modes 0 and 1).
 extern "C" void dlia_norm(void* out, void* x, const void* delta, const float* partial, int splits, long pM,
                           const void* pbias, const void* w, const void* b, const int* row_idx, int rows, int H,
-                          long ldx, long ldo, float eps, int mode, float* qscale, hipStream_t stream) {
+                          long ldx, long ldo, float eps, int mode, float* qscale, hipStream_t stream, int enter) {
   if (rows <= 0) return;
   dim3 grid(rows), block(kNormThreads);
   bf16* o = (bf16*)out; bf16* xx = (bf16*)x;
   const bf16* d = (const bf16*)delta; const bf16* ww = (const bf16*)w; const bf16* bb = (const bf16*)b;
   const bf16* pb = (const bf16*)pbias;
-  const int src = partial ? 2 : (delta ? 1 : 0);
+  const int src = enter ? 3 : partial ? 2 : (delta ? 1 : 0);
 #define DLIA_NORM(MODE, SRC)                                                                                      \
   do {                                                                                                            \
     if (qscale) hipLaunchKernelGGL((norm_kernel<MODE, SRC, true>), grid, block, 0, stream, o, xx, d, partial,     \
@@ -165,8 +201,8 @@ extern "C" void dlia_norm(void* out, void* x, const void* delta, const float* pa
     else hipLaunchKernelGGL((norm_kernel<MODE, SRC, false>), grid, block, 0, stream, o, xx, d, partial,           \
                             splits, pM, pb, ww, bb, row_idx, H, ldx, ldo, eps, qscale);                           \
   } while (0)
-  if (mode == 0)      { if (src == 0) DLIA_NORM(0, 0); else if (src == 1) DLIA_NORM(0, 1); else DLIA_NORM(0, 2); }
-  else if (mode == 1) { if (src == 0) DLIA_NORM(1, 0); else if (src == 1) DLIA_NORM(1, 1); else DLIA_NORM(1, 2); }
+  if (mode == 0)      { if (src == 0) DLIA_NORM(0, 0); else if (src == 1) DLIA_NORM(0, 1); else if (src == 2) DLIA_NORM(0, 2); else DLIA_NORM(0, 3); }
+  else if (mode == 1) { if (src == 0) DLIA_NORM(1, 0); else if (src == 1) DLIA_NORM(1, 1); else if (src == 2) DLIA_NORM(1, 2); else DLIA_NORM(1, 3); }
   else                { qscale = nullptr; if (src == 1) DLIA_NORM(2, 1); else if (src == 2) DLIA_NORM(2, 2); }
 #undef DLIA_NORM
 }

@@ -331,6 +331,33 @@ def test_gemm_partials_consumed_by_norm_and_rope(K):
         assert_close(o3, ref.rmsnorm(hn[rows.long()], g, 1e-5), 3e-2, 2e-2, "row-gathered norm over partials")
 
 
+@pytest.mark.parametrize("M,H,S", [(1, 64, 1), (3, 2048, 16), (64, 4096, 5), (7, 520, 3)])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_step_enters_and_leaves_without_copies(K, M, H, S, mode):
+    """The first norm that takes the stream over from the step's input, and the last fold into the output buffer with the rows' counters: bits of
+    a copy and the norm, of the fold and a copy."""
+    g = torch.Generator(device=DEV).manual_seed(M + H)
+    r = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    src, w, b = bf(r(M, H)), bf(r(H)), bf(r(H)) if mode else None
+    h, h2 = bf(r(M, H)), src.clone()
+    out, want = torch.empty_like(h), torch.empty_like(h)
+    K.norm_enter(out, None, h, src, w, b, 1e-5, mode)
+    K.norm(want, h2, None, None, 1, None, w, b, None, 1e-5, mode)
+    assert torch.equal(out, want) and torch.equal(h, src)
+    if H % 16 == 0:
+        q, q2 = (torch.zeros(M, H, device=DEV, dtype=torch.uint8) for _ in range(2))
+        sc, sc2 = (torch.zeros(M, device=DEV) for _ in range(2))
+        h.zero_()
+        K.norm_enter(q, sc, h, src, w, b, 1e-5, mode)
+        K.norm_q(q2, sc2, src.clone(), None, None, 1, None, w, b, 1e-5, mode)
+        assert torch.equal(q, q2) and torch.equal(sc, sc2) and torch.equal(h, src)
+    part, bias, count = r(S, M, H), bf(r(H)) if mode else None, torch.arange(M + 2, device=DEV, dtype=torch.int32)
+    out.zero_()
+    K.fold_out(out, h, part, S, bias, count[:M])
+    K.norm(want, h, None, part, S, bias, w, None, None, 1e-5, 2)
+    assert torch.equal(out, h) and count.tolist() == [i + 1 for i in range(M)] + [M, M + 1]
+
+
 @pytest.mark.parametrize("M", [257, 300, 520])
 @pytest.mark.parametrize("epi", [0, 3, 4, 5])
 def test_gemm_a8w8_large_m(K, M, epi):
