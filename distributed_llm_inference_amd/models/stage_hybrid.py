@@ -795,8 +795,8 @@ class HybridGpuStage(GpuStage):
                     tr = 128 if (self.wmode == "bf16" and T * e.top >= 1024 and H % 32 == 0 and e.ff % 32 == 0) else 32
                     nt = (T * e.top + tr - 1) // tr + e.experts
                     eact, ey, ya = wk.eact[:tr * nt * e.ff].view(tr * nt, e.ff), wk.ey[:tr * nt * H].view(tr * nt, H), view(wk.ya, H)
-                    K.moe_route(wk.sel, wk.wts, z2[:, :e.experts], e.top, e.groups, e.keep, e.scale)
-                    K.moe_plan(wk.tiles, wk.row_tok, wk.pair_row, wk.sel, T * e.top, e.top, e.experts, tr)
+                    K.moe_route_plan(wk.sel, wk.wts, z2[:, :e.experts], e.top, e.groups, e.keep, e.scale, None, False, 2, True, wk.tiles, wk.row_tok,
+                                     wk.pair_row, e.experts, tr, None)
                     K.moe_up(eact, xn, p["w_gate_e"], p["w_up_e"], wk.tiles, wk.row_tok, nt, e.limit, tr)
                     K.moe_down(ey, eact, p["w_down_e"], wk.tiles, wk.row_tok, nt, tr)
                     K.moe_combine(ya, ey, wk.pair_row, wk.wts, e.top)
@@ -1186,9 +1186,8 @@ class HybridGpuStage(GpuStage):
                 tr = 128 if (self.wmode == "bf16" and T * e.top >= 1024 and H % 32 == 0 and e.ff % 32 == 0) else 32
                 nt = (T * e.top + tr - 1) // tr + e.experts
                 eact, ey, ya = wk.eact[:tr * nt * e.ff].view(tr * nt, e.ff), wk.ey[:tr * nt * H].view(tr * nt, H), view(wk.ya, H)
-                K.moe_route(wk.sel, wk.wts, z2[:, :e.outputs], e.top, e.groups, e.keep, e.scale, p["correction"], e.score == "softmax",
-                            e.group_rank, e.renorm)
-                K.moe_plan(wk.tiles, wk.row_tok, wk.pair_row, wk.sel, T * e.top, e.top, e.experts, tr)
+                K.moe_route_plan(wk.sel, wk.wts, z2[:, :e.outputs], e.top, e.groups, e.keep, e.scale, p["correction"], e.score == "softmax",
+                                 e.group_rank, e.renorm, wk.tiles, wk.row_tok, wk.pair_row, e.experts, tr, None)
                 K.moe_up(eact, xn, p["w_gate_e"], p["w_up_e"], wk.tiles, wk.row_tok, nt, e.limit if e.act != "silu" else 0.0, tr)
                 K.moe_down(ey, eact, p["w_down_e"], wk.tiles, wk.row_tok, nt, tr)
                 K.moe_combine(ya, ey, wk.pair_row, wk.wts, e.top, h if e.identity else None)

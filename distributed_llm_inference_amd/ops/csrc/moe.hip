@@ -94,12 +94,84 @@ __device__ __forceinline__ void route_token(int t, int* __restrict__ sel, float*
   for (int r = 0; r < top; ++r) wts[(long)t * top + r] *= inv;
 }
 
+// The same for up to 32 experts in up to 8 groups: the scores, formed once, stay in LDS (a column a thread, `ks` apart), what may be chosen is one
+// 32-bit mask, nothing is divided by the group's size. Same choices and weights to the last bit. (64 tokens of 16 experts in 4 groups,
+// with the plan: 20.2 -> 10.4 us, 300 of 16 in 2 27 -> 13; the general form evaluates exponentials and divides at every comparison.)
+constexpr int kFewExperts = 32, kFewGroups = 8;
+
+__device__ __forceinline__ void route_few(int t, int* __restrict__ sel, float* __restrict__ wts, const float* __restrict__ logits, long ld, int E,
+                                          int top, int groups, int keep, float scale, const float* __restrict__ corr, int softmax, int group_rank,
+                                          int renorm, float* kept, float* gscore, int ks) {
+  const float* z = logits + (long)t * ld;
+  const int per = E / groups;
+#pragma unroll 8
+  for (int e = 0; e < E; ++e) kept[e * ks] = z[e];
+  float zmax = 0.f, zinv = 1.f;
+  if (softmax) {
+    zmax = -INFINITY;
+    for (int e = 0; e < E; ++e) zmax = fmaxf(zmax, kept[e * ks]);
+    float sum = 0.f;
+#pragma unroll 4
+    for (int e = 0; e < E; ++e) { const float x = expf(kept[e * ks] - zmax); kept[e * ks] = x; sum += x; }
+    zinv = 1.f / sum;
+#pragma unroll 4
+    for (int e = 0; e < E; ++e) kept[e * ks] *= zinv;
+  } else {
+#pragma unroll 4
+    for (int e = 0; e < E; ++e) kept[e * ks] = 1.f / (1.f + expf(-kept[e * ks]));
+  }
+  auto choice = [&](int e) { return corr ? kept[e * ks] + corr[e] : kept[e * ks]; };
+  unsigned open = ~0u;
+  if (keep < groups) {
+    for (int g = 0; g < groups; ++g) {
+      float a = -INFINITY, b = -INFINITY;             // the block's best two choice scores
+      for (int e = g * per; e < (g + 1) * per; ++e) {
+        const float s = choice(e);
+        if (s > a) { b = a; a = s; } else if (s > b) b = s;
+      }
+      gscore[g * ks] = a + (group_rank >= 2 && b > -INFINITY ? b : 0.f);
+    }
+    unsigned taken = 0u;
+    open = 0u;
+    for (int r = 0; r < keep; ++r) {
+      int best = -1; float bs = -INFINITY;
+      for (int g = 0; g < groups; ++g) {
+        if (taken >> g & 1u) continue;
+        const float gs = gscore[g * ks];
+        if (best < 0 || gs > bs) { bs = gs; best = g; }
+      }
+      if (best >= 0) { taken |= 1u << best; open |= ((1u << per) - 1u) << (best * per); }       // (per < 32: more than one group)
+    }
+  }
+  float total = 0.f;
+  for (int r = 0; r < top; ++r) {
+    int best = -1; float bs = -INFINITY;
+    for (int e = 0; e < E; ++e) {
+      const float s = choice(e);
+      if ((open >> e & 1u) && (best < 0 || s > bs)) { bs = s; best = e; }
+    }
+    if (best < 0) best = 0;
+    open &= ~(1u << best);
+    const float w = kept[best * ks];
+    sel[(long)t * top + r] = best;
+    wts[(long)t * top + r] = w;
+    total += w;
+  }
+  const float inv = renorm ? scale / (total + 1e-20f) : scale;
+  for (int r = 0; r < top; ++r) wts[(long)t * top + r] *= inv;
+}
+
 __global__ __launch_bounds__(64) void moe_route_kernel(int* __restrict__ sel, float* __restrict__ wts,
                                                        const float* __restrict__ logits, long ld, int T, int E, int top,
                                                        int groups, int keep, float scale, const float* __restrict__ corr,
                                                        int softmax, int group_rank, int renorm) {
+  __shared__ float kept[kFewExperts * 64], gscore[kFewGroups * 64];
   const int t = blockIdx.x * 64 + threadIdx.x;
-  if (t < T) route_token(t, sel, wts, logits, ld, E, top, groups, keep, scale, corr, softmax, group_rank, renorm);
+  if (t >= T) return;
+  if (E <= kFewExperts && groups <= kFewGroups)
+    route_few(t, sel, wts, logits, ld, E, top, groups, keep, scale, corr, softmax, group_rank, renorm, kept + threadIdx.x, gscore + threadIdx.x, 64);
+  else
+    route_token(t, sel, wts, logits, ld, E, top, groups, keep, scale, corr, softmax, group_rank, renorm);
 }
 
 // Lays out the pairs of one layer. expert(i): the expert of pair i (i / top is its token). 1024 threads.
@@ -155,7 +227,12 @@ __global__ __launch_bounds__(1024) void moe_route_plan_kernel(int* __restrict__ 
                                                               int experts, int max_rows, int tile_rows, float* __restrict__ row_w) {
   __shared__ int count[kMoeMaxExperts], start[kMoeMaxExperts], fill[kMoeMaxExperts];
   __shared__ int ntiles;
-  for (int t = threadIdx.x; t < T; t += 1024) route_token(t, sel, wts, logits, ld, E, top, groups, keep, scale, corr, softmax, group_rank, renorm);
+  __shared__ float kept[kFewExperts * 256], gscore[kFewGroups * 256];
+  const bool few = E <= kFewExperts && groups <= kFewGroups && T <= 256;
+  for (int t = threadIdx.x; t < T; t += 1024) {
+    if (few) route_few(t, sel, wts, logits, ld, E, top, groups, keep, scale, corr, softmax, group_rank, renorm, kept + t, gscore + t, 256);
+    else route_token(t, sel, wts, logits, ld, E, top, groups, keep, scale, corr, softmax, group_rank, renorm);
+  }
   __threadfence_block();
   __syncthreads();
   plan_pairs(tiles, row_tok, pair_row, T * top, top, experts, max_rows, tile_rows, count, start, fill, &ntiles,
@@ -184,16 +261,23 @@ __global__ __launch_bounds__(1024) void moe_table_plan_kernel(int* __restrict__ 
              });
 }
 
-template <typename OT>
+// V entries of a row per thread (1900 rows of 3584, bf16 out: 18.1 us with one, 12.1 with four).
+template <typename OT, int V>
 __global__ __launch_bounds__(256) void glu_act_kernel(OT* __restrict__ act, long lda, const float* __restrict__ z, long ldz, int F,
                                                       float limit, int gated) {
   const long m = blockIdx.y;
-  const int c = blockIdx.x * 256 + threadIdx.x;
+  const int c = (blockIdx.x * 256 + threadIdx.x) * V;
   if (c >= F) return;
   const float* zr = z + m * ldz;
-  float v = expert_act(zr[c], zr[F + c], limit);
-  if (gated) v *= 1.f / (1.f + expf(-zr[2 * F]));
-  act[m * lda + c] = (OT)v;
+  const Unit<V> g = ldu<V>(zr + c), u = ldu<V>(zr + F + c);
+  const float all = gated ? 1.f / (1.f + expf(-zr[2 * F])) : 1.f;
+  Unit<V> o;
+#pragma unroll
+  for (int e = 0; e < V; ++e) {
+    o.v[e] = expert_act(g.v[e], u.v[e], limit);
+    if (gated) o.v[e] *= all;
+  }
+  stu<V>(act + m * lda + c, o);
 }
 
 // Row tiles of the plan: 32 rows. Where experts have several of them and the blocks fill the chip (fp32 prompts above all) a workgroup of four waves covers one
@@ -869,7 +953,10 @@ extern "C" void dlia_moe_table_plan(int* tiles, int* row_tok, int* pair_row, con
 
 extern "C" void dlia_glu_act(void* act, int out_f32, long lda, const float* z, long ldz, int M, int F, float limit, int gated, hipStream_t stream) {
   if (M <= 0 || F <= 0) return;
-  const dim3 grid((F + 255) / 256, M);
-  if (out_f32) hipLaunchKernelGGL(dlia::glu_act_kernel<float>, grid, dim3(256), 0, stream, (float*)act, lda, z, ldz, F, limit, gated);
-  else hipLaunchKernelGGL(dlia::glu_act_kernel<dlia::bf16>, grid, dim3(256), 0, stream, (dlia::bf16*)act, lda, z, ldz, F, limit, gated);
+  const bool wide = F % 4 == 0 && ldz % 4 == 0 && lda % 4 == 0 && dlia::al16_(z) && (uintptr_t)act % (out_f32 ? 16 : 8) == 0;
+  const dim3 grid(((wide ? F / 4 : F) + 255) / 256, M);
+#define DLIA_GLU(OT, V) hipLaunchKernelGGL((dlia::glu_act_kernel<OT, V>), grid, dim3(256), 0, stream, (OT*)act, lda, z, ldz, F, limit, gated)
+  if (out_f32) { if (wide) DLIA_GLU(float, 4); else DLIA_GLU(float, 1); }
+  else { if (wide) DLIA_GLU(dlia::bf16, 4); else DLIA_GLU(dlia::bf16, 1); }
+#undef DLIA_GLU
 }

@@ -453,6 +453,39 @@ def test_experts_tiles_in_pairs_where_they_measured_faster(T, E, top, cols, K, p
 
 
 @gpu
+@pytest.mark.parametrize("E,groups,keep,top", [(32, 1, 1, 5), (32, 8, 3, 6), (32, 2, 1, 4), (31, 1, 1, 31), (8, 8, 2, 2), (24, 12, 5, 3), (33, 3, 2, 4), (1, 1, 1, 1)])
+@pytest.mark.parametrize("T", [1, 65, 257])
+def test_routing_of_few_and_many_experts_chooses_the_same(E, groups, keep, top, T):
+    """On either side of the 32 experts and 8 groups whose scores stay in LDS: choices of the equations in 64 bits (experts 0 and 1 tie: the lower
+    index), weights within a few roundings of theirs."""
+    from distributed_llm_inference_amd import ops
+    K = ops.load()
+    g = torch.Generator().manual_seed(E + T)
+    z, corr = torch.randn(T, E, generator=g) * 1.5, torch.randn(E, generator=g) * 0.5
+    z[:, 1:2], corr[1:2] = z[:, :1], corr[:1]             # (logits in steps give sums of two scores that only rounding tells apart: one tie, and no grid)
+    i32 = lambda n: torch.zeros(n, dtype=torch.int32, device="cuda")
+    for softmax, c, rank, renorm in ((False, None, 2, True), (True, corr, 1, False), (False, corr, 2, False)):
+        s = torch.softmax(z.double(), -1) if softmax else torch.sigmoid(z.double())
+        pick = s + c.double() if c is not None else s.clone()
+        if groups > 1 and keep < groups:
+            gs = pick.view(T, groups, -1).topk(min(rank, E // groups), -1).values.sum(-1)
+            kept = torch.zeros(T, groups, dtype=torch.bool).scatter_(1, gs.argsort(dim=-1, descending=True, stable=True)[:, :keep], True)
+            pick = pick.masked_fill(~kept.repeat_interleave(E // groups, 1), float("-inf"))
+        n = min(top, keep * (E // groups))
+        idx = pick.argsort(dim=-1, descending=True, stable=True)[:, :n]
+        w = s.gather(1, idx)
+        w = w / (w.sum(-1, keepdim=True) + 1e-20) * 1.5 if renorm else w * 1.5
+        sel, wts, nt = i32(T * n), torch.zeros(T * n, device="cuda"), (T * n + 31) // 32 + E
+        sel2, wts2, tiles, rows, pairs = i32(T * n), torch.zeros(T * n, device="cuda"), i32(1 + nt), i32(32 * nt), i32(T * n)
+        dc = c.cuda() if c is not None else None
+        K.moe_route(sel, wts, z.cuda(), n, groups, keep, 1.5, dc, softmax, rank, renorm)
+        K.moe_route_plan(sel2, wts2, z.cuda(), n, groups, keep, 1.5, dc, softmax, rank, renorm, tiles, rows, pairs, E, 32, None)
+        assert torch.equal(sel, sel2) and torch.equal(wts, wts2)
+        got, gw = sel.cpu().view(T, n).long(), wts.cpu().double().view(T, n)
+        assert torch.equal(got, idx) and bool(((gw - w).abs() <= 2.0 ** -19 * w).all())
+
+
+@gpu
 @pytest.mark.parametrize("counts,kind,N", [([1, 128, 129, 256, 300, 700], 0, 8200), ([1, 128, 129, 256, 300, 700], 1, 4100), ([700, 0, 129, 1, 257, 384], 2, 8200),
                                            ([(37 * i) % 401 for i in range(80)], 0, 640), ([(37 * i) % 401 for i in range(80)], 1, 328)])      # (more than 64 tiles)
 @pytest.mark.parametrize("k", [64, 128, 192, 256, 320, 448])
