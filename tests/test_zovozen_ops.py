@@ -130,6 +130,44 @@ def test_post_norm_add_hip(out_dtype):
     close(out.float(), x, tol)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("H", [1, 256, 2047, 2048, 2049, 4096, 4097])      # rows in registers (8 and 16 entries a thread), and the loop
+def test_post_norm_add_row_lengths_hip(H):
+    K, dev, T, eps = _K(), "cuda", 3, 1e-6
+    x, ya, yb, w = rnd(T, H, seed=1), rnd(T, H, seed=2, std=3.0), rnd(T, H, seed=3, std=0.2), 1.0 + rnd(H, seed=4, std=0.2)
+    f = lambda t: t.float().to(dev).contiguous()
+    for out_dtype, tol in ((torch.float32, 2e-5), (torch.bfloat16, 1e-2)):
+        h, out = f(x), torch.zeros(T + 1, H, device=dev, dtype=out_dtype)
+        K.post_norm_add(out[:T], h, f(ya), f(yb), 0.7, 0.6, f(w), eps)
+        ref = x + O.rms(0.7 * ya + 0.6 * yb, eps, w)
+        close(h, ref)
+        close(out[:T].float(), ref, tol)
+        assert not out[T].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,d,dims", [(16, 4, 128, 64), (17, 1, 121, 0), (32, 8, 128, 128), (5, 5, 103, 102), (3, 1, 5, 2)])
+def test_preparation_on_both_sides_of_the_registers_hip(H, G, d, dims):
+    """Projections of up to and over 2048 query and 512 key entries: the first are kept in registers, the rest pass through a loop."""
+    from distributed_llm_inference_amd.models.rope import rope_table
+    K, dev, dv = _K(), "cuda", 16
+    _, eps, _, base, _, z_all, _, P = _attention_case(H, G, d, dv, dims, False)
+    T, z = 5, z_all[:5]
+    f = lambda t: t.float().to(dev).contiguous()
+    cos, sin = rope_table(dims, base, None, 400, dev) if dims else (None, None)
+    kc, vc = torch.zeros(2, G, 32, d, device=dev), torch.zeros(2, G, 32, dv, device=dev)
+    table = torch.tensor([[-1, -1], [1, 0]], dtype=torch.int32, device=dev)
+    tok_pos, tok_seq, *_ = _meta([(1, T, 30)], dev)                 # tokens 30 to 34: both blocks
+    q = torch.zeros(T, H * d, device=dev)
+    K.mix_prep(f(z), H, G, d, dv, f(P["q.norm"]), f(P["k.norm"]), eps, dims, cos, sin, True, None, q, kc, vc, False, tok_pos, tok_seq, table)
+    pos = torch.arange(30, 30 + T)
+    qr, kr = O.rms(z[:, :H * d], eps, P["q.norm"]).view(T, H, d), O.rms(z[:, H * d:(H + G) * d], eps, P["k.norm"]).view(T, G, d)
+    close(q, O.rotate_half_partial(qr, pos, dims, base, 1.0).reshape(T, -1), 2e-5)
+    rows = lambda c: torch.cat([c[1, :, 30:], c[0, :, :3]], 1).transpose(0, 1)
+    close(rows(kc), O.rotate_half_partial(kr, pos, dims, base, 1.0), 2e-5)
+    close(rows(vc), O.rms(z[:, (H + G) * d:].view(T, G, dv), eps), 2e-5)
+
+
 def _prep_and_attend(K, dev, dtype, tile, H, G, d, dv, chunk, dims, mixed, z_all, gate, P, steps, scale, eps, base, factor, direct=False):
     """Runs mix_prep + attention over `steps` ([[(slot, first token, count)]]: the sequences of every step) on a paged cache whose
     blocks are in no order; returns {slot: outputs [T, H dv]}."""
