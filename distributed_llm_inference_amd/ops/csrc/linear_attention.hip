@@ -134,6 +134,10 @@ __global__ __launch_bounds__(256) void la_decode_kernel(LaArgs p) {
 }
 
 // ---- portions: what a chunk adds to a state ---------------------------------------------------------------------------
+// Two workgroups a CU (LDS), and about four rounds of them for a long prompt: what one of them waits for is what the launch costs. So the
+// loads are asked for ahead of the decays, and a full chunk's products have no branch between them. 1900 tokens of 32 heads of 128 x 128
+// (32 MFMA cycles a product: 13 us; 125 MB: 26 us), us a launch: decays per head 69 -> 48, per channel (rank 16) 112 -> 99, of which half is the
+// decays. The heads of a chunk on one XCD (its rows read through one L2) gave nothing here and cost the read-outs 5 %.
 __device__ __forceinline__ long la_chunk_row(int t0, int b) { return t0 / kLaChunk + b; }     // (rows of different sequences never meet)
 
 __global__ __launch_bounds__(256) void la_local_kernel(LaArgs p) {
@@ -147,9 +151,36 @@ __global__ __launch_bounds__(256) void la_local_kernel(LaArgs p) {
   if (nt <= 0 || slot < 0 || slot >= p.state_rows) return;   // (whole workgroup)
   const int tid = threadIdx.x, d = p.d, dv = p.dv;
   const long tq = (long)t0 + chunk * kLaChunk, crow = la_chunk_row(t0, b) + chunk;
-  const int c = tid & 63, qt = tid >> 6, ch = db * kLaCh + c;
+  const int c = tid & 63, qt = __builtin_amdgcn_readfirstlane(tid >> 6), ch = db * kLaCh + c;
   const bool ok = ch < d;
   const float* zq = p.z + tq * p.ldz;
+  // The keys and the first values are asked for ahead of the decays, whose logarithms take as long as the loads.
+  float kreg[kLaQuarter];
+  f32x4 v[kLaChunk / 8];
+  // every thread: four neighbouring columns of every eighth token
+  const int cc = (tid & 31) * 4, r8 = tid >> 5;
+  auto ask_values = [&](int v0) {
+    const float* src = zq + p.col_v + (long)h * dv + v0 + cc;
+#pragma unroll
+    for (int i = 0; i < kLaChunk / 8; ++i) {
+      const int row = r8 + i * 8;
+      v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (row < nt) {
+        if (p.vec) { if (v0 + cc < dv) v[i] = *reinterpret_cast<const f32x4*>(src + (long)row * p.ldz); }
+        else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (v0 + cc + e < dv) v[i][e] = src[(long)row * p.ldz + e];
+        }
+      }
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < kLaQuarter; ++i) {
+    const int row = qt * kLaQuarter + i;
+    kreg[i] = ok && row < nt ? (zq + (long)row * p.ldz + p.col_k + h * d)[ch] : 0.f;
+  }
+  ask_values(0);
   float f[kLaQuarter];                                       // factor of this thread's 16 tokens in its channel
   if (p.head_decay) {
     const float l2 = p.head_decay[p.H + h];
@@ -199,38 +230,39 @@ __global__ __launch_bounds__(256) void la_local_kernel(LaArgs p) {
 #pragma unroll
   for (int i = 0; i < kLaQuarter; ++i) {
     const int row = qt * kLaQuarter + i;
-    ks[row * KST + c] = ok && row < nt ? zq[(long)row * p.ldz + p.col_k + h * d + ch] * f[i] : 0.f;
+    ks[row * KST + c] = ok && row < nt ? kreg[i] * f[i] : 0.f;
   }
   const int wave = tid >> 6, lane = tid & 63, r16 = lane & 15, kq = lane >> 4;
   float* dst = p.ws_state + (crow * p.H + h) * (long)d * dv;
   for (int v0 = 0; v0 < dv; v0 += kLaVals) {
     __syncthreads();
-    {
-      // every thread: four neighbouring columns of every eighth token, all loads in flight before the first is parked
-      const int cc = (tid & 31) * 4, r8 = tid >> 5;
-      const float* src = zq + p.col_v + (long)h * dv + v0 + cc;
-      f32x4 v[kLaChunk / 8];
+    if (v0 > 0) ask_values(v0);
 #pragma unroll
-      for (int i = 0; i < kLaChunk / 8; ++i) {
-        const int row = r8 + i * 8;
-        v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (row < nt) {
-          if (p.vec) { if (v0 + cc < dv) v[i] = *reinterpret_cast<const f32x4*>(src + (long)row * p.ldz); }
-          else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (v0 + cc + e < dv) v[i][e] = src[(long)row * p.ldz + e];
-          }
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < kLaChunk / 8; ++i) *reinterpret_cast<f32x4*>(vs + (r8 + i * 8) * VST + cc) = v[i];
-    }
+    for (int i = 0; i < kLaChunk / 8; ++i) *reinterpret_cast<f32x4*>(vs + (r8 + i * 8) * VST + cc) = v[i];
     __syncthreads();
     if (db * kLaCh + wave * 16 >= d) continue;               // (no barrier until the next round's, which every wave reaches)
     float a[16];
 #pragma unroll
     for (int s = 0; s < 16; ++s) a[s] = ks[(s * 4 + kq) * KST + wave * 16 + r16];
+    if (nt == kLaChunk) {                                    // two column tiles at a time, nothing between their products
+      for (int ct = 0; ct < kLaVals / 16 && v0 + ct * 16 < dv; ct += 2) {
+        f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int s = 0; s < 16; ++s)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) acc[u] = mfma4(a[s], vs[(s * 4 + kq) * VST + (ct + u) * 16 + r16], acc[u]);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int col = v0 + (ct + u) * 16 + r16;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int row = db * kLaCh + wave * 16 + kq * 4 + r;
+            if (row < d && col < dv) dst[(long)row * dv + col] = acc[u][r];
+          }
+        }
+      }
+      continue;
+    }
 #pragma unroll
     for (int ct = 0; ct < kLaVals / 16; ++ct) {
       if (v0 + ct * 16 >= dv) break;
@@ -291,13 +323,17 @@ __global__ __launch_bounds__(256) void la_carry_kernel(LaArgs p) {
 // ---- portions: read-outs ------------------------------------------------------------------------------------------------
 // Eight waves. Score tiles (query quarter I, key quarter J <= I): wave w forms tiles w and w + 8 of the ten. Values: wave w owns
 // the column tiles w, w + 8, ... of 16 columns for all 64 tokens.
+// A wave's rows are addressed from scalar registers: with an address a lane for each of its loads the kernel of decays per channel took 212
+// registers, one workgroup a CU; now 128 and two. 1900 tokens of 32 heads of 128 x 128, us a launch: fp32 out, decays per channel 135 -> 96, per head 88 -> 80
+// (products 23, 190 MB of reads and writes 40).
 template <typename OT, int NCT, bool HEAD>
-__global__ __launch_bounds__(512) void la_out_kernel(LaArgs p) {
+__global__ __launch_bounds__(512, NCT == 1 ? 4 : 2) void la_out_kernel(LaArgs p) {
   constexpr int ST = kLaCh + 4;
   __shared__ __attribute__((aligned(16))) float qs[kLaChunk * ST];
   __shared__ __attribute__((aligned(16))) float ks[kLaChunk * ST];
   __shared__ __attribute__((aligned(16))) float ps[kLaChunk * ST];
-  __shared__ float tot[4][kLaCh];
+  __shared__ __attribute__((aligned(16))) float tot[4][kLaCh];
+  __shared__ __attribute__((aligned(16))) float lead[4][kLaCh];          // exp2 of the quarters' sums in front of quarter I
   __shared__ float red[8][kLaChunk];
   const int h = blockIdx.x, b = blockIdx.y, chunk = blockIdx.z;
   const int t0 = p.q_start[b], n = p.q_start[b + 1] - t0, slot = p.slots[b];
@@ -326,17 +362,18 @@ __global__ __launch_bounds__(512) void la_out_kernel(LaArgs p) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int ch = db * kLaCh + (i >> 2) * 16 + kq * 4 + (i & 3);
-        sreg[u][i] = ch < d && col < dv ? S[(long)ch * dv + col] : 0.f;
+        sreg[u][i] = ch < d && col < dv ? S[ch * dv + col] : 0.f;
       }
     }
     __syncthreads();
     {
-      const int c = tid & 63, r8 = tid >> 6, ch = db * kLaCh + c, qt = r8 >> 1;
+      // (the row is the wave's: its address in scalar registers)
+      const int c = lane, r8 = __builtin_amdgcn_readfirstlane(wave), ch = db * kLaCh + c, qt = r8 >> 1;
       const bool ok = ch < d;
       float total = 0.f;
-      const long gc = (long)h * d + ch;
+      const int gc = h * d + ch;
       if constexpr (!HEAD) {
-        if (ok && qt * kLaQuarter < nt) total = p.g[(tq + min(qt * kLaQuarter + kLaQuarter - 1, nt - 1)) * p.H * d + gc];
+        if (ok && qt * kLaQuarter < nt) total = (p.g + (tq + min(qt * kLaQuarter + kLaQuarter - 1, nt - 1)) * p.H * d)[gc];
         if (!(r8 & 1)) tot[qt][c] = total;
       }
 #pragma unroll
@@ -344,10 +381,11 @@ __global__ __launch_bounds__(512) void la_out_kernel(LaArgs p) {
         const int row = r8 * 8 + i;
         float q = 0.f, k = 0.f;
         if (ok && row < nt) {
-          q = zq[(long)row * p.ldz + p.col_q + h * d + ch] * p.qscale;
-          k = zq[(long)row * p.ldz + p.col_k + h * d + ch];
+          const float* zr = zq + (long)row * p.ldz + h * d;
+          q = (zr + p.col_q)[ch] * p.qscale;
+          k = (zr + p.col_k)[ch];
           if constexpr (!HEAD) {
-            const float g = p.g[(tq + row) * p.H * d + gc];
+            const float g = (p.g + (tq + row) * p.H * d)[gc];
             q *= ex2(g);
             k *= ex2(total - g);
           }
@@ -357,6 +395,13 @@ __global__ __launch_bounds__(512) void la_out_kernel(LaArgs p) {
       }
     }
     __syncthreads();
+    if constexpr (!HEAD) {
+      if (wave < 4) {
+        float f = 0.f;
+        for (int m = 0; m < wave; ++m) f += tot[m][lane];
+        lead[wave][lane] = ex2(f);
+      }
+    }
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const int x = wave + 8 * s;
@@ -387,17 +432,17 @@ __global__ __launch_bounds__(512) void la_out_kernel(LaArgs p) {
         f32x4 qa = *reinterpret_cast<const f32x4*>(qs + (I * 16 + r16) * ST + c);
         const f32x4 kb = *reinterpret_cast<const f32x4*>(ks + (J * 16 + r16) * ST + c);
         if constexpr (!HEAD) {
+          f32x4 f = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (I == J) f = -*reinterpret_cast<const f32x4*>(&tot[I][c]);
+          for (int m = J + 1; m < I; ++m) f += *reinterpret_cast<const f32x4*>(&tot[m][c]);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            float f = I == J ? -tot[I][c + e] : 0.f;
-            for (int m = J + 1; m < I; ++m) f += tot[m][c + e];
-            qa[e] *= ex2(f);
-          }
+          for (int e = 0; e < 4; ++e) qa[e] *= ex2(f[e]);
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) sc[s] = mfma4(qa[e], kb[e], sc[s]);
       }
     }
+    if constexpr (!HEAD) __syncthreads();                    // (`lead` is written)
 #pragma unroll
     for (int I = 0; I < 4; ++I) {
       if (I >= mt || wave * 16 >= dv) break;
@@ -405,14 +450,10 @@ __global__ __launch_bounds__(512) void la_out_kernel(LaArgs p) {
       for (int k4 = 0; k4 < 4; ++k4) {
         const int c = k4 * 16 + kq * 4;
         f32x4 qa = *reinterpret_cast<const f32x4*>(qs + (I * 16 + r16) * ST + c);
-        if constexpr (!HEAD) {
+        if (!HEAD && I > 0) {
+          const f32x4 f = *reinterpret_cast<const f32x4*>(&lead[I][c]);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            float f = 0.f;
-#pragma unroll
-            for (int m = 0; m < I; ++m) f += tot[m][c + e];
-            if (I > 0) qa[e] *= ex2(f);
-          }
+          for (int e = 0; e < 4; ++e) qa[e] *= f[e];
         }
 #pragma unroll
         for (int u = 0; u < NCT; ++u)
