@@ -13,6 +13,8 @@
 //                   matrix M [H, H] (scores of head h are sum_g M[h, g] q_g . k) the mix is carried by the query: q leaves
 //                   as H rows of G * d entries, row h holding for every key head c the sum over the heads g of c's group of
 //                   M[h, g] q_g, and the keys of all G heads are ONE cache row of G * d entries that every head reads.
+// The fused multiply-adds of the sums and of the rotation are written out: which product of a pair is rounded would otherwise change with the
+// unrolling, and a stack whose gates are exponential shows it.
 // Norm statistics, rotation and the mix are fp32; outputs take the GEMMs' / the cache's type (bf16 or fp32).
 #include "common.h"
 #include "launch.h"
@@ -135,9 +137,9 @@ __global__ __launch_bounds__(kPostThreads) void mix_prep_kernel(
     for (int i = threadIdx.x; i < H * H; i += kPostThreads) ms[i % H * H + i / H] = mix[i];
   float sq = 0.f, sk = 0.f;
 #pragma unroll
-  for (int u = 0; u < NQ; ++u) sq += q0[u] * q0[u];
+  for (int u = 0; u < NQ; ++u) sq = __builtin_fmaf(q0[u], q0[u], sq);
 #pragma unroll
-  for (int u = 0; u < NK; ++u) sk += k0[u] * k0[u];
+  for (int u = 0; u < NK; ++u) sk = __builtin_fmaf(k0[u], k0[u], sk);
   for (int i = threadIdx.x + NQ * kPostThreads; i < qn; i += kPostThreads) { const float v = zr[i]; qs[i] = v; sq += v * v; }
   for (int i = threadIdx.x + NK * kPostThreads; i < kn; i += kPostThreads) { const float v = zr[qn + i]; ks[i] = v; sk += v * v; }
   if (qw) {
@@ -165,8 +167,8 @@ __global__ __launch_bounds__(kPostThreads) void mix_prep_kernel(
       for (int p = p0; p < half; p += 1 << lg) {
         const float c = p == p0 ? c0 : cs[p], s = p == p0 ? s0 : sn[p];
         const float e = v[p], f = v[p + half];
-        v[p] = e * c - f * s;
-        v[p + half] = f * c + e * s;
+        v[p] = __builtin_fmaf(e, c, -(f * s));
+        v[p + half] = __builtin_fmaf(f, c, e * s);
       }
     }
   }
