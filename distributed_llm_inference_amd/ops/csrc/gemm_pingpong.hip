@@ -84,9 +84,9 @@ typedef int i32x8 __attribute__((ext_vector_type(8)));
 // 1.1 % (60.98 against 60.30 ms per step, four position-balanced runs each) — more than half of what the guided
 // sampler it serves brings.
 // TAIL: the tiles behind an XCD's last whole round run as two halves of 128 rows each, on twice as many workgroups (the launcher's rule;
-// never with K splits). A half walks K in two phases a K-tile, q0: A0 x B0, q1: A0 x B1, over three K-tiles of three half-tiles (144 KiB):
-// q0 of K-tile t asks for A0 and B0 of t + 2, q1 for its B1, into the slots that t - 1 was read from two phases before, and at q1 a wave
-// waits until only the four pieces it asked for in q0 may be on their way: all of t + 1 has landed.
+// K splits are then walked one behind the other and added up in registers). A half walks K in two phases a K-tile, q0: A0 x B0, q1: A0 x B1, over
+// three K-tiles of three half-tiles (144 KiB): q0 of K-tile t asks for A0 and B0 of t + 2, q1 for its B1, into the slots that t - 1 was read from two
+// phases before, and at q1 a wave waits until only the four pieces it asked for in q0 may be on their way: all of t + 1 has landed.
 // ACT: the activation of a feed-forward in the epilogue, on the fp32 sums, instead of a launch that reads them back (an instantiation each, for the
 // registers' sake): 1 gelu_tanh(gate) * up from weights whose first N / 2 rows are the gate's: B0 takes gate columns and B1 the up columns of
 // the same places, so both meet in one wave; p.bias [N]. 2 xIELU with the coefficients p.coef [2], N a multiple of 256, rows of out in
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
   const int tiles_total = p.K >> (F8 ? 7 : 6), KT = tiles_total * 2;   // K-tile = 128 bytes of an x row
   const int per = (tiles_total + p.splitk - 1) / p.splitk;
   const int c0 = ks * per;
-  const int n = min(tiles_total, c0 + per) - c0;   // K-tiles of this split (>= 1 by the launcher)
+  const int n = TAIL ? tiles_total : min(tiles_total, c0 + per) - c0;   // K-tiles of this split (>= 1 by the launcher)
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
 
   // diagnostic mask 16: every workgroup of an XCD loads the same two panels (all L2 hits)
@@ -262,6 +262,15 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
       if constexpr (kind == 0) pp_dma_pair(asrc[0][0] + cc * 128, asrc[0][1] + cc * 128, dst);
       else pp_dma_pair(bsrc[kind - 1] + cc * 2048, bsrc[kind - 1] + cc * 2048, dst);
     };
+    // The sums of a K split join those before it in the registers of the missing half: the bits of the splits below, without their slabs. Done
+    // while the other group multiplies: a quarter's sums in the interval in which this group reads the fragments of the other.
+    int border = per < n ? per : n + 1;              // first K-tile of the next split
+    auto join = [](f32x4 (&a)[4][2], f32x4 (&sum)[4][2]) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) { sum[i][j] += a[i][j]; a[i][j] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+    };
     auto half_phase = [&](auto q_c, int t, auto buf_c) {
       constexpr int q = decltype(q_c)::value, here = decltype(buf_c)::value * 3, there = (decltype(buf_c)::value + 2) % 3 * 3;
       if constexpr (q == 1) pp_wait_vm<4>();
@@ -282,6 +291,8 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (q == 0) { fetch(ic<0>{}, t + 2, there); fetch(ic<1>{}, t + 2, there + 1); }
       else fetch(ic<2>{}, t + 2, there + 2);
+      if constexpr (q == 0) { if (t == border) { join(acc[0][1], acc[1][1]); border += per; } }
+      else if (t + 1 == border) join(acc[0][0], acc[1][0]);
       pp_barrier();
       cluster(acc[0][q], q ? b1 : b0);
       pp_barrier();
@@ -295,6 +306,13 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
       half_phase(ic<0>{}, t, ic<0>{}); half_phase(ic<1>{}, t, ic<0>{});
       if (t + 1 < n) { half_phase(ic<0>{}, t + 1, ic<1>{}); half_phase(ic<1>{}, t + 1, ic<1>{}); }
       if (t + 2 < n) { half_phase(ic<0>{}, t + 2, ic<2>{}); half_phase(ic<1>{}, t + 2, ic<2>{}); }
+    }
+    if (per < n) {
+#pragma unroll
+      for (int f = 0; f < 16; ++f) {
+        f32x4& a = acc[0][f >> 3][(f >> 1) & 3][f & 1];
+        a = acc[1][f >> 3][(f >> 1) & 3][f & 1] + a;
+      }
     }
   } else {
   // prologue: K-tile 0 whole, A0 and B0 of K-tile 1
@@ -329,11 +347,12 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
   if (!TAIL && p.splitk > 1) {
     // ---- sum the K splits of this tile ------------------------------------------------------
     // Each workgroup first draws a ticket from the tile's arrival counter. All but the last to
-    // arrive store their accumulators (write-through, register order) to their slab and raise the
-    // tile's second counter; the last one, which never stores, waits until that counter shows
-    // every slab complete — a wait for workgroups that are already running and wait for nothing
-    // themselves, so it cannot deadlock whatever else is resident — adds the slabs to its
-    // registers and runs the fused epilogue.
+    // arrive store their accumulators (write-through, register order) to their ticket's slab and raise the
+    // tile's second counter (low four bits; three bits a ticket above them say which split it drew); the last
+    // one, which never stores, waits until that counter shows every slab complete — a wait for workgroups that
+    // are already running and wait for nothing themselves, so it cannot deadlock whatever else is resident —
+    // adds its registers and the slabs in the order of the splits, whoever came last, so that a step repeats its bits
+    // (added in the order of arrival, a router behind it saw other ties every time), and runs the fused epilogue.
     const int tile = cb * mblocks + mblk;
     int* const arrived = p.counters + 2 * tile;
     int* const stored = arrived + 1;
@@ -352,28 +371,50 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // every storing wave drains, then one lane signals
       __syncthreads();
-      if (tid == 0) __hip_atomic_fetch_add(stored, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (tid == 0) __hip_atomic_fetch_add(stored, 1 + (ks << (4 + 3 * ticket)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       return;                                                // whole workgroup
     }
     if (tid == 0) {
-      while (__hip_atomic_load(stored, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != p.splitk - 1)
+      int word;
+      while (((word = __hip_atomic_load(stored, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) & 15) != p.splitk - 1)
         __builtin_amdgcn_s_sleep(8);
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      lds_word[1] = word;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    for (int s = 0; s < p.splitk - 1; ++s) {
-      const f32x4* src = reinterpret_cast<const f32x4*>(slabs + (long)s * kPPSlab) + tid;
+    const int drew = __builtin_amdgcn_readfirstlane(lds_word[1]);
+    auto load8 = [&](int s, int f0, f32x4 (&t)[8]) {         // eight fragments of split s
+      int from = 0;                                          // the ticket that it drew
+      for (int i = 1; i < p.splitk - 1; ++i)
+        if (((drew >> (4 + 3 * i)) & 7) == s) from = i;
+      const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(slabs + (long)from * kPPSlab, 0, kPPSlab * 4, 0x00020000);
 #pragma unroll
-      for (int f0 = 0; f0 < 32; f0 += 8) {
-        f32x4 t[8];
+      for (int u = 0; u < 8; ++u)
+        t[u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, tid * 16, (f0 + u) * (kPPThreads * 16), 0));
+    };
 #pragma unroll
-        for (int u = 0; u < 8; ++u) t[u] = src[(f0 + u) * kPPThreads];
+    for (int f0 = 0; f0 < 32; f0 += 8) {
+      f32x4 t[8], sum[8];
+      if (ks > 0) {
+        load8(0, f0, sum);
+#pragma unroll 1
+        for (int s = 1; s < ks; ++s) {
+          load8(s, f0, t);
+#pragma unroll
+          for (int u = 0; u < 8; ++u) sum[u] += t[u];
+        }
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-          const int f = f0 + u;
-          acc[f >> 4][(f >> 3) & 1][(f >> 1) & 3][f & 1] += t[u];
+          f32x4& a = acc[f0 >> 4][(f0 >> 3) & 1][u >> 1][u & 1];
+          a = sum[u] + a;
         }
+      }
+#pragma unroll 1
+      for (int s = ks + 1; s < p.splitk; ++s) {
+        load8(s, f0, t);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc[f0 >> 4][(f0 >> 3) & 1][u >> 1][u & 1] += t[u];
       }
     }
     if (tid == 0) {                                          // both counters back to zero for the next launch
@@ -971,8 +1012,9 @@ static int pp_splitk(int M, int N, int ktiles, int want = 0) {
 // Tiles per XCD that run whole in front of halves (TAIL), or -1: no halves. An XCD's 32 CUs take its tiles in rounds of 32; where the last round has
 // at most 16, its tiles go out as halves of 128 rows, which cost 0.55 (half the chip) to 0.8 (all of it) of a round: 1531 rows, N 14336, K 4096
 // (42 tiles) 162 -> 141 us, fp32 out 175 -> 150; 1290 rows (42) 160 -> 137; 2048 rows, N 28672 (112) 417 -> 402. With up to 16 tiles in all
-// the halves stand against K splits, whose sums cost 17 to 37 us whatever K is: 1024 rows, N = K =
-// 4096 47 -> 42 us, 2048 rows 63 -> 57, 300 rows 48 -> 39; K 14336 102 / 129, 173 / 182, 143 / 154. They meet between 79 and 126 K-tiles.
+// the halves stand against K splits, whose sums cost 17 to 37 us whatever K is (a half adds up the same splits in registers, about 0.7 us each): 1024 rows, N = K =
+// 4096 46.8 -> 46.5 us, 2048 rows 61 -> 57, 300 rows 48 -> 45, e4m3 38 -> 28, 42 -> 34, 31 -> 26; K 14336 102 / 129, 173 / 182, 143 / 154. They meet between
+// 79 and 126 K-tiles.
 // `alone`: the caller wants the chip filled (beside another stream's kernels an idle CU is theirs, and halves move more bytes a product).
 extern "C" int dlia_gemm_pingpong_whole(int M, int N, int ktiles, int alone) {
   const int per_xcd = ((packed_ntiles(N) + 15) / 16 + 7) / 8 * ((M + 255) / 256), rest = per_xcd % 32;
@@ -1029,6 +1071,19 @@ extern "C" void dlia_gemm_pingpong(const dlia::GemmParams* p, hipStream_t stream
   else                         launch_pingpong<false>(p, stream);
 }
 
+// K splits and halves of a GEMM. Splits need room for their slabs behind p.partial; halves add up the same splits themselves, and where whole
+// rounds run in front of them there are none.
+static void choose_splits(dlia::GemmParams& p, int ktiles, long ws_floats, int wg_target, bool halves) {
+  const int s = pp_splitk(p.M, p.N, ktiles, wg_target);
+  const long tiles = (long)((p.M + 255) / 256) * ((p.ntiles + 15) / 16);
+  p.full_items = halves ? dlia_gemm_pingpong_whole(p.M, p.N, ktiles, wg_target > 128) : -1;
+  if (p.partial && s > 1 && ws_floats >= tiles * (s - 1) * kPPSlab + kPPCounters) {
+    p.splitk = s;
+    p.counters = reinterpret_cast<int*>(p.partial + ws_floats - kPPCounters);
+    if (p.full_items > 0) p.full_items = -1;
+  }
+}
+
 // out[M,N] = epi(x[M,K] @ Wp^T) for bf16 weights and more than 256 rows (epilogues 0..5 as
 // dlia_gemm_skinny). `chunk_max` (may be null; then ldc / n_valid are ignored): see GemmParams. `workspace` (may be null) of `ws_floats` floats: lets thin shapes split K; its
 // last 4096 words are the arrival counters (zero when first handed over, zero after every launch).
@@ -1047,13 +1102,7 @@ extern "C" void dlia_gemm_large(void* out, const void* x, const void* wp, const 
   p.act = epi == 4 ? 1 : (epi == 5 ? 2 : 0);
   p.out_f32 = out_f32; p.partial_only = 0; p.splitk = 1; p.group_n = 1; p.full_items = -1; p.counters = nullptr;
   if (dlia_gemm_large_choice(-1) == 2 && chunk_max == nullptr) { dlia_gemm_rows(&p, stream); return; }
-  p.full_items = chunk_max ? -1 : dlia_gemm_pingpong_whole(M, N, K / 64, wg_target > 128);
-  const int s = p.full_items >= 0 ? 1 : pp_splitk(M, N, K / 64, wg_target);
-  const long tiles = (long)((M + 255) / 256) * ((p.ntiles + 15) / 16);
-  if (workspace && s > 1 && ws_floats >= tiles * (s - 1) * kPPSlab + kPPCounters) {
-    p.splitk = s;
-    p.counters = reinterpret_cast<int*>(workspace + ws_floats - kPPCounters);
-  }
+  choose_splits(p, K / 64, ws_floats, wg_target, chunk_max == nullptr);
   dlia_gemm_pingpong(&p, stream);
 }
 
@@ -1067,13 +1116,7 @@ extern "C" void dlia_gemm_large_act(void* out, const void* x, const void* wp, co
   p.bias = act == 1 ? (const bf16*)bias : nullptr; p.residual = nullptr; p.ldr = 0; p.coef = coef;
   p.partial = workspace; p.M = M; p.N = N; p.K = K; p.ntiles = packed_ntiles(N);
   p.act = 0; p.out_f32 = 0; p.partial_only = 0; p.splitk = 1; p.group_n = 1; p.counters = nullptr;
-  p.full_items = dlia_gemm_pingpong_whole(M, N, K / 64, wg_target > 128);
-  const int s = p.full_items >= 0 ? 1 : pp_splitk(M, N, K / 64, wg_target);
-  const long tiles = (long)((M + 255) / 256) * ((p.ntiles + 15) / 16);
-  if (workspace && s > 1 && ws_floats >= tiles * (s - 1) * kPPSlab + kPPCounters) {
-    p.splitk = s;
-    p.counters = reinterpret_cast<int*>(workspace + ws_floats - kPPCounters);
-  }
+  choose_splits(p, K / 64, ws_floats, wg_target, true);
   if (act == 1) launch_pingpong<false, false, 1>(&p, stream);
   else launch_pingpong<false, false, 2>(&p, stream);
 }
@@ -1094,12 +1137,6 @@ extern "C" void dlia_gemm_a8w8_large(void* out, const void* xq, const float* xsc
   p.act = epi == 4 ? 1 : (epi == 5 ? 2 : 0);
   p.out_f32 = out_f32; p.partial_only = 0; p.splitk = 1; p.group_n = 1; p.full_items = -1; p.counters = nullptr;
   if (dlia_gemm_large_choice(-1) == 2) { p.partial = nullptr; dlia_gemm_rows_f8(&p, stream); return; }
-  p.full_items = dlia_gemm_pingpong_whole(M, N, K / 128, wg_target > 128);
-  const int s = p.full_items >= 0 ? 1 : pp_splitk(M, N, K / 128, wg_target);
-  const long tiles = (long)((M + 255) / 256) * ((p.ntiles + 15) / 16);
-  if (workspace && s > 1 && ws_floats >= tiles * (s - 1) * kPPSlab + kPPCounters) {
-    p.splitk = s;
-    p.counters = reinterpret_cast<int*>(workspace + ws_floats - kPPCounters);
-  }
+  choose_splits(p, K / 128, ws_floats, wg_target, true);
   launch_pingpong<true>(&p, stream);
 }

@@ -639,6 +639,41 @@ def test_gemm_large_m_with_the_feed_forwards_activation(K, M, F, Kd, act, pad):
     assert int(ws[-4096:].view(torch.int32).abs().sum()) == 0
 
 
+@pytest.mark.parametrize("f8", [False, True], ids=["bf16", "e4m3"])
+@pytest.mark.parametrize("M,N,Kd,target", [(300, 4096, 4096, 256), (300, 4096, 9088, 256), (1024, 4096, 14336, 256), (600, 2048, 14336, 256), (2011, 4096, 8192, 256),
+                                           (257, 1000, 9088, 1), (512, 1536, 4096, 1)])
+def test_gemm_large_m_adds_its_k_splits_in_order(K, M, N, Kd, target, f8):
+    """Halves (up to 80 K-tiles alone) and tiles split in K, even and uneven splits: the fp32 sums of the splits, each by itself (a launch whose other inputs
+    are zero), added in their order, to the bit and every time."""
+    kt, tiles = Kd // (128 if f8 else 64), (M + 255) // 256 * ((N + 255) // 256)
+    S = min(8, (target if target > 1 else 128) // tiles)
+    while S > 1 and kt // S < 8:
+        S -= 1
+    per, piece = (kt + S - 1) // S, Kd // kt
+    assert S > 1
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    if f8:
+        x, w = (torch.randn(r, Kd, device=DEV, generator=g).to(torch.float8_e4m3fn).view(torch.uint8) for r in (M, N))
+        wp, sc = packing.pack_weight_a8w8(w.view(torch.float8_e4m3fn).float())
+        xs, sc = torch.ones(M, device=DEV), torch.ones_like(sc)
+        run = lambda out, x, ws, t: K.gemm_a8w8(out, x, xs, wp, sc, None, None, ws, N, 0, t, 0)
+    else:
+        x, wp = bf(torch.randn(M, Kd, device=DEV, generator=g)), packing.pack_weight(bf(torch.randn(N, Kd, device=DEV, generator=g)))
+        run = lambda out, x, ws, t: K.gemm(out, x, wp, None, None, ws, N, 0, t, 0)
+    want = None
+    for s in range(S):
+        part, lone = torch.zeros_like(x), torch.empty(M, N, device=DEV)
+        part[:, s * per * piece:(s + 1) * per * piece] = x[:, s * per * piece:(s + 1) * per * piece]
+        run(lone, part, None, 1)
+        want = lone if want is None else want + lone
+    ws, out = torch.zeros(int(K.gemm_ws_floats(M, N, Kd)) + 4096, device=DEV), torch.empty(M, N, device=DEV)
+    for _ in range(5):
+        out.zero_()
+        run(out, x, ws, target)
+        assert torch.equal(out, want)
+    assert int(ws[-4096:].view(torch.int32).abs().sum()) == 0
+
+
 def test_gemm_large_m_halves_where_they_measured_faster(K):
     whole = K.gemm_large_whole          # us: whole tiles or K splits against halves
     assert whole(1531, 14336, 64, True) == 32 and whole(2048, 28672, 64, True) == 96 and whole(1290, 14336, 64, True) == 32          # 162 / 141, 417 / 402, 160 / 137
