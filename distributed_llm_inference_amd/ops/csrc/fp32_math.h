@@ -26,10 +26,15 @@ __device__ __forceinline__ float sigmoid_c(float x) {
   return x > 0.f ? 1.f - q : q;
 }
 
-__device__ __forceinline__ float sqrt_c(float x) {                 // (x no negative number)
-  const float s = __builtin_amdgcn_sqrtf(x);
-  const float r = __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * __builtin_amdgcn_rcpf(s), s);
-  return x > 0.f ? r : s;
+// The instruction takes no input below the normal range (it would be 0, and its inverse infinite): small ones are scaled by 2^32 and back.
+// x no negative number, finite. 0.50 / 0.29 either way.
+__device__ __forceinline__ float sqrt_c(float x) {
+  const bool low = x < 0x1p-96f;
+  const float y = low ? x * 0x1p32f : x;
+  const float s = __builtin_amdgcn_sqrtf(y);
+  const float r = __builtin_fmaf(__builtin_fmaf(-s, s, y), 0.5f * __builtin_amdgcn_rcpf(s), s);
+  const float v = y > 0.f ? r : s;
+  return low ? v * 0x1p-16f : v;
 }
 
 // (1 - e) / (1 + e), e = exp(-2 |y|); below 1/4, where 1 - e cancels, the odd series (what it leaves out is under 2^-26 there)

@@ -233,6 +233,38 @@ def test_recurrent_unit_hip(W, nb, taps, over_workgroups):
     close(torch.cat(got_b), ref_b, 5e-5)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("portions,over_workgroups", [((1,) * 40, False), ((40,), False), ((7, 300), False), ((300, 9), True)])
+def test_recurrent_unit_of_closed_gates_hip(portions, over_workgroups):
+    """Decay gates so far negative that 1 - a^2 falls below the normal range, and to 0, with decay rates from 0.002 up: finite, and within 2^-20 of the terms
+    summed. A gate r below the normal range may be 0: its root is then off by up to sqrt(2 c 2^-126), c being the rate."""
+    K, dev, T = _K(), "cuda", sum(portions)
+    lam = torch.tensor([-8.0, -6.5, -5.0, -3.5, 0.0, 3.0], dtype=F64).repeat_interleave(11)
+    W = len(lam)
+    gr = torch.stack([torch.linspace(-104.0, -60.0, W, dtype=F64)[torch.randperm(W, generator=torch.Generator().manual_seed(t))] for t in range(T)]).float()
+    u, gi, clam = rnd(T, W, seed=1).float(), rnd(T, W, seed=2).float(), (8.0 * O.softplus(lam)).float()
+    la = -clam.to(F64) * torch.sigmoid(gr.to(F64))
+    b = torch.sqrt(-torch.expm1(2 * la)) * torch.sigmoid(gi.to(F64)) * u.to(F64)
+    S, want = torch.zeros(W, dtype=F64), []
+    for t in range(T):
+        S = torch.exp(la[t]) * S + b[t]
+        want.append(S)
+    bound = 2.0 ** -20 * b.abs().cumsum(0) + (torch.sqrt(2 * clam.to(F64) * 2.0 ** -126) * u.to(F64).abs()).cumsum(0)
+    state, got, at = torch.full((2, W), 5.0, device=dev), [], 0
+    for n in portions:
+        i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+        sl = slice(at, at + n)
+        out = torch.zeros(n, W, device=dev)
+        ws = torch.zeros(int(K.rglru_scan_ws_floats(n, 1, W)), device=dev) if over_workgroups else None
+        K.rglru_scan(out, u[sl].to(dev), torch.cat([gr, gi], 1)[sl].to(dev), torch.full((n, W), 3.0, device=dev), clam.to(dev), state, i32([0, n]), i32([at]), i32([1]),
+                     W, n, ws)
+        got.append(out.cpu().to(F64))
+        at += n
+        assert bool(((state[1].cpu().to(F64) - want[at - 1]).abs() <= bound[at - 1]).all())
+    g = float(torch.nn.functional.gelu(torch.tensor(3.0, dtype=F64), approximate="tanh"))
+    assert bool(((torch.cat(got) - g * torch.stack(want)).abs() <= g * bound).all())
+
+
 BLOCKS = [(16, 48, 512, 3), (9, 40, 520, 4), (40, 36, 128, 3), (300, 72, 1088, 5), (200, 448, 128, 32), (1900, 448, 128, 32), (500, 1020, 1024, 2)]
 
 
