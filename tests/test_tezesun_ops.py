@@ -265,6 +265,22 @@ def test_recurrent_unit_of_closed_gates_hip(portions, over_workgroups):
     assert bool(((torch.cat(got) - g * torch.stack(want)).abs() <= g * bound).all())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rate", [0.05, 3.0])
+def test_recurrent_unit_of_one_token_to_the_last_places_hip(rate):
+    """A token's input alone, sqrt(1 - a^2): half of what the gate (two units in the last place) and the series (one) leave, and the root's half unit."""
+    K, dev, W = _K(), "cuda", 1 << 18
+    gr = torch.linspace(-5.0, 5.0, W).to(dev)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    state = torch.zeros(1, W, device=dev)
+    one = torch.ones(1, W, device=dev)
+    K.rglru_scan(torch.zeros(1, W, device=dev), one, torch.cat([gr, 100.0 * one[0]])[None], one, torch.full((W,), rate, device=dev), state, i32([0, 1]), i32([0]), i32([0]),
+                 W, 1, None)
+    want = torch.sqrt(-torch.expm1(-2.0 * torch.full((), rate, device=dev).to(F64) * torch.sigmoid(gr.to(F64))))
+    unit = 2.0 ** (torch.frexp(want).exponent.to(F64) - 24)
+    assert float(((state[0].to(F64) - want).abs() / unit).max()) <= 2.0
+
+
 BLOCKS = [(16, 48, 512, 3), (9, 40, 520, 4), (40, 36, 128, 3), (300, 72, 1088, 5), (200, 448, 128, 32), (1900, 448, 128, 32), (500, 1020, 1024, 2)]
 
 
