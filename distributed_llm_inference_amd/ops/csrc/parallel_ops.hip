@@ -544,25 +544,16 @@ __global__ __launch_bounds__(512) void multi_rows_kernel(
 // weights of those 8 keys ARE the lane's B fragment of O^T += V^T . P^T when the A fragment takes the same keys in the same
 // order, which it can because values sit key-contiguous in the cache: two 8-byte loads per 16 value entries. Both maps of a
 // head use the same value fragments. Blocks in front of the window are skipped except those that hold kept first tokens.
-// Bound by vector work: per score a cap, a mask and an exponential. So tanh and exp are made of the hardware exponential (2-norm errors against
-// 64 bits are the same to 2e-5 of themselves with tanhf and expf), masks are for blocks that some row does not see in full, accumulators
-// are rescaled only where a maximum has moved, and the tiles with most keys start first. 32 heads of two maps of 64, values of 128,
-// cap 30: three prompts of 1531 tokens together 327 -> 96 us, one of 1531 648 -> 183, 16 of 100 113 -> 58; 64 single tokens behind 500 54 -> 45.
+// Bound by vector work: per score a cap, a mask and an exponential. So tanh and exp are made of the hardware exponential (fp32_math.h: no less
+// exact than tanhf and expf), masks are for blocks that some row does not see in full, accumulators are rescaled only where a maximum has
+// moved, and the tiles with most keys start first. 32 heads of two maps of 64, values of 128,
+// cap 30: three prompts of 1531 tokens together 322 -> 111 us, one of 1531 648 -> 216, 16 of 100 113 -> 63; 64 single tokens behind 500 54 -> 51.
 // Single-token steps over ONE key row for all heads (Gk == 1 < G): with many key / value heads a tile takes 16 consecutive heads
 // whatever their value head, so that the long key rows are read once per 16 heads instead of once per value head; the value
 // product then runs once per value head of the tile, one after the other. With few value heads a tile per value head is
 // faster (64 sequences at 1024 tokens, key rows of 4 x 128: 17 against 30 us per layer; key rows of 8 x 128: a step of four
 // layers 2.47 against 2.12 ms).
 __host__ __device__ inline bool tile_all_heads(int G, int Gk) { return Gk == 1 && G > 4; }
-
-// tanh within 2 units in the last place or so: (1 - e) / (1 + e), e = exp(-2 |y|), and below 1/4, where 1 - e cancels, the odd series (what it
-// leaves out is under 2^-26 there). A third of the instructions of tanhf, whose two cases both run in a wave that holds both.
-__device__ __forceinline__ float tanh_score(float y) {
-  const float e = __builtin_amdgcn_exp2f(fabsf(y) * -2.8853900817779268f), y2 = y * y;
-  const float big = copysignf((1.f - e) * __builtin_amdgcn_rcpf(1.f + e), y);
-  const float small = y * __builtin_fmaf(y2, __builtin_fmaf(y2, __builtin_fmaf(y2, __builtin_fmaf(y2, 62.f / 2835.f, -17.f / 315.f), 2.f / 15.f), -1.f / 3.f), 1.f);
-  return y2 < 0.0625f ? small : big;
-}
 
 template <int MAPS, int DVT, bool HEADROWS, int KS>
 __global__ __launch_bounds__(256) void tile_attention_kernel(
@@ -699,7 +690,7 @@ __global__ __launch_bounds__(256) void tile_attention_kernel(
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         sv[i] = s[a][i >> 2][i & 3] * scale;
-        if (softcap > 0.f) sv[i] = softcap * tanh_score(sv[i] * inv_cap);
+        if (softcap > 0.f) sv[i] = softcap * tanh_c(sv[i] * inv_cap);
       }
       if (!whole) {
 #pragma unroll
@@ -715,10 +706,10 @@ __global__ __launch_bounds__(256) void tile_attention_kernel(
       bm = fmaxf(bm, __shfl_xor(bm, 16, 64));
       bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
       const float m_new = fmaxf(m[a], bm), m_safe = m_new == -INFINITY ? 0.f : m_new;      // (nothing seen so far: exp(-inf) below)
-      const float corr = __builtin_amdgcn_exp2f((m[a] - m_safe) * 1.4426950408889634f);
+      const float corr = exp_c(m[a] - m_safe);
       float p[8], add = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) { p[i] = __builtin_amdgcn_exp2f((sv[i] - m_safe) * 1.4426950408889634f); add += p[i]; }
+      for (int i = 0; i < 8; ++i) { p[i] = exp_c(sv[i] - m_safe); add += p[i]; }
       lsum[a] = lsum[a] * corr + add;
       m[a] = m_new;
       if (__ballot(corr != 1.f) != 0) {

@@ -412,6 +412,70 @@ def test_tile_attention_hip(H, G, d, dv, maps, window, keep, cap, dims, inter):
 
 
 @pytest.mark.gpu
+def test_tile_attention_caps_and_weights_to_the_last_places_hip():
+    """What the key splits of single-token steps leave for the merge, in fp32: the capped score of one key (the cap a power of two: the tanh's error alone) and
+    values of a first block rescaled by the weight that a second block's maximum leaves them. One unit in the last place and a rounding each."""
+    K, dev, bf, B, H, d, dv = _K(), "cuda", torch.bfloat16, 1024, 16, 8, 8
+    i32 = lambda v: v.to(torch.int32).to(dev)
+    units = lambda got, want: float(((got.to(F64) - want).abs() / 2.0 ** (torch.frexp(want).exponent.to(F64) - 24)).max())
+
+    def parts(x, blocks, cap):
+        q = torch.zeros(B, H, d, device=dev, dtype=bf)
+        q[:, :, 0] = x
+        kc, vt = torch.zeros(2, 1, 32, d, device=dev, dtype=bf), torch.zeros(2, 1, dv, 32, device=dev, dtype=bf)
+        kc[-1, :, :, 0], vt[0] = 1.0, 1.0                     # block 0: scores of 0, values of 1; block 1: scores of x, values of 0
+        part = torch.zeros(int(K.tile_attention_part_floats(B, H, 1, dv, 1)), device=dev)
+        assert part.numel() == B * H * (dv + 2)               # (one split)
+        n = torch.full((B,), 31 if blocks == [1] else 63)
+        K.tile_attention(torch.zeros(B, H * dv, device=dev, dtype=bf), q.view(B, -1), d, kc, vt, i32(torch.arange(B + 1)), i32(n), i32(torch.arange(B)),
+                         i32(torch.tensor(blocks)).repeat(B, 1), 1, H, d, dv, 1, 1.0, 0, 0, cap, 0.0, 1.0, 1e-5, None, part)
+        return part.view(B, H, dv + 2)
+
+    for lo, hi in ((0.5, 8.0), (-40.0, -2.0)):
+        x = torch.linspace(lo, hi, B * H, device=dev).view(B, H).to(bf)
+        assert units(parts(x, [1], 8.0)[:, :, dv], 8.0 * torch.tanh(x.to(F64) / 8.0)) <= 1.5
+    x = torch.linspace(0.25, 80.0, B * H, device=dev).view(B, H).to(bf)
+    assert units(parts(x, [0, 1], 0.0)[:, :, :dv], (32.0 * torch.exp(-x.to(F64)))[:, :, None].expand(-1, -1, dv)) <= 1.5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("window,keep,chunk", [(100, 0, 0), (100, 70, 0), (64, 33, 0), (31, 300, 0), (1, 1, 0), (0, 0, 96), (70, 0, 96), (0, 0, 1)])
+@pytest.mark.parametrize("H,G,d,dv,cap", [(4, 2, 64, 64, 0.0), (8, 1, 72, 128, 20.0), (3, 3, 128, 24, 0.0)])
+@pytest.mark.parametrize("lens", [[(0, 200), (300, 131), (0, 0), (64, 1), (95, 33)], [(401, 17)], [(33, 1), (0, 1), (200, 1)]])
+def test_tile_attention_blocks_seen_in_full_hip(lens, H, G, d, dv, cap, window, keep, chunk):
+    """Blocks without masks on the edges of windows, kept first tokens and chunks; the tiles of sequences of different lengths, last ones first, an empty one
+    among them. Weights are rounded to bf16 (the sum is of the unrounded ones), the result once more; fp32 scores move a weight by less than 2^-11 of itself."""
+    K, dev, bf = _K(), "cuda", torch.bfloat16
+    lens = [(c, n) for c, n in lens if n or max(m for _, m in lens) > 1]
+    nb, B = [(c + n + 31) // 32 for c, n in lens], len(lens)
+    table = torch.full((B, max(nb) + 1), -1, dtype=torch.int32)
+    perm = torch.randperm(sum(nb), generator=torch.Generator().manual_seed(5)).int().split(nb)
+    for b in range(B):
+        table[b, :nb[b]] = perm[b]
+    kc, vt = rnd(sum(nb), G, 32, d, seed=1).to(bf), rnd(sum(nb), G, dv, 32, seed=2).to(bf)
+    starts = torch.tensor([0] + [n for _, n in lens]).cumsum(0)
+    q, mq = rnd(int(starts[-1]), H * d, seed=3).to(bf), max(n for _, n in lens)
+    out = torch.full((len(q), H * dv), 9.0, device=dev, dtype=bf)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    part = torch.zeros(int(K.tile_attention_part_floats(B, H, G, dv, 1)), device=dev)
+    K.tile_attention(out, q.to(dev), d, kc.to(dev), vt.to(dev), starts.int().to(dev), i32([c for c, _ in lens]), i32(list(range(B))), table.to(dev), mq, H, d, dv, 1,
+                     d ** -0.5, window, keep, cap, 0.0, 1.0, 1e-5, None, part, chunk)
+    for b, (c, n) in enumerate(lens):
+        blk = table[b, :nb[b]].long()
+        k, v = kc[blk].to(F64).permute(1, 0, 2, 3).reshape(G, -1, d)[:, :c + n], vt[blk].to(F64).permute(1, 0, 3, 2).reshape(G, -1, dv)[:, :c + n]
+        i, j = torch.arange(c, c + n)[:, None], torch.arange(c + n)[None]
+        see = (j <= i) & (((i - j < window) | (j < keep)) if window else True) & ((j >= i // chunk * chunk) if chunk else True)
+        rows = slice(int(starts[b]), int(starts[b + 1]))
+        for h in range(H):
+            s = q[rows, h * d:(h + 1) * d].to(F64) @ k[h // (H // G)].T * d ** -0.5
+            s = cap * torch.tanh(s / cap) if cap else s
+            w = torch.softmax(s.masked_fill(~see, float("-inf")), -1)
+            want, room = w @ v[h // (H // G)], w @ v[h // (H // G)].abs()
+            got = out[rows, h * dv:(h + 1) * dv].cpu().to(F64)
+            assert bool(((got - want).abs() <= (2.0 ** -8 + 2.0 ** -11) * room + 2.0 ** -8 * want.abs() + 1e-6).all()), (b, h)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,G,Gk,d,dv,window,keep,cap,chunk,sink", [
     (16, 4, 1, 64, 64, 0, 0, 0.0, 0, True), (8, 8, 1, 16, 4, 0, 0, 0.0, 0, False), (24, 3, 1, 48, 68, 90, 5, 0.0, 0, True), (40, 2, 2, 32, 128, 0, 0, 20.0, 0, False),
     (16, 1, 1, 576, 512, 0, 0, 0.0, 130, True), (16, 1, 1, 592, 64, 0, 0, 0.0, 0, False), (16, 16, 1, 64, 128, 70, 0, 0.0, 0, False)])
