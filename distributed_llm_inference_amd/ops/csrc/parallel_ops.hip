@@ -1009,7 +1009,7 @@ __global__ __launch_bounds__(64) void rglru_stretch_kernel(
 template <typename OT, int V>
 __global__ __launch_bounds__(256) void xielu_kernel(OT* __restrict__ act, const float* __restrict__ z, int M, int F, long ldz,
                                                     long lda, const float* __restrict__ pq) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  const long i = ((long)blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
   const int units = F / V;
   if (i >= (long)M * units) return;
   const int m = (int)(i / units), c = (int)(i % units) * V;
@@ -1173,7 +1173,8 @@ extern "C" void dlia_xielu(void* act, int out_f32, const float* z, int M, int F,
   const long n = (long)M * F;
   if (n <= 0) return;
   const bool wide = F % 4 == 0 && ldz % 4 == 0 && lda % 4 == 0 && al16_(z) && (uintptr_t)act % (out_f32 ? 16 : 8) == 0;
-  const dim3 grid((unsigned)((wide ? n / 4 : n) + 255) / 256);
+  const long blocks = ((wide ? n / 4 : n) + 255) / 256, row = 1L << 22;      // (a dimension of a launch has less than 2^32 threads)
+  const dim3 grid((unsigned)(blocks < row ? blocks : row), (unsigned)((blocks + row - 1) / row));
 #define DLIA_XIELU(OT, V) hipLaunchKernelGGL((xielu_kernel<OT, V>), grid, dim3(256), 0, stream, (OT*)act, z, M, F, ldz, lda, pq)
   if (out_f32) { if (wide) DLIA_XIELU(float, 4); else DLIA_XIELU(float, 1); }
   else { if (wide) DLIA_XIELU(bf16, 4); else DLIA_XIELU(bf16, 1); }

@@ -358,6 +358,18 @@ def test_xielu_rows_in_pieces_and_one_by_one(M, F, ld, dt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("F", [65537, 65540])
+def test_xielu_of_more_entries_than_a_dimension_has_threads(F):
+    """A little over 2^32 entries one by one, and over 2^30 pieces of four, for which a launch has a second dimension: every row as one row by itself."""
+    K, dev, M = _K(), "cuda", F
+    z, pq = rnd(1, F, seed=1, std=2.0).float().to(dev), torch.tensor([0.8, 1.05], device=dev)
+    one, act = torch.zeros(1, F, device=dev, dtype=torch.bfloat16), torch.full((M, F), 7.0, device=dev, dtype=torch.bfloat16)
+    K.xielu(one, z, pq)
+    K.xielu(act, z.expand(M, F), pq)
+    assert all(torch.equal(a, one.expand(len(a), F)) for a in act.split(4096))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,G,d,dv,maps,window,keep,cap,dims,inter", [
     (4, 2, 16, 24, 2, 40, 5, 10.0, 8, True), (2, 1, 8, 8, 1, 0, 0, 0.0, 8, False), (3, 3, 24, 70, 2, 3, 50, 0.0, 4, True),
     (2, 2, 72, 130, 1, 33, 0, 3.0, 0, False), (6, 1, 40, 16, 2, 64, 1, 25.0, 10, True), (1, 1, 104, 300, 1, 0, 0, 0.0, 16, False),
