@@ -81,9 +81,8 @@ __global__ __launch_bounds__(kPPThreads, 2) void moe_pingpong_kernel(bf16* __res
   const int n0 = cblk * BO;          // first output column of the workgroup
   const int n = K / 64;                                         // K-tiles
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
-  // Every XCD begins an eighth of K further and goes round: the rows they read at one time lie on different memory channels (3 % at 1900
-  // tokens), and the workgroups of one XCD still meet in its L2.
-  const int turn = (int)(blockIdx.x & 7) * n / 8;
+  // (Every workgroup walks K from its start, as the ring does: begun an eighth further on each XCD, for the memory channels' sake, it took 0 to 2 %
+  // less, and a row's bits depended on the step's other rows.)
 
   // ---- the pieces this wave brings in: rows 16 wave + 8 e + lane / 8 of every half-tile, 16-byte slot XOR-ed with (row / 2) % 8 ----
   // Nothing is masked: a row without a token reads token 0 or its own stale row, a weight row beyond N reads row 0, and neither
@@ -105,9 +104,7 @@ __global__ __launch_bounds__(kPPThreads, 2) void moe_pingpong_kernel(bf16* __res
   // half 0 / 1 of the rows (WHICH 0) or of the weights (1), K-tile c, to LDS offset `at`
   auto issue = [&](auto which_c, auto half_c, int c, int at) {
     constexpr int which = decltype(which_c)::value, h = decltype(half_c)::value;
-    int cc = min(c, n - 1) + turn;
-    cc = cc >= n ? cc - n : cc;
-    const long off = (long)cc * 128;
+    const long off = (long)min(c, n - 1) * 128;
     const char* const (&s)[2] = which ? bsrc[h] : asrc[h];
     pp_dma_pair(s[0] + off, s[1] + off, lds0 + at + wave * 2048);
   };

@@ -486,6 +486,44 @@ def test_routing_of_few_and_many_experts_chooses_the_same(E, groups, keep, top, 
 
 
 @gpu
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_experts_of_prompts_do_not_depend_on_the_other_rows(kind):
+    """A row's result is the same to the bit whatever else the step brings: other places in the plan, pairs of tiles and single ones."""
+    from distributed_llm_inference_amd import ops
+    K = ops.load()
+    E, N, k, tr, bf = 8, 2048, 1024, 128, torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(kind)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    w, w2, x_all = (r(E, N, k) * k ** -0.5).to(bf), (r(E, N, k) * k ** -0.5).to(bf), r(5000, k).to(bf)
+    sel_all = torch.randint(0, E, (5000,), device="cuda", generator=g, dtype=torch.int32)
+
+    def run(rows):
+        T = len(rows)
+        nt = (T + tr - 1) // tr + E
+        tiles, row_tok, pair_row = (torch.zeros(n, dtype=torch.int32, device="cuda") for n in (1 + nt, tr * nt, T))
+        K.moe_plan(tiles, row_tok, pair_row, sel_all[rows].contiguous(), T, 1, E, tr)
+        x, at = x_all[rows], pair_row.long()
+        if kind == 0:
+            a, out = torch.zeros(tr * nt, k, device="cuda", dtype=bf), torch.zeros(tr * nt, N, device="cuda")
+            a[at] = x
+            K.moe_down(out, a, w, tiles, row_tok, nt, tr)
+        else:
+            out = torch.zeros(tr * nt, N, device="cuda", dtype=bf)
+            K.moe_up(out, x, w if kind == 1 else None, w2, tiles, row_tok, nt, 7.0 if kind == 1 else 0.0, tr)
+        return out[at], K.moe_pairs(nt, E, 2 * N if kind == 1 else N, k)
+
+    whole, pairs = run(torch.arange(5000, device="cuda"))
+    assert pairs
+    seen = set()
+    for n in (4100, 2500, 1100):
+        rows = torch.randperm(5000, generator=torch.Generator().manual_seed(n))[:n].cuda()
+        part, pairs = run(rows)
+        seen.add(bool(pairs))
+        assert torch.equal(part, whole[rows]), n
+    assert seen == {True, False}
+
+
+@gpu
 @pytest.mark.parametrize("counts,kind,N", [([1, 128, 129, 256, 300, 700], 0, 8200), ([1, 128, 129, 256, 300, 700], 1, 4100), ([700, 0, 129, 1, 257, 384], 2, 8200),
                                            ([(37 * i) % 401 for i in range(80)], 0, 640), ([(37 * i) % 401 for i in range(80)], 1, 328)])      # (more than 64 tiles)
 @pytest.mark.parametrize("k", [64, 128, 192, 256, 320, 448])
