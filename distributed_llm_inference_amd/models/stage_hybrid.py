@@ -353,6 +353,10 @@ class HybridGpuStage(GpuStage):
         # more than 256 rows: the tile kernel, spread over the whole chip when a shape has few tiles
         self.K.gemm(out, x, wp, b, None, wk.ws, p[name + "_n"], 1 if b is not None else 0, 256 if x.shape[0] > self.decode_rows else 0, 0)
 
+    def _act_in_gemm(self, T: int) -> bool:
+        """Whether T rows take the feed-forward's activation in the large GEMM's epilogue: more than the weight streams take, and no other kernel chosen."""
+        return T > max(self.decode_rows, 256) and self.K.large_gemm_default()
+
     def _mm_parts(self, wk, out: torch.Tensor, x: torch.Tensor, p, name: str, cols: int) -> torch.Tensor:
         """x . W^T for a consumer that adds up the partial results of key splits while it reads them: [splits, T, cols] in the step's
         GEMM workspace for steps on the weight-streaming kernel (valid until the next GEMM), else [T, cols] in `out`."""
@@ -593,7 +597,7 @@ class HybridGpuStage(GpuStage):
             K.norm32(xn if after_mixer is not None else None, h, yo, p["ln1b_w"], after_mixer, None, eps, 1.0)
             if ls.ff:
                 act = view(wk.act, p["ff_cols"])
-                if "w_gu_p" in p and T > max(self.decode_rows, 256) and ls.ff % 16 == 0:
+                if "w_gu_p" in p and ls.ff % 16 == 0 and self._act_in_gemm(T):
                     K.gemm_act(act, xn, p["w_gu_p"], p.get("w_gu_b"), None, wk.ws, 2 * ls.ff, 1, 256)
                 elif "w_gu_p" in p:
                     gu = view(wk.gu, 2 * ls.ff)
@@ -998,7 +1002,7 @@ class HybridGpuStage(GpuStage):
             self._mm(wk, ya, mixed, p, "w_o")
             if ls.ff:
                 z2, act, yb = view(wk.z2, self._cols(p, "w_up")), view(wk.act, ls.ff), view(wk.yb, self._cols(p, "w_down"))
-                if "w_up_p" in p and T > max(self.decode_rows, 256) and ls.ff % 256 == 0:
+                if "w_up_p" in p and ls.ff % 256 == 0 and self._act_in_gemm(T):
                     K.gemm_act(act, xn, p["w_up_p"], None, p["pq"], wk.ws, ls.ff, 2, 256)
                 else:
                     self._mm(wk, z2, xn, p, "w_up")

@@ -252,6 +252,9 @@ int64_t large_gemm_kernel(int64_t which) {
   return before == 4 ? 6 : (before == 2 && narrow_before ? 4 : before);
 }
 
+// whether the default kernel is the one chosen (the activations of gemm_act are in its epilogue alone)
+bool large_gemm_default() { return dlia_gemm_large_choice(-1) == 0; }
+
 // out[M, N_out] = epi(x[M,K] @ W^T); wp = packed weights (uint8 view of the packed image).
 // epi: 0 none, 1 +bias, 2 +residual, 3 +bias+residual, 4 swiglu, 5 +bias -> gelu_tanh.
 // wscale given: wp holds fp8 e4m3 weights (1 byte each) and wscale one fp32 scale per packed row.
@@ -1018,6 +1021,7 @@ TORCH_LIBRARY(dlia, m) {
   m.def("gemm_splitk(int M, int N, int K) -> int");
   m.def("gemm_large_whole(int M, int N, int ktiles, bool alone) -> int");
   m.def("large_gemm_kernel(int which) -> int");
+  m.def("large_gemm_default() -> bool");
   m.def("gemm_ws_floats(int M, int N, int K) -> int");
   m.def("attention_ws_floats(int B, int max_q_len, int Hq, int Hkv, int D, int splits) -> int");
   m.def("paged_attention(Tensor(a!) out, Tensor qkv, Tensor kv_cache, Tensor q_start, Tensor ctx_lens, Tensor block_table, Tensor? slots, Tensor? partial, int max_q_len, int Hq, int Hkv, int D, float scale, int splits) -> ()");
@@ -1073,6 +1077,7 @@ TORCH_LIBRARY_IMPL(dlia, CompositeExplicitAutograd, m) {
   m.impl("gemm_splitk", &gemm_splitk);
   m.impl("gemm_large_whole", &gemm_large_whole);
   m.impl("large_gemm_kernel", &large_gemm_kernel);
+  m.impl("large_gemm_default", &large_gemm_default);
   m.impl("gemm_ws_floats", &gemm_ws_floats);
   m.impl("gemm_config", &gemm_config);
   m.impl("gemm_any_form", &gemm_any_form);

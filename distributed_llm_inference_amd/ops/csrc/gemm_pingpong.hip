@@ -1107,7 +1107,7 @@ extern "C" void dlia_gemm_large(void* out, const void* x, const void* wp, const 
 }
 
 // The same with a feed-forward's activation: act 1 gelu_tanh(gate) * up, out [M, N / 2] (N / 2 a multiple of 16; weight rows: the gate's, then
-// the up projection's; bias [N] or null), act 2 xIELU, out [M, N], N a multiple of 256, coef [2]. bf16 out. Always the kernel above, whatever else is chosen.
+// the up projection's; bias [N] or null), act 2 xIELU, out [M, N], N a multiple of 256, coef [2]. bf16 out. The kernel above: callers ask whether it is the one chosen.
 extern "C" void dlia_gemm_large_act(void* out, const void* x, const void* wp, const void* bias, const float* coef, float* workspace, long ws_floats,
                                     int M, int N, int K, long ldx, long ldo, int act, int wg_target, hipStream_t stream) {
   if (M <= 0 || N <= 0) return;

@@ -72,10 +72,11 @@ extern "C" void dlia_gemm_a8w8_large(void* out, const void* xq, const float* xsc
                                      const void* bias, const void* residual, float* workspace, long ws_floats, int M,
                                      int N, int K, long ldx, long ldo, long ldr, int epi, int out_f32, int wg_target,
                                      hipStream_t stream);
-// kernel for bf16 GEMMs of more than 256 rows: 0 = 256 x 256 ping-pong tiles (default), 2 = the loader-wave
-// kernel of gemm_rows.hip; which < 0 only reads; returns the previous choice
+// more than 256 rows and a feed-forward's activation: act 1 gelu_tanh(gate) * up, 2 xIELU (gemm_pingpong.hip)
 void dlia_gemm_large_act(void* out, const void* x, const void* wp, const void* bias, const float* coef, float* workspace, long ws_floats,
                          int M, int N, int K, long ldx, long ldo, int act, int wg_target, hipStream_t stream);
+// kernel for bf16 GEMMs of more than 256 rows: 0 = 256 x 256 ping-pong tiles (default), 2 = the loader-wave
+// kernel of gemm_rows.hip; which < 0 only reads; returns the previous choice
 int dlia_gemm_large_choice(int which);
 // the large-M kernel's in-launch split-K: factor for a shape, and the workspace floats it needs (slabs + counters)
 int dlia_gemm_pingpong_splitk(int M, int N, int K);

@@ -674,6 +674,37 @@ def test_gemm_large_m_adds_its_k_splits_in_order(K, M, N, Kd, target, f8):
     assert int(ws[-4096:].view(torch.int32).abs().sum()) == 0
 
 
+@pytest.mark.parametrize("model", ["tiny-letarax-gpu-test", "tiny-tezesun-gpu-test"])
+@pytest.mark.parametrize("which", [0, 2, 6])
+def test_feed_forwards_activation_follows_the_chosen_kernel(K, model, which):
+    """Prompts of hybrid stacks: the activation is in the default kernel's epilogue; with another kernel chosen, the GEMM by that one and a launch of its own."""
+    from distributed_llm_inference_amd.models import weights as W_
+    from distributed_llm_inference_amd.models.partition import StagePlan
+    from distributed_llm_inference_amd.models.spec import BUILTIN_SPECS
+    from distributed_llm_inference_amd.models.stage_hybrid import HybridGpuStage
+    from distributed_llm_inference_amd.runtime.batch import StepBatch
+    spec, n = BUILTIN_SPECS[model], 300
+    plan = StagePlan(0, 1, 0, spec.num_layers, True, True)
+    ex = HybridGpuStage(spec, plan, W_.random_stage_weights(spec, plan, seed=1, device=DEV, dtype=torch.bfloat16), max_slots=1, max_seq_len=512, num_blocks=16,
+                        max_tokens=512, max_batch=1, dtype="bf16")
+    calls, ops = [], ex.K
+
+    class Watched:
+        def __getattr__(self, name):
+            calls.append(name)
+            return getattr(ops, name)
+
+    ex.K = Watched()
+    prev = K.large_gemm_kernel(which)
+    try:
+        ex.forward(StepBatch(slots=[0], q_lens=[n], ctx_lens=[0], sample=[1], temperature=[0.0], top_k=[1], top_p=[1.0], seeds=[1], sample_steps=[0],
+                             table_slots=[0], table_blocks=[list(range(10))], score_rows=[n - 1]), torch.arange(n, dtype=torch.int32) % spec.vocab_size)
+    finally:
+        K.large_gemm_kernel(prev)
+    assert ("gemm_act" in calls) == (which == 0)
+    assert any(c in calls for c in ("gated_gelu", "xielu")) == (which != 0)
+
+
 def test_gemm_large_m_halves_where_they_measured_faster(K):
     whole = K.gemm_large_whole          # us: whole tiles or K splits against halves
     assert whole(1531, 14336, 64, True) == 32 and whole(2048, 28672, 64, True) == 96 and whole(1290, 14336, 64, True) == 32          # 162 / 141, 417 / 402, 160 / 137
