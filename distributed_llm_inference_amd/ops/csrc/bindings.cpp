@@ -852,8 +852,8 @@ void gemm_any(Tensor out, const Tensor& x, const Tensor& w, OptTensor bias, int6
 }
 
 // the kernel that gemm_any or gemm_blocks takes by its sizes where its rows are in whole 16-byte pieces (`dlia_gemm_any_form`)
-int64_t gemm_any_form(int64_t M, int64_t N, int64_t K, int64_t blocks, bool f32, int64_t epi) {
-  return dlia_gemm_any_form((int)M, (int)N, (int)K, (int)blocks, f32, (int)epi);
+int64_t gemm_any_form(int64_t M, int64_t N, int64_t K, int64_t blocks, bool f32, int64_t epi, bool out_f32) {
+  return dlia_gemm_any_form((int)M, (int)N, (int)K, (int)blocks, f32, (int)epi, out_f32);
 }
 
 void gated_gelu(Tensor act, const Tensor& gu) {
@@ -997,7 +997,7 @@ TORCH_LIBRARY(dlia, m) {
   m.def("paged_attention_capped(Tensor(a!) out, Tensor q, Tensor kv_cache, Tensor q_start, Tensor ctx_lens, Tensor block_table, Tensor? slots, int max_q_len, int Hq, int Hkv, int D, float scale, int window, float softcap, Tensor? gate) -> ()");
   m.def("value_mix(Tensor(a!) qkv, Tensor(b!) vfirst, Tensor? lam, int mix, int v_off, int v_cols) -> ()");
   m.def("gemm_any(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int epi) -> ()");
-  m.def("gemm_any_form(int M, int N, int K, int blocks, bool f32, int epi) -> int");
+  m.def("gemm_any_form(int M, int N, int K, int blocks, bool f32, int epi, bool out_f32=False) -> int");
   m.def("kv_store(Tensor qkv, Tensor(a!)? vfirst, Tensor? lam, int mix, Tensor(b!) kcache, Tensor(c!) vcache, Tensor tok_pos, Tensor tok_seq, Tensor block_table, int G, int d, int dv, int q_cols) -> ()");
   m.def("window_attention(Tensor(a!) out, Tensor qkv, Tensor kcache, Tensor vcache, Tensor tok_pos, Tensor tok_seq, Tensor block_table, int H, int G, int d, int dv, float scale, int window, bool sink) -> ()");
   m.def("short_conv(Tensor(a!) y, Tensor z, Tensor(b!) carry, Tensor taps, Tensor q_start, Tensor ctx, Tensor slots, int max_q) -> ()");

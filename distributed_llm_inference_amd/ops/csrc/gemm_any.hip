@@ -398,14 +398,16 @@ __global__ __launch_bounds__(256) void gated_gelu_kernel(bf16* __restrict__ act,
 // 64 is measured (fp32, K 4096: 77, 60, 45 and 25 us; 28 where a CU has one 32 x 32 tile to itself). bf16 chooses by the same numbers: of
 // 159 shapes (17 to 2048 rows, N and K 64 to 8192) of either type the tile taken was within 8 % of the best of the four, but for 400 rows,
 // N 8192, K 2048 (bf16 40 us where 64 x 64 takes 34, fp32 166 and 152).
-extern "C" int dlia_gemm_any_form(int M, int N, int K, int blocks, int f32, int epi) {
+extern "C" int dlia_gemm_any_form(int M, int N, int K, int blocks, int f32, int epi, int out_f32) {
   const int bk = f32 ? 32 : 64;
   if (M <= 16 && K >= 8 * bk) return 1;
   if (K % bk) return 0;
   auto rounds = [&](int bm, int bn) { return (int)(((long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * blocks + 255) / 256); };
   const int r66 = rounds(64, 64), r46 = rounds(48, 64), r36 = rounds(32, 64), r33 = rounds(32, 32);
   const double t66 = r66, t46 = epi == 0 ? r46 * 0.77 : 1e30, t36 = r36 * 0.58, t33 = epi == 0 ? (r33 == 1 ? 0.36 : r33 * 0.33) : 1e30;
-  if (f32 && K == bk && r66 >= 4) return 0;    // (a single stage and the chip full: 2048 rows, N 4096, K 32 19.1 us, the general kernel 16.4)
+  // (a single stage and the chip full: the stores are what is left, in fp32 the general kernel's have less in front of them. fp32, 2048 rows, N 4096, K 32
+  // 19.1 us, the general kernel 16.4; 16-bit operands, K 64, 32 products of 1900 rows, N 640: fp32 out 65.6, 51.7, 16-bit out the tiles take 0.9 of it over 40 shapes)
+  if ((f32 || out_f32) && K == bk && r66 >= 4) return 0;
   const bool split = K >= 16 * bk;             // (below that the rings are filled once or twice: nothing to hide)
   const double best = r66 > 6 ? t66 : fmin(fmin(t66, t46), fmin(t36, t33));        // (with many rounds the last one is small change: 32 products of 1900 rows, N 128, K 448 23 us, in tiles of 48 rows 27)
   if (t66 == best) return split && r66 == 1 ? 64642 : 64641;
@@ -424,7 +426,7 @@ static void launch_any_epi(void* C, const void* A, const void* W, const float* b
   constexpr int VEC = 16 / sizeof(T);
   const int vec_ok = K % VEC == 0 && lda % VEC == 0 && ldw % VEC == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 &&
                      a_step % VEC == 0 && w_step % VEC == 0;
-  const int form = vec_ok ? dlia_gemm_any_form(M, N, K, blocks, sizeof(T) == 4, EPI) : 0;
+  const int form = vec_ok ? dlia_gemm_any_form(M, N, K, blocks, sizeof(T) == 4, EPI, sizeof(OT) == 4) : 0;
   if (form == 1) {
     constexpr int NT = EPI == 0 ? 1 : 2;
     hipLaunchKernelGGL((gemm_any_rows_kernel<T, OT, EPI, NT>), dim3((N + 16 * NT - 1) / (16 * NT), 1, blocks), dim3(512), 0, stream, DLIA_ANY_ARGS, a_step, w_step, c_step);

@@ -124,7 +124,7 @@ void dlia_gated_headnorm(void* out, int out_f32, const float* o, const float* ga
 // ---- gemm_any.hip ---------------------------------------------------------------------------
 // C[M,N] = A[M,K] . W[N,K]^T (+ bias), any shape, row-major W; epi 1: gated pair (interleaved gate / up tiles) ->
 // gelu_tanh(gate) * up, N / 2 columns
-int dlia_gemm_any_form(int M, int N, int K, int blocks, int f32, int epi);
+int dlia_gemm_any_form(int M, int N, int K, int blocks, int f32, int epi, int out_f32);
 void dlia_gemm_any(void* C, int out_f32, const void* A, const void* W, int in_f32, const float* bias, int M, int N, int K,
                    long lda, long ldw, long ldc, int epi, hipStream_t stream);
 // `blocks` independent products in one launch: block b reads A + b * a_step, W + b * w_step, bias + b * N and writes

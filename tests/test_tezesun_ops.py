@@ -291,6 +291,14 @@ def test_block_products_reach_streams_and_tiles():
         assert {form(M, N, k, nb, f32, 0) for M, N, k, nb in BLOCKS} >= {1, 64642, 64641, 48641, 32324, 32321}
 
 
+def test_block_products_of_one_stage_by_their_output():
+    from distributed_llm_inference_amd import ops
+    form = ops.load(build_if_missing=True).gemm_any_form
+    for M, N, nb in ((1900, 640, 32), (312, 640, 32), (1900, 4096, 1), (700, 640, 8)):          # us in tiles / general, fp32 out: 65.6 / 51.7, 15.9 / 13.3, 15.4 / 14.1, 9.9 / 9.0
+        assert form(M, N, 64, nb, False, 0, True) == 0 and form(M, N, 64, nb, False, 0, False) != 0 and form(M, N, 32, nb, True, 0, True) == 0
+    assert form(312, 448, 64, 8, False, 0, True) == form(312, 448, 64, 8, False, 0, False) != 0                                             # (the chip not full)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("dt,ot", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32), (torch.bfloat16, torch.bfloat16)])
@@ -311,6 +319,12 @@ def test_block_products_streams_and_tiles_hip(M, N, k, nb, dt, ot, bias):
         bound = (k + 1) * 2.0 ** -24 * mag + (2.0 ** -8 * ref.abs() if ot == torch.bfloat16 else 0.0)
         assert bool(((out[:, i * os_:i * os_ + N].double() - ref).abs() <= bound).all()), i
         assert bool((out[:, i * os_ + N:(i + 1) * os_] == 7.0).all()), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ot", [torch.float32, torch.bfloat16])
+def test_block_products_of_one_stage_hip(ot):
+    test_block_products_streams_and_tiles_hip(313, 636, 64, 32, torch.bfloat16, ot, True)
 
 
 @pytest.mark.gpu
