@@ -26,7 +26,7 @@ constexpr int kPostThreads = 256;
 
 // N > 0: rows of up to N * 256 entries in registers, a thread's entries of all operands asked for at once. A few hundred rows are about a
 // workgroup a CU, so a launch lasts as long as one row's loads, and a loop that reads an entry, adds and reads the next pays the memory's
-// latency for each. Entries are dealt to threads and added in the order of the loop (N = 0, any length): the same bits.
+// latency for each. Entries are dealt to threads and added in the order of the loop (N = 0, any length), the multiply-adds written out: the same bits.
 // Two operands, us a launch: 1 row of 2048 5.6 -> 3.2, 300 of 2048 6.8 -> 4.2, 32 of 4096 9.6 -> 4.4, 2048 of 4096 31.9 -> 20.6. Rows of more than 4096
 // entries stay in the loop (16 entries take 78 registers; more was not tried).
 template <typename OT, int N>
@@ -54,13 +54,13 @@ __global__ __launch_bounds__(kPostThreads) void post_norm_add_kernel(
       float ss = 0.f;
 #pragma unroll
       for (int u = 0; u < N; ++u) {
-        y[u] = br ? a * y[u] + b * y2[u] : a * y[u];
-        if ((int)threadIdx.x + u * kPostThreads < H) ss += y[u] * y[u];
+        y[u] = br ? __builtin_fmaf(b, y2[u], a * y[u]) : a * y[u];
+        if ((int)threadIdx.x + u * kPostThreads < H) ss = __builtin_fmaf(y[u], y[u], ss);
       }
       ss = block_sum(ss, scratch);
       const float r = 1.f / sqrtf(ss / H + eps);
 #pragma unroll
-      for (int u = 0; u < N; ++u) v[u] += y[u] * r * g[u];
+      for (int u = 0; u < N; ++u) v[u] = __builtin_fmaf(y[u] * r, g[u], v[u]);
     }
 #pragma unroll
     for (int u = 0; u < N; ++u) {
@@ -74,14 +74,14 @@ __global__ __launch_bounds__(kPostThreads) void post_norm_add_kernel(
   if (ya) {
     float ss = 0.f;
     for (int i = threadIdx.x; i < H; i += kPostThreads) {
-      const float y = br ? a * ar[i] + b * br[i] : a * ar[i];
-      ss += y * y;
+      const float y = br ? __builtin_fmaf(b, br[i], a * ar[i]) : a * ar[i];
+      ss = __builtin_fmaf(y, y, ss);
     }
     ss = block_sum(ss, scratch);
     const float r = 1.f / sqrtf(ss / H + eps);
     for (int i = threadIdx.x; i < H; i += kPostThreads) {
-      const float y = br ? a * ar[i] + b * br[i] : a * ar[i];
-      xr[i] += y * r * w[i];
+      const float y = br ? __builtin_fmaf(b, br[i], a * ar[i]) : a * ar[i];
+      xr[i] = __builtin_fmaf(y * r, w[i], xr[i]);
     }
   }
   if (!out) return;
@@ -191,11 +191,11 @@ __global__ __launch_bounds__(kPostThreads) void mix_prep_kernel(
             if (vec8) {
               const f32x4 m0 = *reinterpret_cast<const f32x4*>(mr), m1 = *reinterpret_cast<const f32x4*>(mr + 4);
 #pragma unroll
-              for (int u = 0; u < 8; ++u) acc[u] += (u < 4 ? m0[u] : m1[u - 4]) * qv;
+              for (int u = 0; u < 8; ++u) acc[u] = __builtin_fmaf(u < 4 ? m0[u] : m1[u - 4], qv, acc[u]);
             } else {
 #pragma unroll
               for (int u = 0; u < 8; ++u)
-                if (h0 + u < H) acc[u] += mr[u] * qv;
+                if (h0 + u < H) acc[u] = __builtin_fmaf(mr[u], qv, acc[u]);
             }
           }
 #pragma unroll

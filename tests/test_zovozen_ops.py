@@ -146,6 +146,21 @@ def test_post_norm_add_row_lengths_hip(H):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("two", [False, True])
+@pytest.mark.parametrize("H,times", [(12, 64), (129, 4), (129, 16), (256, 4), (256, 16), (257, 4), (512, 16), (514, 4), (1024, 4), (2048, 4), (2049, 4), (4096, 4)])
+def test_post_norm_add_of_all_row_lengths_has_the_same_bits_hip(H, times, two):
+    """A row followed by zeros, `times` as long, its entries times sqrt(times) and the weights divided by it: sums, quotient and results are the same to
+    the bit, however many entries a thread of either kernel holds."""
+    K, dev, T, k = _K(), "cuda", 3, {4: 2.0, 16: 4.0, 64: 8.0}[times]
+    x, ya, yb, w = (t.float().to(dev) for t in (rnd(T, H, seed=1), rnd(T, H, seed=2, std=3.0), rnd(T, H, seed=3, std=0.2), 1.0 + rnd(H, seed=4, std=0.2)))
+    long = lambda t, f: torch.cat([t * f, t.new_zeros(*t.shape[:-1], (times - 1) * H)], -1).contiguous()
+    h, out, h2, out2 = x.clone(), torch.zeros(T, H, device=dev), long(x, 1.0), torch.zeros(T, times * H, device=dev)
+    K.post_norm_add(out, h, ya, yb if two else None, 0.7, 0.6, w, 1e-6)
+    K.post_norm_add(out2, h2, long(ya, k), long(yb, k) if two else None, 0.7, 0.6, long(w, 1 / k), 1e-6)
+    assert torch.equal(out, out2[:, :H]) and torch.equal(h, h2[:, :H]) and torch.equal(h, out) and not out2[:, H:].any()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,G,d,dims", [(16, 4, 128, 64), (17, 1, 121, 0), (32, 8, 128, 128), (5, 5, 103, 102), (3, 1, 5, 2)])
 def test_preparation_on_both_sides_of_the_registers_hip(H, G, d, dims):
     """Projections of up to and over 2048 query and 512 key entries: the first are kept in registers, the rest pass through a loop."""
