@@ -27,8 +27,9 @@ constexpr int kPostThreads = 256;
 // N > 0: rows of up to N * 256 entries in registers, a thread's entries of all operands asked for at once. A few hundred rows are about a
 // workgroup a CU, so a launch lasts as long as one row's loads, and a loop that reads an entry, adds and reads the next pays the memory's
 // latency for each. Entries are dealt to threads and added in the order of the loop (N = 0, any length), the multiply-adds written out: the same bits.
-// Two operands, us a launch: 1 row of 2048 5.6 -> 3.2, 300 of 2048 6.8 -> 4.2, 32 of 4096 9.6 -> 4.4, 2048 of 4096 31.9 -> 20.6. Rows of more than 4096
-// entries stay in the loop (16 entries take 78 registers; more was not tried).
+// Two operands, us a launch: 1 row of 2048 6.5 -> 3.1, 256 of 2048 7.5 -> 3.9, 256 of 1024 4.8 -> 3.2, 256 of 256 2.9 -> 2.65 (with the eight predicated
+// loads of the longest rows 3.2; 2048 such rows 4.4 -> 4.2, with eight 5.6), 32 of 4096 9.6 -> 4.4, 2048 of 4096 31.9 -> 20.6. Rows of
+// more than 4096 entries stay in the loop (16 entries take 78 registers; more was not tried).
 template <typename OT, int N>
 __global__ __launch_bounds__(kPostThreads) void post_norm_add_kernel(
     OT* __restrict__ out, long ldo, float* __restrict__ x, long ldx, const float* __restrict__ ya, long ldya,
@@ -241,7 +242,8 @@ extern "C" void dlia_post_norm_add(void* out, int out_f32, long ldo, float* x, l
   hipLaunchKernelGGL((dlia::post_norm_add_kernel<OT, N>), dim3(T), dim3(dlia::kPostThreads), 0, stream, (OT*)out, ldo, x, ldx, ya, ldya, yb, \
                      ldyb, a, b, w, H, eps)
 #define DLIA_POST_ROW(OT)                                                                                                     \
-  if (H <= 2048) DLIA_POST(OT, 8); else if (H <= 4096) DLIA_POST(OT, 16); else DLIA_POST(OT, 0)
+  if (H <= 256) DLIA_POST(OT, 1); else if (H <= 512) DLIA_POST(OT, 2); else if (H <= 1024) DLIA_POST(OT, 4);                  \
+  else if (H <= 2048) DLIA_POST(OT, 8); else if (H <= 4096) DLIA_POST(OT, 16); else DLIA_POST(OT, 0)
   if (out_f32 || !out) { DLIA_POST_ROW(float); }
   else { DLIA_POST_ROW(dlia::bf16); }
 #undef DLIA_POST_ROW
