@@ -89,7 +89,7 @@ __global__ __launch_bounds__(kPostThreads) void post_norm_add_kernel(
   for (int i = threadIdx.x; i < H; i += kPostThreads) orow[i] = (OT)xr[i];      // (each thread re-reads what it wrote itself)
 }
 
-template <typename T, typename QT>
+template <typename T, typename QT, int NQ, int NK>
 __global__ __launch_bounds__(kPostThreads) void mix_prep_kernel(
     const float* __restrict__ z, long ldz, int H, int G, int d, int dv, const float* __restrict__ qw, const float* __restrict__ kw,
     float eps, int dims, const float* __restrict__ cos_t, const float* __restrict__ sin_t, int table_pos, int v_unit,
@@ -107,8 +107,8 @@ __global__ __launch_bounds__(kPostThreads) void mix_prep_kernel(
   // A token's first entries of q and k, their norm weights and the way to its cache row are asked for together, ahead of everything that waits
   // (as in post_norm_add: a launch of some hundred tokens lasts as long as one token's loads). With the mix read 16 bytes at a time and
   // dealt over blockIdx.y, fp32, us a launch: 16 heads of 128 on 4 key heads, 1 token 13.4 -> 7.5, 300 15.8 -> 9.8; 32 heads on 8, 64 tokens
-  // 37.7 -> 14.6; without a mix 300 tokens 8.0 -> 7.0, 2048 tokens of 32 heads 40.3 -> 34.6; 6 heads of 10, 100 tokens, 5.7 -> 6.1.
-  constexpr int NQ = 8, NK = 2;
+  // 37.7 -> 14.6; without a mix 300 tokens 8.0 -> 7.0, 2048 tokens of 32 heads 40.3 -> 34.6. NQ and NK by the length (predicated loads that nobody
+  // needs cost a short row 0.5 us: 4 heads of 64, 64 tokens, 4.3 -> 4.8 with eight, 4.25 with one).
   float q0[NQ], k0[NK], wq[NQ], wk[NK];
 #pragma unroll
   for (int u = 0; u < NQ; ++u) {
@@ -141,8 +141,8 @@ __global__ __launch_bounds__(kPostThreads) void mix_prep_kernel(
   for (int u = 0; u < NQ; ++u) sq = __builtin_fmaf(q0[u], q0[u], sq);
 #pragma unroll
   for (int u = 0; u < NK; ++u) sk = __builtin_fmaf(k0[u], k0[u], sk);
-  for (int i = threadIdx.x + NQ * kPostThreads; i < qn; i += kPostThreads) { const float v = zr[i]; qs[i] = v; sq += v * v; }
-  for (int i = threadIdx.x + NK * kPostThreads; i < kn; i += kPostThreads) { const float v = zr[qn + i]; ks[i] = v; sk += v * v; }
+  for (int i = threadIdx.x + NQ * kPostThreads; i < qn; i += kPostThreads) { const float v = zr[i]; qs[i] = v; sq = __builtin_fmaf(v, v, sq); }
+  for (int i = threadIdx.x + NK * kPostThreads; i < kn; i += kPostThreads) { const float v = zr[qn + i]; ks[i] = v; sk = __builtin_fmaf(v, v, sk); }
   if (qw) {
     sq = block_sum(sq, scratch);
     sk = block_sum(sk, scratch);
@@ -261,15 +261,20 @@ extern "C" int dlia_mix_prep(const float* z, long ldz, int T, int H, int G, int 
   // the mixed query rows of few tokens: several workgroups a token, each preparing the token and mixing its share of the heads
   int gy = 1;
   while (mix && q_out && 16 * gy <= H && 2 * gy * T <= 1024) gy *= 2;
-#define DLIA_PREP(CT, QT)                                                                                                      \
-  hipLaunchKernelGGL((dlia::mix_prep_kernel<CT, QT>), dim3(T, gy), dim3(dlia::kPostThreads), lds, stream, z, ldz, H, G, d, dv, qw, kw, eps, \
-                     dims, cos_t, sin_t, table_pos, v_unit, mix, (QT*)q_out, ldqo, (CT*)kcache, Gk, (CT*)vcache, v_t, tok_pos, tok_seq, \
+#define DLIA_PREP_N(CT, QT, NQ, NK)                                                                                            \
+  hipLaunchKernelGGL((dlia::mix_prep_kernel<CT, QT, NQ, NK>), dim3(T, gy), dim3(dlia::kPostThreads), lds, stream, z, ldz, H, G, d, dv, qw, kw, eps, dims, cos_t, sin_t, table_pos, v_unit, mix, (QT*)q_out, ldqo, (CT*)kcache, Gk, (CT*)vcache, v_t, tok_pos, tok_seq, \
                      block_table, max_blocks, num_blocks, table_rows)
+#define DLIA_PREP(CT, QT)                                                                                                      \
+  do {                                                                                                                         \
+    if (H * d <= 256) DLIA_PREP_N(CT, QT, 1, 1); else if (H * d <= 512) DLIA_PREP_N(CT, QT, 2, 1);                             \
+    else if (H * d <= 1024) DLIA_PREP_N(CT, QT, 4, 1); else DLIA_PREP_N(CT, QT, 8, 2);                                         \
+  } while (0)
   if (cache_f32) {
     if (q_f32) DLIA_PREP(float, float); else return 1;
   } else {
     if (q_f32) DLIA_PREP(dlia::bf16, float); else DLIA_PREP(dlia::bf16, dlia::bf16);
   }
 #undef DLIA_PREP
+#undef DLIA_PREP_N
   return 0;
 }

@@ -183,6 +183,14 @@ def test_preparation_on_both_sides_of_the_registers_hip(H, G, d, dims):
     close(rows(vc), O.rms(z[:, (H + G) * d:].view(T, G, dv), eps), 2e-5)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,d,dims", [(4, 1, 64, 64), (4, 2, 65, 64), (2, 2, 256, 128), (8, 8, 64, 32), (8, 1, 128, 128), (6, 3, 171, 170)])
+def test_preparation_of_short_rows_hip(H, G, d, dims):
+    """On both sides of 256, 512 and 1024 query and 256 key entries: as many in registers as there are."""
+    test_preparation_on_both_sides_of_the_registers_hip(H, G, d, dims)
+
+
+
 def _prep_and_attend(K, dev, dtype, tile, H, G, d, dv, chunk, dims, mixed, z_all, gate, P, steps, scale, eps, base, factor, direct=False):
     """Runs mix_prep + attention over `steps` ([[(slot, first token, count)]]: the sequences of every step) on a paged cache whose
     blocks are in no order; returns {slot: outputs [T, H dv]}."""
