@@ -261,8 +261,9 @@ __global__ __launch_bounds__(1024) void moe_table_plan_kernel(int* __restrict__ 
              });
 }
 
-// V entries of a row per thread (1900 rows of 3584, bf16 out: 18.1 us with one, 12.1 with four).
-template <typename OT, int V>
+// V entries of a row per thread (1900 rows of 3584, bf16 out: 18.1 us with one, 11 with four). LIMITED at compile time: with both forms of the activation in
+// sight the compiler evaluates both and selects (256 rows of 8192, one entry a thread, 5.2 -> 6.5 us).
+template <typename OT, int V, bool LIMITED>
 __global__ __launch_bounds__(256) void glu_act_kernel(OT* __restrict__ act, long lda, const float* __restrict__ z, long ldz, int F,
                                                       float limit, int gated) {
   const long m = blockIdx.y;
@@ -270,12 +271,13 @@ __global__ __launch_bounds__(256) void glu_act_kernel(OT* __restrict__ act, long
   if (c >= F) return;
   const float* zr = z + m * ldz;
   const Unit<V> g = ldu<V>(zr + c), u = ldu<V>(zr + F + c);
-  const float all = gated ? 1.f / (1.f + expf(-zr[2 * F])) : 1.f;
   Unit<V> o;
 #pragma unroll
-  for (int e = 0; e < V; ++e) {
-    o.v[e] = expert_act(g.v[e], u.v[e], limit);
-    if (gated) o.v[e] *= all;
+  for (int e = 0; e < V; ++e) o.v[e] = LIMITED ? expert_act_limited(g.v[e], u.v[e], limit) : expert_act_free(g.v[e], u.v[e]);
+  if (gated) {
+    const float all = 1.f / (1.f + expf(-zr[2 * F]));
+#pragma unroll
+    for (int e = 0; e < V; ++e) o.v[e] *= all;
   }
   stu<V>(act + m * lda + c, o);
 }
@@ -953,9 +955,15 @@ extern "C" void dlia_moe_table_plan(int* tiles, int* row_tok, int* pair_row, con
 
 extern "C" void dlia_glu_act(void* act, int out_f32, long lda, const float* z, long ldz, int M, int F, float limit, int gated, hipStream_t stream) {
   if (M <= 0 || F <= 0) return;
-  const bool wide = F % 4 == 0 && ldz % 4 == 0 && lda % 4 == 0 && dlia::al16_(z) && (uintptr_t)act % (out_f32 ? 16 : 8) == 0;
+  // (fewer entries are spread over more threads: 16 rows of 2048 2.0 us, 2.1 in fours; 1024 of 96 2.1, 2.35; 64 of 8192 2.3, 2.4; from the line on
+  // 256 rows of 2048 2.6, 2.4, 1024 of 3584 7.8, 6.2)
+  const bool wide = M >= 128 && F >= 512 && (long)M * F >= 1 << 19 && F % 4 == 0 && ldz % 4 == 0 && lda % 4 == 0 && dlia::al16_(z) && (uintptr_t)act % (out_f32 ? 16 : 8) == 0;
   const dim3 grid(((wide ? F / 4 : F) + 255) / 256, M);
-#define DLIA_GLU(OT, V) hipLaunchKernelGGL((dlia::glu_act_kernel<OT, V>), grid, dim3(256), 0, stream, (OT*)act, lda, z, ldz, F, limit, gated)
+#define DLIA_GLU(OT, V)                                                                                                              \
+  do {                                                                                                                              \
+    if (limit > 0.f) hipLaunchKernelGGL((dlia::glu_act_kernel<OT, V, true>), grid, dim3(256), 0, stream, (OT*)act, lda, z, ldz, F, limit, gated); \
+    else hipLaunchKernelGGL((dlia::glu_act_kernel<OT, V, false>), grid, dim3(256), 0, stream, (OT*)act, lda, z, ldz, F, limit, gated);            \
+  } while (0)
   if (out_f32) { if (wide) DLIA_GLU(float, 4); else DLIA_GLU(float, 1); }
   else { if (wide) DLIA_GLU(dlia::bf16, 4); else DLIA_GLU(dlia::bf16, 1); }
 #undef DLIA_GLU

@@ -360,6 +360,24 @@ def test_experts_by_token_id_hip(dtype, H, ff, experts, top, T):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("limit,gated", [(0.0, False), (0.0, True), (1.3, False), (1.3, True)])
+@pytest.mark.parametrize("M,F,pad", [(127, 4128, 0), (128, 4096, 0), (1025, 512, 4), (1025, 511, 4), (128, 4096, 1), (3, 20, 0)])
+def test_shared_experts_activation_hip(M, F, pad, limit, gated):
+    """Entries in fours (128 rows and 2^19 entries on, whole pieces) and one by one. Sigmoid, its products and the gate: a dozen roundings of fp32, and one
+    of bf16."""
+    K, dev = _K(), "cuda"
+    z = rnd(M, 2 * F + (4 if gated and not pad else pad + gated), seed=F, std=2.0).float()
+    for dtype in (torch.float32, torch.bfloat16):
+        act = torch.full((M + 1, F), 7.0, device=dev, dtype=dtype)
+        K.glu_act(act[:M], z.to(dev), limit, gated)
+        g, u = z[:, :F].to(F64), z[:, F:2 * F].to(F64)
+        gv, uv = (g.clamp(max=limit), u.clamp(-limit, limit) + 1.0) if limit else (g, u)
+        want = gv * torch.sigmoid((1.702 if limit else 1.0) * gv) * uv * (torch.sigmoid(z[:, 2 * F:2 * F + 1].to(F64)) if gated else 1.0)
+        bound = (12 * 2.0 ** -24 * (1.0 + gv.abs()) + (2.0 ** -8 if dtype == torch.bfloat16 else 0.0)) * want.abs() + 12 * 2.0 ** -24 * gv.abs()
+        assert bool(((act[:M].cpu().to(F64) - want).abs() <= bound).all()) and bool((act[M] == 7.0).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("F", [33, 40, 3000])
 def test_polynomial_hip(dtype, F):
