@@ -266,6 +266,34 @@ def test_latent_attention_hip(D, R, H, window):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("window", [0, 40, 4000])        # (a window shorter than the portions' tiles: sequence after sequence; otherwise last tiles first)
+@pytest.mark.parametrize("D,R,H", [(40, 32, 4), (576, 512, 3)])
+def test_latent_attention_of_several_sequences_hip(D, R, H, window):
+    """Tiles of sequences of different lengths in both orders, an empty one among them: each as by itself, to the bit."""
+    K, dev, bf = _K(), "cuda", torch.bfloat16
+    lens = [(100, 33), (0, 700), (50, 0), (300, 301), (64, 1)]
+    nb = [(c + n + 31) // 32 for c, n in lens]
+    perm, table = _blocks(sum(nb), 4).int().split(nb), torch.full((len(lens), max(nb)), -1, dtype=torch.int32)
+    for b in range(len(lens)):
+        table[b, :nb[b]] = perm[b]
+    kc, vt = rnd(sum(nb), 1, 32, D, seed=1).to(dev, bf), rnd(sum(nb), 1, R, 32, seed=2).to(dev, bf)
+
+    def run(seqs):
+        i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+        q = torch.cat([rnd(lens[b][1], H * D, seed=10 + b) for b in seqs]).to(dev, bf)
+        out = torch.full((len(q), H * R), 9.0, device=dev, dtype=bf)
+        starts = torch.tensor([0] + [lens[b][1] for b in seqs]).cumsum(0)
+        K.latent_attention(out, q, kc, vt, starts.int().to(dev), i32([lens[b][0] for b in seqs]), i32(seqs), table.to(dev), max(lens[b][1] for b in seqs), H,
+                           1.5 * D ** -0.5, window, None)
+        return out.split([lens[b][1] for b in seqs])
+
+    together = run(list(range(len(lens))))
+    for b in range(len(lens)):
+        if lens[b][1]:
+            assert torch.equal(together[b], run([b, 0] if lens[b][1] == 1 else [b])[0]), b           # (a token by itself has another kernel)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("R,dr,H,d,base", [(24, 8, 3, 16, 100.0), (300, 64, 2, 10, 500000.0), (14, 6, 1, 4, 7.0)])
 def test_latent_rows_into_the_cache_hip(dtype, R, dr, H, d, base):
