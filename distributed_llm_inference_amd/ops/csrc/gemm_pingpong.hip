@@ -1012,15 +1012,25 @@ static int pp_splitk(int M, int N, int ktiles, int want = 0) {
 // Tiles per XCD that run whole in front of halves (TAIL), or -1: no halves. An XCD's 32 CUs take its tiles in rounds of 32; where the last round has
 // at most 16, its tiles go out as halves of 128 rows, which cost 0.55 (half the chip) to 0.8 (all of it) of a round: 1531 rows, N 14336, K 4096
 // (42 tiles) 162 -> 141 us, fp32 out 175 -> 150; 1290 rows (42) 160 -> 137; 2048 rows, N 28672 (112) 417 -> 402. With up to 16 tiles in all
-// the halves stand against K splits, whose sums cost 17 to 37 us whatever K is (a half adds up the same splits in registers, about 0.7 us each): 1024 rows, N = K =
-// 4096 46.8 -> 46.5 us, 2048 rows 61 -> 57, 300 rows 48 -> 45, e4m3 38 -> 28, 42 -> 34, 31 -> 26; K 14336 102 / 129, 173 / 182, 143 / 154. They meet between
-// 79 and 126 K-tiles.
+// the halves stand against `s` K splits and add up the same splits in registers, so that the sums are the same either way. us by the two sides of the
+// comparison, fitted to 280 shapes (300 to 2011 rows, N 1024 to 6144, 16 to 80 K-tiles, bf16 and e4m3 alike; splits 3 us rms off, halves 1.5): a K-tile
+// and a split more of a half; rounds of an XCD's splits, a slab more and its bytes. It takes the slower side of 14 by 3 to 6 %; halves whatever the
+// sizes took that of 66, by up to 35 % (300 rows, N 1024, 80 K-tiles 40 us in splits, 54). 1024 rows, N = K = 4096 46.8 -> 46.5 us, 2048 rows 61 -> 57,
+// 300 rows 48 -> 45, 1531 rows, N 3072 70 -> 45; e4m3 38 -> 28, 42 -> 34, 31 -> 26. K 14336 102 / 129, 173 / 182, 143 / 154: not beyond 80 K-tiles.
 // `alone`: the caller wants the chip filled (beside another stream's kernels an idle CU is theirs, and halves move more bytes a product).
-extern "C" int dlia_gemm_pingpong_whole(int M, int N, int ktiles, int alone) {
-  const int per_xcd = ((packed_ntiles(N) + 15) / 16 + 7) / 8 * ((M + 255) / 256), rest = per_xcd % 32;
+static int pp_whole(int M, int N, int ktiles, int alone, int s) {
+  const int nb = (packed_ntiles(N) + 15) / 16, mb = (M + 255) / 256, per_xcd = (nb + 7) / 8 * mb, rest = per_xcd % 32;
   if (!alone || rest == 0 || rest > 16) return -1;
-  return per_xcd > 32 || ktiles <= 80 ? per_xcd - rest : -1;
+  if (per_xcd > 32) return s > 1 ? -1 : per_xcd - rest;         // (whole tiles in front have no splits)
+  if (ktiles > 80) return -1;
+  if (s > 1) {
+    const double halves = 7.0 + ktiles * (0.46 + per_xcd / 70.0) + 0.85 * (s - 1);
+    const double splits = 9.5 + 1.2 * ((per_xcd * s + 31) / 32) * ((ktiles + s - 1) / s) + (s - 1) * (2.6 + mb * nb / 18.5);
+    if (halves > splits) return -1;
+  }
+  return 0;
 }
+extern "C" int dlia_gemm_pingpong_whole(int M, int N, int ktiles, int alone) { return pp_whole(M, N, ktiles, alone, pp_splitk(M, N, ktiles, 256)); }
 extern "C" int dlia_gemm_pingpong_splitk(int M, int N, int K) { return pp_splitk(M, N, K / 64); }
 // Workspace the split needs: slabs [tiles][S][256 x 256]; the arrival counters are the LAST
 // kPPCounters words of whatever workspace the caller hands over (so that workspaces shared with
@@ -1071,17 +1081,15 @@ extern "C" void dlia_gemm_pingpong(const dlia::GemmParams* p, hipStream_t stream
   else                         launch_pingpong<false>(p, stream);
 }
 
-// K splits and halves of a GEMM. Splits need room for their slabs behind p.partial; halves add up the same splits themselves, and where whole
-// rounds run in front of them there are none.
+// K splits and halves of a GEMM. Splits need room for their slabs behind p.partial.
 static void choose_splits(dlia::GemmParams& p, int ktiles, long ws_floats, int wg_target, bool halves) {
   const int s = pp_splitk(p.M, p.N, ktiles, wg_target);
   const long tiles = (long)((p.M + 255) / 256) * ((p.ntiles + 15) / 16);
-  p.full_items = halves ? dlia_gemm_pingpong_whole(p.M, p.N, ktiles, wg_target > 128) : -1;
   if (p.partial && s > 1 && ws_floats >= tiles * (s - 1) * kPPSlab + kPPCounters) {
     p.splitk = s;
     p.counters = reinterpret_cast<int*>(p.partial + ws_floats - kPPCounters);
-    if (p.full_items > 0) p.full_items = -1;
   }
+  p.full_items = halves ? pp_whole(p.M, p.N, ktiles, wg_target > 128, p.splitk) : -1;
 }
 
 // out[M,N] = epi(x[M,K] @ Wp^T) for bf16 weights and more than 256 rows (epilogues 0..5 as

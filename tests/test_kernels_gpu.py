@@ -711,6 +711,8 @@ def test_gemm_large_m_halves_where_they_measured_faster(K):
     assert whole(1024, 4096, 64, True) == 0 and whole(2048, 4096, 64, True) == 0 and whole(300, 14336, 64, True) == 0               # 47 / 42, 63 / 57, 57 / 44
     assert whole(1024, 4096, 224, True) == -1 and whole(2048, 4096, 224, True) == -1 and whole(2048, 8192, 64, True) == -1          # 102 / 129, 173 / 182, full rounds
     assert whole(2048, 6144, 64, True) == -1 and whole(1531, 14336, 64, False) == -1                                                # more than half a round; beside another stream
+    assert whole(300, 1024, 80, True) == -1 and whole(512, 2048, 64, True) == -1 and whole(762, 2048, 80, True) == -1               # 40 / 54, 40 / 45, 45 / 54
+    assert whole(1531, 3072, 80, True) == 0 and whole(2011, 1024, 64, True) == 0 and whole(300, 1024, 32, True) == 0                # 83 / 55, 72 / 47, 27 / 25
 
 
 def test_gemm_pingpong_exact_on_integer_data_with_asymmetric_operands(K):
