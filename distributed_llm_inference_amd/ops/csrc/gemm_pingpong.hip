@@ -83,16 +83,17 @@ typedef int i32x8 __attribute__((ext_vector_type(8)));
 // (220 instead of 256 VGPRs, a different main loop): with it compiled into every GEMM, bench.py's default point lost
 // 1.1 % (60.98 against 60.30 ms per step, four position-balanced runs each) — more than half of what the guided
 // sampler it serves brings.
-// TAIL: the tiles behind an XCD's last whole round run as two halves of 128 rows each, on twice as many workgroups (the launcher's rule;
-// K splits are then walked one behind the other and added up in registers). A half walks K in two phases a K-tile, q0: A0 x B0, q1: A0 x B1, over
-// three K-tiles of three half-tiles (144 KiB): q0 of K-tile t asks for A0 and B0 of t + 2, q1 for its B1, into the slots that t - 1 was read from two
-// phases before, and at q1 a wave waits until only the four pieces it asked for in q0 may be on their way: all of t + 1 has landed.
+// TAIL: the tiles behind an XCD's last whole round run as two halves of 128 rows each, on twice as many workgroups (the launcher's rule; 2: no whole
+// tiles, and K splits walked one behind the other and added up in registers; with that in sight whole tiles take 1 % longer). A half walks K in
+// two phases a K-tile, q0: A0 x B0, q1: A0 x B1, over three K-tiles of three half-tiles (144 KiB): q0 of K-tile t asks for A0 and B0 of t + 2, q1 for its
+// B1, into the slots that t - 1 was read from two phases before, and at q1 a wave waits until only the four pieces it asked for in q0 may be
+// on their way: all of t + 1 has landed.
 // ACT: the activation of a feed-forward in the epilogue, on the fp32 sums, instead of a launch that reads them back (an instantiation each, for the
 // registers' sake): 1 gelu_tanh(gate) * up from weights whose first N / 2 rows are the gate's: B0 takes gate columns and B1 the up columns of
 // the same places, so both meet in one wave; p.bias [N]. 2 xIELU with the coefficients p.coef [2], N a multiple of 256, rows of out in
 // 16-byte pieces. bf16 out. K 4096, width 14336, two launches against
 // one, 300 / 1531 / 2048 rows: gated 111 / 300 / 383 -> 101 / 271 / 350 us, xIELU (fp32 between the two) 60 / 169 / 222 -> 59 / 159 / 205.
-template <bool F8, bool CMAX = false, bool TAIL = false, int ACT = 0>
+template <bool F8, bool CMAX = false, int TAIL = 0, int ACT = 0>
 __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams p) {
   static_assert(!(CMAX && TAIL), "the chunk maxima of a half tile would need their own rows");
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -107,7 +108,7 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
   const int nb = (p.ntiles + 15) >> 4;           // 256-column blocks (the last may have one column half only)
   // ... and the K splits of one tile are neighbours in that order: dispatched together, done together.
   const int within = blockIdx.x >> 3;
-  const bool half = TAIL && within >= p.full_items;
+  const bool half = TAIL == 2 || (TAIL && within >= p.full_items);
   const int ks = TAIL ? 0 : within % p.splitk, rest = TAIL ? (half ? p.full_items + ((within - p.full_items) >> 1) : within) : within / p.splitk;
   const int cb = (rest / mblocks) * 8 + (blockIdx.x & 7);
   if (cb >= nb) return;                          // grid padded to 8 column blocks; whole workgroup, before any barrier
@@ -264,8 +265,8 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
     };
     // The sums of a K split join those before it in the registers of the missing half: the bits of the splits below, without their slabs. Done
     // while the other group multiplies: a quarter's sums in the interval in which this group reads the fragments of the other.
-    int border = per < n ? per : n + 1;              // first K-tile of the next split
-    auto join = [](f32x4 (&a)[4][2], f32x4 (&sum)[4][2]) {
+    [[maybe_unused]] int border = per;               // first K-tile of the next split
+    [[maybe_unused]] auto join = [](f32x4 (&a)[4][2], f32x4 (&sum)[4][2]) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -291,8 +292,10 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (q == 0) { fetch(ic<0>{}, t + 2, there); fetch(ic<1>{}, t + 2, there + 1); }
       else fetch(ic<2>{}, t + 2, there + 2);
-      if constexpr (q == 0) { if (t == border) { join(acc[0][1], acc[1][1]); border += per; } }
-      else if (t + 1 == border) join(acc[0][0], acc[1][0]);
+      if constexpr (TAIL == 2) {
+        if constexpr (q == 0) { if (t == border) { join(acc[0][1], acc[1][1]); border += per; } }
+        else if (t + 1 == border) join(acc[0][0], acc[1][0]);
+      }
       pp_barrier();
       cluster(acc[0][q], q ? b1 : b0);
       pp_barrier();
@@ -307,7 +310,7 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
       if (t + 1 < n) { half_phase(ic<0>{}, t + 1, ic<1>{}); half_phase(ic<1>{}, t + 1, ic<1>{}); }
       if (t + 2 < n) { half_phase(ic<0>{}, t + 2, ic<2>{}); half_phase(ic<1>{}, t + 2, ic<2>{}); }
     }
-    if (per < n) {
+    if constexpr (TAIL == 2) {
 #pragma unroll
       for (int f = 0; f < 16; ++f) {
         f32x4& a = acc[0][f >> 3][(f >> 1) & 3][f & 1];
@@ -395,26 +398,33 @@ __global__ __launch_bounds__(kPPThreads, 2) void gemm_pingpong_kernel(GemmParams
     };
 #pragma unroll
     for (int f0 = 0; f0 < 32; f0 += 8) {
-      f32x4 t[8], sum[8];
+      auto own = [&](int u) -> f32x4& { return acc[f0 >> 4][(f0 >> 3) & 1][u >> 1][u & 1]; };
+      auto add = [](f32x4 (&to)[8], const f32x4 (&t)[8]) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) to[u] += t[u];
+      };
+      f32x4 t[8], t2[8], sum[8];
       if (ks > 0) {
         load8(0, f0, sum);
+        int s = 1;
 #pragma unroll 1
-        for (int s = 1; s < ks; ++s) {
-          load8(s, f0, t);
+        for (; s + 1 < ks; s += 2) { load8(s, f0, t); load8(s + 1, f0, t2); add(sum, t); add(sum, t2); }
+        if (s < ks) { load8(s, f0, t); add(sum, t); }
 #pragma unroll
-          for (int u = 0; u < 8; ++u) sum[u] += t[u];
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          f32x4& a = acc[f0 >> 4][(f0 >> 3) & 1][u >> 1][u & 1];
-          a = sum[u] + a;
-        }
+        for (int u = 0; u < 8; ++u) own(u) = sum[u] + own(u);
       }
+      int s = ks + 1;
 #pragma unroll 1
-      for (int s = ks + 1; s < p.splitk; ++s) {
+      for (; s + 1 < p.splitk; s += 2) {
+        load8(s, f0, t);
+        load8(s + 1, f0, t2);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) own(u) = own(u) + t[u] + t2[u];
+      }
+      if (s < p.splitk) {
         load8(s, f0, t);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) acc[f0 >> 4][(f0 >> 3) & 1][u >> 1][u & 1] += t[u];
+        for (int u = 0; u < 8; ++u) own(u) += t[u];
       }
     }
     if (tid == 0) {                                          // both counters back to zero for the next launch
@@ -1044,7 +1054,7 @@ extern "C" long dlia_gemm_pingpong_ws_floats(int M, int N, int K) {
 // bf16, M > 256 (any M is correct; below that the weight-streaming kernels are faster), K a
 // multiple of 64; `p` fully set up by the caller. p->splitk > 1 needs p->partial = slabs for
 // [tiles][splitk - 1] and p->counters = two zero words per tile (the kernel leaves them zero).
-template <bool F8, bool CMAX = false, bool TAIL = false, int ACT = 0>
+template <bool F8, bool CMAX = false, int TAIL = 0, int ACT = 0>
 static void launch_pingpong_kernel(const dlia::GemmParams* p, int workgroups, hipStream_t stream) {
   constexpr int lds = TAIL ? kPPTailLds : kPPLds;
   static const bool once = [] {
@@ -1060,11 +1070,13 @@ static void launch_pingpong(const dlia::GemmParams* p, hipStream_t stream) {
   const int nb = (p->ntiles + 15) / 16, nb8 = (nb + 7) / 8 * 8, mblocks = (p->M + 255) / 256;
   if constexpr (!CMAX) {
     if (p->full_items >= 0) {
-      launch_pingpong_kernel<F8, false, true, ACT>(p, 8 * (p->full_items + 2 * (nb8 / 8 * mblocks - p->full_items)), stream);
+      const int workgroups = 8 * (p->full_items + 2 * (nb8 / 8 * mblocks - p->full_items));
+      if (p->splitk > 1) launch_pingpong_kernel<F8, false, 2, ACT>(p, workgroups, stream);
+      else launch_pingpong_kernel<F8, false, 1, ACT>(p, workgroups, stream);
       return;
     }
   }
-  launch_pingpong_kernel<F8, CMAX, false, ACT>(p, nb8 * mblocks * p->splitk, stream);
+  launch_pingpong_kernel<F8, CMAX, 0, ACT>(p, nb8 * mblocks * p->splitk, stream);
 }
 static void launch_quad(const dlia::GemmParams* p, hipStream_t stream) {
   static const bool once = [] {
