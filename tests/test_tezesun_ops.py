@@ -372,6 +372,21 @@ def test_xielu_rows_in_pieces_and_one_by_one(M, F, ld, dt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,F,ld", [(512, 1024, 1024), (511, 1024, 1024), (514, 1022, 1024), (520, 1024, 1025), (1, 1 << 19, 1 << 19)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_xielu_on_both_sides_of_the_line(M, F, ld, dt):
+    """2^19 entries, from which on a thread takes four where the rows allow: the same entries one by one, to the bit."""
+    K, dev = _K(), "cuda"
+    z, pq = rnd(M, ld, seed=1, std=2.0).float().to(dev)[:, :F], torch.tensor([0.8, 1.05], device=dev)
+    act, few = torch.full((M, F), 7.0, device=dev, dtype=dt), torch.full((M, F), 7.0, device=dev, dtype=dt)
+    K.xielu(act, z, pq)
+    for m in range(0, M, 64):
+        for c in range(0, F, 4096):
+            K.xielu(few[m:m + 64, c:c + 4096], z[m:m + 64, c:c + 4096], pq)
+    assert torch.equal(act, few) and not bool((few == 7.0).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("F", [65537, 65540])
 def test_xielu_of_more_entries_than_a_dimension_has_threads(F):
     """A little over 2^32 entries one by one, and over 2^30 pieces of four, for which a launch has a second dimension: every row as one row by itself."""
