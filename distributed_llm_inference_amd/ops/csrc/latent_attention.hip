@@ -47,8 +47,10 @@ __global__ __launch_bounds__((64 * lat_waves<KS, SPLITV>())) void latent_attenti
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r16 = lane & 15, kq = lane >> 4;
   // the last tiles of all sequences first: they have the most keys (one prompt of 1900 tokens of 32 heads, 475 workgroups of 1 to 60 blocks,
   // 229 -> 179 us; two of 1100 and 800 138 either way)
-  // (within a window shorter than the portions all tiles have about the same, and neighbours share their keys: 512 of 1900 107 us, 112 so)
-  const bool even = p.window > 0 && (long)p.window * p.H < (long)p.tiles_per_seq * (SPLITV ? 16 : 16 * NW);
+  // (within a window shorter than the portions all tiles have about the same, and neighbours share their keys: 512 of 1900 107 us, 112 so; tiles that
+  // leave half of the chip to their key splits have no first: 16 portions of 60 21.1 us, 22.2 so, one of 600 of 8 heads 28.4, 29.9. Single tokens:
+  // a sequence's tiles are on one XCD so, 32 behind 700 33.6 -> 30.2)
+  const bool even = (!SPLITV && gridDim.x <= 128) || (p.window > 0 && (long)p.window * p.H < (long)p.tiles_per_seq * (SPLITV ? 16 : 16 * NW));
   const int seqs = gridDim.x / p.tiles_per_seq, b = even ? blockIdx.x / p.tiles_per_seq : blockIdx.x % seqs;
   const int ti = even ? blockIdx.x % p.tiles_per_seq : p.tiles_per_seq - 1 - blockIdx.x / seqs;
   const int t0 = p.q_start[b], n = p.q_start[b + 1] - t0, c0 = p.ctx[b], slot = p.slots[b];

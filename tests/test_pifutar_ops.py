@@ -267,7 +267,7 @@ def test_latent_attention_hip(D, R, H, window):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("window", [0, 40, 4000])        # (a window shorter than the portions' tiles: sequence after sequence; otherwise last tiles first)
-@pytest.mark.parametrize("D,R,H", [(40, 32, 4), (576, 512, 3)])
+@pytest.mark.parametrize("D,R,H", [(40, 32, 16), (576, 512, 8)])          # (440 workgroups together, more than run at once)
 def test_latent_attention_of_several_sequences_hip(D, R, H, window):
     """Tiles of sequences of different lengths in both orders, an empty one among them: each as by itself, to the bit."""
     K, dev, bf = _K(), "cuda", torch.bfloat16
