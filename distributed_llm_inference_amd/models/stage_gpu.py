@@ -215,6 +215,9 @@ class GpuStage:
         self._gemm_cfg: Dict[tuple, tuple] = {}
         self._ones = torch.ones(H, device=dev, dtype=bf)
         self.scale = 1.0 / math.sqrt(spec.head_dim)
+        # Rows up to which a step runs on `gemm_thin` (RMSNorm, bf16 weights): the kernel's limit on rows times hidden size. Below a hidden size of
+        # 1024 its waves have less than a chunk of K each; there steps of any number of rows up to 128 keep kernels that add K up alike.
+        self._thin_rows = min(16, 32767 // H) if self.wmode == "bf16" and spec.is_llama and 1024 <= H <= 4096 else 0
 
     def _init_limits(self, spec, plan, device, max_slots, max_seq_len, max_tokens, max_batch, use_graphs, graph_sizes):
         """What every executor on this library shares, whatever its layers are: the kernel library, the
@@ -449,7 +452,7 @@ class GpuStage:
         return c
 
     def _layers(self, wk: _Work, T: int, B: int, tok_pos, tok_seq, q_start, ctx, slots, max_q: int, splits: int,
-                alone: bool = False, lead_decode: int = 0, entry: Optional[torch.Tensor] = None):
+                alone: bool = False, lead_decode: int = 0, entry: Optional[torch.Tensor] = None, leave: Optional[torch.Tensor] = None):
         """Runs this stage's decoder layers on wk.h[:T] (decode regime: or on the rows `entry`, which wk.h takes over). Returns the pending split-K partial
         (splits, bias) of the last down projection that the caller still has to fold into h
         (decode regime), or None when h is final. `lead_decode`: the first that many sequences of a
@@ -503,6 +506,30 @@ class GpuStage:
                 else:
                     self._gemm(wk, act, x2, p, "w_fc", p["b_fc"], None, lws, I, 5, tg, 0)
                     self._gemm(wk, h, act, p, "w_down", p["b_down"], h, lws, H, 3, tg, 0)
+            return None
+        if T <= self._thin_rows:
+            # few rows: every GEMM's sums are complete inside its workgroups, so the residual is added where they are formed and the
+            # next GEMM normalises the rows itself (`leave`: where the last block's rows go instead of wk.h)
+            src = h if entry is None else entry
+            z = wk.ws[:T * s.qkv_size].view(T, s.qkv_size)
+            last, skip = len(self.layers) - 1, 1 if self.plan.skip_attn_first else 0
+            for li, p in enumerate(self.layers):
+                to = leave if leave is not None and li == last else h
+                if "w_qkv" in p:
+                    if self.kv8:        # (an e4m3 row's scale needs the whole head)
+                        K.gemm_thin(z, src, p["w_qkv"], p["ln1_w"], s.norm_eps, None, None, s.qkv_size, 6)
+                        self._kvwrite(li, qkv, wk.ws, 1, p.get("b_qkv"), tok_pos, tok_seq)
+                    else:
+                        K.gemm_thin_qkv(qkv, src, p["w_qkv"], p["ln1_w"], s.norm_eps, p.get("b_qkv"), self.kv[li - skip], self.cos, self.sin,
+                                        tok_pos, tok_seq, self.block_table, Hq, Hkv, D)
+                    attend(li)
+                    o = h if "w_down" in p else to
+                    K.gemm_thin(o, attn, p["w_o"], None, 0.0, p.get("b_o"), src, H, 2)
+                    src = o
+                if "w_down" in p:
+                    K.gemm_thin(act, src, p["w_gu"], p["ln2_w"], s.norm_eps, None, None, 2 * I, 4)
+                    K.gemm_thin(to, act, p["w_down"], None, 0.0, p.get("b_down"), src, H, 2)
+                    src = to
             return None
         # decode regime: weight-streaming GEMMs write fp32 split-K partials which the NEXT kernel
         # (norm / rope) sums while it reads them anyway — no reduce launches, no bf16 round trip
@@ -711,6 +738,9 @@ class GpuStage:
             entry = {"entry": st.hidden_in}
         else:
             wk.h[:B].copy_(st.hidden_in)
+        leaves = "entry" in entry and not self.plan.has_head and B <= self._thin_rows
+        if leaves:
+            entry["leave"] = st.hidden_out
         pend = self._layers(wk, B, B, st.ctx, st.slots, self._arange[:B + 1], st.ctx, st.slots, 1, st.splits, **entry)
         if self.plan.has_head:
             self._head(wk, self._arange, B, B, pend)
@@ -718,6 +748,8 @@ class GpuStage:
             # pipeline, where the feedback hop is local — puts the token into the next step's input ids
             K.sample_step(st.tokens, wk.logits[:B], wk.cmax[:B] if wk.guided else None, st.temperature, st.top_k, st.top_p,
                           st.seeds, st.steps, self.spec.vocab_size, st.ids if self.plan.has_embed else None, st.ctx)
+        elif leaves:
+            K.advance(st.ctx, 1)
         elif self._first_norm_enters and pend is not None:
             K.fold_out(st.hidden_out, wk.h[:B], wk.ws, pend[0], pend[1], st.ctx)
         else:

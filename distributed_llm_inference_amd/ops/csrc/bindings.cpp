@@ -400,6 +400,66 @@ void gemm(Tensor out, const Tensor& x, const Tensor& wp, OptTensor bias, OptTens
   gemm_impl(out, x, wp, c10::nullopt, bias, residual, workspace, N, epi, splitk, ntw);
 }
 
+// At most 16 rows, every sum complete inside a workgroup: epi 2 out = x @ Wp^T + bias + residual, bf16; with RMSNorm(x), K up to 4096, M K up to 32768: epi 4 SwiGLU, bf16,
+// epi 6 fp32 [M, N], epi 7 (gemm_thin_qkv) rotated q | k | v.
+static void gemm_thin_impl(Tensor out, const Tensor& x, const Tensor& wp, OptTensor norm_w, double eps, OptTensor bias, OptTensor residual, int64_t N,
+                           int64_t epi, const dlia::ThinRope* rope) {
+  check_dev(out, "out"); check_bf16(x, "x"); check_rows(x, "x"); check_bf16(wp, "wp");
+  const int64_t M = x.size(0), K = x.size(1), n_out = epi == 4 ? N / 2 : N;
+  DLIA_CHECK(M <= 16, "gemm_thin: at most 16 rows");
+  DLIA_CHECK(K % 128 == 0 && N > 0 && N % 4 == 0, "gemm_thin: K a multiple of 128, N of 4");
+  DLIA_CHECK(epi != 4 || N % 32 == 0, "swiglu needs gate/up tile pairs");
+  DLIA_CHECK(wp.is_contiguous() && wp.numel() == (N + 127) / 128 * 128 * K && reinterpret_cast<uintptr_t>(wp.data_ptr()) % 16 == 0, "packed weight size");
+  DLIA_CHECK(out.scalar_type() == (epi == 6 ? at::kFloat : at::kBFloat16) && out.dim() == 2 && out.stride(1) == 1 && out.size(0) >= M && out.size(1) >= n_out &&
+             out.stride(0) % 4 == 0 && reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0, "gemm_thin: out");
+  DLIA_CHECK(out.data_ptr() != x.data_ptr(), "gemm_thin: other workgroups read x while out is written");
+  const void* np = nullptr; const void* bp = nullptr; const void* rp = nullptr; long ldr = 0;
+  DLIA_CHECK(norm_w.has_value() == (epi != 2) && (epi == 2 || (K <= 4096 && M * K <= 32768)), "gemm_thin: RMSNorm with epi 4, 6 and 7, K up to 4096, M K up to 32768");
+  if (norm_w.has_value()) {
+    check_bf16(*norm_w, "norm_w");
+    DLIA_CHECK(norm_w->is_contiguous() && norm_w->numel() == K && reinterpret_cast<uintptr_t>(norm_w->data_ptr()) % 16 == 0, "norm_w");
+    np = norm_w->data_ptr();
+  }
+  if (bias.has_value()) {
+    check_bf16(*bias, "bias");
+    DLIA_CHECK((epi == 2 || epi == 7) && bias->is_contiguous() && bias->numel() == N && reinterpret_cast<uintptr_t>(bias->data_ptr()) % 8 == 0, "gemm_thin: bias");
+    bp = bias->data_ptr();
+  }
+  DLIA_CHECK(residual.has_value() == (epi == 2), "gemm_thin: epi 2 adds a residual");
+  if (residual.has_value()) {
+    check_bf16(*residual, "residual");
+    DLIA_CHECK(residual->dim() == 2 && residual->stride(1) == 1 && residual->size(0) >= M && residual->size(1) >= N && residual->stride(0) % 4 == 0 &&
+               reinterpret_cast<uintptr_t>(residual->data_ptr()) % 8 == 0, "gemm_thin: residual");
+    rp = residual->data_ptr(); ldr = residual->stride(0);
+  }
+  dlia_gemm_thin(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), wp.data_ptr(), np, (float)eps, bp, rp, ldr, (int)M, (int)N, (int)K, (int)epi,
+                 rope, cur_stream());
+}
+
+void gemm_thin(Tensor out, const Tensor& x, const Tensor& wp, OptTensor norm_w, double eps, OptTensor bias, OptTensor residual, int64_t N, int64_t epi) {
+  DLIA_ON_DEVICE_OF(out);
+  DLIA_CHECK(epi == 2 || epi == 4 || epi == 6, "gemm_thin: epi 2, 4 or 6");
+  gemm_thin_impl(out, x, wp, norm_w, eps, bias, residual, N, epi, nullptr);
+}
+
+// q | k | v of RMSNorm(x): + bias, rotated; q to the front of qkv's rows, k and v to the paged bf16 cache.
+void gemm_thin_qkv(Tensor qkv, const Tensor& x, const Tensor& wp, const Tensor& norm_w, double eps, OptTensor bias, Tensor kv_cache, const Tensor& cos_t,
+                   const Tensor& sin_t, const Tensor& tok_pos, const Tensor& tok_seq, const Tensor& block_table, int64_t Hq, int64_t Hkv, int64_t D) {
+  DLIA_ON_DEVICE_OF(qkv);
+  DLIA_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128");
+  const int64_t T = x.size(0);
+  auto g = check_kv(kv_cache, Hkv, D);
+  check_i32(tok_pos, "tok_pos"); check_i32(tok_seq, "tok_seq"); check_i32(block_table, "block_table");
+  DLIA_CHECK(tok_pos.numel() >= T && tok_seq.numel() >= T && block_table.dim() == 2, "gemm_thin_qkv: metadata shapes");
+  check_f32(cos_t, "cos"); check_f32(sin_t, "sin");
+  DLIA_CHECK(cos_t.dim() == 2 && cos_t.size(0) > 0 && cos_t.size(1) == D / 2 && sin_t.sizes() == cos_t.sizes() && cos_t.is_contiguous() && sin_t.is_contiguous(),
+             "rope tables [P, D/2]");
+  const dlia::ThinRope r = {kv_cache.data_ptr(), cos_t.data_ptr<float>(), sin_t.data_ptr<float>(), tok_pos.data_ptr<int>(), tok_seq.data_ptr<int>(),
+                            block_table.data_ptr<int>(), (int)Hq, (int)Hkv, (int)D, (int)block_table.size(1), (int)g.num_blocks, (int)cos_t.size(0)};
+  // tok_seq values index block_table rows: the caller guarantees tok_seq < block_table.size(0)
+  gemm_thin_impl(qkv, x, wp, norm_w, eps, bias, c10::nullopt, (Hq + 2 * Hkv) * D, 7, &r);
+}
+
 void gemm_w8(Tensor out, const Tensor& x, const Tensor& wp, const Tensor& wscale, OptTensor bias, OptTensor residual,
              OptTensor workspace, int64_t N, int64_t epi, int64_t splitk, int64_t ntw) {
   gemm_impl(out, x, wp, wscale, bias, residual, workspace, N, epi, splitk, ntw);
@@ -1011,6 +1071,9 @@ TORCH_LIBRARY(dlia, m) {
   m.def("rope_kvwrite(Tensor(a!) qkv, Tensor? partial, int splits, Tensor? pbias, Tensor(b!) kv_cache, Tensor cos, Tensor sin, Tensor tok_pos, Tensor tok_seq, Tensor block_table, int Hq, int Hkv, int D, bool use_rope) -> ()");
   m.def("rope_kvwrite8(Tensor(a!) qkv, Tensor? partial, int splits, Tensor? pbias, Tensor(b!) kv_cache, Tensor(c!) kv_scale, Tensor cos, Tensor sin, Tensor tok_pos, Tensor tok_seq, Tensor block_table, int Hq, int Hkv, int D, bool use_rope) -> ()");
   m.def("paged_attention8(Tensor(a!) out, Tensor qkv, Tensor kv_cache, Tensor kv_scale, Tensor q_start, Tensor ctx_lens, Tensor block_table, Tensor? slots, Tensor? partial, int max_q_len, int Hq, int Hkv, int D, float scale, int splits) -> ()");
+  m.def("gemm_thin(Tensor(a!) out, Tensor x, Tensor wp, Tensor? norm_w, float eps, Tensor? bias, Tensor? residual, int N, int epi) -> ()");
+  m.def("gemm_thin_qkv(Tensor(a!) qkv, Tensor x, Tensor wp, Tensor norm_w, float eps, Tensor? bias, Tensor(b!) kv_cache, Tensor cos_t, Tensor sin_t, "
+        "Tensor tok_pos, Tensor tok_seq, Tensor block_table, int Hq, int Hkv, int D) -> ()");
   m.def("gemm(Tensor(a!) out, Tensor x, Tensor wp, Tensor? bias, Tensor? residual, Tensor? workspace, int N, int epi, int splitk, int ntw) -> ()");
   m.def("gemm_act(Tensor(a!) out, Tensor x, Tensor wp, Tensor? bias, Tensor? coef, Tensor? workspace, int N, int act, int workgroups) -> ()");
   m.def("gemm_w8(Tensor(a!) out, Tensor x, Tensor wp, Tensor wscale, Tensor? bias, Tensor? residual, Tensor? workspace, int N, int epi, int splitk, int ntw) -> ()");
@@ -1058,6 +1121,8 @@ TORCH_LIBRARY_IMPL(dlia, CUDA, m) {
   m.impl("rope_kvwrite8", &rope_kvwrite8);
   m.impl("paged_attention8", &paged_attention8);
   m.impl("gemm", &gemm);
+  m.impl("gemm_thin", &gemm_thin);
+  m.impl("gemm_thin_qkv", &gemm_thin_qkv);
   m.impl("gemm_act", &gemm_act);
   m.impl("gemm_w8", &gemm_w8);
   m.impl("gemm_a8w8", &gemm_a8w8);

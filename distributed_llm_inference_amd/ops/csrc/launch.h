@@ -4,6 +4,14 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+namespace dlia {
+// where gemm_thin.hip puts q | k | v: the paged cache, the rotation's tables and every row's place
+struct ThinRope {
+  void* kv; const float* cos_t; const float* sin_t; const int* tok_pos; const int* tok_seq; const int* block_table;
+  int Hq, Hkv, D, max_blocks, num_blocks, rope_len;
+};
+}  // namespace dlia
+
 extern "C" {
 
 // ---- norm.hip -------------------------------------------------------------------------
@@ -120,6 +128,12 @@ void dlia_norm32(void* out, int out_f32, float* x, const float* y, const float* 
                  int rows, int H, long ldx, long ldy, long ldo, float eps, float off, hipStream_t stream);
 void dlia_gated_headnorm(void* out, int out_f32, const float* o, const float* gate, const float* w, int T, int heads, int dv,
                          long ldo_in, long ldg, long ld_out, float eps, hipStream_t stream);
+
+// ---- gemm_thin.hip --------------------------------------------------------------------------
+// At most 16 rows, no K splits. epi 2: out = x @ Wp^T + bias + residual (bf16); epi 4, 6, 7: x goes through RMSNorm first (K up to 2048): SwiGLU (bf16),
+// fp32 sums, or q | k | v: + bias, rotated, q to out's rows and k, v to the paged cache (`rope`)
+void dlia_gemm_thin(void* out, long ldo, const void* x, long ldx, const void* wp, const void* norm_w, float eps, const void* bias,
+                    const void* residual, long ldr, int M, int N, int K, int epi, const dlia::ThinRope* rope, hipStream_t stream);
 
 // ---- gemm_any.hip ---------------------------------------------------------------------------
 // C[M,N] = A[M,K] . W[N,K]^T (+ bias), any shape, row-major W; epi 1: gated pair (interleaved gate / up tiles) ->
