@@ -89,10 +89,12 @@ constexpr float kNegInf = -__builtin_inff();
 // NW = waves per work item: 4 interleave the item's KV blocks and merge at the end (few items, long
 // contexts); 1 walks all of them alone with no LDS and no barrier (decode over thousands of
 // (sequence, kv head) items, where a 160-token context is 5 blocks and 4 waves would take 2, 1, 1, 1).
-// EXT: 0 plain causal; 1 window, sink and the learned extras; 2 window, capped scores and the entry gate.
+// EXT: 0 plain causal; 1 window, sink and the learned extras; 2 window, capped scores and the entry gate; 3 as 1
+// with one column tile and a bias, whose entries come with the keys (asked for where they are used, a block waits for them: 128 sequences of 700 tokens
+// 78 -> 69 us).
 template <int D, int NT, bool KV8, int NW, bool PF, int EXT = 0>
 __device__ __forceinline__ void paged_attn_body(const AttnParams& p, long item) {
-  constexpr bool WIN = EXT >= 1, LEARNED = EXT == 1, CAPPED = EXT == 2;
+  constexpr bool WIN = EXT >= 1, LEARNED = EXT == 1 || EXT == 3, CAPPED = EXT == 2;
   constexpr int KS = D / 32;      // MFMA k-steps over the head dim (QK^T)
   constexpr int DT = D / 16;      // 16-row tiles of the head dim (PV)
   constexpr int NC = NT * 16;     // query columns per workgroup
@@ -186,9 +188,25 @@ __device__ __forceinline__ void paged_attn_body(const AttnParams& p, long item) 
     u32x4 k[2][KV8 ? KS / 2 : KS];
     u32x4 v[KV8 ? DT / 2 : DT];
     f32x4 sk[2], sv[2];
+    float bias[2][4];                            // LEARNED decode: this lane's entries of the table, on their way with the keys
+  };
+  constexpr bool BIAS_AHEAD = EXT == 3;
+  static_assert(EXT != 3 || NT == 1, "one column tile");
+  auto bias_at = [&](int nt, int kb, int kt, int r) {
+    const int limit = col_qpos[nt] >= 0 ? ctx + col_qpos[nt] : -1;
+    const int dist = min(max(limit - (kb * kBlockTokens + kt * 16 + quad * 4 + r), 0), p.bias_rows - 1);
+    return col_bias[nt][(long)dist * p.Hq];
   };
   auto load_kv = [&](int kb, Raw& r) {
     const int blk = block_of(kb);
+    if constexpr (BIAS_AHEAD) {
+      if (p.bias) {
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) r.bias[kt][e] = bias_at(0, kb, kt, e);
+      }
+    }
     if constexpr (KV8) {
       const unsigned char* kbase = reinterpret_cast<const unsigned char*>(p.kv) + kv_head_base(blk, kvh, p.Hkv, D, 0) + lane * 16;
 #pragma unroll
@@ -257,10 +275,8 @@ __device__ __forceinline__ void paged_attn_body(const AttnParams& p, long item) 
 #pragma unroll
           for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int dist = min(max(limit - (kb * kBlockTokens + kt * 16 + quad * 4 + r), 0), p.bias_rows - 1);
-              st[kt][nt][r] = st[kt][nt][r] * col_temp[nt] + (col_bias[nt] ? col_bias[nt][(long)dist * p.Hq] : 0.f);
-            }
+            for (int r = 0; r < 4; ++r)
+              st[kt][nt][r] = st[kt][nt][r] * col_temp[nt] + (p.bias ? (BIAS_AHEAD ? raw.bias[kt][r] : bias_at(nt, kb, kt, r)) : 0.f);
         }
       }
 #pragma unroll
@@ -426,8 +442,10 @@ __device__ __forceinline__ void paged_attn_body(const AttnParams& p, long item) 
   }
 }
 
-template <int D, int NT, bool KV8, int EXT = 0>
-__global__ __launch_bounds__(256) void paged_attn_kernel(AttnParams p) { paged_attn_body<D, NT, KV8, 4, true, EXT>(p, blockIdx.x); }
+// OCC: waves a SIMD that the registers allow. With a window or the extras the compiler takes a few more than 256 where it may, and a CU holds one
+// workgroup: too few bytes on their way once there are more items than CUs.
+template <int D, int NT, bool KV8, int EXT = 0, int OCC = 1>
+__global__ __launch_bounds__(256, OCC) void paged_attn_kernel(AttnParams p) { paged_attn_body<D, NT, KV8, 4, true, EXT>(p, blockIdx.x); }
 
 // One wave per item, one block in flight per wave, registers capped so that 3 waves share a SIMD:
 // latency is hidden by the other waves instead of by a second set of K/V registers.
@@ -903,23 +921,34 @@ static inline long wave_per_item_threshold() {
   return v;
 }
 
+// (two workgroups a CU, see there, from more items than CUs on: 64 sequences x 8 heads of 512 to 1024 tokens in a step 58 -> 47 us; 32 x 8 of 1125 with either 26)
+template <int D, int NT, int EXT>
+static void launch_attn_sink(const AttnParams& p, long nitems, long thr, hipStream_t stream) {
+  constexpr size_t smem = 4 * NT * 64 * 2 * 4 + 4 * (D / 16) * NT * 64 * 16;
+  constexpr int two = NT == 1 ? 2 : 1;
+  if (NT == 1 && thr > 0 && nitems >= thr) hipLaunchKernelGGL((paged_attn_lean_kernel<D, false, EXT>), dim3((unsigned)nitems), dim3(64), 0, stream, p);
+  else if (nitems > 256) hipLaunchKernelGGL((paged_attn_kernel<D, NT, false, EXT, two>), dim3((unsigned)nitems), dim3(256), smem, stream, p);
+  else hipLaunchKernelGGL((paged_attn_kernel<D, NT, false, EXT>), dim3((unsigned)nitems), dim3(256), smem, stream, p);
+}
+
 template <int D, int NT>
 static void launch_attn(const AttnParams& p, hipStream_t stream) {
   const long nitems = (long)p.B * p.Hkv * p.qtiles * p.splits;
   constexpr size_t smem = 4 * NT * 64 * 2 * 4 + 4 * (D / 16) * NT * 64 * 16;
   const long thr = wave_per_item_threshold();
+  constexpr int two = NT == 1 ? 2 : 1, with_bias = NT == 1 ? 3 : 1;
   const char* pe = getenv("DLIA_ATTN_PERSIST");               // read per launch (a captured graph keeps what it was captured with)
   const long persist = pe ? atol(pe) : 0L;
   if (capped(p) && !p.kv_scale) {                            // capped / entry-gated instantiations (bf16 cache)
     if (NT == 1 && thr > 0 && nitems >= thr)
       hipLaunchKernelGGL((paged_attn_lean_kernel<D, false, 2>), dim3((unsigned)nitems), dim3(64), 0, stream, p);
+    else if (NT == 1 && nitems > 256)
+      hipLaunchKernelGGL((paged_attn_kernel<D, NT, false, 2, two>), dim3((unsigned)nitems), dim3(256), smem, stream, p);
     else
       hipLaunchKernelGGL((paged_attn_kernel<D, NT, false, 2>), dim3((unsigned)nitems), dim3(256), smem, stream, p);
   } else if ((p.window > 0 || p.sink) && !p.kv_scale) {      // windowed / sink instantiations (bf16 cache)
-    if (NT == 1 && thr > 0 && nitems >= thr)
-      hipLaunchKernelGGL((paged_attn_lean_kernel<D, false, 1>), dim3((unsigned)nitems), dim3(64), 0, stream, p);
-    else
-      hipLaunchKernelGGL((paged_attn_kernel<D, NT, false, 1>), dim3((unsigned)nitems), dim3(256), smem, stream, p);
+    if (NT == 1 && p.bias) launch_attn_sink<D, NT, with_bias>(p, nitems, thr, stream);
+    else                   launch_attn_sink<D, NT, 1>(p, nitems, thr, stream);
   } else if (NT == 1 && thr > 0 && nitems >= thr && persist > 0 && nitems >= persist * 4 && !p.kv_scale) {
     hipLaunchKernelGGL((paged_attn_lean_persist_kernel<D, false>), dim3((unsigned)persist), dim3(256), 0, stream, p, nitems);
   } else if (NT == 1 && thr > 0 && nitems >= thr) {
