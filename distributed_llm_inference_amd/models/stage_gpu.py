@@ -213,6 +213,7 @@ class GpuStage:
         if not defer_kv:
             self.allocate_kv(num_blocks if num_blocks is not None else self.kv_budget_blocks())
         self._gemm_cfg: Dict[tuple, tuple] = {}
+        self._gemm_spread: Dict[tuple, int] = {}
         self._ones = torch.ones(H, device=dev, dtype=bf)
         self.scale = 1.0 / math.sqrt(spec.head_dim)
         # Rows up to which a step runs on `gemm_thin` (RMSNorm, bf16 weights): the kernel's limit on rows times hidden size. Below a hidden size of
@@ -451,6 +452,16 @@ class GpuStage:
             self._gemm_cfg[key] = c
         return c
 
+    def _spread(self, M: int, N: int, K: int) -> int:
+        """Workgroups that a GEMM of more than 256 rows is spread over when it has the chip for itself."""
+        key = (M, N, K)
+        t = self._gemm_spread.get(key)
+        if t is None:
+            if len(self._gemm_spread) > 4096:        # (every prompt length has its own)
+                self._gemm_spread.clear()
+            t = self._gemm_spread[key] = int(self.K.gemm_spread(M, N, K // (128 if self.wmode == "fp8" else 64))) if M > 256 else 256
+        return t
+
     def _layers(self, wk: _Work, T: int, B: int, tok_pos, tok_seq, q_start, ctx, slots, max_q: int, splits: int,
                 alone: bool = False, lead_decode: int = 0, entry: Optional[torch.Tensor] = None, leave: Optional[torch.Tensor] = None):
         """Runs this stage's decoder layers on wk.h[:T] (decode regime: or on the rows `entry`, which wk.h takes over). Returns the pending split-K partial
@@ -487,25 +498,27 @@ class GpuStage:
             # fused bias / residual / activation epilogues; the 256 x 256 kernel (bf16 and e4m3) splits
             # K inside the launch on shapes with fewer tiles than CUs and needs the workspace for that
             lws = wk.ws if self.wmode in ("bf16", "fp8") else None
-            # workgroups a thin GEMM is spread over: the whole chip for a step that runs alone (prefill
-            # chunk on the eager path), half of it for decode micro-batches that overlap on two streams
-            tg = 256 if alone else 1
+            # workgroups a thin GEMM is spread over: what takes least for a step that runs alone (prefill chunk on the eager path, the
+            # steps of a stage with a single decode micro-batch: 2 layers of Llama-3-8B with the head, 2048 rows, 3821 -> 3641 us), half
+            # the chip at most for decode micro-batches that overlap on two streams
+            alone = alone or self.decode_states == 1
+            tg = lambda n, k: self._spread(T, n, k) if alone else 1
             for li, p in enumerate(self.layers):
                 if "w_qkv" in p:            # attention block (absent from a first layer whose attention ran upstream)
                     x1 = norm(None, 1, None, p["ln1_w"], p.get("ln1_b"))
-                    self._gemm(wk, qkv, x1, p, "w_qkv", p.get("b_qkv"), None, lws, s.qkv_size, 1 if "b_qkv" in p else 0, tg, 0)
+                    self._gemm(wk, qkv, x1, p, "w_qkv", p.get("b_qkv"), None, lws, s.qkv_size, 1 if "b_qkv" in p else 0, tg(s.qkv_size, H), 0)
                     self._kvwrite(li, qkv, None, 1, None, tok_pos, tok_seq)
                     attend(li)
-                    self._gemm(wk, h, attn, p, "w_o", p.get("b_o"), h, lws, H, 3 if "b_o" in p else 2, tg, 0)
+                    self._gemm(wk, h, attn, p, "w_o", p.get("b_o"), h, lws, H, 3 if "b_o" in p else 2, tg(H, s.q_size), 0)
                 if "w_down" not in p:       # MLP block runs on the next stage
                     continue
                 x2 = norm(None, 1, None, p["ln2_w"], p.get("ln2_b"))
                 if llama:
-                    self._gemm(wk, act, x2, p, "w_gu", None, None, lws, 2 * I, 4, tg, 0)
-                    self._gemm(wk, h, act, p, "w_down", None, h, lws, H, 2, tg, 0)
+                    self._gemm(wk, act, x2, p, "w_gu", None, None, lws, 2 * I, 4, tg(2 * I, H), 0)
+                    self._gemm(wk, h, act, p, "w_down", None, h, lws, H, 2, tg(H, I), 0)
                 else:
-                    self._gemm(wk, act, x2, p, "w_fc", p["b_fc"], None, lws, I, 5, tg, 0)
-                    self._gemm(wk, h, act, p, "w_down", p["b_down"], h, lws, H, 3, tg, 0)
+                    self._gemm(wk, act, x2, p, "w_fc", p["b_fc"], None, lws, I, 5, tg(I, H), 0)
+                    self._gemm(wk, h, act, p, "w_down", p["b_down"], h, lws, H, 3, tg(H, I), 0)
             return None
         if T <= self._thin_rows:
             # few rows: every GEMM's sums are complete inside its workgroups, so the residual is added where they are formed and the

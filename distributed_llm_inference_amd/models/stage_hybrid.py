@@ -166,6 +166,7 @@ class HybridGpuStage(GpuStage):
         # latent attention in bf16: DLIA_LATENT_ATTN=0 keeps it on the general tile kernel (A/B)
         self._latent_fast = os.environ.get("DLIA_LATENT_ATTN", "1") != "0"
         self._part_cfg: Dict[tuple, tuple] = {}
+        self._gemm_spread: Dict[tuple, int] = {}
         self._shapes = []                        # (N, K, has_bias) of every packed GEMM, for the workspace
         # Attention layers whose keys and values have one size, 64 or 128, with up to 16 query heads per key / value head run
         # on the library's MFMA attention kernels (fragment-ordered cache, the windowed / sink instantiations), bf16 only;
@@ -350,8 +351,9 @@ class HybridGpuStage(GpuStage):
             self.K.gemm_any(out, x, p[name], p.get("b_" + name[2:]), 0)
             return
         b = p.get(name + "_b")
-        # more than 256 rows: the tile kernel, spread over the whole chip when a shape has few tiles
-        self.K.gemm(out, x, wp, b, None, wk.ws, p[name + "_n"], 1 if b is not None else 0, 256 if x.shape[0] > self.decode_rows else 0, 0)
+        # more than 256 rows: the tile kernel, with K splits when a shape has few tiles
+        T, K = x.shape
+        self.K.gemm(out, x, wp, b, None, wk.ws, p[name + "_n"], 1 if b is not None else 0, self._spread(T, p[name + "_n"], K) if T > self.decode_rows else 0, 0)
 
     def _act_in_gemm(self, T: int) -> bool:
         """Whether T rows take the feed-forward's activation in the large GEMM's epilogue: more than the weight streams take, and no other kernel chosen."""
@@ -598,7 +600,7 @@ class HybridGpuStage(GpuStage):
             if ls.ff:
                 act = view(wk.act, p["ff_cols"])
                 if "w_gu_p" in p and ls.ff % 16 == 0 and self._act_in_gemm(T):
-                    K.gemm_act(act, xn, p["w_gu_p"], p.get("w_gu_b"), None, wk.ws, 2 * ls.ff, 1, 256)
+                    K.gemm_act(act, xn, p["w_gu_p"], p.get("w_gu_b"), None, wk.ws, 2 * ls.ff, 1, self._spread(T, 2 * ls.ff, xn.shape[1]))
                 elif "w_gu_p" in p:
                     gu = view(wk.gu, 2 * ls.ff)
                     self._mm(wk, gu, xn, p, "w_gu")
@@ -1003,7 +1005,7 @@ class HybridGpuStage(GpuStage):
             if ls.ff:
                 z2, act, yb = view(wk.z2, self._cols(p, "w_up")), view(wk.act, ls.ff), view(wk.yb, self._cols(p, "w_down"))
                 if "w_up_p" in p and ls.ff % 256 == 0 and self._act_in_gemm(T):
-                    K.gemm_act(act, xn, p["w_up_p"], None, p["pq"], wk.ws, ls.ff, 2, 256)
+                    K.gemm_act(act, xn, p["w_up_p"], None, p["pq"], wk.ws, ls.ff, 2, self._spread(T, ls.ff, xn.shape[1]))
                 else:
                     self._mm(wk, z2, xn, p, "w_up")
                     K.xielu(act, z2, p["pq"])

@@ -555,6 +555,8 @@ void gemm_a8w8(Tensor out, const Tensor& xq, const Tensor& xscale, const Tensor&
 
 // 256 x 256 tiles per XCD in front of those that run as halves of 128 rows, -1: none do (ktiles: 128-byte pieces of a row of x)
 int64_t gemm_large_whole(int64_t M, int64_t N, int64_t ktiles, bool alone) { return dlia_gemm_pingpong_whole((int)M, (int)N, (int)ktiles, alone); }
+// the `splitk` (workgroups to spread over) that a caller with the chip for itself passes to gemm, gemm_a8w8 and gemm_act above 256 rows
+int64_t gemm_spread(int64_t M, int64_t N, int64_t ktiles) { return dlia_gemm_pingpong_spread((int)M, (int)N, (int)ktiles); }
 int64_t gemm_splitk(int64_t M, int64_t N, int64_t K) { return dlia_gemm_skinny_splitk((int)M, (int)N, (int)K); }
 
 // [ntw, splitk] the weight-streaming kernel would use for this shape
@@ -1082,6 +1084,7 @@ TORCH_LIBRARY(dlia, m) {
   m.def("quant_rows(Tensor(a!) q, Tensor(b!) scale, Tensor x) -> ()");
   m.def("gemm_config(int M, int N, int K, int epi, bool allow_split) -> int[]");
   m.def("gemm_splitk(int M, int N, int K) -> int");
+  m.def("gemm_spread(int M, int N, int ktiles) -> int");
   m.def("gemm_large_whole(int M, int N, int ktiles, bool alone) -> int");
   m.def("large_gemm_kernel(int which) -> int");
   m.def("large_gemm_default() -> bool");
@@ -1141,6 +1144,7 @@ TORCH_LIBRARY_IMPL(dlia, CUDA, m) {
 TORCH_LIBRARY_IMPL(dlia, CompositeExplicitAutograd, m) {
   m.impl("gemm_splitk", &gemm_splitk);
   m.impl("gemm_large_whole", &gemm_large_whole);
+  m.impl("gemm_spread", &gemm_spread);
   m.impl("large_gemm_kernel", &large_gemm_kernel);
   m.impl("large_gemm_default", &large_gemm_default);
   m.impl("gemm_ws_floats", &gemm_ws_floats);

@@ -1040,6 +1040,27 @@ static int pp_whole(int M, int N, int ktiles, int alone, int s) {
   }
   return 0;
 }
+// Workgroups a caller with the chip for itself asks for (`wg_target`): as many K splits as take least, not as many as fit. us of a launch of s splits, fitted
+// to 300 launches of 16 to 224 K-tiles and 16 to 256 tiles (2.5 % rms): a K-tile takes longer once more than 150 workgroups draw power and L2 bandwidth, a slab its
+// write and its read. Over 54 shapes (300 to 2048 rows, N 2048 to 8192) the number chosen is 0.4 % off the best, all that fit 5 %: N 4096, 300 rows, K 4096 / 7168 /
+// 14336 45.9 / 56.6 / 75.2 -> 38.1 / 47.7 / 68.7; N 2048, K 5632, 1024 rows 53.9 -> 43.5. (Halves where they take less than either.)
+static int pp_spread(int M, int N, int ktiles) {
+  const int tiles = ((M + 255) / 256) * ((packed_ntiles(N) + 15) / 16), most = pp_splitk(M, N, ktiles, 256);
+  if (most <= 1) return 256;
+  auto us = [&](int s) {
+    const double w = tiles * s, ktile = 0.937 + 0.389 * std::max(0.0, w - 150.0) / 96.0;
+    return 7.8 + ktile * ((ktiles + s - 1) / s) + (s > 1 ? 4.4 : 0.0) + (s - 1) * (2.54 + 0.0285 * tiles);
+  };
+  int best = 1;
+  for (int s = 2; s <= most; ++s)
+    if (us(s) < us(best)) best = s;
+  if (pp_whole(M, N, ktiles, 1, most) >= 0) {
+    const int nb = (packed_ntiles(N) + 15) / 16, per_xcd = (nb + 7) / 8 * ((M + 255) / 256);
+    if (per_xcd > 32 || 7.0 + ktiles * (0.46 + per_xcd / 70.0) + 0.85 * (most - 1) <= us(best)) return 256;
+  }
+  return std::max(2, tiles * best);                // (1 asks for the default)
+}
+extern "C" int dlia_gemm_pingpong_spread(int M, int N, int ktiles) { return pp_spread(M, N, ktiles); }
 extern "C" int dlia_gemm_pingpong_whole(int M, int N, int ktiles, int alone) { return pp_whole(M, N, ktiles, alone, pp_splitk(M, N, ktiles, 256)); }
 extern "C" int dlia_gemm_pingpong_splitk(int M, int N, int K) { return pp_splitk(M, N, K / 64); }
 // Workspace the split needs: slabs [tiles][S][256 x 256]; the arrival counters are the LAST

@@ -88,6 +88,7 @@ void dlia_gemm_large_act(void* out, const void* x, const void* wp, const void* b
 int dlia_gemm_large_choice(int which);
 // the large-M kernel's in-launch split-K: factor for a shape, and the workspace floats it needs (slabs + counters)
 int dlia_gemm_pingpong_splitk(int M, int N, int K);
+int dlia_gemm_pingpong_spread(int M, int N, int ktiles);
 int dlia_gemm_pingpong_whole(int M, int N, int ktiles, int alone);
 long dlia_gemm_pingpong_ws_floats(int M, int N, int K);
 
