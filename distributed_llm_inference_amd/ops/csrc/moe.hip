@@ -437,21 +437,29 @@ __global__ __launch_bounds__(256) void moe_down_kernel(float* __restrict__ y, co
 // holds the row tile against 16 NJ columns (of gate and up alike) over ALL of K; its four waves take K in turns, U whole k-steps (a
 // cache line or two of every row) at a time with the next piece on its way, and their partial tiles meet in LDS, added in the order
 // of the waves. Workgroups are many and short, so the chip stays even, and no half of a tile without a token is loaded or
-// multiplied. Rows of a power of two of bytes put one k of every row on the same memory channels: workgroups begin at different
+// multiplied. RT 2: the workgroup of an expert's first, third, ... tile takes the one behind it along. Rows of a power of two of bytes put one k of every row on the same memory channels: workgroups begin at different
 // places of K and go round. Two column tiles a wave halve the traffic of the token rows, which at 16 rows an expert equals the
 // weights'. (Before: 64 columns of a tile in each workgroup, every wave over all of K with its own columns: 448 or 512 workgroups on
 // 256 CUs, all on the same channels.) 8 experts, two a token, gate and up [3584, 4096], down [4096, 3584], bf16: 4 tokens 90 -> 51
 // and 75 -> 32 us, 64 tokens (470 and 235 MB) 116 -> 95 and 76 -> 50 us (4.9 and 4.7 TB/s), 160 tokens 216 -> 157 and 148 -> 96.
-template <typename T, typename OT, int KIND, bool FAST, int NW, int U, int NJ>
-__global__ __launch_bounds__(64 * NW) void moe_stream_kernel(OT* __restrict__ out, const T* __restrict__ x, const T* __restrict__ w0,
+template <typename T, typename OT, int KIND, bool FAST, int NW, int U, int NJ, int RT = 1>
+__global__ __launch_bounds__(64 * NW, RT > 1 ? 2 : 1) void moe_stream_kernel(OT* __restrict__ out, const T* __restrict__ x, const T* __restrict__ w0,
                                                              const T* __restrict__ w1, const int* __restrict__ tiles,
                                                              const int* __restrict__ row_tok, int N, int K, long ldx, long ldo, float limit,
                                                              int vec_ok, const float* __restrict__ row_w) {
   constexpr int VEC = 16 / (int)sizeof(T), KS = 4 * VEC, CH = U * KS, NG = KIND == 1 ? 2 : 1;
-  __shared__ f32x4 part[NW][2][NG * NJ][64];
+  constexpr int HM = 2 * RT;                                       // 16-row halves of RT tiles
+  __shared__ f32x4 part[NW][HM][NG * NJ][64];
   const int tile = blockIdx.y;
   if (tile >= tiles[0]) return;
   const int e = tiles[1 + tile];
+  int follows = 0;                                                 // RT 2: an expert's tiles two at a time, by the workgroup of the first
+  if constexpr (RT > 1) {
+    int before = 0;
+    while (before < tile && tiles[tile - before] == e) ++before;
+    if (before & 1) return;
+    follows = tile + 1 < tiles[0] && tiles[2 + tile] == e;
+  }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
   const int n0 = blockIdx.x * 16 * NJ;
   const int* rows = row_tok + (long)tile * kMoeTile;
@@ -463,17 +471,20 @@ __global__ __launch_bounds__(64 * NW) void moe_stream_kernel(OT* __restrict__ ou
     wr[j * NG] = w0 + wrow;
     if constexpr (KIND == 1) wr[j * NG + 1] = w1 + wrow;
   }
-  const T* ar[2]; bool av[2];
+  const T* ar[HM]; bool av[HM];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int tok = rows[i * 16 + r16];
+  for (int i = 0; i < HM; ++i) {
+    const int tok = i < 2 || follows ? rows[i * 16 + r16] : -1;
     av[i] = tok >= 0;
     ar[i] = x + (KIND == 0 ? (long)tile * kMoeTile + i * 16 + r16 : (long)(av[i] ? tok : 0)) * ldx;
   }
-  const bool both = __ballot(av[1]) != 0;
-  f32x4 acc[2][NG * NJ];
+  int halves = 1;                                                  // with a token (their rows are filled from the front)
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 1; i < HM; ++i)
+    if (__ballot(av[i]) != 0) halves = i + 1;
+  f32x4 acc[HM][NG * NJ];
+#pragma unroll
+  for (int i = 0; i < HM; ++i)
 #pragma unroll
     for (int g = 0; g < NG * NJ; ++g) acc[i][g] = f32x4{0.f, 0.f, 0.f, 0.f};
   auto run = [&](auto halves) {
@@ -516,15 +527,20 @@ __global__ __launch_bounds__(64 * NW) void moe_stream_kernel(OT* __restrict__ ou
       }
     }
   };
-  if (both) run(std::integral_constant<int, 2>{});
-  else run(std::integral_constant<int, 1>{});
+  if (halves == 1) run(std::integral_constant<int, 1>{});
+  else if (RT == 1 || halves == 2) run(std::integral_constant<int, 2>{});
+  else if constexpr (RT > 1) {
+    if (halves == 3) run(std::integral_constant<int, 3>{});
+    else run(std::integral_constant<int, 4>{});
+  }
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < HM; ++i)
 #pragma unroll
     for (int g = 0; g < NG * NJ; ++g) part[wave][i][g][lane] = acc[i][g];
   __syncthreads();
-  for (int q = wave; q < 2 * NJ; q += NW) {
-    const int i = q & 1, j = q >> 1, col = n0 + j * 16 + r16;
+  const int used = follows ? HM : 2;
+  for (int q = wave; q < used * NJ; q += NW) {
+    const int i = q % used, j = q / used, col = n0 + j * 16 + r16;
     f32x4 s[NG];
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
@@ -846,17 +862,23 @@ static void launch_moe_stream(OT* out, const T* x, const T* w0, const T* w1, con
   // 2048, 64 tokens: 27.6 us against 30.7; 3584 x 4096, 4 tokens: 51 against 58, 64 tokens 101 against 96; by the row tiles there
   // are, not the experts: 2048 x 2048, 300 / 400 tokens in 19 / 25 tiles 86 / 107 us against 70 / 89); fp32 pieces are half as deep and its
   // workgroups last longer (64 tokens: 68 against 60).
-#define DLIA_ST(FAST, U, NJ)                                                                                                               \
-  hipLaunchKernelGGL((dlia::moe_stream_kernel<T, OT, KIND, FAST, 4, U, NJ>), dim3((N + 16 * NJ - 1) / (16 * NJ), max_tiles), dim3(256), 0, \
+#define DLIA_ST(FAST, U, NJ, RT)                                                                                                               \
+  hipLaunchKernelGGL((dlia::moe_stream_kernel<T, OT, KIND, FAST, 4, U, NJ, RT>), dim3((N + 16 * NJ - 1) / (16 * NJ), max_tiles), dim3(256), 0, \
                      stream, out, x, w0, w1, tiles, row_tok, N, K, ldx, ldo, limit, ok, row_w)
   if constexpr (KIND == 1 && sizeof(T) == 2)
     if (max_tiles - experts <= 1 || (long)(N + 31) / 32 * likely_tiles(max_tiles, experts) < 768) {
-      if (ok && K % (256 / (int)sizeof(T)) == 0) DLIA_ST(true, 4, 1);
-      else DLIA_ST(false, 4, 1);
+      if (ok && K % (256 / (int)sizeof(T)) == 0) DLIA_ST(true, 4, 1, 1);
+      else DLIA_ST(false, 4, 1, 1);
       return;
     }
-  if (ok && K % (128 / (int)sizeof(T)) == 0) DLIA_ST(true, 2, 2);
-  else DLIA_ST(false, 2, 2);
+  // Tiles of one expert two a workgroup from 16 rows an expert on, where some have more than a tile: its weights then come once for 64 rows. us, a tile a
+  // workgroup against two, gated 3584 x 4096, two of 8 experts: 96 / 128 / 160 / 200 / 300 tokens 102 / 130 / 153 / 158 / 226 -> 100 / 121 / 127 / 134 / 192, down 61 / 80 / 93 / 102 / 143 ->
+  // 61 / 68 / 72 / 83 / 133; with one tile each the same (64 tokens 92, 52). Not in fp32, whose tiles are bound by the matrix rate (a prompt of 300 tokens, one expert of 8
+  // taking all of them, the step 4317 -> 4530).
+  constexpr int two = sizeof(T) == 2 ? 2 : 1;
+  if (ok && K % (128 / (int)sizeof(T)) == 0 && 2 * (max_tiles - experts) >= experts) DLIA_ST(true, 2, 2, two);
+  else if (ok && K % (128 / (int)sizeof(T)) == 0) DLIA_ST(true, 2, 2, 1);
+  else DLIA_ST(false, 2, 2, 1);
 #undef DLIA_ST
 }
 
