@@ -390,12 +390,16 @@ __global__ __launch_bounds__(256) void multi_attention_kernel(
 // accumulators of its own, so a value head's rows reach no other head. A lane's 16 bytes of a value row are one row of each of four
 // 16-entry tiles. Bound by what a CU takes from the caches (512 KB a round at key rows of 512 and four value heads of 128). Against a
 // wave per (token, head) with a key row per lane (16 bytes of 64 rows a load): 16 heads on key rows of 512, values 4 x 128, a prompt
-// of 300 / 2000 tokens 309 -> 77 / 9330 -> 1440 us, 24 sequences of 1000 tokens 944 -> 194, one 608 -> 184. Error against 64 bits,
+// of 300 / 2000 tokens 309 -> 77 / 9330 -> 1440 us, 24 sequences of 1000 tokens 944 -> 194, one 608 -> 184. The rounds begin at
+// multiples of four, so that four keys in a row lie in one block and an address serves them all; the values of 16 keys travel while 16
+// are multiplied, and only a part round clears any: one accumulator set then stays within the 128 registers that let two workgroups
+// share a CU. Against a load of each key's block and address, waited for 16 keys at a time, that and the exact count of units took
+// prompts of 300 / 1000 tokens 64 -> 53 / 384 -> 286 us, 24 sequences of 1000 tokens 192 -> 164. The same for the keys spills. Error against 64 bits,
 // mean over rows: 3.5e-7 -> 2.9e-7, 6.9e-7 -> 4.1e-7 (sums in four parts, and by rounds of 128 keys). Below 16 keys, where the contexts of a
 // batch can only be for its first tokens, the two barriers and the copy of the queries cost 0.5 to 1 us more than that wave (8 heads of
 // 64 on two key rows, 6 keys: 7.7 -> 8.8 us), with a value head per head 2.5 to 4 (10 keys: 8.6 -> 11.9); at 31 keys 14.6 -> 10.
 template <int UPW>
-__global__ __launch_bounds__(512) void multi_rows_kernel(
+__global__ __launch_bounds__(512, UPW == 1 ? 4 : 2) void multi_rows_kernel(
     float* __restrict__ out, long ldo, const float* __restrict__ q, long ldq, int q_head, const float* __restrict__ kcache, int k_row,
     const float* __restrict__ vcache, int v_row, int v_off, const int* __restrict__ tok_pos, const int* __restrict__ tok_seq,
     const int* __restrict__ block_table, int max_blocks, int num_blocks, int table_rows, int H, int G, int d, int dv, float scale,
@@ -429,14 +433,15 @@ __global__ __launch_bounds__(512) void multi_rows_kernel(
   for (int u = 0; u < UPW; ++u)
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[u][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  typedef int i32x4 __attribute__((ext_vector_type(4)));
   int buf = 0;
   for (int seg = kept > 0 ? 0 : 1; seg < 2; ++seg) {
     const int j_lo = seg == 0 ? 0 : lo, j_hi = seg == 0 ? kept - 1 : pos;
-    for (int j0 = j_lo; j0 <= j_hi; j0 += KT, buf ^= 1) {
+    for (int j0 = j_lo & ~3; j0 <= j_hi; j0 += KT, buf ^= 1) {      // (four keys in a row are of one block)
       float* S = sc + buf * KT * LS;
       int* B = bk + buf * KT;
       const int j = j0 + wave * 16 + r16;
-      int blk = j <= j_hi ? table[j / kParBlock] : -1;
+      int blk = j >= j_lo && j <= j_hi ? table[j / kParBlock] : -1;
       if (blk >= num_blocks) blk = -1;
       if (kq == 0) B[wave * 16 + r16] = blk;
       if (j0 + wave * 16 <= j_hi) {
@@ -464,7 +469,7 @@ __global__ __launch_bounds__(512) void multi_rows_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int key = sub * 16 + kq * 4 + i;
-          p[sub][i] = B[key] >= 0 ? S[key * LS + r16] : -INFINITY;      // (keys beyond the last have no block)
+          p[sub][i] = B[key] >= 0 ? S[key * LS + r16] : -INFINITY;      // (keys before the first and beyond the last have no block)
           bm = fmaxf(bm, p[sub][i]);
         }
       }
@@ -493,20 +498,31 @@ __global__ __launch_bounds__(512) void multi_rows_kernel(
         f32x4 o[4];                                  // (the part of these 128 keys, added as one)
 #pragma unroll
         for (int c = 0; c < 4; ++c) o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        f32x4 v[2][4];                               // values of 16 keys multiplied while the next 16 travel
+        auto fetch = [&](f32x4 (&to)[4], int sub) {
+          const int key = sub * 16 + kq * 4;
+          const i32x4 b4 = *reinterpret_cast<const i32x4*>(B + key);
+          const int b = max(max(b4[0], b4[1]), max(b4[2], b4[3]));
+          const float* vr = vb + (((long)max(b, 0) * G + gv) * kParBlock + (j0 + key) % kParBlock) * v_row;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) to[i] = *reinterpret_cast<const f32x4*>(vr + i * v_row);
+        };
+        fetch(v[0], 0);
 #pragma unroll
         for (int sub = 0; sub < NW; ++sub) {
           if (sub >= nsub) break;
-          f32x4 v[4];
+          if (sub + 1 < NW) fetch(v[(sub + 1) & 1], sub + 1);       // (beyond the last keys: block -1, read as block 0)
+          f32x4(&now)[4] = v[sub & 1];
+          const i32x4 b4 = *reinterpret_cast<const i32x4*>(B + sub * 16 + kq * 4);
+          if (__any(min(min(b4[0], b4[1]), min(b4[2], b4[3])) < 0)) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int key = sub * 16 + kq * 4 + i, b = B[key];
-            v[i] = *reinterpret_cast<const f32x4*>(vb + (((long)max(b, 0) * G + gv) * kParBlock + (j0 + key) % kParBlock) * v_row);
-            if (b < 0) v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int i = 0; i < 4; ++i)
+              if (b4[i] < 0) now[i] = f32x4{0.f, 0.f, 0.f, 0.f};
           }
 #pragma unroll
           for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i][c], p[sub][i], o[c], 0, 0, 0);
+            for (int c = 0; c < 4; ++c) o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(now[i][c], p[sub][i], o[c], 0, 0, 0);
         }
 #pragma unroll
         for (int c = 0; c < 4; ++c) acc[u][c] = acc[u][c] * corr + o[c];
@@ -1114,7 +1130,10 @@ extern "C" void dlia_multi_attention(void* out, long ldo, const float* q, long l
   // chip is full as well (300 tokens, 4 key rows of 128 for 16 heads: 166 against 86 us; 16 heads on one row of 512: 309 against 77),
   // with one or two the tile is mostly empty and only steps that do not fill the chip gain. The workspace in LDS holds rows up to 576.
   const int heads = H / Gk, ht = heads < 16 ? heads : 16, tiles = (heads + 15) / 16;
-  const int units = ((ht + H / G - 2) / (H / G) + 1) * ((dv + 63) / 64);      // (value heads that 16 heads may touch)
+  const int group = H / G;
+  const bool even = (heads % ht == 0 || Gk == 1) && (ht % group == 0 || group % ht == 0);      // (tiles begin and end with value heads)
+  const int touched = even ? (ht + group - 1) / group : (ht + group - 2) / group + 1;
+  const int units = touched * ((dv + 63) / 64);      // (value heads that 16 heads may touch)
   if (f32 && maps == 1 && vec && heads >= 4 && d % 16 == 0 && d <= 576 && dv % 4 == 0 && v_row % 4 == 0 && v_off % 4 == 0 &&
       (uintptr_t)vcache % 16 == 0 && units <= 16 && num_blocks > 0 && Gk * tiles <= 65535) {
     const size_t lds = (16 * (size_t)(d + 4) + 2 * 128 * 20 + 2 * 128) * 4;
@@ -1122,7 +1141,7 @@ extern "C" void dlia_multi_attention(void* out, long ldo, const float* q, long l
   hipLaunchKernelGGL(multi_rows_kernel<UPW>, dim3(T, Gk * tiles), dim3(512), lds, stream, (float*)out, ldo, q, ldq, q_head,           \
                      (const float*)kcache, k_row, (const float*)vcache, v_row, v_off, tok_pos, tok_seq, block_table, max_blocks, num_blocks, \
                      table_rows, H, G, d, dv, scale, window, keep_first, softcap, gate, ldg, Gk, chunk, sink)
-    if (units <= 8) DLIA_ROWS(1);
+    if (units <= 8) DLIA_ROWS(1);                      // (16 heads of four value heads of 128 on the other form: 64 us for 53)
     else DLIA_ROWS(2);
 #undef DLIA_ROWS
     return;
