@@ -276,7 +276,7 @@ extern "C" void dlia_gemm_a8w8(void* out, const void* xq, const float* xscale, c
   int antw, as;
   dlia_gemm_skinny_config(M, N, K, epi, workspace != nullptr, &antw, &as);
   if (splitk <= 0) splitk = as;
-  if (ntw <= 0 || ntw > 2) ntw = 2;
+  if (ntw <= 0 || ntw > 2) ntw = antw;
   if (epi == 4) ntw = 2;
   if (workspace == nullptr) splitk = 1;
   const int chunks = K / (128 * a8w8_ksub(M, K));

@@ -572,9 +572,27 @@ extern "C" void dlia_gemm_skinny_config(int M, int N, int K, int epi, int allow_
     // A fused epilogue (bias / residual / activation: anything but "partials only") needs a reduce
     // launch after a split, ~5 us of a decode step that is a chain of ~5 us kernels. From 64
     // workgroups on, the unsplit launch is faster than split + reduce: TinyLlama gate/up (88
-    // workgroups unsplit, 4 splits before) 1.155 -> 1.113 ms per token at batch 1, 1.66 -> 1.54 at 64;
-    // GPT-2's fc (24 workgroups) keeps its split (0.507 against 0.518 ms unsplit).
+    // workgroups unsplit, 4 splits before) 1.155 -> 1.113 ms per token at batch 1, 1.66 -> 1.54 at 64.
     if (epi != 6 && nblocks >= 64) s = 1;
+    // Up to 128 rows such launches (but the gated one, whose pairs of tiles are one wave's) take 64 columns a workgroup instead, twice the
+    // workgroups with no second pass: a workgroup streams its columns at the latency of its loads, whatever else the chip does. One that
+    // walks up to 1024 of K is done before a reduce could start, and from 65 blocks of 128 columns on (9472: 23.6 whole, 27.1 as two) twice
+    // that many fill the chip unsplit; else as few splits as give 192 workgroups, none shorter than 512 of K. 64 rows, K 4096, bf16 weights, with the reduce, before / after: N 4096 (8 -> 4 splits) 16.3 / 14.2 us,
+    // 8192 (1 -> 2) 29.8 / 20.4, 12352 (unsplit) 31.7 / 25.3, 14336 (unsplit) 32.5 / 26.9, 16 rows of K 768, N 2304 (2 splits -> unsplit)
+    // 7.3 / 5.3; e4m3 weights the same way, N 8192: 26.4 / 18.0, e4m3 products 16.6 / 13.7. From 16512 columns on one pass of 128 columns
+    // is faster (18432: 34.5 against 43.2), and from 8320 on over more than 4096 of K two splits of it are (N 12288, K 8192, 64 rows: 58.4
+    // unsplit, 45.6 with 64 columns, 41.8 so).
+    if (epi != 6 && epi != 4 && M <= 128 && nblocks <= 128) {
+      if (nblocks > 64 && chunks > 32) {
+        *ntw_out = 2; *splitk_out = 2;
+        return;
+      }
+      s = 1;
+      if (chunks > 8 && nblocks <= 64)
+        while (nblocks * 2 * s < (forced > 0 ? forced : 192) && chunks / (s * 2) >= 4) s *= 2;
+      *ntw_out = 1; *splitk_out = s;
+      return;
+    }
   }
   *ntw_out = ntw; *splitk_out = s;
 }
